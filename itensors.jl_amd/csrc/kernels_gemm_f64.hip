@@ -19,11 +19,23 @@
 //
 // Tiles: 256 threads = 4 wave64s in a 2x2 grid; each wave owns a
 // (BM/2) x (BN/2) sub-tile as (BM/32) x (BN/32) MFMA 16x16 blocks of FP64
-// accumulators. A and B K-slices (BK = 16) are double-buffered in LDS: the
-// next slice is fetched into registers while the current one is multiplied,
-// then written to the other buffer, with one barrier per slice. The MFMA is
+// accumulators and multiplies only the blocks that hold outputs. The MFMA is
 // issued as D = B^T A^T so that each lane's accumulators run down a column
 // of C, which makes the column-major epilogue stores contiguous.
+//
+// K loop: the slices (16 real or 8 complex values of k) of all pairs form one
+// sequence. Slice s is multiplied from one LDS buffer while slice s + 1 goes
+// from registers to the other and slice s + 2 is loaded, one barrier per
+// slice; the fragments of each half slice are read while the other half's
+// MFMAs run. What bounds it: the FP64 matrix pipe (76 TF/s measured with
+// MFMAs alone; one instruction takes 64 cycles) and, with it, every vector
+// instruction, which FP64 MFMAs do not overlap. The loop before this one
+// spent about 150 of them per slice and wave on addresses, masks and alpha
+// and waited for each slice's loads within the slice; this one spends about
+// 8, in 16-byte loads and LDS accesses. Measured, 64x64 tiles, MI355X:
+// 4096^3 real 2.63 -> 2.21 ms, 2048^3 complex 0.95 ms (72 TF/s); the grouped
+// products of the chi = 4096 U(1) network 0.385 -> 0.313 ms each; dense
+// chi = 1024 network (5120 x 4096 x 1024) 0.84 -> 0.71 ms.
 //
 // Complex data (interleaved re/im) uses the 4-real-product form on the same
 // tiles, with conj(A)/conj(B) folded into the sign of the imaginary parts.
@@ -31,6 +43,7 @@
 // NDTensors/src/array/mul.jl:1-4) and the per-pair loop of
 // NDTensors/src/blocksparse/contract_generic.jl:78-129.
 #include <algorithm>
+#include <type_traits>
 
 #include "itg_internal.h"
 
@@ -41,39 +54,222 @@ namespace {
 typedef double v4d __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int BK = 16;
-constexpr int PAD = 1;
+// A K slice of a tile holds 8 chunks of 16 bytes along K: 16 real or 8
+// complex values.
+constexpr int kChunksK = 8;
+
+// 16 bytes at an address that need only be aligned to the element (NDTensors'
+// block offsets put Float64 blocks on 8-byte boundaries).
+struct __attribute__((aligned(8))) Chunk {
+  double x, y;
+};
+
+// One operand of the tile: R rows (of M or N) by one K slice, moved from
+// global memory to LDS in 16-byte chunks (two real values along the
+// operand's contiguous mode, or one complex value). KC: the values of a row
+// are contiguous along K (A stored K x M, B stored K x N), else along the rows.
+//
+// FP64 MFMAs and vector-ALU instructions do not overlap on a SIMD (a slice's
+// cycles add up to MFMA busy + 4 per VALU instruction), so the steady state
+// is kept free of the latter: a uniform base that advances per slice plus
+// fixed 32-bit offsets for the loads, fixed LDS addresses, and every special
+// case (conj, alpha, partial slices) behind a uniform branch.
+template <int R, int CPLX, int KC>
+struct Operand {
+  static constexpr int CE = CPLX ? 1 : 2;          // elements per chunk
+  static constexpr int ES = CPLX ? 16 : 8;         // bytes per element
+  static constexpr int BK = kChunksK * CE;         // contracted values per slice
+  static constexpr int NCH = R * kChunksK / kThreads;  // chunks per thread
+  static constexpr int RC = R / CE;                // chunks along the rows (KC = 0)
+  static constexpr bool kLines = !CPLX && !KC;     // LDS rows of one k, else of one chunk of k
+  // padded so that the lanes of a fragment read (kLines) or of a chunk write
+  // fall on different banks
+  static constexpr int kRowBytes = kLines ? (R + 8) * 8 : (R + 1) * 16;
+  // 16 bytes in front: a chunk moved back by one row may start at row -1
+  static constexpr int kBytes = 16 + (kLines ? BK : kChunksK) * kRowBytes;
+  // LDS distance of a thread's consecutive chunks
+  static constexpr int kStep = KC ? kThreads / kChunksK * 16 : kThreads / RC * kRowBytes;
+
+  double2 v[NCH];     // the slice in flight
+  const char* base;   // uniform: the next fast slice's first element
+  uint32_t off[NCH];  // byte offsets of this thread's chunks from base
+  uint32_t mask;      // masked slices: bit 2 * r + e of element e of chunk r
+  int wr, rd;         // LDS offsets: first chunk written, first fragment read
+
+  // chunk r of this thread: first row / first k inside the tile
+  static __device__ __forceinline__ int row(int tid, int r) {
+    const int idx = tid + r * kThreads;
+    return KC ? idx / kChunksK : (idx % RC) * CE;
+  }
+  static __device__ __forceinline__ int kofs(int tid, int r) {
+    const int idx = tid + r * kThreads;
+    return KC ? (idx % kChunksK) * CE : idx / RC;
+  }
+  // LDS offset of (row, k)
+  static __device__ __forceinline__ int at(int row_, int k) {
+    return 16 + (kLines ? k * kRowBytes + row_ * 8 : (k / CE) * kRowBytes + row_ * 16);
+  }
+  // Rows past the end re-read the last ones: they only feed outputs that are
+  // not stored. A real chunk along the rows moves back by one when its second
+  // row is past the end, in global memory and in LDS alike.
+  static __device__ __forceinline__ int clamp_row(int g, int rows) {
+    return min(g, rows - (KC ? 1 : CE));
+  }
+  __device__ __forceinline__ void init(int r0, int rows, int w0, int l16, int lk, int tid) {
+    wr = at(KC ? row(tid, 0) : clamp_row(r0 + row(tid, 0), rows) - r0, kofs(tid, 0));
+    rd = 16 + (kLines ? 2 * lk * kRowBytes + (w0 + l16) * 8 : lk * kRowBytes + (w0 + l16) * 16);
+  }
+  // whether the byte offsets of a slice fit 32 bits (with room to spare)
+  static __device__ __forceinline__ bool fits(int ld, int r0, int rows) {
+    return (int64_t)ld * (KC ? min(R, rows - r0) : BK) <= (INT64_C(1) << 31) / ES;
+  }
+  // first slice of a pair's block: rows r0.. of `rows`, leading dimension ld
+  __device__ __forceinline__ void start(const double* __restrict__ X, int64_t block, int64_t ld,
+                                        int r0, int rows, int tid) {
+    const int rb = max(clamp_row(r0, rows), 0);
+    base = reinterpret_cast<const char*>(X) + (block + (KC ? rb * ld : rb)) * ES;
+#pragma unroll
+    for (int r = 0; r < NCH; ++r) {
+      const uint32_t dr = (uint32_t)(clamp_row(r0 + row(tid, r), rows) - rb);
+      const uint32_t k = (uint32_t)kofs(tid, r);
+      off[r] = (KC ? dr * (uint32_t)ld + k : k * (uint32_t)ld + dr) * ES;
+    }
+  }
+  // Buffer loads: a scalar base and a 32-bit lane offset, with no address
+  // arithmetic on the vector ALU.
+  __device__ __forceinline__ void load_fast(int64_t ld) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, 0xffffffffu, 0x00027000);
+#pragma unroll
+    for (int r = 0; r < NCH; ++r)
+      v[r] = __builtin_bit_cast(
+          double2, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[r], 0, 0));
+    base += (KC ? 1 : ld) * (BK * ES);
+  }
+  // a slice that reaches past K (or a block of one row, or one that does not
+  // fit): element by element from clamped addresses, with a mask of the
+  // elements that are inside
+  __device__ __forceinline__ void load_masked(const double* __restrict__ X, int64_t block,
+                                              int64_t ld, int r0, int rows, int k0, int K,
+                                              int tid) {
+    mask = 0u;
+#pragma unroll
+    for (int r = 0; r < NCH; ++r) {
+#pragma unroll
+      for (int e = 0; e < CE; ++e) {
+        const int g = r0 + row(tid, r) + (KC ? 0 : e), k = k0 + kofs(tid, r) + (KC ? e : 0);
+        if (g < rows && k < K) mask |= 1u << (2 * r + e);
+        const int64_t gc = min(g, rows - 1), kc = min(k, K - 1);
+        const int64_t o = block + (KC ? gc * ld + kc : kc * ld + gc);
+        if (CPLX)
+          v[r] = reinterpret_cast<const double2*>(X)[o];
+        else if (e == 0)
+          v[r].x = X[o];
+        else
+          v[r].y = X[o];
+      }
+    }
+  }
+  __device__ __forceinline__ void store_fast(char* S) const {
+#pragma unroll
+    for (int r = 0; r < NCH; ++r) {
+      Chunk c;
+      c.x = v[r].x;
+      c.y = v[r].y;
+      *reinterpret_cast<Chunk*>(S + wr + r * kStep) = c;
+    }
+  }
+  __device__ __forceinline__ void store_masked(char* S, int tid) const {
+#pragma unroll
+    for (int r = 0; r < NCH; ++r) {
+      double2 c = v[r];
+      if (!(mask >> (2 * r) & 1u)) c.x = 0.0;
+      if (!(mask >> (2 * r + CE - 1) & 1u)) c.y = 0.0;
+      *reinterpret_cast<double2*>(S + at(row(tid, r), kofs(tid, r))) = c;
+    }
+  }
+  __device__ __forceinline__ void conj() {
+#pragma unroll
+    for (int r = 0; r < NCH; ++r) v[r].y = -v[r].y;
+  }
+  __device__ __forceinline__ void scale(double re, double im) {
+#pragma unroll
+    for (int r = 0; r < NCH; ++r)
+      v[r] = CPLX ? make_double2(re * v[r].x - im * v[r].y, re * v[r].y + im * v[r].x)
+                  : make_double2(re * v[r].x, re * v[r].y);
+  }
+  // The fragments of one wave for half a slice (Q = 0, 1), two values per
+  // row: f[h][i], row w0 + 16 i + l16. Real: the MFMA steps h = 0, 1 take
+  // k = 8 Q + 2 lk + h in lane group lk, the same map for both operands and
+  // both storage orders; complex: h = real, imaginary part of k = 4 Q + lk.
+  template <int F>
+  __device__ __forceinline__ void frags(const char* S, int Q, double (&f)[2][F]) const {
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+      if (kLines) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          f[h][i] = *reinterpret_cast<const double*>(S + rd + (8 * Q + h) * kRowBytes + i * 128);
+      } else {
+        const double2 c =
+            *reinterpret_cast<const double2*>(S + rd + 4 * Q * kRowBytes + i * 256);
+        f[0][i] = c.x;
+        f[1][i] = c.y;
+      }
+    }
+  }
+};
+
+// A workgroup barrier that waits for LDS accesses only (the global loads of
+// the next slice stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xF | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The pair table is never written while a launch runs: scalar loads.
+typedef const __attribute__((address_space(4))) GemmPair* PairTable;
+
+// Waves per SIMD the register allocation leaves room for.
+template <int BM, int BN, int CPLX>
+constexpr int kWavesPerSimd = CPLX ? (BM * BN <= 4096 ? 3 : 2) : (BM * BN <= 4096 ? 4 : 2);
 
 template <int BM, int BN, int CPLX, int TA, int TB>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, (kWavesPerSimd<BM, BN, CPLX>))
     gemm_f64_kernel(const GemmPair* __restrict__ pairs, const GemmGroup* __restrict__ groups,
                     const int2* __restrict__ tiles, const double* __restrict__ Ag,
                     const double* __restrict__ Bg, double* __restrict__ Cg, unsigned flags,
                     double ga_re, double ga_im, double beta_re, double beta_im) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int NA = BM * BK / kThreads;  // A elements loaded per thread
-  constexpr int NB = BN * BK / kThreads;
   constexpr int NPLANE = CPLX ? 2 : 1;
+  using OpA = Operand<BM, CPLX, TA ? 1 : 0>;
+  using OpB = Operand<BN, CPLX, TB ? 0 : 1>;
+  constexpr int BK = OpA::BK;
 
-  __shared__ double As[2][NPLANE][BK][BM + PAD];
-  __shared__ double Bs[2][NPLANE][BK][BN + PAD];
+  __shared__ __attribute__((aligned(16))) char smem[2][OpA::kBytes + OpB::kBytes];
 
   const int2 tt = tiles[blockIdx.x];
   if (tt.x < 0) return;  // padding slot of the XCD-balanced table
   const GemmGroup grp = groups[tt.x];
-  const int tiles_m = (grp.M + BM - 1) / BM;
+  const int M = grp.M, N = grp.N;
+  const int tiles_m = (M + BM - 1) / BM;
   const int tm = tt.y % tiles_m, tn = tt.y / tiles_m;
   const int m0 = tm * BM, n0 = tn * BN;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm0 = (wave & 1) * WM, wn0 = (wave >> 1) * WN;
   const int l16 = lane & 15, lk = lane >> 4;
 
-  const double sa = (flags & 1u) ? -1.0 : 1.0;  // conj(A): negate Im(A)
-  const double sb = (flags & 2u) ? -1.0 : 1.0;
+  // 16 x 16 blocks of this wave that hold outputs; the rest is padding
+  const int nfm = min(max((M - m0 - wm0 + 15) / 16, 0), FM);
+  const int nfn = min(max((N - n0 - wn0 + 15) / 16, 0), FN);
+  // a chunk of two rows needs two rows
+  const bool wide = CPLX || ((TA || M >= 2) && (!TB || N >= 2));
 
   v4d acc[NPLANE][FM][FN];
 #pragma unroll
@@ -83,142 +279,181 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[c][i][j] = v4d{0.0, 0.0, 0.0, 0.0};
 
-  double ra[NPLANE][NA], rb[NPLANE][NB];
-
-  for (int p = grp.p0; p < grp.p1; ++p) {
-    const GemmPair pr = pairs[p];
-    const int K = pr.K;
-    const int M = grp.M, N = grp.N;
-    const double al_re = ga_re * pr.alpha_re - ga_im * pr.alpha_im;
-    const double al_im = ga_re * pr.alpha_im + ga_im * pr.alpha_re;
-
-    // Loads are unconditional from clamped (in-block) addresses so that they
-    // issue back to back and their latency overlaps the MFMAs; out-of-range
-    // elements are zeroed, and alpha / conj applied, when the registers are
-    // written to LDS.
-    unsigned ina = 0u, inb = 0u;
-    auto load_regs = [&](int k0) {
-      ina = inb = 0u;
-#pragma unroll
-      for (int r = 0; r < NA; ++r) {
-        const int idx = tid + r * kThreads;
-        const int m = TA ? idx / BK : idx % BM;
-        const int k = TA ? idx % BK : idx / BM;
-        const int gm = m0 + m, gk = k0 + k;
-        if (gm < M && gk < K) ina |= 1u << r;
-        const int gmc = min(gm, M - 1), gkc = min(gk, K - 1);
-        const int64_t off = TA ? ((int64_t)gmc * pr.lda + gkc) : ((int64_t)gkc * pr.lda + gmc);
-        if (CPLX) {
-          const double2 v = reinterpret_cast<const double2*>(Ag)[pr.off_a + off];
-          ra[0][r] = v.x;
-          ra[NPLANE - 1][r] = v.y;
-        } else {
-          ra[0][r] = Ag[pr.off_a + off];
-        }
+  OpA a;
+  OpB b;
+  a.init(m0, M, wm0, l16, lk, tid);
+  b.init(n0, N, wn0, l16, lk, tid);
+  const PairTable ptab = (PairTable)(uintptr_t)pairs;
+  // The slices of all pairs form one sequence: one slice is multiplied from
+  // LDS while the next one is in registers, on its way there.
+  int p = grp.p0 - 1, k0 = 0, K = 0;
+  int64_t off_a = 0, off_b = 0;
+  int lda = 0, ldb = 0;
+  bool masked = false, fast = false;   // of the slice in registers; of its pair
+  bool special = false;                // conj or alpha to apply to its pair
+  double al_re = 1.0, al_im = 0.0;
+  // issue the loads of the next slice; false when there is none
+  auto load_next = [&]() -> bool {
+    k0 += BK;
+    if (k0 >= K) {
+      do {
+        if (++p >= grp.p1) return false;
+        K = ptab[p].K;
+      } while (K <= 0);
+      k0 = 0;
+      off_a = ptab[p].off_a;
+      off_b = ptab[p].off_b;
+      lda = ptab[p].lda;
+      ldb = ptab[p].ldb;
+      const double are = ptab[p].alpha_re, aim = ptab[p].alpha_im;
+      al_re = ga_re * are - ga_im * aim;
+      al_im = ga_re * aim + ga_im * are;
+      special = al_re != 1.0 || (CPLX && (al_im != 0.0 || (flags & 3u)));
+      fast = wide && OpA::fits(lda, m0, M) && OpB::fits(ldb, n0, N);
+      if (fast) {
+        a.start(Ag, off_a, lda, m0, M, tid);
+        b.start(Bg, off_b, ldb, n0, N, tid);
       }
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        const int idx = tid + r * kThreads;
-        const int n = TB ? idx % BN : idx / BK;
-        const int k = TB ? idx / BN : idx % BK;
-        const int gn = n0 + n, gk = k0 + k;
-        if (gn < N && gk < K) inb |= 1u << r;
-        const int gnc = min(gn, N - 1), gkc = min(gk, K - 1);
-        const int64_t off = TB ? ((int64_t)gkc * pr.ldb + gnc) : ((int64_t)gnc * pr.ldb + gkc);
-        if (CPLX) {
-          const double2 v = reinterpret_cast<const double2*>(Bg)[pr.off_b + off];
-          rb[0][r] = v.x;
-          rb[NPLANE - 1][r] = v.y;
-        } else {
-          rb[0][r] = Bg[pr.off_b + off];
-        }
-      }
-    };
-    auto store_lds = [&](int buf) {
-#pragma unroll
-      for (int r = 0; r < NA; ++r) {
-        const int idx = tid + r * kThreads;
-        const int m = TA ? idx / BK : idx % BM;
-        const int k = TA ? idx % BK : idx / BM;
-        const bool in = (ina >> r) & 1u;
-        if (CPLX) {
-          const double x = in ? ra[0][r] : 0.0;
-          const double y = in ? sa * ra[NPLANE - 1][r] : 0.0;
-          As[buf][0][k][m] = al_re * x - al_im * y;
-          As[buf][NPLANE - 1][k][m] = al_re * y + al_im * x;
-        } else {
-          As[buf][0][k][m] = in ? al_re * ra[0][r] : 0.0;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        const int idx = tid + r * kThreads;
-        const int n = TB ? idx % BN : idx / BK;
-        const int k = TB ? idx / BN : idx % BK;
-        const bool in = (inb >> r) & 1u;
-        Bs[buf][0][k][n] = in ? rb[0][r] : 0.0;
-        if (CPLX) Bs[buf][NPLANE - 1][k][n] = in ? sb * rb[NPLANE - 1][r] : 0.0;
-      }
-    };
-
-    if (K <= 0) continue;
-    // every wave is past the previous pair's last read of buffer 0 (the
-    // barrier that closes each K-slice), so it can be refilled here
-    load_regs(0);
-    store_lds(0);
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += BK) {
-      const bool more = k0 + BK < K;
-      if (more) load_regs(k0 + BK);
-      // every fragment of the slice is read before the first MFMA (each kk
-      // into its own registers), so the reads of later kk land while the
-      // MFMAs of earlier ones run; left to itself the scheduler reuses one
-      // register set and waits for each kk's reads with lgkmcnt(0)
-      constexpr int NKK = BK / 4;
-      double af[NKK][NPLANE][FM], bf[NKK][NPLANE][FN];
-#pragma unroll
-      for (int q = 0; q < NKK; ++q)
-#pragma unroll
-        for (int c = 0; c < NPLANE; ++c) {
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-            af[q][c][i] = As[buf][c][4 * q + lk][wm0 + i * 16 + l16];
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            bf[q][c][j] = Bs[buf][c][4 * q + lk][wn0 + j * 16 + l16];
-        }
-#pragma unroll
-      for (int q = 0; q < NKK; ++q)
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            if (CPLX) {
-              // re += Bre*Are - Bim*Aim ; im += Bre*Aim + Bim*Are
-              acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[q][0][j], af[q][0][i],
-                                                                  acc[0][i][j], 0, 0, 0);
-              acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                  -bf[q][NPLANE - 1][j], af[q][NPLANE - 1][i], acc[0][i][j], 0, 0, 0);
-              acc[NPLANE - 1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                  bf[q][0][j], af[q][NPLANE - 1][i], acc[NPLANE - 1][i][j], 0, 0, 0);
-              acc[NPLANE - 1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                  bf[q][NPLANE - 1][j], af[q][0][i], acc[NPLANE - 1][i][j], 0, 0, 0);
-            } else {
-              acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[q][0][j], af[q][0][i],
-                                                                  acc[0][i][j], 0, 0, 0);
-            }
-          }
-      __builtin_amdgcn_sched_group_barrier(0x100, NKK * NPLANE * (FM + FN), 0);  // DS reads
-      __builtin_amdgcn_sched_group_barrier(0x008, NKK * FM * FN * (CPLX ? 4 : 1), 0);  // MFMAs
-      __builtin_amdgcn_sched_barrier(0);
-      // the other buffer was last read in the previous slice, before the
-      // barrier that ended it
-      if (more) store_lds(buf ^ 1);
-      __syncthreads();
-      buf ^= 1;
     }
-  }
+    masked = !fast || k0 + BK > K;
+    if (!masked) {
+      a.load_fast(lda);
+      b.load_fast(ldb);
+    } else {
+      a.load_masked(Ag, off_a, lda, m0, M, k0, K, tid);
+      b.load_masked(Bg, off_b, ldb, n0, N, k0, K, tid);
+    }
+    return true;
+  };
+  auto adjust = [&]() {
+    if (special) {
+      asm volatile("; conj, alpha");  // stays a branch: it is almost never taken
+      if (CPLX && (flags & 1u)) a.conj();
+      if (CPLX && (flags & 2u)) b.conj();
+      if (al_re != 1.0 || (CPLX && al_im != 0.0)) a.scale(al_re, al_im);
+    }
+  };
+  auto store_any = [&](char* S) {
+    adjust();
+    if (!masked) {
+      a.store_fast(S);
+      b.store_fast(S + OpA::kBytes);
+    } else {
+      a.store_masked(S, tid);
+      b.store_masked(S + OpA::kBytes, tid);
+    }
+  };
+
+  // The K loop of a wave with NM x NN live 16 x 16 blocks (0 x 0: only its
+  // share of the loads). Every wave of the workgroup passes the same
+  // barriers, whichever form it runs.
+  auto k_loop = [&](auto nm, auto nn) {
+    constexpr int NM = decltype(nm)::value, NN = decltype(nn)::value;
+    constexpr bool LIVE = NM > 0 && NN > 0;
+    double fa[2][2][LIVE ? NM : 1], fb[2][2][LIVE ? NN : 1];  // [half slice][h][block]
+    auto frags = [&](int Q, const char* S) {
+      if constexpr (LIVE) {
+        a.template frags<NM>(S, Q, fa[Q]);
+        b.template frags<NN>(S + OpA::kBytes, Q, fb[Q]);
+      }
+    };
+    auto mfmas = [&](int Q) {
+      if constexpr (LIVE) {
+#pragma unroll
+        for (int h = 0; h < (CPLX ? 1 : 2); ++h)
+#pragma unroll
+          for (int i = 0; i < NM; ++i)
+#pragma unroll
+            for (int j = 0; j < NN; ++j) {
+              if (CPLX) {
+                // re += Bre*Are - Bim*Aim ; im += Bre*Aim + Bim*Are
+                acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[Q][0][j], fa[Q][0][i],
+                                                                    acc[0][i][j], 0, 0, 0);
+                acc[NPLANE - 1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    fb[Q][0][j], fa[Q][1][i], acc[NPLANE - 1][i][j], 0, 0, 0);
+                acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-fb[Q][1][j], fa[Q][1][i],
+                                                                    acc[0][i][j], 0, 0, 0);
+                acc[NPLANE - 1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    fb[Q][1][j], fa[Q][0][i], acc[NPLANE - 1][i][j], 0, 0, 0);
+              } else {
+                acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[Q][h][j], fa[Q][h][i],
+                                                                    acc[0][i][j], 0, 0, 0);
+              }
+            }
+      }
+    };
+    // one slice from S; the registers (a full slice) go to T and the next
+    // full slice of the pair is loaded. The halves of a slice are read one
+    // half ahead of their MFMAs; T was last read before the previous barrier.
+    auto steady = [&](const char* S, char* T) {
+      adjust();
+      a.store_fast(T);
+      b.store_fast(T + OpA::kBytes);
+      frags(1, S);
+      __builtin_amdgcn_sched_barrier(0);
+      a.load_fast(lda);
+      b.load_fast(ldb);
+      mfmas(0);
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();
+      frags(0, T);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(1);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (!load_next()) return;
+    store_any(smem[0]);
+    bool more = load_next();
+    lds_barrier();
+    int buf = 0;
+    frags(0, smem[0]);
+    while (more) {
+      // Slices whose successor is a full slice of the same pair, then one
+      // whose successor may be a partial slice or the next pair's first.
+      int n = masked ? 0 : (K - k0) / BK - 1;
+      k0 += max(n, 0) * BK;
+      if (n > 0 && buf) {
+        steady(smem[1], smem[0]);
+        buf = 0;
+        --n;
+      }
+      for (; n >= 2; n -= 2) {
+        steady(smem[0], smem[1]);
+        steady(smem[1], smem[0]);
+      }
+      if (n > 0) {
+        steady(smem[0], smem[1]);
+        buf = 1;
+      }
+      store_any(smem[buf ^ 1]);
+      frags(1, smem[buf]);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(0);
+      more = load_next();
+      lds_barrier();
+      buf ^= 1;
+      frags(0, smem[buf]);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(1);
+    }
+    frags(1, smem[buf]);
+    __builtin_amdgcn_sched_barrier(0);
+    mfmas(0);
+    mfmas(1);
+  };
+  using std::integral_constant;
+  if (nfm == FM && nfn == FN)
+    k_loop(integral_constant<int, FM>{}, integral_constant<int, FN>{});
+  else if (nfm == 0 || nfn == 0)
+    k_loop(integral_constant<int, 0>{}, integral_constant<int, 0>{});
+  else if (nfm <= FM / 2 && nfn <= FN / 2)
+    k_loop(integral_constant<int, FM / 2>{}, integral_constant<int, FN / 2>{});
+  else if (nfm <= FM / 2)
+    k_loop(integral_constant<int, FM / 2>{}, integral_constant<int, FN>{});
+  else if (nfn <= FN / 2)
+    k_loop(integral_constant<int, FM>{}, integral_constant<int, FN / 2>{});
+  else
+    k_loop(integral_constant<int, FM>{}, integral_constant<int, FN>{});
 
   // Epilogue. v_mfma_f64_16x16x4_f64 leaves D[i][j] in lane j + 16*(i%4),
   // register i/4 (rows interleaved across the four lane groups), so with
@@ -227,13 +462,13 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     const int gm = m0 + wm0 + i * 16 + l16;
-    if (gm >= grp.M) continue;
+    if (gm >= M) continue;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int gn = n0 + wn0 + j * 16 + lk + 4 * r;
-        if (gn >= grp.N) continue;
+        if (gn >= N) continue;
         const int64_t o = grp.off_c + gm + (int64_t)gn * grp.ldc;
         if (CPLX) {
           double2 out = make_double2(acc[0][i][j][r], acc[NPLANE - 1][i][j][r]);
