@@ -210,7 +210,7 @@ int pick_cfg(itg_handle* h, const ExecPlan& ep, int cplx, int prec) {
   if (ep.tuned[cplx][prec] >= 0) return ep.tuned[cplx][prec];
   auto it = h->tuned.find(tune_key(ep, cplx, prec));
   if (it != h->tuned.end()) return it->second;
-  return prec != 0 ? default_split_cfg(ep) : default_gemm_cfg(ep, cplx);
+  return kDefaultCfg;
 }
 
 itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void* T1,

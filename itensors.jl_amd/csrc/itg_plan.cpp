@@ -1305,25 +1305,6 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
   return "";
 }
 
-int default_gemm_cfg(const ExecPlan&, int) {
-  // 64x64 tiles whatever the block size. Timed on MI355X against the other
-  // shapes (128x128, 128x64, 64x128 real; 128x64 complex) on the two-site
-  // network's GEMMs at chi = 1024 (one 5120 x 4096 x 1024 block), the
-  // chi = 4096 U(1) blocks (about 410 on a side) and 4096^3 / 2048^3
-  // products, 64x64 is the fastest or within 3 % of it, and the large tiles
-  // are slower by up to 30 % (128x128 real) and 14 % (128x64 complex): four
-  // waves per SIMD hide the fill latency that the larger register tiles
-  // cannot.
-  return 0;
-}
-
-int default_split_cfg(const ExecPlan& ep) {
-  int64_t tiles = 0;
-  for (const GemmGroup& G : ep.h_groups)
-    if (G.M > 0 && G.N > 0) tiles += (int64_t)((G.M + 127) / 128) * ((G.N + 63) / 64);
-  return tiles >= 2 * 256 ? 2 : 0;
-}
-
 int mixed_big_cfg(int cplx) { return cplx ? 2 : 1; }
 
 // Key of a cached launch: the mixed choice's tile shapes depend on the

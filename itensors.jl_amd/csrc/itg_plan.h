@@ -235,11 +235,20 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err,
                     KernelTimer* kt = nullptr, bool may_build = true);
-// Tile cfg picked by the built-in heuristic (the autotuner may override).
-int default_gemm_cfg(const ExecPlan& ep, int cplx);
-// Split-precision tile: 2 (128 x 64, three LDS stages, one workgroup per CU)
-// when that shape still gives two workgroups per CU, else 0 (64 x 64).
-int default_split_cfg(const ExecPlan& ep);
+// Tile shape of plans that were not tuned: 64x64, FP64 and split precision
+// alike, whatever the block size.
+// FP64, timed on MI355X against the other shapes (128x128, 128x64, 64x128
+// real; 128x64 complex): the fastest or within 3 % of it for the two-site
+// network's GEMMs at chi = 1024 (one 5120 x 4096 x 1024 block), the chi = 4096
+// U(1) blocks (about 410 on a side: 0.63 ms for the two GEMMs, 128x128 0.86,
+// 128x64 0.74), the 256-network batch and a 4096^3 product (2.04-2.11 ms,
+// 128x128 1.99-2.07): the padding and the last wave of large tiles cost more
+// than the panels they save.
+// Split, 64x64 (two workgroups per CU, three LDS stages) against 128x64 (one,
+// four): U(1) chi = 4096 0.43 against 0.51 ms for the two GEMMs, dense complex
+// chi = 1536 11.8 against 12.1 ms, 3001 x 777 x 500 0.039 against 0.046 ms,
+// 4096^3 1.36 against 1.38 ms.
+constexpr int kDefaultCfg = 0;
 hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, int cplx, hipStream_t s,
                               bool may_build = true);
 // XCD-balanced workgroup -> {group, tile} table for tile shape tc.
