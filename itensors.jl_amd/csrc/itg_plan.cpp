@@ -1345,13 +1345,19 @@ hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, int cplx, hipStream_t s, bo
 }
 
 // Workgroup w of a launch is dispatched to XCD w % kXcds. Cut the tiles of
-// every group into chunks (a group's tiles in tm-fastest order; big groups
-// are split so that every XCD gets several chunks), assign chunks to XCDs
-// largest-work-first to the least loaded one, and interleave the per-XCD
-// lists so each XCD runs its own chunks back to back: the tiles of a chunk
-// share their A and B panels through that XCD's L2.
+// every group into chunks (big groups are split so that every XCD gets
+// several chunks), assign chunks to XCDs largest-work-first to the least
+// loaded one, and interleave the per-XCD lists so each XCD runs its own
+// chunks back to back: the tiles of a chunk share their A and B panels
+// through that XCD's L2. A group's tiles are taken in strips of kStrip tile
+// columns, row by row inside a strip, so that the tiles that run together
+// form a patch with few panels: down whole columns, a 4096^3 FP64 product
+// missed L2 for 9 GB. Measured against that order (MI355X): 4096^3 FP64 2.11 ->
+// 2.04 ms, chi = 1536 complex network in split precision 11.8 -> 11.4 ms, the
+// U(1) networks (blocks of at most 7 tiles a side) level; strips of 4 and 16
+// within 1 % of 8.
 std::vector<int2> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, int filter) {
-  constexpr int kXcds = 8;
+  constexpr int kXcds = 8, kStrip = 8;
   struct Chunk {
     int32_t g, t0, t1;
     double work;
@@ -1386,7 +1392,13 @@ std::vector<int2> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, int filter)
     for (int x = 1; x < kXcds; ++x)
       if (load[x] < load[best]) best = x;
     load[best] += c.work;
-    for (int32_t t = c.t0; t < c.t1; ++t) bins[best].push_back(int2{c.g, t});
+    const GemmGroup& G = ep.h_groups[(size_t)c.g];
+    const int tm = (G.M + tc.bm - 1) / tc.bm, tn = (G.N + tc.bn - 1) / tc.bn;
+    for (int32_t t = c.t0; t < c.t1; ++t) {
+      const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
+      const int width = std::min(kStrip, tn - strip * kStrip);
+      bins[best].push_back(int2{c.g, r / width + (strip * kStrip + r % width) * tm});
+    }
   }
   size_t len = 0;
   for (auto& b : bins) len = std::max(len, b.size());

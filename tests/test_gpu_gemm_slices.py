@@ -38,7 +38,7 @@ def blas():
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 70, 17), (70, 1, 16), (2, 3, 40), (16, 17, 15),
                                    (33, 48, 31), (64, 64, 64), (65, 63, 33), (81, 129, 100),
-                                   (257, 31, 47)])
+                                   (257, 31, 47), (70, 1100, 40)])
 def test_shapes_and_orders(blas, m, n, k, ta, tb, cplx):
     ND = blas
     rng = np.random.default_rng(m * 1000003 + n * 1009 + k)
