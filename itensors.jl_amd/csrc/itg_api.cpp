@@ -1392,9 +1392,7 @@ itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void*
     cands = {0, 2};  // split tiles 64 x 64 and 128 x 64
     if (!cplx) cands.push_back(3);  // 64 x 64 with A in registers
   } else {
-    for (int c = 0; c < gemm_num_cfgs(); ++c)
-      if (gemm_cfg_ok(c, cplx)) cands.push_back(c);
-    cands.push_back(kCfgMixed);
+    cands = {kDefaultCfg};  // the FP64 GEMM has one tile shape
   }
   for (int cfg : cands) {
     // warm-up, then 3 timed runs

@@ -78,8 +78,27 @@ struct GemmGroup {
   int32_t M, N;
   int32_t ldc;
   int32_t p0, p1;
+  // the first pair with K > 0 (its index pf, p1 if there is none): a workgroup
+  // of the FP64 GEMM needs no further read to issue its first loads
+  int32_t pf;
+  int64_t off_a, off_b;
+  int32_t K, lda, ldb;
   int32_t pad;
 };
+inline void set_first_pair(GemmGroup* g, const GemmPair* pairs) {
+  g->pf = g->p0;
+  while (g->pf < g->p1 && pairs[g->pf].K <= 0) ++g->pf;
+  g->off_a = g->off_b = 0;
+  g->K = g->lda = g->ldb = 0;
+  if (g->pf < g->p1) {
+    const GemmPair& p = pairs[g->pf];
+    g->off_a = p.off_a;
+    g->off_b = p.off_b;
+    g->K = p.K;
+    g->lda = p.lda;
+    g->ldb = p.ldb;
+  }
+}
 
 // ------------------------------------------------------------ kernel launch
 // Events that the kernels launched by this thread record their own start
@@ -302,21 +321,24 @@ hipError_t launch_fiber(hipStream_t s, int cplx, int nf, const FiberGroup* group
 // elements each; host helper that must agree with the kernel).
 int64_t direct_group_tiles(const DirectGroup* g, int nr);
 
-// Grouped GEMM (FP64 MFMA). cfg selects the tile shape; ta/tb: A stored
-// K x M / B stored N x K. `tiles` holds one {group, tile index in group} per
-// workgroup ({-1, -1} = idle slot), laid out so that workgroup w runs on
-// XCD w % 8.
+// Grouped GEMM (FP64 MFMA, 64 x 64 tiles); ta/tb: A stored K x M / B stored
+// N x K. `tiles` holds one entry per workgroup, laid out so that workgroup w
+// runs on XCD w % 8. quarters: every entry runs as four workgroups, one per
+// 32 x 32 quarter of its tile (entries: a multiple of 8).
+struct GemmTile {
+  int32_t g;       // group; < 0: idle slot
+  int32_t m0, n0;  // first row / column
+  int32_t pad;
+};
+// Tile shapes by cfg: 0 = 64 x 64 (FP64 and split GEMM), 2 = 128 x 64 (split).
 struct GemmTileCfg {
   int bm, bn;
 };
-int gemm_num_cfgs();
 GemmTileCfg gemm_cfg(int cfg);
-bool gemm_cfg_ok(int cfg, int cplx);
-hipError_t launch_gemm_f64(hipStream_t s, int cfg, int cplx, int ta, int tb,
-                           const GemmPair* pairs, const GemmGroup* groups, const int2* tiles,
-                           int64_t grid_size, const void* A, const void* B, void* C,
-                           unsigned flags, double ga_re, double ga_im, double beta_re,
-                           double beta_im);
+hipError_t launch_gemm_f64(hipStream_t s, int cplx, int ta, int tb, const GemmPair* pairs,
+                           const GemmGroup* groups, const GemmTile* tiles, int64_t entries,
+                           bool quarters, const void* A, const void* B, void* C, unsigned flags,
+                           double ga_re, double ga_im, double beta_re, double beta_im);
 
 // Split-K form of the grouped FP64 GEMM: the GEMM kernel writes S partial
 // sums of each output block (one per slice of its contracted extent) into a
@@ -419,8 +441,8 @@ hipError_t launch_slice(hipStream_t s, int prec, int cplx, int nsets, const Slic
 // aim: take each pair's factor from alpha_im instead of alpha (the second
 // pass of a product with complex per-pair factors).
 hipError_t launch_split_gemm(hipStream_t s, int prec, int cplx, int wmb, int comp, int sets,
-                             const SplitPair* pairs, const GemmGroup* groups, const int2* tiles,
-                             int64_t grid, const void* planesA, const void* planesB,
+                             const SplitPair* pairs, const GemmGroup* groups,
+                             const GemmTile* tiles, int64_t grid, const void* planesA, const void* planesB,
                              const void* expA, const void* expB, void* C, double ga,
                              double beta, int aim = 0);
 // x[i] = beta * x[i] for i < n (complex when cplx).

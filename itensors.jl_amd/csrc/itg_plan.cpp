@@ -775,6 +775,7 @@ std::string build_ksplit(ExecPlan* ep, hipStream_t s) {
         kin += take;
       }
       h.p1 = (int32_t)sp.size();
+      set_first_pair(&h, sp.data());
       sg.push_back(h);
     }
     poff += S[g] * mn;
@@ -783,7 +784,7 @@ std::string build_ksplit(ExecPlan* ep, hipStream_t s) {
   ExecPlan tab;
   tab.h_groups = sg;
   tab.h_pairs = sp;
-  std::vector<int2> tiles_tab = xcd_tile_table(tab, gemm_cfg(0));
+  std::vector<GemmTile> tiles_tab = xcd_tile_table(tab, gemm_cfg(0), nullptr);
   // skinny: (entry, first row) per workgroup, 256 rows of the long side
   std::vector<int2> rows;
   if (skinny)
@@ -795,7 +796,7 @@ std::string build_ksplit(ExecPlan* ep, hipStream_t s) {
   if ((e = ep->ks_pairs.upload(sp.data(), std::max<size_t>(sp.size(), 1) * sizeof(GemmPair), s)) !=
           hipSuccess ||
       (e = ep->ks_groups.upload(sg.data(), sg.size() * sizeof(GemmGroup), s)) != hipSuccess ||
-      (e = ep->ks_tiles.upload(tiles_tab.data(), tiles_tab.size() * sizeof(int2), s)) !=
+      (e = ep->ks_tiles.upload(tiles_tab.data(), tiles_tab.size() * sizeof(GemmTile), s)) !=
           hipSuccess ||
       (e = ep->ks_red.upload(red.data(), red.size() * sizeof(KsReduce), s)) != hipSuccess ||
       (skinny && (e = ep->ks_rows.upload(rows.data(), rows.size() * sizeof(int2), s)) !=
@@ -1133,6 +1134,7 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
     g.p0 = (int32_t)granges[gi].first;
     g.p1 = (int32_t)granges[gi].second;
     double cost = 0;
+    set_first_pair(&g, ep->h_pairs.data());
     for (size_t q = granges[gi].first; q < granges[gi].second; ++q)
       cost += 2.0 * (double)M * (double)N * (double)ep->h_pairs[q].K;
     ep->group_cost[gi] = cost;
@@ -1305,44 +1307,57 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
   return "";
 }
 
-int mixed_big_cfg(int cplx) { return cplx ? 2 : 1; }
-
-// Key of a cached launch: the mixed choice's tile shapes depend on the
-// element type (a plan is shared by real and complex tensors of one block
-// structure), every other tile table does not.
-int gemm_launch_key(int cfg, int cplx) {
-  if (cfg == kCfgMixed) return kCfgMixed + (cplx ? 1 : 0);
-  return gemm_cfg_ok(cfg, cplx) ? cfg : 0;
-}
-
-hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, int cplx, hipStream_t s, bool may_build) {
-  if (cfg != kCfgMixed && !gemm_cfg_ok(cfg, cplx)) cfg = 0;
-  const int key = gemm_launch_key(cfg, cplx);
-  auto it = ep.launches.find(key);
-  if (it != ep.launches.end()) return hipSuccess;
+hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, hipStream_t s, bool may_build) {
+  if (ep.launches.count(cfg)) return hipSuccess;
   if (!may_build) return hipErrorNotReady;
   std::unique_ptr<GemmLaunch> gl(new GemmLaunch);
-  gl->cfg = cfg;
+  std::vector<GemmTile> table = xcd_tile_table(ep, gemm_cfg(cfg), gl->quarters);
+  gl->grid = (int64_t)table.size();
   hipError_t e;
-  if (cfg == kCfgMixed) {
-    const int big = mixed_big_cfg(cplx);
-    std::vector<int2> t1 = xcd_tile_table(ep, gemm_cfg(big), 1);
-    std::vector<int2> t2 = xcd_tile_table(ep, gemm_cfg(0), 2);
-    gl->cfg = big;
-    gl->grid = (int64_t)t1.size();
-    gl->cfg2 = 0;
-    gl->grid2 = (int64_t)t2.size();
-    if ((e = gl->tiles.upload(t1.data(), t1.size() * sizeof(int2), s)) != hipSuccess) return e;
-    if ((e = gl->tiles2.upload(t2.data(), t2.size() * sizeof(int2), s)) != hipSuccess) return e;
-  } else {
-    std::vector<int2> table = xcd_tile_table(ep, gemm_cfg(cfg));
-    gl->grid = (int64_t)table.size();
-    if ((e = gl->tiles.upload(table.data(), table.size() * sizeof(int2), s)) != hipSuccess)
-      return e;
-  }
-  ep.launches[key] = std::move(gl);
+  if ((e = gl->tiles.upload(table.data(), table.size() * sizeof(GemmTile), s)) != hipSuccess)
+    return e;
+  ep.launches[cfg] = std::move(gl);
   return hipSuccess;
 }
+
+namespace {
+// Whether the FP64 GEMM runs a table of 64 x 64 tiles faster as four 32 x 32
+// quarters each. cost[x]: of the tiles of XCD x, in their order (16 x 16 blocks
+// times contracted values). A quarter costs 1.42 (real) or 1.08 (complex: four
+// products per value loaded) of a fourth of its tile on a full CU, but a
+// product with fewer tiles than the chip has CUs, or a few long ones, leaves
+// CUs idle: the tiles are laid on the XCD's 32 CUs in order, each on the least
+// loaded, and a CU that holds few of them runs slower by `lone` (one, two,
+// three tiles; latency is not hidden). A lone quarter, bound by latency alone,
+// takes about as long as the MFMAs of its whole tile. Measured on MI355X, whole
+// -> quarters (K = 2048 unless said): real 512 x 1024 79 -> 58 us, 1024 x 1024
+// 91 -> 113, 2048 x 2048 272 -> 386; 128 x 1280 x 128 (K = 128) 9.4 -> 6.5 us;
+// complex 1024 x 1024 273 -> 289, the chi = 1500 U(1) network's last product
+// 134 -> 112 us.
+bool quarters_faster(const std::vector<std::vector<double>>& cost, int cplx) {
+  constexpr int kCus = 32, kMaxTiles = 256;  // per XCD; beyond 8 tiles a CU whole tiles win
+  const double lone[2][3] = {{1.32, 1.23, 1.08}, {1.15, 1.02, 1.0}};
+  const double quarter = cplx ? 1.08 : 1.42;
+  double t_whole = 0.0, t_quarters = 0.0;
+  for (const std::vector<double>& c : cost) {
+    if (c.size() > kMaxTiles) return false;
+    double load[kCus] = {0.0}, all = 0.0, longest = 0.0;
+    int n[kCus] = {0};
+    for (double t : c) {
+      const int b = (int)(std::min_element(load, load + kCus) - load);
+      load[b] += t;
+      ++n[b];
+      all += t;
+      longest = std::max(longest, t);
+    }
+    for (int b = 0; b < kCus; ++b)
+      if (n[b])
+        t_whole = std::max(t_whole, load[b] * (n[b] <= 3 ? lone[cplx][n[b] - 1] : 1.0));
+    t_quarters = std::max({t_quarters, quarter * all / kCus, 0.97 * longest});
+  }
+  return t_quarters < 0.9 * t_whole;
+}
+}  // namespace
 
 // Workgroup w of a launch is dispatched to XCD w % kXcds. Cut the tiles of
 // every group into chunks (big groups are split so that every XCD gets
@@ -1356,20 +1371,19 @@ hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, int cplx, hipStream_t s, bo
 // 2.04 ms, chi = 1536 complex network in split precision 11.8 -> 11.4 ms, the
 // U(1) networks (blocks of at most 7 tiles a side) level; strips of 4 and 16
 // within 1 % of 8.
-std::vector<int2> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, int filter) {
+std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* quarters) {
   constexpr int kXcds = 8, kStrip = 8;
   struct Chunk {
     int32_t g, t0, t1;
-    double work;
+    double k;     // contracted values of one of its tiles
+    double work;  // of all of them
   };
   std::vector<Chunk> chunks;
   int64_t total = 0;
   std::vector<int32_t> gt(ep.h_groups.size());
   for (size_t g = 0; g < ep.h_groups.size(); ++g) {
     const GemmGroup& G = ep.h_groups[g];
-    const bool big = G.M >= tc.bm && G.N >= tc.bn;
-    const bool keep = filter == 0 || (filter == 1 && big) || (filter == 2 && !big);
-    gt[g] = (!keep || G.M <= 0 || G.N <= 0)
+    gt[g] = (G.M <= 0 || G.N <= 0)
                 ? 0
                 : ((G.M + tc.bm - 1) / tc.bm) * ((G.N + tc.bn - 1) / tc.bn);
     total += gt[g];
@@ -1380,31 +1394,46 @@ std::vector<int2> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, int filter)
     for (int p = ep.h_groups[g].p0; p < ep.h_groups[g].p1; ++p) k += std::max(ep.h_pairs[p].K, 1);
     for (int64_t t0 = 0; t0 < gt[g]; t0 += unit) {
       const int64_t t1 = std::min<int64_t>(gt[g], t0 + unit);
-      chunks.push_back(Chunk{(int32_t)g, (int32_t)t0, (int32_t)t1, k * (double)(t1 - t0)});
+      chunks.push_back(Chunk{(int32_t)g, (int32_t)t0, (int32_t)t1, k, k * (double)(t1 - t0)});
     }
   }
   std::stable_sort(chunks.begin(), chunks.end(),
                    [](const Chunk& a, const Chunk& b) { return a.work > b.work; });
-  std::vector<std::vector<int2>> bins(kXcds);
+  std::vector<std::vector<Chunk>> mine(kXcds);
   std::vector<double> load(kXcds, 0.0);
   for (const Chunk& c : chunks) {
     int best = 0;
     for (int x = 1; x < kXcds; ++x)
       if (load[x] < load[best]) best = x;
     load[best] += c.work;
-    const GemmGroup& G = ep.h_groups[(size_t)c.g];
-    const int tm = (G.M + tc.bm - 1) / tc.bm, tn = (G.N + tc.bn - 1) / tc.bn;
-    for (int32_t t = c.t0; t < c.t1; ++t) {
-      const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
-      const int width = std::min(kStrip, tn - strip * kStrip);
-      bins[best].push_back(int2{c.g, r / width + (strip * kStrip + r % width) * tm});
-    }
+    mine[best].push_back(c);
   }
+  // an XCD starts its longest tiles first
+  for (auto& m : mine)
+    std::stable_sort(m.begin(), m.end(), [](const Chunk& a, const Chunk& b) { return a.k > b.k; });
+  std::vector<std::vector<GemmTile>> bins(kXcds);
+  std::vector<std::vector<double>> cost(kXcds);  // of each tile: its 16 x 16 blocks times k
+  for (int x = 0; x < kXcds; ++x)
+    for (const Chunk& c : mine[x]) {
+      const GemmGroup& G = ep.h_groups[(size_t)c.g];
+      const int tm = (G.M + tc.bm - 1) / tc.bm, tn = (G.N + tc.bn - 1) / tc.bn;
+      for (int32_t t = c.t0; t < c.t1; ++t) {
+        const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
+        const int width = std::min(kStrip, tn - strip * kStrip);
+        const GemmTile T{c.g, r / width * tc.bm, (strip * kStrip + r % width) * tc.bn, 0};
+        bins[x].push_back(T);
+        if (quarters)
+          cost[x].push_back((double)((std::min(G.M - T.m0, tc.bm) + 15) / 16) *
+                            ((std::min(G.N - T.n0, tc.bn) + 15) / 16) * c.k);
+      }
+    }
   size_t len = 0;
   for (auto& b : bins) len = std::max(len, b.size());
-  std::vector<int2> table(len * kXcds, int2{-1, -1});
+  std::vector<GemmTile> table(len * kXcds, GemmTile{-1, 0, 0, 0});
   for (int x = 0; x < kXcds; ++x)
     for (size_t i = 0; i < bins[x].size(); ++i) table[i * kXcds + x] = bins[x][i];
+  if (quarters)
+    for (int cplx = 0; cplx < 2; ++cplx) quarters[cplx] = quarters_faster(cost, cplx);
   return table;
 }
 
@@ -1571,7 +1600,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
   // with A in registers; otherwise 64 x 64
   const int wmb = cfg == 2 ? 2 : (cfg == 3 && !cplx ? 3 : 1);
   const int tcfg = wmb == 2 ? 2 : 0;  // the FP64 tile table of the same shape
-  if ((e = ensure_gemm_launch(ep, tcfg, 0, s, may_build)) != hipSuccess) {
+  if ((e = ensure_gemm_launch(ep, tcfg, s, may_build)) != hipSuccess) {
     *err = e == hipErrorNotReady ? std::string(kTablesMissing)
                                  : std::string("gemm table upload: ") + hipGetErrorString(e);
     return e;
@@ -1590,7 +1619,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
         TimeScope ts(kt, "split_gemm_kernel", s);
         e = launch_split_gemm(s, prec, cplx, wmb, comp, split_sets(comp, conja, conjb),
                               (const SplitPair*)ep.s_pairs.p, (const GemmGroup*)ep.s_groups.p,
-                              (const int2*)gl.tiles.p, gl.grid, planesA, planesB, expA, expB,
+                              (const GemmTile*)gl.tiles.p, gl.grid, planesA, planesB, expA, expB,
                               part ? S2 : S1, 1.0, 0.0, part);
       }
     if (e != hipSuccess) {
@@ -1636,7 +1665,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     TimeScope ts(kt, "split_gemm_kernel", s);
     e = launch_split_gemm(s, prec, cplx, wmb, comp, split_sets(comp, conja, conjb),
                           (const SplitPair*)ep.s_pairs.p, (const GemmGroup*)ep.s_groups.p,
-                          (const int2*)gl.tiles.p, gl.grid, planesA, planesB, expA, expB, C, a_re,
+                          (const GemmTile*)gl.tiles.p, gl.grid, planesA, planesB, expA, expB, C, a_re,
                           beta_k);
   }
   if (e != hipSuccess) {
@@ -1751,9 +1780,9 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
                                ep.ks_nrows, A, B, w, gflags, a_re, a_im);
     } else {
       TimeScope ts(kt, "gemm_f64_kernel", s);
-      e = launch_gemm_f64(s, 0, cplx, ep.ta, ep.tb, (const GemmPair*)ep.ks_pairs.p,
-                          (const GemmGroup*)ep.ks_groups.p, (const int2*)ep.ks_tiles.p,
-                          ep.ks_grid, A, B, w, gflags, a_re, a_im, 0.0, 0.0);
+      e = launch_gemm_f64(s, cplx, ep.ta, ep.tb, (const GemmPair*)ep.ks_pairs.p,
+                          (const GemmGroup*)ep.ks_groups.p, (const GemmTile*)ep.ks_tiles.p,
+                          ep.ks_grid, false, A, B, w, gflags, a_re, a_im, 0.0, 0.0);
     }
     if (e == hipSuccess) {
       TimeScope ts(kt, "ksplit_reduce_kernel", s);
@@ -1765,30 +1794,23 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
       return e;
     }
   } else {
-  if ((e = ensure_gemm_launch(ep, cfg, cplx, s, may_build)) != hipSuccess) {
+  if ((e = ensure_gemm_launch(ep, kDefaultCfg, s, may_build)) != hipSuccess) {
     *err = e == hipErrorNotReady ? std::string(kTablesMissing)
                                  : std::string("gemm table upload: ") + hipGetErrorString(e);
     return e;
   }
-  GemmLaunch& gl = *ep.launches[gemm_launch_key(cfg, cplx)];
+  GemmLaunch& gl = *ep.launches[kDefaultCfg];
   {
     TimeScope ts(kt, "gemm_f64_kernel", s);
-    e = launch_gemm_f64(s, gl.cfg, cplx, ep.ta, ep.tb, (const GemmPair*)ep.g_pairs.p,
-                        (const GemmGroup*)ep.g_groups.p, (const int2*)gl.tiles.p, gl.grid, A, B,
-                        C, gflags, a_re, a_im, gbr, gbi);
-  }
-  if (e == hipSuccess && gl.cfg2 >= 0) {
-    TimeScope ts(kt, "gemm_f64_kernel", s);
-    e = launch_gemm_f64(s, gl.cfg2, cplx, ep.ta, ep.tb, (const GemmPair*)ep.g_pairs.p,
-                        (const GemmGroup*)ep.g_groups.p, (const int2*)gl.tiles2.p, gl.grid2, A, B,
-                        C, gflags, a_re, a_im, gbr, gbi);
+    e = launch_gemm_f64(s, cplx, ep.ta, ep.tb, (const GemmPair*)ep.g_pairs.p,
+                        (const GemmGroup*)ep.g_groups.p, (const GemmTile*)gl.tiles.p, gl.grid,
+                        gl.quarters[cplx], A, B, C, gflags, a_re,
+                        a_im, gbr, gbi);
   }
   if (e != hipSuccess) {
     char what[160];
-    std::snprintf(what, sizeof what,
-                  "gemm launch (tile cfg %d / %d, workgroups %lld / %lld, %s, ta %d, tb %d): ",
-                  gl.cfg, gl.cfg2, (long long)gl.grid, (long long)gl.grid2,
-                  cplx ? "complex" : "real", ep.ta, ep.tb);
+    std::snprintf(what, sizeof what, "gemm launch (workgroups %lld, %s, ta %d, tb %d): ",
+                  (long long)gl.grid, cplx ? "complex" : "real", ep.ta, ep.tb);
     *err = std::string(what) + hipGetErrorString(e);
     return e;
   }

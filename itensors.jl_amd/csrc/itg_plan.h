@@ -111,17 +111,11 @@ struct PermuteLaunch {
   DevBuf blocks, prefix;
 };
 
-// Tile-shape choice "mixed": groups whose output block fills large tiles
-// use the large shape, the others 64x64, as two grouped launches.
-constexpr int kCfgMixed = 16;
-
+// Workgroup table of a tile shape (FP64: gemm cfg 0; split: cfg 0 or 2).
 struct GemmLaunch {
-  int cfg = -1;
-  int64_t grid = 0;  // workgroups, including idle padding slots
-  DevBuf tiles;      // int2 {group, tile} per workgroup
-  int cfg2 = -1;     // second launch of a mixed choice (64x64 part)
-  int64_t grid2 = 0;
-  DevBuf tiles2;
+  int64_t grid = 0;   // entries, idle padding included
+  bool quarters[2] = {false, false};  // FP64, real / complex: 32 x 32 workgroups
+  DevBuf tiles;       // GemmTile per entry
 };
 
 struct ExecPlan {
@@ -249,11 +243,10 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
 // chi = 1536 11.8 against 12.1 ms, 3001 x 777 x 500 0.039 against 0.046 ms,
 // 4096^3 1.36 against 1.38 ms.
 constexpr int kDefaultCfg = 0;
-hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, int cplx, hipStream_t s,
-                              bool may_build = true);
-// XCD-balanced workgroup -> {group, tile} table for tile shape tc.
-// filter: 0 = every group, 1 = only groups with M, N >= the tile, 2 = the rest.
-std::vector<int2> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, int filter = 0);
+hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, hipStream_t s, bool may_build = true);
+// XCD-balanced tile table for tile shape tc. quarters (optional, two values):
+// whether the FP64 GEMM should run it as quarter tiles (real, complex).
+std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* quarters);
 
 // Two consecutive matrix-form fiber contractions run as one pass (see
 // ChainGroup). Built from the two steps' plans; the device tables live here.

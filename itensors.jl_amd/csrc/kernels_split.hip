@@ -459,7 +459,7 @@ __device__ inline v4i lds_read16_untracked(uint32_t addr) {
 template <int S, int CPLX, int WM>
 __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
     split_gemm_kernel(const SplitPair* __restrict__ pairs, const GemmGroup* __restrict__ groups,
-                      const int2* __restrict__ tiles, const int8_t* __restrict__ planesA,
+                      const GemmTile* __restrict__ tiles, const int8_t* __restrict__ planesA,
                       const int8_t* __restrict__ planesB, const int32_t* __restrict__ expA,
                       const int32_t* __restrict__ expB, double* __restrict__ Cg, double ga,
                       double beta, int comp, int sets, int nsetsA, int nsetsB, int aim) {
@@ -487,12 +487,10 @@ __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
   static_assert(NSTAGE - 2 <= 2, "wait_newer covers at most two newer stages");
   __shared__ v4i lds[NSTAGE * (A_ST + B_ST)];
 
-  const int2 tt = tiles[blockIdx.x];
-  if (tt.x < 0) return;
-  const GemmGroup grp = groups[tt.x];
-  const int tiles_m = (grp.M + BM - 1) / BM;
-  const int tm = tt.y % tiles_m, tn = tt.y / tiles_m;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const GemmTile& tt = tiles[blockIdx.x];
+  if (tt.g < 0) return;
+  const GemmGroup grp = groups[tt.g];
+  const int m0 = tt.m0, n0 = tt.n0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm0 = (wave % WM) * 32, wn0 = (wave / WM) * 32;
@@ -649,11 +647,10 @@ __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
 template <int S>
 __global__ void __launch_bounds__(128, 1)
     split_gemm_areg_kernel(const SplitPair* __restrict__ pairs,
-                           const GemmGroup* __restrict__ groups, const int2* __restrict__ tiles,
+                           const GemmGroup* __restrict__ groups, const GemmTile* __restrict__ tiles,
                            const int8_t* planesA, const int8_t* __restrict__ planesB,
                            const int32_t* __restrict__ expA, const int32_t* __restrict__ expB,
                            double* __restrict__ Cg, double ga, double beta) {
-  constexpr int BM = 64;
   constexpr int NL = S;
   constexpr int B_ST = S * 2 * BN;  // 16-byte LDS slots of one B stage
   constexpr int NLD = S * 2;        // wave loads (64 rows x 16 bytes) per B stage
@@ -662,12 +659,10 @@ __global__ void __launch_bounds__(128, 1)
   constexpr int NSTAGE = 3;
   __shared__ v4i lds[NSTAGE * B_ST];
 
-  const int2 tt = tiles[blockIdx.x];
-  if (tt.x < 0) return;
-  const GemmGroup grp = groups[tt.x];
-  const int tiles_m = (grp.M + BM - 1) / BM;
-  const int tm = tt.y % tiles_m, tn = tt.y / tiles_m;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const GemmTile& tt = tiles[blockIdx.x];
+  if (tt.g < 0) return;
+  const GemmGroup grp = groups[tt.g];
+  const int m0 = tt.m0, n0 = tt.n0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, lh = lane >> 5;
@@ -836,7 +831,7 @@ int64_t slice_block_wgs(int32_t rows, int32_t kparts) {
 namespace {
 template <int CPLX, int WM>
 hipError_t launch_sg(hipStream_t s, int comp, int sets, const SplitPair* pairs,
-                     const GemmGroup* groups, const int2* tiles, int64_t grid,
+                     const GemmGroup* groups, const GemmTile* tiles, int64_t grid,
                      const void* planesA, const void* planesB, const void* expA,
                      const void* expB, void* C, double ga, double beta, int aim) {
   const int ns = CPLX ? 3 : 1;
@@ -849,7 +844,7 @@ hipError_t launch_sg(hipStream_t s, int comp, int sets, const SplitPair* pairs,
 }  // namespace
 
 hipError_t launch_split_gemm(hipStream_t s, int prec, int cplx, int wmb, int comp, int sets,
-                             const SplitPair* pairs, const GemmGroup* groups, const int2* tiles,
+                             const SplitPair* pairs, const GemmGroup* groups, const GemmTile* tiles,
                              int64_t grid, const void* planesA, const void* planesB,
                              const void* expA, const void* expB, void* C, double ga,
                              double beta, int aim) {

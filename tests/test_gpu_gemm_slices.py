@@ -1,8 +1,9 @@
-"""FP64 grouped GEMM at the sizes where its K loop changes form: tile and
-slice remainders, one row or column, one slice or less, two pairs with
-different K, operands in every storage order, blocks at odd element offsets,
-alpha and conj; and leading dimensions whose slices do not fit 32-bit
-offsets.
+"""FP64 grouped GEMM at the sizes where it changes form: tile and slice
+remainders, every number of live 16-row and 16-column blocks of a tile, one
+row or column, one slice or less, pairs with different K, few tiles (run as
+quarters) and many (run whole, several strips of tile columns), operands in
+every storage order, blocks at odd element offsets, alpha and conj; and
+leading dimensions whose slices do not fit 32-bit offsets.
 
 Tolerance: a sum of K products in any order is within K * eps of the exact
 one, relative to the sum of the products' magnitudes (real; a complex product
@@ -38,7 +39,8 @@ def blas():
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 70, 17), (70, 1, 16), (2, 3, 40), (16, 17, 15),
                                    (33, 48, 31), (64, 64, 64), (65, 63, 33), (81, 129, 100),
-                                   (257, 31, 47), (70, 1100, 40)])
+                                   (257, 31, 47), (70, 1100, 40), (1030, 1100, 33),
+                                   (2100, 2055, 20)])
 def test_shapes_and_orders(blas, m, n, k, ta, tb, cplx):
     ND = blas
     rng = np.random.default_rng(m * 1000003 + n * 1009 + k)
@@ -63,14 +65,15 @@ def test_shapes_and_orders(blas, m, n, k, ta, tb, cplx):
 
 
 @pytest.mark.parametrize("cplx", [False, True])
-def test_pairs_of_different_length(cplx):
+@pytest.mark.parametrize("m,n", [((37, 66), 70), ((370, 666), 2100)])
+def test_pairs_of_different_length(m, n, cplx):
     """Output blocks summing over blocks of 5, 16, 33 and 100 values of k."""
     import itg
     from itg import ndtensors as ND
     rng = np.random.default_rng(3)
     q = [itg.QN(("Sz", i)) for i in range(4)]
-    i = itg.Index([(itg.QN(("Sz", 0)), 37), (itg.QN(("Sz", 1)), 66)], "i", dir=itg.Out)
-    j = itg.Index([(itg.QN(("Sz", 0)), 70)], "j", dir=itg.In)
+    i = itg.Index([(itg.QN(("Sz", 0)), m[0]), (itg.QN(("Sz", 1)), m[1])], "i", dir=itg.Out)
+    j = itg.Index([(itg.QN(("Sz", 0)), n)], "j", dir=itg.In)
     k = itg.Index(list(zip(q, (5, 16, 33, 100))), "k", dir=itg.Out)
     s = itg.Index([(itg.QN(("Sz", -x)), 1) for x in range(4)], "s", dir=itg.Out)
     dt = np.complex128 if cplx else np.float64
