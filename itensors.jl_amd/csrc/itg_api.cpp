@@ -24,9 +24,28 @@ static_assert(ITG_FLAG_KEEP_SLICES_1 == kFlagKeep1 && ITG_FLAG_KEEP_SLICES_2 == 
                   (ITG_FLAG_CONJ_A | ITG_FLAG_CONJ_B) == kFlagConj,
               "execution flag values");
 
+namespace {
+// Tables of one call that are needed on the device only until its kernel has
+// run: written to pinned memory, copied on the stream, used by the kernel;
+// `done` is recorded after it. A handle keeps a ring of these, so that a call
+// neither allocates nor waits; it is freed with the handle.
+struct Stage {
+  void* host = nullptr;
+  void* dev = nullptr;
+  size_t bytes = 0;
+  hipEvent_t done = nullptr;
+  bool used = false;
+};
+constexpr int kStages = 4;
+// larger tables get a buffer of their own for the call
+constexpr size_t kStageMax = (size_t)4 << 20;
+}  // namespace
+
 struct itg_handle {
   int device = 0;
   hipStream_t stream = nullptr;
+  Stage stages[kStages];
+  int next_stage = 0;
   std::string err;
   void* ws = nullptr;
   size_t ws_bytes = 0;
@@ -158,6 +177,69 @@ itg_status widen_operands(itg_handle* h, itg_dtype dt, int64_t n1, const void* T
     return hip_fail(h, e, "widen launch");
   return ITG_OK;
 }
+
+void free_stage(Stage* st) {
+  if (st->used) (void)hipEventSynchronize(st->done);
+  if (st->done) (void)hipEventDestroy(st->done);
+  if (st->dev) (void)hipFree(st->dev);
+  if (st->host) (void)hipHostFree(st->host);
+  *st = Stage{};
+}
+
+// Device copies of up to two host tables for the kernel the caller launches
+// next on the handle's stream; finish() after that launch. Not under capture
+// (a replay would copy from memory that later calls rewrite).
+class CallTables {
+ public:
+  explicit CallTables(itg_handle* h) : h_(h) {}
+  ~CallTables() { finish(); }
+  hipError_t put(const void* a, size_t na, const void* b, size_t nb) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(h_->stream, &cs);
+    if (e != hipSuccess) return e;
+    if (cs != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
+    off_ = al256(na);
+    const size_t n = off_ + al256(nb);
+    Stage* st = &own_;
+    if (n <= kStageMax) {
+      st = &h_->stages[h_->next_stage];
+      h_->next_stage = (h_->next_stage + 1) % kStages;
+      if (st->used && (e = hipEventSynchronize(st->done)) != hipSuccess) return e;
+    }
+    if (st->bytes < n) {
+      free_stage(st);
+      const size_t b = std::min(std::max(n, (size_t)1 << 16) * 2, std::max(n, kStageMax));
+      if ((e = hipHostMalloc(&st->host, b, hipHostMallocDefault)) != hipSuccess ||
+          (e = hipMalloc(&st->dev, b)) != hipSuccess ||
+          (e = hipEventCreateWithFlags(&st->done, hipEventDisableTiming)) != hipSuccess) {
+        free_stage(st);
+        return e;
+      }
+      st->bytes = b;
+    }
+    st_ = st;
+    std::memcpy(st->host, a, na);
+    std::memcpy((char*)st->host + off_, b, nb);
+    return hipMemcpyAsync(st->dev, st->host, n, hipMemcpyHostToDevice, h_->stream);
+  }
+  const void* first() const { return st_->dev; }
+  const void* second() const { return (const char*)st_->dev + off_; }
+  void finish() {
+    if (!st_) return;
+    if (hipEventRecord(st_->done, h_->stream) == hipSuccess)
+      st_->used = true;
+    else  // the tables may still be read: wait here instead
+      (void)hipStreamSynchronize(h_->stream);
+    if (st_ == &own_) free_stage(&own_);
+    st_ = nullptr;
+  }
+
+ private:
+  itg_handle* h_;
+  Stage own_;
+  Stage* st_ = nullptr;
+  size_t off_ = 0;
+};
 
 // One past the last element a block list's blocks occupy (diag: each block
 // stores min(dims) elements).
@@ -385,6 +467,7 @@ itg_status itg_destroy(itg_handle* h) {
       if (gr) (void)hipGraphDestroy(gr);
       h->stream = h->pre_capture;
     }
+    for (Stage& st : h->stages) free_stage(&st);
     if (h->ws || !h->retired.empty()) (void)hipStreamSynchronize(h->stream);
     if (h->ws) (void)hipFree(h->ws);
     if (h->ws32) (void)hipFree(h->ws32);
@@ -640,20 +723,20 @@ itg_status itg_permute(itg_handle* h, itg_dtype dtype, int ndim, const int64_t* 
   bl.offs.push_back(0);
   bl.nnz = n;
   PermuteLaunch pl;
-  {
-    hipError_t e = build_permute_launch(&pl, ndim, p0, bl, nullptr, h->stream);
-    if (e != hipSuccess) return hip_fail(h, e, "permute tables");
-  }
+  std::vector<PermBlock> blocks;
+  std::vector<int64_t> prefix;
+  build_permute_tables(&pl, ndim, p0, bl, nullptr, nullptr, &blocks, &prefix);
+  CallTables tab(h);
+  hipError_t e = tab.put(blocks.data(), blocks.size() * sizeof(PermBlock), prefix.data(),
+                         prefix.size() * sizeof(int64_t));
+  if (e != hipSuccess) return hip_fail(h, e, "permute tables");
   const int cplx = dtype == ITG_C128 || dtype == ITG_C64;
   const double a_re = alpha ? alpha[0] : 1.0, a_im = (alpha && cplx) ? alpha[1] : 0.0;
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
-  hipError_t e = launch_permute(h->stream, elt_code(dtype), pl.nm, pl.perm, (const PermBlock*)pl.blocks.p,
-                                (const int64_t*)pl.prefix.p, pl.nblk, pl.tiles, pl.kind, src, dst,
-                                a_re, a_im, b_re, b_im);
+  e = launch_permute(h->stream, elt_code(dtype), pl.nm, pl.perm, (const PermBlock*)tab.first(),
+                     (const int64_t*)tab.second(), pl.nblk, pl.tiles, pl.kind, src, dst, a_re,
+                     a_im, b_re, b_im);
   if (e != hipSuccess) return hip_fail(h, e, "permute launch");
-  // the tables are freed when `pl` goes out of scope: wait for the kernel
-  e = hipStreamSynchronize(h->stream);
-  if (e != hipSuccess) return hip_fail(h, e, "permute");
   return ITG_OK;
 }
 
@@ -1219,11 +1302,16 @@ itg_status itg_bs_chain_destroy(itg_bs_chain* c) {
   return ITG_OK;
 }
 
-itg_status itg_bs_permute_ex(itg_handle* h, itg_dtype dtype, int N, int64_t nblk,
-                             const int64_t* blockdims, const int64_t* offs_src,
-                             const int64_t* offs_dst, const uint8_t* fresh, const int32_t* perm,
-                             const void* src, void* dst, const double* alpha, const double* beta,
-                             int32_t* nonzero) {
+}  // extern "C"
+
+namespace {
+// itg_bs_permute_ex without its final wait; nonzero flags are on the host
+// when it returns.
+itg_status bs_permute_run(itg_handle* h, itg_dtype dtype, int N, int64_t nblk,
+                          const int64_t* blockdims, const int64_t* offs_src,
+                          const int64_t* offs_dst, const uint8_t* fresh, const int32_t* perm,
+                          const void* src, void* dst, const double* alpha, const double* beta,
+                          int32_t* nonzero) {
   if (!h) return ITG_ERR_INVALID;
   if (!dtype_any(dtype)) return fail(h, ITG_ERR_UNSUPPORTED, "unsupported dtype");
   if (N < 0 || N > kMaxModes) return fail(h, ITG_ERR_UNSUPPORTED, "too many modes");
@@ -1261,31 +1349,48 @@ itg_status itg_bs_permute_ex(itg_handle* h, itg_dtype dtype, int N, int64_t nblk
   if (fresh) fr.assign(fresh, fresh + nblk);
   DeviceGuard g(h->device);
   PermuteLaunch pl;
-  hipError_t e = build_permute_launch(&pl, N, p0, bl, &od, h->stream, fresh ? &fr : nullptr);
+  std::vector<PermBlock> blocks;
+  std::vector<int64_t> prefix;
+  build_permute_tables(&pl, N, p0, bl, &od, fresh ? &fr : nullptr, &blocks, &prefix);
+  CallTables tab(h);
+  hipError_t e = tab.put(blocks.data(), blocks.size() * sizeof(PermBlock), prefix.data(),
+                         prefix.size() * sizeof(int64_t));
   if (e != hipSuccess) return hip_fail(h, e, "permute tables");
   DevBuf nz;
-  if (nonzero) {
-    std::vector<int32_t> zero((size_t)nblk, 0);
-    if ((e = nz.upload(zero.data(), zero.size() * sizeof(int32_t), h->stream)) != hipSuccess)
-      return hip_fail(h, e, "flag buffer");
-  }
+  if (nonzero && (e = nz.reserve((size_t)nblk * sizeof(int32_t))) != hipSuccess)
+    return hip_fail(h, e, "flag buffer");
   const int cplx = dtype == ITG_C128 || dtype == ITG_C64;
   const double a_re = alpha ? alpha[0] : 1.0, a_im = (alpha && cplx) ? alpha[1] : 0.0;
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
   KernelTimer* kt = active_timer(h);
   if (kt) kt->begin("permute_kernel", h->stream);
-  e = launch_permute(h->stream, elt_code(dtype), pl.nm, pl.perm, (const PermBlock*)pl.blocks.p,
-                     (const int64_t*)pl.prefix.p, pl.nblk, pl.tiles, pl.kind, src, dst, a_re,
+  e = launch_permute(h->stream, elt_code(dtype), pl.nm, pl.perm, (const PermBlock*)tab.first(),
+                     (const int64_t*)tab.second(), pl.nblk, pl.tiles, pl.kind, src, dst, a_re,
                      a_im, b_re, b_im, nonzero ? (int32_t*)nz.p : nullptr);
   if (kt) kt->end(h->stream);
   if (e != hipSuccess) return hip_fail(h, e, "permute launch");
   if (nonzero) {
     e = hipMemcpyAsync(nonzero, nz.p, (size_t)nblk * sizeof(int32_t), hipMemcpyDeviceToHost,
                        h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);  // nz is freed on return
     if (e != hipSuccess) return hip_fail(h, e, "flag download");
   }
-  // the tables (and the flags) are freed when the locals go out of scope
-  e = hipStreamSynchronize(h->stream);
+  return ITG_OK;
+}
+}  // namespace
+
+extern "C" {
+
+itg_status itg_bs_permute_ex(itg_handle* h, itg_dtype dtype, int N, int64_t nblk,
+                             const int64_t* blockdims, const int64_t* offs_src,
+                             const int64_t* offs_dst, const uint8_t* fresh, const int32_t* perm,
+                             const void* src, void* dst, const double* alpha, const double* beta,
+                             int32_t* nonzero) {
+  itg_status st = bs_permute_run(h, dtype, N, nblk, blockdims, offs_src, offs_dst, fresh, perm, src,
+                                 dst, alpha, beta, nonzero);
+  if (st != ITG_OK || nblk == 0) return st;
+  DeviceGuard g(h->device);
+  hipError_t e = hipStreamSynchronize(h->stream);
   if (e != hipSuccess) return hip_fail(h, e, "permute");
   return ITG_OK;
 }
@@ -1298,8 +1403,8 @@ itg_status itg_bs_permute(itg_handle* h, itg_dtype dtype, int N, int64_t nblk,
   if (nblk > 0 && offs_src)
     for (int64_t b = 0; b < nblk; ++b)
       if (offs_src[b] < 0) return fail(h, ITG_ERR_INVALID, "negative source offset");
-  return itg_bs_permute_ex(h, dtype, N, nblk, blockdims, offs_src, offs_dst, nullptr, perm, src,
-                           dst, nullptr, nullptr, nullptr);
+  return bs_permute_run(h, dtype, N, nblk, blockdims, offs_src, offs_dst, nullptr, perm, src, dst,
+                        nullptr, nullptr, nullptr);
 }
 
 itg_status itg_bs_copy(itg_handle* h, itg_dtype dtype, int64_t nblk, int nmodes,
@@ -1351,15 +1456,15 @@ itg_status itg_bs_copy(itg_handle* h, itg_dtype dtype, int64_t nblk, int nmodes,
     prefix.push_back(prefix.back() + copy_block_wgs(n));
   }
   DeviceGuard g(h->device);
-  DevBuf tb, tp;
-  hipError_t e;
-  if ((e = tb.upload(cb.data(), cb.size() * sizeof(CopyBlock), h->stream)) != hipSuccess ||
-      (e = tp.upload(prefix.data(), prefix.size() * sizeof(int64_t), h->stream)) != hipSuccess)
-    return hip_fail(h, e, "copy tables");
+  CallTables tab(h);
+  hipError_t e = tab.put(cb.data(), cb.size() * sizeof(CopyBlock), prefix.data(),
+                         prefix.size() * sizeof(int64_t));
+  if (e != hipSuccess) return hip_fail(h, e, "copy tables");
   KernelTimer* kt = active_timer(h);
   if (kt) kt->begin("copy_blocks_kernel", h->stream);
-  e = launch_copy_blocks(h->stream, dtype == ITG_C128, std::max(nmodes, 1), (const CopyBlock*)tb.p,
-                         (const int64_t*)tp.p, nblk, prefix.back(), src, dst);
+  e = launch_copy_blocks(h->stream, dtype == ITG_C128, std::max(nmodes, 1),
+                         (const CopyBlock*)tab.first(), (const int64_t*)tab.second(), nblk,
+                         prefix.back(), src, dst);
   if (kt) kt->end(h->stream);
   if (e != hipSuccess) return hip_fail(h, e, "copy launch");
   e = hipStreamSynchronize(h->stream);

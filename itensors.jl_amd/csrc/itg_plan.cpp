@@ -181,9 +181,10 @@ Merged merge_modes(int n, const int* perm) {
   return m;
 }
 
-hipError_t build_permute(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
-                         const std::vector<int64_t>* dst_offs, hipStream_t s,
-                         const std::vector<uint8_t>* fresh = nullptr) {
+// Host tables of a grouped permutation (see build_permute_launch).
+void permute_tables(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
+                    const std::vector<int64_t>* dst_offs, const std::vector<uint8_t>* fresh,
+                    std::vector<PermBlock>* blocks_out, std::vector<int64_t>* prefix_out) {
   Merged m = merge_modes(n, perm);
   if (m.nm == 0) {  // 0-dim tensor: one mode of extent 1
     m.nm = 1;
@@ -197,11 +198,12 @@ hipError_t build_permute(PermuteLaunch* pl, int n, const int* perm, const BlockL
   int q = 0;
   for (int i = 0; i < m.nm; ++i)
     if (m.perm[i] == 0) q = i;
-  std::vector<PermBlock> blocks(bl.nblk());
-  std::vector<int64_t> prefix(bl.nblk() + 1, 0);
+  std::vector<PermBlock>& blocks = *blocks_out;
+  std::vector<int64_t>& prefix = *prefix_out;
+  blocks.assign((size_t)bl.nblk(), PermBlock{});
+  prefix.assign((size_t)bl.nblk() + 1, 0);
   for (int64_t b = 0; b < bl.nblk(); ++b) {
     PermBlock& pb = blocks[b];
-    std::memset(&pb, 0, sizeof(pb));
     pb.off_src = bl.offs[b];
     pb.off_dst = dst_offs ? (*dst_offs)[b] : bl.offs[b];
     pb.fresh = fresh ? (*fresh)[b] : 0;
@@ -217,18 +219,25 @@ hipError_t build_permute(PermuteLaunch* pl, int n, const int* perm, const BlockL
     }
     pb.nelem = (int32_t)acc;
     for (int i = 0; i < kMaxModes; ++i) {
+      pb.ddim[i] = 1;
+      pb.dmul[i] = 1;  // x / 1
       if (i < m.nm) {
         pb.ddim[i] = (uint32_t)sdim[m.perm[i]];
         pb.sstr[i] = sstr[m.perm[i]];
-      } else {
-        pb.ddim[i] = 1;
+        fastdiv_consts(std::max<uint32_t>(pb.ddim[i], 1), &pb.dmul[i], &pb.dshr[i]);
       }
-      fastdiv_consts(std::max<uint32_t>(pb.ddim[i], 1), &pb.dmul[i], &pb.dshr[i]);
     }
     prefix[b + 1] = prefix[b] + permute_block_tiles(m.nm, q, pb.ddim, pl->kind);
   }
   pl->nblk = bl.nblk();
   pl->tiles = prefix.back();
+}
+
+hipError_t build_permute(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
+                         const std::vector<int64_t>* dst_offs, hipStream_t s) {
+  std::vector<PermBlock> blocks;
+  std::vector<int64_t> prefix;
+  permute_tables(pl, n, perm, bl, dst_offs, nullptr, &blocks, &prefix);
   hipError_t e = pl->blocks.upload(blocks.data(), blocks.size() * sizeof(PermBlock), s);
   if (e != hipSuccess) return e;
   return pl->prefix.upload(prefix.data(), prefix.size() * sizeof(int64_t), s);
@@ -669,10 +678,10 @@ bool build_fiber_tables(const Structure& st, const BlockList& b1, const BlockLis
 
 }  // namespace
 
-hipError_t build_permute_launch(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
-                                const std::vector<int64_t>* dst_offs, hipStream_t s,
-                                const std::vector<uint8_t>* fresh) {
-  return build_permute(pl, n, perm, bl, dst_offs, s, fresh);
+void build_permute_tables(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
+                          const std::vector<int64_t>* dst_offs, const std::vector<uint8_t>* fresh,
+                          std::vector<PermBlock>* blocks, std::vector<int64_t>* prefix) {
+  permute_tables(pl, n, perm, bl, dst_offs, fresh, blocks, prefix);
 }
 
 // ----------------------------------------------------------- exec plan

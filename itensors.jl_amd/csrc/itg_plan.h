@@ -210,13 +210,14 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
                                const std::vector<int>& Xp, const std::vector<int>& Xq,
                                const std::vector<PairSpec>& pairs, bool swap, hipStream_t s);
 
-// Build the device tables of a grouped permutation (dst offsets default to
-// the src offsets; a negative src offset marks an absent source block, whose
-// values are zero). perm: new mode i = old mode perm[i], 0-based. fresh
-// (optional, per block): 1 = the dst block is new, written without being read.
-hipError_t build_permute_launch(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
-                                const std::vector<int64_t>* dst_offs, hipStream_t s,
-                                const std::vector<uint8_t>* fresh = nullptr);
+// The host tables of a grouped permutation (dst offsets default to the src
+// offsets; a negative src offset marks an absent source block, whose values
+// are zero). perm: new mode i = old mode perm[i], 0-based. fresh (optional,
+// per block): 1 = the dst block is new, written without being read. Sets pl's
+// shape fields; the caller puts the tables on the device.
+void build_permute_tables(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
+                          const std::vector<int64_t>* dst_offs, const std::vector<uint8_t>* fresh,
+                          std::vector<PermBlock>* blocks, std::vector<int64_t>* prefix);
 
 // Launch the plan. ws: workspace of at least exec_workspace_bytes().
 // alpha_cplx: the call's alpha has a nonzero imaginary part.

@@ -168,7 +168,8 @@ class Index:
         return self.space[b - 1][0]
 
     def __eq__(self, other):
-        return isinstance(other, Index) and (self.id, self.plev, self.tags) == (other.id, other.plev, other.tags)
+        return isinstance(other, Index) and self.id == other.id and self.plev == other.plev \
+            and self.tags == other.tags
 
     def __hash__(self):
         return hash((self.id, self.plev, self.tags))
@@ -176,14 +177,21 @@ class Index:
     def __repr__(self):
         return f"(dim={self.dim}|id={self.id % 1000}|{self.tags!r}){chr(39) * self.plev}"
 
+    def _with(self, plev, dir, id):
+        """This index's space and tags (already checked) under another prime
+        level, arrow and id."""
+        i = Index.__new__(Index)
+        i.space, i.tags, i.plev, i.dir, i.id = self.space, self.tags, plev, dir, id
+        return i
+
     def prime(self, n=1):
-        return Index(self.space, self.tags, self.plev + n, self.dir, self.id)
+        return self._with(int(self.plev + n), self.dir, self.id)
 
     def sim(self):
-        return Index(self.space, self.tags, self.plev, self.dir)
+        return self._with(self.plev, self.dir, next(_next_id))
 
     def dag(self):
-        return Index(self.space, self.tags, self.plev, -self.dir, self.id)
+        return self._with(self.plev, -self.dir, self.id)
 
 
 def dag_index(i):
@@ -225,7 +233,7 @@ def compute_contraction_labels(Ais, Bis):
     ncont = 0
     for i, a in enumerate(Ais):
         for j, b in enumerate(Bis):
-            if a == b:
+            if a.id == b.id and a == b:
                 if have_qns and a.dir != -b.dir:
                     raise ValueError(
                         f"Attempting to contract IndexSet {Ais} with IndexSet {Bis}: QN indices "

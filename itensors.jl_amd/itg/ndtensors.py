@@ -19,7 +19,9 @@ raise.
 from __future__ import annotations
 
 import ctypes
+import itertools
 import math
+import operator
 from collections import OrderedDict
 
 import numpy as np
@@ -587,22 +589,16 @@ def contract_(R, labelsR, T1, labels1, T2, labels2, alpha=1.0, beta=0.0, *, prec
     dev = R.data.device
     h = _handle(dev)
     dt = _dtype_code(R.eltype)
-    lR, l1, l2 = _lib.i64(labelsR), _lib.i64(labels1), _lib.i64(labels2)
-    dR, d1, d2 = _lib.i64(R.dims), _lib.i64(T1.dims), _lib.i64(T2.dims)
     a, _ka = _lib.scalar2(alpha)
     b, _kb = _lib.scalar2(beta)
     flags = (_lib.ITG_FLAG_CONJ_A if conj1 else 0) | (_lib.ITG_FLAG_CONJ_B if conj2 else 0)
-    p = _lib.PREC[prec or _precision[0]]
-    args = []
-    for arr in (dR, lR, d1, l1, d2, l2):
-        ptr, keep = _lib.ptr64(arr)
-        args.append((ptr, keep))
+    ints = _lib.ints
     st = _lib.lib().itg_contract_dense_ex(
         h.h, dt,
-        len(R.dims), args[0][0], args[1][0], _ptr(R.data),
-        len(T1.dims), args[2][0], args[3][0], _ptr(T1.data),
-        len(T2.dims), args[4][0], args[5][0], _ptr(T2.data),
-        a, b, p, flags)
+        len(R.dims), ints(R.dims), ints(labelsR), _ptr(R.data),
+        len(T1.dims), ints(T1.dims), ints(labels1), _ptr(T1.data),
+        len(T2.dims), ints(T2.dims), ints(labels2), _ptr(T2.data),
+        a, b, _lib.PREC[prec or _precision[0]], flags)
     h.check(st)
     return R
 
@@ -945,25 +941,32 @@ def permutedims(T, perm):
         R = DenseTensor(torch.empty_like(T.data), dims)
         return permutedims_(R, T, perm)
     h = _handle(T.data.device)
+    N = T.ndims
+    if len(perm) != N:
+        raise ValueError("permutation length does not match the tensor")
     blocks = list(T.blockoffsets)
-    bd = _lib.i64([d for b in blocks for d in T.blockdims_of(b)])
-    offs = _lib.i64(list(T.blockoffsets.values()))
-    keep = []
-
-    def pp(a):
-        p, k = _lib.ptr64(a)
-        keep.append(k)
-        return p
-
+    nb = len(blocks)
+    # every block's dims: its sector coordinates looked up in the modes'
+    # sector sizes laid end to end
+    coords = np.fromiter(itertools.chain.from_iterable(blocks), dtype=np.int64,
+                         count=nb * N).reshape(nb, N)
+    sizes = np.array([d for bd in T.blockdims for d in bd], dtype=np.int64)
+    first = np.cumsum([0] + [len(bd) for bd in T.blockdims])[:N]
+    bd = sizes[coords - 1 + first] if N else np.zeros((nb, 0), dtype=np.int64)
+    offs = np.fromiter(T.blockoffsets.values(), dtype=np.int64, count=nb)
     # output offsets accumulate in block order (blockoffsets.jl:103-111)
-    dst = []
-    acc = 0
-    for b in blocks:
-        dst.append(acc)
-        acc += math.prod(T.blockdims_of(b))
-    out = torch.empty(acc, dtype=T.eltype, device=T.data.device)
+    ends = np.cumsum(bd.prod(axis=1))
+    nnz = int(ends[-1]) if nb else 0
+    dst = np.concatenate([[0], ends[:-1]]).astype(np.int64) if nb else ends
+    out = torch.empty(nnz, dtype=T.eltype, device=T.data.device)
     p32, _k32 = _lib.ptr32(list(perm))
-    h.check(_lib.lib().itg_bs_permute(h.h, _dtype_code(T.eltype), T.ndims, len(blocks), pp(bd),
-                                      pp(offs), pp(_lib.i64(dst)), p32, _ptr(T.data), _ptr(out)))
-    new_offs = OrderedDict((tuple(b[p - 1] for p in perm), o) for b, o in zip(blocks, dst))
-    return BlockSparseTensor(out, new_offs, tuple(T.blockdims[p - 1] for p in perm))
+    (pbd, _k1), (poffs, _k2), (pdst, _k3) = (
+        _lib.ptr64(np.ascontiguousarray(a)) for a in (bd.reshape(-1), offs, dst))
+    h.check(_lib.lib().itg_bs_permute(h.h, _dtype_code(T.eltype), N, nb, pbd, poffs, pdst, p32,
+                                      _ptr(T.data), _ptr(out)))
+    if N > 1:
+        moved = map(operator.itemgetter(*(p - 1 for p in perm)), blocks)
+    else:
+        moved = blocks
+    new_offs = OrderedDict(zip(moved, dst.tolist()))
+    return BlockSparseTensor._checked(out, new_offs, tuple(T.blockdims[p - 1] for p in perm), nnz)
