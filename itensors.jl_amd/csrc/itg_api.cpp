@@ -733,8 +733,8 @@ itg_status itg_permute(itg_handle* h, itg_dtype dtype, int ndim, const int64_t* 
   const int cplx = dtype == ITG_C128 || dtype == ITG_C64;
   const double a_re = alpha ? alpha[0] : 1.0, a_im = (alpha && cplx) ? alpha[1] : 0.0;
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
-  e = launch_permute(h->stream, elt_code(dtype), pl.nm, pl.perm, (const PermBlock*)tab.first(),
-                     (const int64_t*)tab.second(), pl.nblk, pl.tiles, pl.kind, src, dst, a_re,
+  e = launch_permute(h->stream, elt_code(dtype), pl.nm, (const PermBlock*)tab.first(),
+                     (const int64_t*)tab.second(), pl.nblk, pl.tiles, src, dst, a_re,
                      a_im, b_re, b_im);
   if (e != hipSuccess) return hip_fail(h, e, "permute launch");
   return ITG_OK;
@@ -1364,8 +1364,8 @@ itg_status bs_permute_run(itg_handle* h, itg_dtype dtype, int N, int64_t nblk,
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
   KernelTimer* kt = active_timer(h);
   if (kt) kt->begin("permute_kernel", h->stream);
-  e = launch_permute(h->stream, elt_code(dtype), pl.nm, pl.perm, (const PermBlock*)tab.first(),
-                     (const int64_t*)tab.second(), pl.nblk, pl.tiles, pl.kind, src, dst, a_re,
+  e = launch_permute(h->stream, elt_code(dtype), pl.nm, (const PermBlock*)tab.first(),
+                     (const int64_t*)tab.second(), pl.nblk, pl.tiles, src, dst, a_re,
                      a_im, b_re, b_im, nonzero ? (int32_t*)nz.p : nullptr);
   if (kt) kt->end(h->stream);
   if (e != hipSuccess) return hip_fail(h, e, "permute launch");

@@ -19,10 +19,11 @@ constexpr int kMaxKModes = 8;
 // Column-major tensors; offsets and strides are in ELEMENTS of the dtype.
 
 // One block of a grouped permutation: dst = alpha*perm(src) + beta*dst,
-// described in the DST block's mode order (dst mode 0 fastest) after mode
-// merging (nm modes, uniform per launch): the dst dims with their division
-// constants and the src stride of every dst mode, all computed on the host,
-// so the kernels walk the modes with compile-time indices only.
+// described in the DST block's mode order (dst mode 0 fastest) after dropping
+// the block's modes of size 1 and merging modes that stay adjacent: the dst
+// dims with their division constants and the src stride of every dst mode,
+// all computed on the host, so the kernels walk the modes with compile-time
+// indices only (nm of them, the most any block of the launch has).
 struct PermBlock {
   int64_t off_src;            // < 0: no source block (its values are zero)
   int64_t off_dst;
@@ -32,7 +33,12 @@ struct PermBlock {
   uint32_t dshr[kMaxModes];
   int32_t nelem;
   int32_t fresh;              // 1: the dst block is new (written, never read)
+  // 0: streamed in dst order; else the dst mode with src stride 1, and tiles
+  // of t0 (along dst mode 0) x tq (along dst mode q) go through LDS
+  int32_t q;
+  uint32_t t0, t0mul, t0shr, tq, tqmul, tqshr;
 };
+constexpr int kPermTile = 1024;  // elements per workgroup
 // Division constants of d >= 1 for dividends below 2^31 (Granlund and
 // Montgomery, "Division by invariant integers using multiplication", 1994,
 // fig. 4.1): q = (umulhi(x, mul) + x) >> shr.
@@ -148,21 +154,17 @@ inline hipError_t launch_kernel(void (*kernel)(KArgs...), dim3 grid, dim3 block,
 
 // Element types of the data-movement kernels.
 enum EltCode { kEltF64 = 0, kEltC128 = 1, kEltF32 = 2, kEltC64 = 3 };
-// Grouped permutation. perm[i] = src mode feeding dst mode i (0-based).
-// tile_prefix has nblk+1 entries (workgroups before block b). elt: EltCode
-// (0 / 1 = the cplx flag of the FP64 paths). nzflags (optional, nblk ints,
-// cleared by the launcher): set to 1 for every block with a written value
-// that is not zero.
-hipError_t launch_permute(hipStream_t s, int elt, int nm, const int32_t* perm_host,
-                          const PermBlock* blocks_dev, const int64_t* tile_prefix_dev,
-                          int64_t nblk, int64_t total_tiles, int mode_kind,
-                          const void* src, void* dst, double a_re, double a_im,
-                          double b_re, double b_im, int32_t* nzflags = nullptr);
-// Number of workgroups a block of the permutation needs (host helper that
-// must agree with the kernel's tiling). ddim: the block's dst dims; q: the
-// dst mode fed by src mode 0. mode_kind: 0 = src mode 0 stays dst mode 0
-// (streamed), 1 = 2-D tile transpose of dst mode 0 and dst mode q.
-int64_t permute_block_tiles(int nm, int q, const uint32_t* ddim, int mode_kind);
+// Grouped permutation. tile_prefix has nblk+1 entries (workgroups before
+// block b). elt: EltCode (0 / 1 = the cplx flag of the FP64 paths). nzflags
+// (optional, nblk ints, cleared by the launcher): set to 1 for every block
+// with a written value that is not zero.
+hipError_t launch_permute(hipStream_t s, int elt, int nm, const PermBlock* blocks_dev,
+                          const int64_t* tile_prefix_dev, int64_t nblk, int64_t total_tiles,
+                          const void* src, void* dst, double a_re, double a_im, double b_re,
+                          double b_im, int32_t* nzflags = nullptr);
+// Chooses a block's form (q, t0, tq) from its ddim, sstr and nelem, and
+// returns its workgroups.
+int64_t permute_block_plan(int nm, PermBlock* b);
 
 // One block of a grouped strided copy (element offsets and strides; modes
 // in traversal order, mode 0 fastest; nelem = product of dims < 2^31).

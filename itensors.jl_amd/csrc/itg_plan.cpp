@@ -142,92 +142,44 @@ std::string analyze_labels(int NR, const int64_t* lR, int N1, const int64_t* l1,
 // --------------------------------------------------------- permutations
 namespace {
 
-// Merge src modes that stay adjacent (and in order) under perm. Returns the
-// merged permutation and, for each merged mode, the range of original modes.
-struct Merged {
-  int nm = 0;
-  int32_t perm[kMaxModes];
-  int first[kMaxModes], last[kMaxModes];  // original src modes of merged src mode
-};
-
-Merged merge_modes(int n, const int* perm) {
-  // group dst positions into runs where perm[j+1] == perm[j] + 1
-  Merged m;
-  int run_of_src[kMaxModes];
-  int runs = 0;
-  int run_first[kMaxModes], run_last[kMaxModes];
-  for (int j = 0; j < n; ++j) {
-    if (j > 0 && perm[j] == perm[j - 1] + 1) {
-      run_last[runs - 1] = perm[j];
-    } else {
-      run_first[runs] = perm[j];
-      run_last[runs] = perm[j];
-      runs++;
-    }
-  }
-  // merged src mode index = rank of run by its first src mode
-  int order[kMaxModes];
-  for (int r = 0; r < runs; ++r) order[r] = r;
-  std::sort(order, order + runs, [&](int a, int b) { return run_first[a] < run_first[b]; });
-  int merged_index_of_run[kMaxModes];
-  for (int i = 0; i < runs; ++i) merged_index_of_run[order[i]] = i;
-  m.nm = runs;
-  for (int r = 0; r < runs; ++r) {
-    m.perm[r] = merged_index_of_run[r];
-    m.first[merged_index_of_run[r]] = run_first[r];
-    m.last[merged_index_of_run[r]] = run_last[r];
-  }
-  (void)run_of_src;
-  return m;
-}
-
-// Host tables of a grouped permutation (see build_permute_launch).
+// Host tables of a grouped permutation (see build_permute_tables).
 void permute_tables(PermuteLaunch* pl, int n, const int* perm, const BlockList& bl,
                     const std::vector<int64_t>* dst_offs, const std::vector<uint8_t>* fresh,
                     std::vector<PermBlock>* blocks_out, std::vector<int64_t>* prefix_out) {
-  Merged m = merge_modes(n, perm);
-  if (m.nm == 0) {  // 0-dim tensor: one mode of extent 1
-    m.nm = 1;
-    m.perm[0] = 0;
-    m.first[0] = 0;
-    m.last[0] = -1;
-  }
-  pl->nm = m.nm;
-  for (int i = 0; i < kMaxModes; ++i) pl->perm[i] = i < m.nm ? m.perm[i] : 0;
-  pl->kind = (m.nm <= 1 || m.perm[0] == 0) ? 0 : 1;
-  int q = 0;
-  for (int i = 0; i < m.nm; ++i)
-    if (m.perm[i] == 0) q = i;
   std::vector<PermBlock>& blocks = *blocks_out;
   std::vector<int64_t>& prefix = *prefix_out;
   blocks.assign((size_t)bl.nblk(), PermBlock{});
   prefix.assign((size_t)bl.nblk() + 1, 0);
+  pl->nm = 1;
   for (int64_t b = 0; b < bl.nblk(); ++b) {
     PermBlock& pb = blocks[b];
     pb.off_src = bl.offs[b];
     pb.off_dst = dst_offs ? (*dst_offs)[b] : bl.offs[b];
     pb.fresh = fresh ? (*fresh)[b] : 0;
     const int32_t* d = bl.d(b);
-    int64_t sdim[kMaxModes], sstr[kMaxModes];
-    int64_t acc = 1;
-    for (int i = 0; i < m.nm; ++i) {  // merged src modes
-      int64_t prod = 1;
-      for (int k = m.first[i]; k <= m.last[i]; ++k) prod *= d[k];
-      sdim[i] = prod;
+    int64_t sstr[kMaxModes], acc = 1;
+    for (int i = 0; i < n; ++i) {
       sstr[i] = acc;
-      acc *= prod;
+      acc *= d[i];
     }
     pb.nelem = (int32_t)acc;
-    for (int i = 0; i < kMaxModes; ++i) {
-      pb.ddim[i] = 1;
-      pb.dmul[i] = 1;  // x / 1
-      if (i < m.nm) {
-        pb.ddim[i] = (uint32_t)sdim[m.perm[i]];
-        pb.sstr[i] = sstr[m.perm[i]];
-        fastdiv_consts(std::max<uint32_t>(pb.ddim[i], 1), &pb.dmul[i], &pb.dshr[i]);
+    // dst modes of more than one value, neighbours merged when they are
+    // neighbours in the source too
+    int nm = 0;
+    for (int i = 0; i < kMaxModes; ++i) pb.ddim[i] = 1;
+    for (int i = 0; i < n && acc > 0; ++i) {
+      const int m = perm[i];
+      if (d[m] == 1) continue;
+      if (nm > 0 && sstr[m] == pb.sstr[nm - 1] * pb.ddim[nm - 1]) {
+        pb.ddim[nm - 1] *= (uint32_t)d[m];
+      } else {
+        pb.ddim[nm] = (uint32_t)d[m];
+        pb.sstr[nm++] = sstr[m];
       }
     }
-    prefix[b + 1] = prefix[b] + permute_block_tiles(m.nm, q, pb.ddim, pl->kind);
+    pl->nm = std::max(pl->nm, nm);
+    for (int i = 0; i < kMaxModes; ++i) fastdiv_consts(pb.ddim[i], &pb.dmul[i], &pb.dshr[i]);
+    prefix[b + 1] = prefix[b] + permute_block_plan(nm, &pb);
   }
   pl->nblk = bl.nblk();
   pl->tiles = prefix.back();
@@ -1645,8 +1597,8 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
         }
       }
       TimeScope ts(kt, "permute_kernel", s);
-      e = launch_permute(s, cplx, ep.pC.nm, ep.pC.perm, (const PermBlock*)ep.pC.blocks.p,
-                         (const int64_t*)ep.pC.prefix.p, ep.pC.nblk, ep.pC.tiles, ep.pC.kind, S1,
+      e = launch_permute(s, cplx, ep.pC.nm, (const PermBlock*)ep.pC.blocks.p,
+                         (const int64_t*)ep.pC.prefix.p, ep.pC.nblk, ep.pC.tiles, S1,
                          R, a_re, a_im, b_re, b_im);
       if (e != hipSuccess) *err = std::string("permute launch: ") + hipGetErrorString(e);
       return e;
@@ -1683,8 +1635,8 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
   }
   if (ep.permC) {
     TimeScope ts(kt, "permute_kernel", s);
-    e = launch_permute(s, cplx, ep.pC.nm, ep.pC.perm, (const PermBlock*)ep.pC.blocks.p,
-                       (const int64_t*)ep.pC.prefix.p, ep.pC.nblk, ep.pC.tiles, ep.pC.kind, C, R,
+    e = launch_permute(s, cplx, ep.pC.nm, (const PermBlock*)ep.pC.blocks.p,
+                       (const int64_t*)ep.pC.prefix.p, ep.pC.nblk, ep.pC.tiles, C, R,
                        1.0, 0.0, b_re, b_im);
     if (e != hipSuccess) *err = std::string("permute launch: ") + hipGetErrorString(e);
   }
@@ -1742,8 +1694,8 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
   if (ep.permA) {
     {
       TimeScope ts(kt, "permute_kernel", s);
-      e = launch_permute(s, cplx, ep.pA.nm, ep.pA.perm, (const PermBlock*)ep.pA.blocks.p,
-                         (const int64_t*)ep.pA.prefix.p, ep.pA.nblk, ep.pA.tiles, ep.pA.kind, A,
+      e = launch_permute(s, cplx, ep.pA.nm, (const PermBlock*)ep.pA.blocks.p,
+                         (const int64_t*)ep.pA.prefix.p, ep.pA.nblk, ep.pA.tiles, A,
                          w, 1.0, 0.0, 0.0, 0.0);
     }
     if (e != hipSuccess) {
@@ -1756,8 +1708,8 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
   if (ep.permB) {
     {
       TimeScope ts(kt, "permute_kernel", s);
-      e = launch_permute(s, cplx, ep.pB.nm, ep.pB.perm, (const PermBlock*)ep.pB.blocks.p,
-                         (const int64_t*)ep.pB.prefix.p, ep.pB.nblk, ep.pB.tiles, ep.pB.kind, B,
+      e = launch_permute(s, cplx, ep.pB.nm, (const PermBlock*)ep.pB.blocks.p,
+                         (const int64_t*)ep.pB.prefix.p, ep.pB.nblk, ep.pB.tiles, B,
                          w, 1.0, 0.0, 0.0, 0.0);
     }
     if (e != hipSuccess) {
@@ -1826,8 +1778,8 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
   }  // split-K
   if (ep.permC) {
     TimeScope ts(kt, "permute_kernel", s);
-    e = launch_permute(s, cplx, ep.pC.nm, ep.pC.perm, (const PermBlock*)ep.pC.blocks.p,
-                       (const int64_t*)ep.pC.prefix.p, ep.pC.nblk, ep.pC.tiles, ep.pC.kind, C, R,
+    e = launch_permute(s, cplx, ep.pC.nm, (const PermBlock*)ep.pC.blocks.p,
+                       (const int64_t*)ep.pC.prefix.p, ep.pC.nblk, ep.pC.tiles, C, R,
                        1.0, 0.0, b_re, b_im);
     if (e != hipSuccess) *err = std::string("permute launch: ") + hipGetErrorString(e);
   }

@@ -104,9 +104,7 @@ constexpr unsigned kFlagConj = 3u;
 
 
 struct PermuteLaunch {
-  int nm = 0;
-  int32_t perm[kMaxModes];
-  int kind = 0;
+  int nm = 0;  // modes of the block descriptors
   int64_t nblk = 0, tiles = 0;
   DevBuf blocks, prefix;
 };

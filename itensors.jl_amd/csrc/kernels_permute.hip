@@ -1,19 +1,27 @@
 // Grouped tensor permutation for gfx950.
 //
 // dst(block b) = alpha * permutedims(src(block b), perm) + beta * dst(block b)
-// for every block of a launch (one block for a dense tensor). The mode
-// permutation is uniform across the launch; block dims differ.
-//
-// Two tilings, chosen on the host from the (merged) permutation:
-//  kind 0: src mode 0 stays the fastest dst mode. Each workgroup streams
-//          kElemsPerWG consecutive dst elements; reads and writes are both
-//          contiguous along mode 0.
-//  kind 1: src mode 0 and src mode perm[0] swap roles. 32x32 tiles staged
-//          through LDS: read along src mode 0, write along dst mode 0, both
-//          coalesced; the other modes are a batch index.
+// for every block of a launch (one block for a dense tensor). Block dims
+// differ, and with them what the permutation looks like once modes of size 1
+// are dropped and neighbours merged, so every block has its own form:
+//  streamed: the block's src mode 0 stays its fastest dst mode (or both of
+//          the modes below are short). A workgroup writes kPermTile
+//          consecutive dst elements; reads run along src mode 0.
+//  tiled:  tiles of dst mode 0 x the dst mode that is src mode 0 go through
+//          LDS: read along src mode 0, written along dst mode 0; the other
+//          modes are a batch index. A tile is 32 x 32, or, when one of the
+//          two modes is shorter, all of it times as much of the other.
+// Bound: HBM. With the form chosen once per launch, from the dims before the
+// unit modes were dropped, every U(1) permutation whose first mode had
+// sectors of size 1 ran as 1 x 32 tiles: chi = 4096 Z(a', b, s1', s2', w'') (360
+// MB moved) in the order (5, 4, 3, 2, 1) 1.45 -> 0.126 ms, (3, 1, 4, 2, 5) 1.83
+// -> 0.071 ms (5.1 TB/s); dense (5, 1024, 2048) -> (1024, 5, 2048) 82 -> 32 us;
+// (1, 3, 4, 5, 2), streamed before and now, 0.074 ms.
 // Replaces NDTensors.permutedims! via Strided.jl (NDTensors/src/array/
 // permutedims.jl:5-24); the alpha/beta form covers _contract_scalar_perm!
 // (NDTensors/src/abstractarray/tensoralgebra/contract.jl:88-113).
+#include <algorithm>
+
 #include "itg_internal.h"
 
 namespace itg {
@@ -23,7 +31,10 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kElemsPerThread = 4;
 constexpr int kElemsPerWG = kThreads * kElemsPerThread;
+static_assert(kElemsPerWG == kPermTile, "permutation tile");
 constexpr int kTile = 32;
+// tile[j * (tq | 1) + i]: at most kPermTile elements, strides of 3 or more
+constexpr int kTileSlots = kPermTile + kPermTile / 2;
 
 template <int CPLX>
 struct Elem;
@@ -108,24 +119,18 @@ __device__ inline void mark_nonzero(int32_t* nzflags, int64_t b, bool nz) {
   if (__syncthreads_or(nz ? 1 : 0) && threadIdx.x == 0) nzflags[b] = 1;
 }
 
-// Kind 0: src mode 0 stays the fastest dst mode. A workgroup streams
-// kElemsPerWG consecutive dst elements of one block: the four loads of a
-// thread are issued back to back (offsets clamped into the block), then the
-// stores; reads and writes run along mode 0.
+// Streamed block: the four loads of a thread are issued back to back (offsets
+// clamped into the block), then the stores. Returns whether a written value
+// is not zero.
 template <typename T, int NM>
-__global__ void __launch_bounds__(kThreads)
-    permute_inner_kernel(const PermBlock* __restrict__ blocks, const int64_t* __restrict__ prefix,
-                         int64_t nblk, const T* __restrict__ src, T* __restrict__ dst,
-                         double a_re, double a_im, double b_re, double b_im,
-                         int32_t* __restrict__ nzflags) {
-  const int64_t wg = blockIdx.x;
-  const int64_t b = find_block(prefix, nblk, wg);
-  const PermBlock& blk = blocks[b];
+__device__ inline bool permute_stream(const PermBlock& blk, uint32_t tile,
+                                      const T* __restrict__ src, T* __restrict__ dst,
+                                      double a_re, double a_im, double b_re, double b_im) {
   const int64_t off_src = blk.off_src, off_dst = blk.off_dst;
   const uint32_t n = (uint32_t)blk.nelem;
   const bool has_src = off_src >= 0;
   const bool use_beta = (b_re != 0.0 || b_im != 0.0) && !blk.fresh;
-  const uint32_t e0 = (uint32_t)(wg - prefix[b]) * kElemsPerWG + threadIdx.x;
+  const uint32_t e0 = tile * kElemsPerWG + threadIdx.x;
   T x[kElemsPerThread], y[kElemsPerThread];
 #pragma unroll
   for (int r = 0; r < kElemsPerThread; ++r) {
@@ -143,23 +148,17 @@ __global__ void __launch_bounds__(kThreads)
       dst[off_dst + e] = v;
     }
   }
-  mark_nonzero(nzflags, b, nz);
+  return nz;
 }
 
-// Kind 1: dst mode 0 (src mode p) and dst mode q (src mode 0) form 32x32
-// tiles staged through LDS: read along src mode 0, written along dst mode 0,
-// both coalesced; the other dst modes are a batch index.
+// Tiled block. A tile's element (j along dst mode 0, i along dst mode q) sits
+// at tile[j * (tq | 1) + i]: an odd stride, so that neither pass conflicts.
 template <typename T, int NM>
-__global__ void __launch_bounds__(kThreads)
-    permute_tile_kernel(const PermBlock* __restrict__ blocks, const int64_t* __restrict__ prefix,
-                        int64_t nblk, int q, const T* __restrict__ src, T* __restrict__ dst,
-                        double a_re, double a_im, double b_re, double b_im,
-                        int32_t* __restrict__ nzflags) {
-  __shared__ T tile[kTile][kTile + 1];
-  const int64_t wg = blockIdx.x;
-  const int64_t b = find_block(prefix, nblk, wg);
-  const PermBlock& blk = blocks[b];
-  // dst strides (column-major over ddim); dst mode q is src mode 0
+__device__ inline bool permute_tiled(const PermBlock& blk, uint32_t t, T* __restrict__ tile,
+                                     const T* __restrict__ src, T* __restrict__ dst, double a_re,
+                                     double a_im, double b_re, double b_im) {
+  const int q = blk.q;
+  // dst strides (column-major over ddim)
   int64_t dstr[NM];
   {
     int64_t acc = 1;
@@ -169,25 +168,20 @@ __global__ void __launch_bounds__(kThreads)
       acc *= blk.ddim[i];
     }
   }
-  uint32_t Dq = 1, Mq = 1, Sq = 0;
+  uint32_t Dq = 1;
   int64_t dstr_q = 1;
 #pragma unroll
   for (int i = 1; i < NM; ++i)
     if (i == q) {
       Dq = blk.ddim[i];
-      Mq = blk.dmul[i];
-      Sq = blk.dshr[i];
       dstr_q = dstr[i];
     }
-  (void)Mq;
-  (void)Sq;
-  const uint32_t D0 = blk.ddim[0];
-  const int64_t sstr0 = blk.sstr[0];  // src stride of dst mode 0 (src mode p)
-  const uint32_t tq_n = (Dq + kTile - 1) / kTile, t0_n = (D0 + kTile - 1) / kTile;
-  uint32_t t = (uint32_t)(wg - prefix[b]);
-  const uint32_t tq = t % tq_n;
+  const uint32_t D0 = blk.ddim[0], T0 = blk.t0, TQ = blk.tq, ld = TQ | 1;
+  const int64_t sstr0 = blk.sstr[0];
+  const uint32_t tq_n = (Dq + TQ - 1) / TQ, t0_n = (D0 + T0 - 1) / T0;
+  const uint32_t i0 = t % tq_n * TQ;
   t /= tq_n;
-  const uint32_t t0 = t % t0_n;
+  const uint32_t j0 = t % t0_n * T0;
   uint32_t bidx = t / t0_n;
   // batch coordinates: every dst mode except 0 and q
   int64_t sbase = 0, dbase = 0;
@@ -200,34 +194,56 @@ __global__ void __launch_bounds__(kThreads)
     dbase += (int64_t)c * dstr[i];
     bidx = qq;
   }
-  const uint32_t iq0 = tq * kTile, j0 = t0 * kTile;
-  const int lx = threadIdx.x % kTile;
-  const int ly = threadIdx.x / kTile;  // 0..7
+  const uint32_t nt = T0 * TQ;
   const bool has_src = blk.off_src >= 0;
-  // read: iq (dst mode q = src mode 0, contiguous in src) along lanes
   if (has_src) {
+    T x[kElemsPerThread];
 #pragma unroll
-    for (int r = 0; r < kTile; r += kThreads / kTile) {
-      const uint32_t iq = iq0 + lx, j = j0 + ly + r;
-      if (iq < Dq && j < D0) tile[ly + r][lx] = src[blk.off_src + sbase + iq + j * sstr0];
+    for (int r = 0; r < kElemsPerThread; ++r) {
+      const uint32_t e = min(threadIdx.x + r * kThreads, nt - 1);
+      const uint32_t j = fdiv(e, blk.tqmul, blk.tqshr), i = e - j * TQ;
+      x[r] = src[blk.off_src + sbase + min(i0 + i, Dq - 1) + min(j0 + j, D0 - 1) * sstr0];
+    }
+#pragma unroll
+    for (int r = 0; r < kElemsPerThread; ++r) {
+      const uint32_t e = min(threadIdx.x + r * kThreads, nt - 1);
+      const uint32_t j = fdiv(e, blk.tqmul, blk.tqshr), i = e - j * TQ;
+      tile[j * ld + i] = x[r];
     }
   }
   __syncthreads();
   const bool use_beta = (b_re != 0.0 || b_im != 0.0) && !blk.fresh;
   bool nz = false;
 #pragma unroll
-  for (int r = 0; r < kTile; r += kThreads / kTile) {
-    const uint32_t j = j0 + lx, iq = iq0 + ly + r;
-    if (iq < Dq && j < D0) {
-      const int64_t o = blk.off_dst + dbase + j + iq * dstr_q;
+  for (int r = 0; r < kElemsPerThread; ++r) {
+    const uint32_t e = threadIdx.x + r * kThreads;
+    const uint32_t i = fdiv(e, blk.t0mul, blk.t0shr), j = e - i * T0;
+    if (e < nt && i0 + i < Dq && j0 + j < D0) {
+      const int64_t o = blk.off_dst + dbase + (j0 + j) + (i0 + i) * dstr_q;
       T y{};
       if (use_beta) y = dst[o];
-      const T x = has_src ? tile[lx][ly + r] : T{};
+      const T x = has_src ? tile[j * ld + i] : T{};
       const T v = axpby(a_re, a_im, x, b_re, b_im, y, use_beta);
       nz |= nonzero(v);
       dst[o] = v;
     }
   }
+  return nz;
+}
+
+template <typename T, int NM>
+__global__ void __launch_bounds__(kThreads)
+    permute_kernel(const PermBlock* __restrict__ blocks, const int64_t* __restrict__ prefix,
+                   int64_t nblk, const T* __restrict__ src, T* __restrict__ dst, double a_re,
+                   double a_im, double b_re, double b_im, int32_t* __restrict__ nzflags) {
+  __shared__ T tile[kTileSlots];
+  const int64_t wg = blockIdx.x;
+  const int64_t b = find_block(prefix, nblk, wg);
+  const PermBlock& blk = blocks[b];
+  const uint32_t t = (uint32_t)(wg - prefix[b]);
+  const bool nz = blk.q == 0
+                      ? permute_stream<T, NM>(blk, t, src, dst, a_re, a_im, b_re, b_im)
+                      : permute_tiled<T, NM>(blk, t, tile, src, dst, a_re, a_im, b_re, b_im);
   mark_nonzero(nzflags, b, nz);
 }
 
@@ -407,38 +423,45 @@ hipError_t launch_axpby_join(hipStream_t s, int64_t n, double a_re, double a_im,
   return hipGetLastError();
 }
 
-int64_t permute_block_tiles(int nm, int q, const uint32_t* ddim, int mode_kind) {
-  int64_t nelem = 1;
-  for (int i = 0; i < nm; ++i) nelem *= ddim[i];
-  if (nelem == 0) return 0;
-  if (mode_kind == 0) return (nelem + kElemsPerWG - 1) / kElemsPerWG;
-  const int64_t D0 = ddim[0], Dq = ddim[q];
-  const int64_t nb = nelem / (D0 * Dq);
-  return ((D0 + kTile - 1) / kTile) * ((Dq + kTile - 1) / kTile) * nb;
+// A mode shorter than a tile side makes the other side longer; below
+// kMinTile elements in all (both modes short) the block is streamed: its
+// dst order is then close to its src order.
+int64_t permute_block_plan(int nm, PermBlock* b) {
+  constexpr uint32_t kMinTile = 256;
+  if (b->nelem <= 0) return 0;
+  int q = 0;
+  for (int i = 1; i < nm; ++i)
+    if (b->sstr[i] == 1) q = i;
+  b->q = 0;
+  b->t0 = b->tq = 1;
+  if (q > 0) {
+    const uint32_t D0 = b->ddim[0], Dq = b->ddim[q];
+    uint32_t t0 = std::min<uint32_t>(D0, kTile), tq = std::min<uint32_t>(Dq, kTile);
+    if (t0 < kTile) tq = std::min<uint32_t>(Dq, kPermTile / t0);
+    else if (tq < kTile) t0 = std::min<uint32_t>(D0, kPermTile / tq);
+    if (t0 * tq >= kMinTile) {
+      b->q = q;
+      b->t0 = t0;
+      b->tq = tq;
+      fastdiv_consts(t0, &b->t0mul, &b->t0shr);
+      fastdiv_consts(tq, &b->tqmul, &b->tqshr);
+      const int64_t nb = b->nelem / ((int64_t)D0 * Dq);
+      return (int64_t)((D0 + t0 - 1) / t0) * ((Dq + tq - 1) / tq) * nb;
+    }
+  }
+  return ((int64_t)b->nelem + kElemsPerWG - 1) / kElemsPerWG;
 }
 
 namespace {
-template <typename T, int NM>
-void launch_perm_nm(hipStream_t s, int kind, int q, dim3 grid, const PermBlock* blocks,
-                    const int64_t* prefix, int64_t nblk, const void* src, void* dst, double a_re,
-                    double a_im, double b_re, double b_im, int32_t* nz) {
-  if (kind == 0)
-    ITG_LAUNCH((permute_inner_kernel<T, NM>), grid, kThreads, 0, s, blocks, prefix, nblk,
-               (const T*)src, (T*)dst, a_re, a_im, b_re, b_im, nz);
-  else
-    ITG_LAUNCH((permute_tile_kernel<T, NM>), grid, kThreads, 0, s, blocks, prefix, nblk, q,
-               (const T*)src, (T*)dst, a_re, a_im, b_re, b_im, nz);
-}
-
 template <typename T>
-void launch_perm_t(hipStream_t s, int nm, int kind, int q, dim3 grid, const PermBlock* blocks,
+void launch_perm_t(hipStream_t s, int nm, dim3 grid, const PermBlock* blocks,
                    const int64_t* prefix, int64_t nblk, const void* src, void* dst, double a_re,
                    double a_im, double b_re, double b_im, int32_t* nz) {
   switch (nm) {
-#define ITG_PERM_NM(N)                                                                        \
-  case N:                                                                                     \
-    launch_perm_nm<T, N>(s, kind, q, grid, blocks, prefix, nblk, src, dst, a_re, a_im, b_re, \
-                         b_im, nz);                                                           \
+#define ITG_PERM_NM(N)                                                                       \
+  case N:                                                                                    \
+    ITG_LAUNCH((permute_kernel<T, N>), grid, kThreads, 0, s, blocks, prefix, nblk,           \
+               (const T*)src, (T*)dst, a_re, a_im, b_re, b_im, nz);                          \
     break;
     ITG_PERM_NM(1)
     ITG_PERM_NM(2)
@@ -454,11 +477,10 @@ void launch_perm_t(hipStream_t s, int nm, int kind, int q, dim3 grid, const Perm
 static_assert(kMaxModes == 8, "permute kernels are instantiated for 1..8 modes");
 }  // namespace
 
-hipError_t launch_permute(hipStream_t s, int elt, int nm, const int32_t* perm_host,
-                          const PermBlock* blocks_dev, const int64_t* tile_prefix_dev,
-                          int64_t nblk, int64_t total_tiles, int mode_kind, const void* src,
-                          void* dst, double a_re, double a_im, double b_re, double b_im,
-                          int32_t* nzflags) {
+hipError_t launch_permute(hipStream_t s, int elt, int nm, const PermBlock* blocks_dev,
+                          const int64_t* tile_prefix_dev, int64_t nblk, int64_t total_tiles,
+                          const void* src, void* dst, double a_re, double a_im, double b_re,
+                          double b_im, int32_t* nzflags) {
   if (nm < 1 || nm > kMaxModes) return hipErrorInvalidValue;
   if (nzflags && nblk > 0) {
     ITG_LAUNCH(fill_i32_kernel, dim3((unsigned)((nblk + kThreads - 1) / kThreads)), kThreads, 0,
@@ -467,30 +489,21 @@ hipError_t launch_permute(hipStream_t s, int elt, int nm, const int32_t* perm_ho
     if (e != hipSuccess) return e;
   }
   if (total_tiles == 0) return hipSuccess;
-  int q = 0;  // dst mode fed by src mode 0
-  for (int i = 0; i < nm; ++i)
-    if (perm_host[i] == 0) q = i;
   const dim3 grid((unsigned)total_tiles);
+#define ITG_PERM_ELT(E, T)                                                                  \
+  case E:                                                                                   \
+    launch_perm_t<T>(s, nm, grid, blocks_dev, tile_prefix_dev, nblk, src, dst, a_re, a_im, \
+                     b_re, b_im, nzflags);                                                  \
+    break;
   switch (elt) {
-    case kEltF64:
-      launch_perm_t<double>(s, nm, mode_kind, q, grid, blocks_dev, tile_prefix_dev, nblk, src,
-                            dst, a_re, a_im, b_re, b_im, nzflags);
-      break;
-    case kEltC128:
-      launch_perm_t<double2>(s, nm, mode_kind, q, grid, blocks_dev, tile_prefix_dev, nblk, src,
-                             dst, a_re, a_im, b_re, b_im, nzflags);
-      break;
-    case kEltF32:
-      launch_perm_t<float>(s, nm, mode_kind, q, grid, blocks_dev, tile_prefix_dev, nblk, src,
-                           dst, a_re, a_im, b_re, b_im, nzflags);
-      break;
-    case kEltC64:
-      launch_perm_t<float2>(s, nm, mode_kind, q, grid, blocks_dev, tile_prefix_dev, nblk, src,
-                            dst, a_re, a_im, b_re, b_im, nzflags);
-      break;
+    ITG_PERM_ELT(kEltF64, double)
+    ITG_PERM_ELT(kEltC128, double2)
+    ITG_PERM_ELT(kEltF32, float)
+    ITG_PERM_ELT(kEltC64, float2)
     default:
       return hipErrorInvalidValue;
   }
+#undef ITG_PERM_ELT
   return hipGetLastError();
 }
 

@@ -1,7 +1,9 @@
 """permutedims calls whose tables go through the handle's staging ring: many
 calls in flight on two streams with different structures, tables too large
 for the ring, orders 1 to 5 with empty sectors, and the refusal under stream
-capture. Values are moved, not computed: compared exactly with numpy."""
+capture; and the forms a block can take (streamed, or tiles whose sides
+follow the block's dims). Values are moved, or scaled by powers of two and
+added once: compared exactly with numpy."""
 import numpy as np
 import pytest
 
@@ -85,3 +87,30 @@ def test_refused_under_capture():
             ND.permutedims(T, (3, 1, 2))
     got = ND.permutedims(T, (3, 1, 2))
     assert torch.equal(got.data, want.data)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
+@pytest.mark.parametrize("dims,perm", [
+    ((1,), (1,)), ((5, 7), (2, 1)), ((2, 600), (2, 1)), ((600, 3), (2, 1)), ((31, 33), (2, 1)),
+    ((32, 32), (2, 1)), ((33, 8), (2, 1)), ((8, 32), (2, 1)), ((16, 16), (2, 1)), ((15, 17), (2, 1)),
+    ((1, 65, 1, 70), (4, 3, 2, 1)), ((3, 5, 130), (3, 1, 2)), ((40, 1, 2, 50), (3, 4, 2, 1)),
+    ((2, 9, 3, 40), (4, 2, 1, 3)), ((70, 2, 3, 5), (3, 1, 4, 2)), ((1030, 2, 1), (2, 3, 1)),
+    ((2, 3, 2, 3, 2, 3, 2, 3), (8, 6, 4, 2, 7, 5, 3, 1)), ((4, 600, 2), (3, 2, 1))])
+def test_block_forms(dims, perm, dtype):
+    import torch
+    from itg import ndtensors as ND
+    rng = np.random.default_rng(sum(dims))
+
+    def draw(shape):
+        x = rng.standard_normal(shape)
+        return (x + 1j * rng.standard_normal(shape) if np.dtype(dtype).kind == "c" else x).astype(
+            dtype)
+
+    p0 = [p - 1 for p in perm]
+    x, y = draw(dims), draw([dims[p] for p in p0])
+    T = ND.DenseTensor.from_numpy(x)
+    assert np.array_equal(ND.permutedims(T, perm).to_numpy(), x.transpose(p0))
+    R = ND.permutedims_(ND.DenseTensor.from_numpy(y), T, perm, alpha=2.0, beta=0.5)
+    wide = np.complex128 if np.dtype(dtype).kind == "c" else np.float64
+    want = (2.0 * x.transpose(p0).astype(wide) + 0.5 * y.astype(wide)).astype(dtype)
+    assert np.array_equal(R.to_numpy(), want)
