@@ -224,7 +224,8 @@ struct FiberPair {
 // group's W in LDS, loads all slots of its fibers at once (A read exactly
 // once) and writes every output.
 constexpr int kFiberSlots = 16, kFiberOuts = 32;
-constexpr int kFibersPerWGMV = 256 * 8;  // 8 rounds of one fiber per thread
+constexpr int kFiberThreads = 256;
+constexpr int kMaxRoundsMV = 8;      // rounds of one fiber per thread in a workgroup, at most
 struct FiberMVGroup {
   int64_t nfib, wg0;
   int32_t fdim[kMaxModes];
@@ -250,12 +251,13 @@ struct FiberCoef {           // W[slot][out] = alpha * B[off_b]
   int32_t slot, out;
 };
 // nf: number of A-free modes (1..kMaxModes). flags bit 0 / 1: conj(A) / conj(B).
+// rounds: fibers per workgroup / kFiberThreads (of the plan's wg_group).
 // smax: slot bound the kernel is unrolled for (4, 8 or 16; >= every group's nslot).
 hipError_t launch_fiber_mv(hipStream_t s, int cplx, int nf, int smax, const FiberMVGroup* groups,
                            const FiberSlot* slots, const FiberOutElem* outs,
                            const FiberCoef* coefs, const int32_t* wg_group, int64_t total_wgs,
-                           const void* A, const void* B, void* C, unsigned flags, double ga_re,
-                           double ga_im, double beta_re, double beta_im);
+                           int rounds, const void* A, const void* B, void* C, unsigned flags,
+                           double ga_re, double ga_im, double beta_re, double beta_im);
 // Two consecutive matrix-form fiber contractions fused, Y = X*B1 then
 // Z = Y*B2, without storing Y. A super-fiber is one value of the modes that
 // are fiber modes of both steps (the other fiber modes of either step have
@@ -267,7 +269,7 @@ hipError_t launch_fiber_mv(hipStream_t s, int cplx, int nf, int smax, const Fibe
 // the same order as the two separate passes, so Z is bit-identical. Slot
 // and output strides are given over the shared modes (fdim order).
 constexpr int kChainX = 16, kChainY = 16, kChainZ = 32;
-constexpr int kFibersPerWGChain = 256 * 4;  // 4 rounds: measured 3 % faster than 8 or 12
+constexpr int kMaxRoundsChain = 4;  // measured 3 % faster than 8 or 12
 struct ChainGroup {
   int64_t nfib, wg0;
   int32_t fdim[kMaxModes];     // extents of the shared modes (1 past nf)
@@ -281,8 +283,8 @@ hipError_t launch_fiber_chain(hipStream_t s, int cplx, int nf, int xm, int ym,
                               const ChainGroup* groups, const FiberSlot* slots,
                               const FiberOutElem* zouts, const uint32_t* ymask,
                               const FiberCoef* coefs1, const FiberCoef* coefs2,
-                              const int32_t* wg_group, int64_t total_wgs, const void* X,
-                              const void* B1, const void* B2, void* Z);
+                              const int32_t* wg_group, int64_t total_wgs, int rounds,
+                              const void* X, const void* B1, const void* B2, void* Z);
 
 // Block-sparse tensor times a block-diagonal one (DiagBlockSparse: blocks
 // (k, ..., k) storing only their diagonals), grouped over the output

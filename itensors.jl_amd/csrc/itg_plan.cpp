@@ -226,6 +226,40 @@ int64_t uf_find(std::vector<int64_t>& par, int64_t x) {
   return x;
 }
 
+// Rounds of kFiberThreads fibers per workgroup for the groups of a matrix-form
+// or chain launch: the most (up to `most`, halving) that still make
+// kFiberWgs workgroups, four for each CU of the chip. More rounds spread the
+// building of W and overlap each round's loads with the one before; with
+// fewer workgroups than that, the rounds of one run in series beside idle
+// CUs. Always 8 rounds (4 for chains) -> this rule, MI355X: one real step of
+// 16384 fibers 24.1 -> 5.8 us, the four steps of a chi = 1024 U(1) gradient
+// 58 -> 39 us, two steps of 256 dense networks of chi 16 to 96 154 -> 149 us;
+// launches beyond 2M fibers are as they were.
+constexpr int64_t kFiberWgs = 1024;
+template <class G>
+int fiber_rounds(const std::vector<G>& groups, int most) {
+  for (int r = most; r > 1; r /= 2) {
+    int64_t n = 0;
+    for (const G& g : groups) n += (g.nfib + r * kFiberThreads - 1) / (r * kFiberThreads);
+    if (n >= kFiberWgs) return r;
+  }
+  return 1;
+}
+
+// Sets each group's first workgroup and appends its index per workgroup to
+// *wgg; returns the number of workgroups.
+template <class G>
+int64_t fiber_workgroups(std::vector<G>* groups, int rounds, std::vector<int32_t>* wgg) {
+  int64_t wgs = 0;
+  for (size_t g = 0; g < groups->size(); ++g) {
+    G& grp = (*groups)[g];
+    grp.wg0 = wgs;
+    wgs += (grp.nfib + rounds * kFiberThreads - 1) / (rounds * kFiberThreads);
+    wgg->resize((size_t)wgs, (int32_t)g);
+  }
+  return wgs;
+}
+
 // Matrix-form FIBER tables (see FiberMVGroup) for the groups comp_granges.
 // Returns "" when built, "-" when the form does not apply (then nothing is
 // set), or an error message.
@@ -245,7 +279,7 @@ std::string build_fiber_mv(const Structure& st, const BlockList& TA, const Block
   std::vector<FiberOutElem> outs;
   std::vector<FiberCoef> coefs;
   std::vector<int32_t> wgg;
-  int64_t wgs = 0, total_fib = 0;
+  int64_t total_fib = 0;
   int smax = 1;
   for (size_t c = 0; c < comp_granges.size(); ++c) {
     FiberMVGroup& G = groups[c];
@@ -363,18 +397,17 @@ std::string build_fiber_mv(const Structure& st, const BlockList& TA, const Block
     G.nw = (int32_t)(coefs.size() - G.w0);
     if (G.nslot > kFiberSlots || G.nout > kFiberOuts || G.nslot < 1) return "-";
     smax = std::max(smax, (int)G.nslot);
-    G.wg0 = wgs;
-    const int64_t n = (nfib + kFibersPerWGMV - 1) / kFibersPerWGMV;
-    for (int64_t w = 0; w < n; ++w) wgg.push_back((int32_t)c);
-    wgs += n;
     total_fib += nfib;
   }
   if (total_fib < 256) return "-";
+  const int rounds = fiber_rounds(groups, kMaxRoundsMV);
+  const int64_t wgs = fiber_workgroups(&groups, rounds, &wgg);
   if (coefs.empty()) coefs.push_back(FiberCoef{});
   if (wgg.empty()) wgg.push_back(0);
   ep->f_a_is_2 = a2;
   ep->f_nf = nf;
   ep->f_wgs = wgs;
+  ep->f_rounds = rounds;
   ep->f_mv = true;
   ep->f_smax = smax <= 4 ? 4 : (smax <= 8 ? 8 : kFiberSlots);
   ep->hfm_groups = groups;
@@ -1671,7 +1704,7 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
       e = launch_fiber_mv(s, cplx, ep.f_nf, ep.f_smax, (const FiberMVGroup*)ep.fm_groups.p,
                           (const FiberSlot*)ep.fm_slots.p, (const FiberOutElem*)ep.fm_outs.p,
                           (const FiberCoef*)ep.fm_coefs.p, (const int32_t*)ep.f_wgg.p, ep.f_wgs,
-                          A, B, R, fl, a_re, a_im, b_re, b_im);
+                          ep.f_rounds, A, B, R, fl, a_re, a_im, b_re, b_im);
     } else {
       TimeScope ts(kt, "fiber_kernel", s);
       e = launch_fiber(s, cplx, ep.f_nf, (const FiberGroup*)ep.f_groups.p,
@@ -1938,7 +1971,6 @@ std::string build_fiber_chain(const ExecPlan& e1, const ExecPlan& e2, hipStream_
   std::vector<uint32_t> ymask;
   std::vector<FiberCoef> coefs1, coefs2;
   std::vector<int32_t> wgg;
-  int64_t wgs = 0;
   int xmax = 1, ymax = 1;
   for (auto& kv : comps) {
     const std::vector<size_t>& G1 = kv.second.first;
@@ -2033,10 +2065,6 @@ std::string build_fiber_chain(const ExecPlan& e1, const ExecPlan& e2, hipStream_
     if (C.nz == 0 || C.nz > kChainZ || C.ny == 0) return "-";
     xmax = std::max(xmax, (int)C.nx);
     ymax = std::max(ymax, (int)C.ny);
-    C.wg0 = wgs;
-    const int64_t n = (C.nfib + kFibersPerWGChain - 1) / kFibersPerWGChain;
-    for (int64_t w = 0; w < n; ++w) wgg.push_back((int32_t)groups.size());
-    wgs += n;
     groups.push_back(C);
   }
   if (groups.empty()) return "-";
@@ -2045,7 +2073,8 @@ std::string build_fiber_chain(const ExecPlan& e1, const ExecPlan& e2, hipStream_
   cp->nf = std::max(ns, 1);
   cp->xm = xmax <= 8 ? 8 : kChainX;
   cp->ym = ymax <= 8 ? 8 : kChainY;
-  cp->wgs = wgs;
+  cp->rounds = fiber_rounds(groups, kMaxRoundsChain);
+  cp->wgs = fiber_workgroups(&groups, cp->rounds, &wgg);
   hipError_t e;
   if ((e = cp->groups.upload(groups.data(), groups.size() * sizeof(ChainGroup), s)) != hipSuccess ||
       (e = cp->slots.upload(slots.data(), slots.size() * sizeof(FiberSlot), s)) != hipSuccess ||
@@ -2069,8 +2098,8 @@ hipError_t exec_chain(const ChainPlan& cp, int cplx, hipStream_t s, const void* 
     e = launch_fiber_chain(s, cplx, cp.nf, cp.xm, cp.ym, (const ChainGroup*)cp.groups.p,
                            (const FiberSlot*)cp.slots.p, (const FiberOutElem*)cp.zouts.p,
                            (const uint32_t*)cp.ymask.p, (const FiberCoef*)cp.coefs1.p,
-                           (const FiberCoef*)cp.coefs2.p, (const int32_t*)cp.wgg.p, cp.wgs, X, B1,
-                           B2, Z);
+                           (const FiberCoef*)cp.coefs2.p, (const int32_t*)cp.wgg.p, cp.wgs,
+                           cp.rounds, X, B1, B2, Z);
   }
   if (e != hipSuccess) *err = std::string("fiber chain kernel launch: ") + hipGetErrorString(e);
   return e;

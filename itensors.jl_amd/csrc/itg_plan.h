@@ -128,6 +128,7 @@ struct ExecPlan {
   int f_nf = 0;
   int f_smax = 0;     // matrix form: slot bound of the kernel (4, 8 or 16) >= every group's nslot
   int64_t f_wgs = 0;
+  int f_rounds = 1;  // matrix form: rounds of kFiberThreads fibers per workgroup
   DevBuf f_groups, f_outs, f_pairs, f_koffs, f_gofs_c, f_gofs_b, f_wgg;
   DevBuf fm_groups, fm_slots, fm_outs, fm_coefs;
   // host copies of the matrix-form tables and the fiber modes (A mode, R
@@ -253,6 +254,7 @@ struct ChainPlan {
   int nf = 0;            // modes of the fiber index (max of both steps)
   int xm = 0, ym = 0;    // unroll bounds (8 or 16) >= every group's nx / ny
   int64_t wgs = 0;
+  int rounds = 1;
   DevBuf groups, slots, zouts, ymask, coefs1, coefs2, wgg;
 };
 // "" on success, "-" when the two steps cannot be fused (the caller runs

@@ -150,12 +150,11 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // Matrix form: out_o = sum_s a_s W[s][o] per fiber, W of the group in LDS.
-// A workgroup builds W once and then streams kMVRounds rounds of one fiber
+// A workgroup builds W once and then streams `rounds` rounds of one fiber
 // per thread; the slots of the next round are loaded before the outputs of
 // the current one are formed, so every wave keeps its A reads in flight
 // behind its arithmetic and stores. Each A value is read once.
-constexpr int kMVRounds = kFibersPerWGMV / kThreads;
-static_assert(kMVRounds * kThreads == kFibersPerWGMV, "whole rounds per workgroup");
+static_assert(kThreads == kFiberThreads, "one fiber per thread and round");
 
 // SM: slot bound (4, 8 or 16) the slot loops are unrolled for; every group
 // of the launch has nslot <= SM.
@@ -163,9 +162,10 @@ template <int CPLX, int NF, int SM>
 __global__ void __launch_bounds__(kThreads)
     fiber_mv_kernel(const FiberMVGroup* __restrict__ groups, const FiberSlot* __restrict__ slots,
                     const FiberOutElem* __restrict__ outs, const FiberCoef* __restrict__ coefs,
-                    const int32_t* __restrict__ wg_group, const double* __restrict__ A,
-                    const double* __restrict__ B, double* __restrict__ C, unsigned flags,
-                    double ga_re, double ga_im, double beta_re, double beta_im) {
+                    const int32_t* __restrict__ wg_group, int rounds,
+                    const double* __restrict__ A, const double* __restrict__ B,
+                    double* __restrict__ C, unsigned flags, double ga_re, double ga_im,
+                    double beta_re, double beta_im) {
   __shared__ double Wre[kFiberSlots * kFiberOuts];
   __shared__ double Wim[CPLX ? kFiberSlots * kFiberOuts : 1];
   // the group's slot and output descriptors, staged once per workgroup
@@ -214,11 +214,11 @@ __global__ void __launch_bounds__(kThreads)
   }
   __syncthreads();
 
-  const int64_t fbase = (wg - fg.wg0) * kFibersPerWGMV;
+  const int64_t fbase = (wg - fg.wg0) * rounds * kThreads;
   const int64_t flast = fg.nfib - 1;
   // rounds holding at least one fiber of the group (uniform)
   const int64_t left = fg.nfib - fbase;
-  const int nrounds = (int)(left >= kFibersPerWGMV ? kMVRounds : (left + kThreads - 1) / kThreads);
+  const int nrounds = left >= rounds * kThreads ? rounds : (int)((left + kThreads - 1) / kThreads);
 
   // coordinates of fiber f (clamped to the group's last fiber: a dead lane
   // reads valid memory and stores nothing)
@@ -340,12 +340,12 @@ __global__ void __launch_bounds__(kThreads)
 template <int CPLX, int SM>
 hipError_t launch_mv(hipStream_t s, int nf, dim3 grid, const FiberMVGroup* groups,
                      const FiberSlot* slots, const FiberOutElem* outs, const FiberCoef* coefs,
-                     const int32_t* wg_group, const void* A, const void* B, void* C,
+                     const int32_t* wg_group, int rounds, const void* A, const void* B, void* C,
                      unsigned flags, double ar, double ai, double br, double bi) {
 #define ITG_NF_CASE(n)                                                                        \
   case n:                                                                                     \
     ITG_LAUNCH((fiber_mv_kernel<CPLX, n, SM>), grid, dim3(kThreads), 0, s, groups, slots,    \
-               outs, coefs, wg_group, (const double*)A, (const double*)B, (double*)C, flags, \
+               outs, coefs, wg_group, rounds, (const double*)A, (const double*)B, (double*)C, flags, \
                ar, ai, br, bi);                                                               \
     return hipGetLastError();
   switch (nf) {
@@ -366,18 +366,18 @@ hipError_t launch_mv(hipStream_t s, int nf, dim3 grid, const FiberMVGroup* group
 template <int CPLX>
 hipError_t launch_mv_sm(hipStream_t s, int nf, int smax, dim3 grid, const FiberMVGroup* groups,
                         const FiberSlot* slots, const FiberOutElem* outs,
-                        const FiberCoef* coefs, const int32_t* wg_group, const void* A,
+                        const FiberCoef* coefs, const int32_t* wg_group, int rounds, const void* A,
                         const void* B, void* C, unsigned flags, double ar, double ai, double br,
                         double bi) {
   switch (smax) {
     case 4:
-      return launch_mv<CPLX, 4>(s, nf, grid, groups, slots, outs, coefs, wg_group, A, B, C,
+      return launch_mv<CPLX, 4>(s, nf, grid, groups, slots, outs, coefs, wg_group, rounds, A, B, C,
                                 flags, ar, ai, br, bi);
     case 8:
-      return launch_mv<CPLX, 8>(s, nf, grid, groups, slots, outs, coefs, wg_group, A, B, C,
+      return launch_mv<CPLX, 8>(s, nf, grid, groups, slots, outs, coefs, wg_group, rounds, A, B, C,
                                 flags, ar, ai, br, bi);
     case kFiberSlots:
-      return launch_mv<CPLX, kFiberSlots>(s, nf, grid, groups, slots, outs, coefs, wg_group, A,
+      return launch_mv<CPLX, kFiberSlots>(s, nf, grid, groups, slots, outs, coefs, wg_group, rounds, A,
                                           B, C, flags, ar, ai, br, bi);
     default:
       return hipErrorInvalidValue;
@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(kThreads, (!CPLX && XM <= 8 && YM <= 8) ? 5 : 
                        const FiberOutElem* __restrict__ zouts,
                        const uint32_t* __restrict__ ymask, const FiberCoef* __restrict__ coefs1,
                        const FiberCoef* __restrict__ coefs2,
-                       const int32_t* __restrict__ wg_group, const double* __restrict__ X,
+                       const int32_t* __restrict__ wg_group, int rounds, const double* __restrict__ X,
                        const double* __restrict__ B1, const double* __restrict__ B2,
                        double* __restrict__ Z) {
   __shared__ double W1re[kChainY * kChainX];
@@ -462,11 +462,10 @@ __global__ void __launch_bounds__(kThreads, (!CPLX && XM <= 8 && YM <= 8) ? 5 : 
   }
   __syncthreads();
 
-  const int64_t fbase = (wg - cg.wg0) * kFibersPerWGChain;
+  const int64_t fbase = (wg - cg.wg0) * rounds * kThreads;
   const int64_t flast = cg.nfib - 1;
   const int64_t left = cg.nfib - fbase;
-  constexpr int kRounds = kFibersPerWGChain / kThreads;
-  const int nrounds = (int)(left >= kFibersPerWGChain ? kRounds : (left + kThreads - 1) / kThreads);
+  const int nrounds = left >= rounds * kThreads ? rounds : (int)((left + kThreads - 1) / kThreads);
 
   auto coords = [&](int64_t f, uint32_t (&c)[NF]) {
     uint32_t rem = (uint32_t)(f < flast ? f : flast);
@@ -610,12 +609,12 @@ template <int CPLX, int XM, int YM>
 hipError_t launch_chain(hipStream_t s, int nf, dim3 grid, const ChainGroup* groups,
                         const FiberSlot* slots, const FiberOutElem* zouts,
                         const uint32_t* ymask, const FiberCoef* coefs1, const FiberCoef* coefs2,
-                        const int32_t* wg_group, const void* X, const void* B1, const void* B2,
+                        const int32_t* wg_group, int rounds, const void* X, const void* B1, const void* B2,
                         void* Z) {
 #define ITG_NF_CASE(n)                                                                        \
   case n:                                                                                     \
     ITG_LAUNCH((fiber_chain_kernel<CPLX, n, XM, YM>), grid, dim3(kThreads), 0, s, groups,    \
-               slots, zouts, ymask, coefs1, coefs2, wg_group, (const double*)X,               \
+               slots, zouts, ymask, coefs1, coefs2, wg_group, rounds, (const double*)X,               \
                (const double*)B1, (const double*)B2, (double*)Z);                             \
     return hipGetLastError();
   switch (nf) {
@@ -634,20 +633,20 @@ hipError_t launch_chain_xy(hipStream_t s, int nf, int xm, int ym, dim3 grid,
                            const ChainGroup* groups, const FiberSlot* slots,
                            const FiberOutElem* zouts, const uint32_t* ymask,
                            const FiberCoef* coefs1, const FiberCoef* coefs2,
-                           const int32_t* wg_group, const void* X, const void* B1,
+                           const int32_t* wg_group, int rounds, const void* X, const void* B1,
                            const void* B2, void* Z) {
   if (xm == 8 && ym == 8)
     return launch_chain<CPLX, 8, 8>(s, nf, grid, groups, slots, zouts, ymask, coefs1, coefs2,
-                                    wg_group, X, B1, B2, Z);
+                                    wg_group, rounds, X, B1, B2, Z);
   if (xm == kChainX && ym == kChainY)
     return launch_chain<CPLX, kChainX, kChainY>(s, nf, grid, groups, slots, zouts, ymask, coefs1,
-                                                coefs2, wg_group, X, B1, B2, Z);
+                                                coefs2, wg_group, rounds, X, B1, B2, Z);
   if (xm == 8 && ym == kChainY)
     return launch_chain<CPLX, 8, kChainY>(s, nf, grid, groups, slots, zouts, ymask, coefs1,
-                                          coefs2, wg_group, X, B1, B2, Z);
+                                          coefs2, wg_group, rounds, X, B1, B2, Z);
   if (xm == kChainX && ym == 8)
     return launch_chain<CPLX, kChainX, 8>(s, nf, grid, groups, slots, zouts, ymask, coefs1,
-                                          coefs2, wg_group, X, B1, B2, Z);
+                                          coefs2, wg_group, rounds, X, B1, B2, Z);
   return hipErrorInvalidValue;
 }
 
@@ -683,15 +682,15 @@ hipError_t launch_c(hipStream_t s, int nf, dim3 grid, const FiberGroup* groups,
 hipError_t launch_fiber_mv(hipStream_t s, int cplx, int nf, int smax,
                            const FiberMVGroup* groups, const FiberSlot* slots,
                            const FiberOutElem* outs, const FiberCoef* coefs,
-                           const int32_t* wg_group, int64_t total_wgs, const void* A,
+                           const int32_t* wg_group, int64_t total_wgs, int rounds, const void* A,
                            const void* B, void* C, unsigned flags, double ga_re, double ga_im,
                            double beta_re, double beta_im) {
   if (total_wgs == 0) return hipSuccess;
   dim3 grid((unsigned)total_wgs);
   if (cplx)
-    return launch_mv_sm<1>(s, nf, smax, grid, groups, slots, outs, coefs, wg_group, A, B, C,
+    return launch_mv_sm<1>(s, nf, smax, grid, groups, slots, outs, coefs, wg_group, rounds, A, B, C,
                            flags, ga_re, ga_im, beta_re, beta_im);
-  return launch_mv_sm<0>(s, nf, smax, grid, groups, slots, outs, coefs, wg_group, A, B, C, flags,
+  return launch_mv_sm<0>(s, nf, smax, grid, groups, slots, outs, coefs, wg_group, rounds, A, B, C, flags,
                          ga_re, ga_im, beta_re, beta_im);
 }
 
@@ -699,15 +698,15 @@ hipError_t launch_fiber_chain(hipStream_t s, int cplx, int nf, int xm, int ym,
                               const ChainGroup* groups, const FiberSlot* slots,
                               const FiberOutElem* zouts, const uint32_t* ymask,
                               const FiberCoef* coefs1, const FiberCoef* coefs2,
-                              const int32_t* wg_group, int64_t total_wgs, const void* X,
+                              const int32_t* wg_group, int64_t total_wgs, int rounds, const void* X,
                               const void* B1, const void* B2, void* Z) {
   if (total_wgs == 0) return hipSuccess;
   dim3 grid((unsigned)total_wgs);
   if (cplx)
     return launch_chain_xy<1>(s, nf, xm, ym, grid, groups, slots, zouts, ymask, coefs1, coefs2,
-                              wg_group, X, B1, B2, Z);
+                              wg_group, rounds, X, B1, B2, Z);
   return launch_chain_xy<0>(s, nf, xm, ym, grid, groups, slots, zouts, ymask, coefs1, coefs2,
-                            wg_group, X, B1, B2, Z);
+                            wg_group, rounds, X, B1, B2, Z);
 }
 
 hipError_t launch_fiber(hipStream_t s, int cplx, int nf, const FiberGroup* groups,
