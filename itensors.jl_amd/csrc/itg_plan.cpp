@@ -2,6 +2,7 @@
 #include "itg_plan.h"
 
 #include <algorithm>
+#include <functional>
 #include <map>
 #include <unordered_map>
 #include <cstdio>
@@ -1328,45 +1329,67 @@ namespace {
 // 91 -> 113, 2048 x 2048 272 -> 386; 128 x 1280 x 128 (K = 128) 9.4 -> 6.5 us;
 // complex 1024 x 1024 273 -> 289, the chi = 1500 U(1) network's last product
 // 134 -> 112 us.
-bool quarters_faster(const std::vector<std::vector<double>>& cost, int cplx) {
+void quarters_faster(const std::vector<std::vector<double>>& cost, bool faster[2]) {
   constexpr int kCus = 32, kMaxTiles = 256;  // per XCD; beyond 8 tiles a CU whole tiles win
   const double lone[2][3] = {{1.32, 1.23, 1.08}, {1.15, 1.02, 1.0}};
-  const double quarter = cplx ? 1.08 : 1.42;
-  double t_whole = 0.0, t_quarters = 0.0;
+  const double quarter[2] = {1.42, 1.08};
+  double t_whole[2] = {0.0, 0.0}, t_quarters[2] = {0.0, 0.0};
+  faster[0] = faster[1] = false;
+  for (const std::vector<double>& c : cost)
+    if (c.size() > kMaxTiles) return;
   for (const std::vector<double>& c : cost) {
-    if (c.size() > kMaxTiles) return false;
-    double load[kCus] = {0.0}, all = 0.0, longest = 0.0;
-    int n[kCus] = {0};
+    std::pair<double, int> cu[kCus];  // load, tiles: a heap, least load first
+    std::fill(cu, cu + kCus, std::make_pair(0.0, 0));
+    double all = 0.0, longest = 0.0;
     for (double t : c) {
-      const int b = (int)(std::min_element(load, load + kCus) - load);
-      load[b] += t;
-      ++n[b];
+      std::pop_heap(cu, cu + kCus, std::greater<>());
+      cu[kCus - 1].first += t;
+      ++cu[kCus - 1].second;
+      std::push_heap(cu, cu + kCus, std::greater<>());
       all += t;
       longest = std::max(longest, t);
     }
-    for (int b = 0; b < kCus; ++b)
-      if (n[b])
-        t_whole = std::max(t_whole, load[b] * (n[b] <= 3 ? lone[cplx][n[b] - 1] : 1.0));
-    t_quarters = std::max({t_quarters, quarter * all / kCus, 0.97 * longest});
+    for (int x = 0; x < 2; ++x) {
+      for (const auto& u : cu)
+        if (u.second)
+          t_whole[x] =
+              std::max(t_whole[x], u.first * (u.second <= 3 ? lone[x][u.second - 1] : 1.0));
+      t_quarters[x] = std::max({t_quarters[x], quarter[x] * all / kCus, 0.97 * longest});
+    }
   }
-  return t_quarters < 0.9 * t_whole;
+  for (int x = 0; x < 2; ++x) faster[x] = t_quarters[x] < 0.9 * t_whole[x];
+}
+
+// First row and column of tile t of group G, in strips of kStrip tile columns
+// taken row by row; returns its live 16 x 16 blocks.
+constexpr int kStrip = 8;
+int tile_blocks(const GemmGroup& G, GemmTileCfg tc, int32_t t, int* m0, int* n0) {
+  const int tm = (G.M + tc.bm - 1) / tc.bm, tn = (G.N + tc.bn - 1) / tc.bn;
+  const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
+  const int width = std::min(kStrip, tn - strip * kStrip);
+  *m0 = r / width * tc.bm;
+  *n0 = (strip * kStrip + r % width) * tc.bn;
+  return ((std::min(G.M - *m0, tc.bm) + 15) / 16) * ((std::min(G.N - *n0, tc.bn) + 15) / 16);
 }
 }  // namespace
 
 // Workgroup w of a launch is dispatched to XCD w % kXcds. Cut the tiles of
 // every group into chunks (big groups are split so that every XCD gets
-// several chunks), assign chunks to XCDs largest-work-first to the least
-// loaded one, and interleave the per-XCD lists so each XCD runs its own
-// chunks back to back: the tiles of a chunk share their A and B panels
-// through that XCD's L2. A group's tiles are taken in strips of kStrip tile
-// columns, row by row inside a strip, so that the tiles that run together
-// form a patch with few panels: down whole columns, a 4096^3 FP64 product
-// missed L2 for 9 GB. Measured against that order (MI355X): 4096^3 FP64 2.11 ->
-// 2.04 ms, chi = 1536 complex network in split precision 11.8 -> 11.4 ms, the
-// U(1) networks (blocks of at most 7 tiles a side) level; strips of 4 and 16
-// within 1 % of 8.
+// several chunks), assign chunks to XCDs largest-work-first (live 16 x 16
+// blocks times contracted values) to the least loaded one, and interleave the
+// per-XCD lists so each XCD runs its own chunks back to back: the tiles of a
+// chunk share their A and B panels through that XCD's L2. A group's tiles are
+// taken in strips of kStrip tile columns, row by row inside a strip, so that
+// the tiles that run together form a patch with few panels: down whole
+// columns, a 4096^3 FP64 product missed L2 for 9 GB. Measured against that
+// order (MI355X): 4096^3 FP64 2.11 -> 2.04 ms, chi = 1536 complex network in
+// split precision 11.8 -> 11.4 ms, the U(1) networks (blocks of at most 7
+// tiles a side) level; strips of 4 and 16 within 1 % of 8. Counting whole
+// tiles as the work instead of their live blocks left one XCD with 4 % more
+// than its share in the chi = 4096 U(1) network's last product: both products
+// 618 -> 604 us; split precision, which computes whole tiles, is level.
 std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* quarters) {
-  constexpr int kXcds = 8, kStrip = 8;
+  constexpr int kXcds = 8;
   struct Chunk {
     int32_t g, t0, t1;
     double k;     // contracted values of one of its tiles
@@ -1388,7 +1411,12 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* q
     for (int p = ep.h_groups[g].p0; p < ep.h_groups[g].p1; ++p) k += std::max(ep.h_pairs[p].K, 1);
     for (int64_t t0 = 0; t0 < gt[g]; t0 += unit) {
       const int64_t t1 = std::min<int64_t>(gt[g], t0 + unit);
-      chunks.push_back(Chunk{(int32_t)g, (int32_t)t0, (int32_t)t1, k, k * (double)(t1 - t0)});
+      double work = 0.0;
+      for (int64_t t = t0; t < t1; ++t) {
+        int m0, n0;
+        work += tile_blocks(ep.h_groups[g], tc, (int32_t)t, &m0, &n0) * k;
+      }
+      chunks.push_back(Chunk{(int32_t)g, (int32_t)t0, (int32_t)t1, k, work});
     }
   }
   std::stable_sort(chunks.begin(), chunks.end(),
@@ -1410,15 +1438,11 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* q
   for (int x = 0; x < kXcds; ++x)
     for (const Chunk& c : mine[x]) {
       const GemmGroup& G = ep.h_groups[(size_t)c.g];
-      const int tm = (G.M + tc.bm - 1) / tc.bm, tn = (G.N + tc.bn - 1) / tc.bn;
       for (int32_t t = c.t0; t < c.t1; ++t) {
-        const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
-        const int width = std::min(kStrip, tn - strip * kStrip);
-        const GemmTile T{c.g, r / width * tc.bm, (strip * kStrip + r % width) * tc.bn, 0};
+        GemmTile T{c.g, 0, 0, 0};
+        const int blocks = tile_blocks(G, tc, t, &T.m0, &T.n0);
         bins[x].push_back(T);
-        if (quarters)
-          cost[x].push_back((double)((std::min(G.M - T.m0, tc.bm) + 15) / 16) *
-                            ((std::min(G.N - T.n0, tc.bn) + 15) / 16) * c.k);
+        if (quarters) cost[x].push_back(blocks * c.k);
       }
     }
   size_t len = 0;
@@ -1426,8 +1450,7 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* q
   std::vector<GemmTile> table(len * kXcds, GemmTile{-1, 0, 0, 0});
   for (int x = 0; x < kXcds; ++x)
     for (size_t i = 0; i < bins[x].size(); ++i) table[i * kXcds + x] = bins[x][i];
-  if (quarters)
-    for (int cplx = 0; cplx < 2; ++cplx) quarters[cplx] = quarters_faster(cost, cplx);
+  if (quarters) quarters_faster(cost, quarters);
   return table;
 }
 
