@@ -323,7 +323,7 @@ itg_status check_reuse(itg_handle* h, const ExecPlan& ep, int cplx, int prec, co
     const unsigned reuse = op == 0 ? kFlagReuse1 : kFlagReuse2;
     if (!(flags & reuse) || (flags & keep)) continue;
     const int side = ep.swap ? 1 - op : op;
-    if (ep.kept_sets[side] != (cplx ? 3 : 1) || ep.kept_src[side] != (op == 0 ? T1 : T2))
+    if (ep.kept_sets[side] != split_sets(cplx) || ep.kept_src[side] != (op == 0 ? T1 : T2))
       return fail(h, ITG_ERR_INVALID,
                   op == 0 ? "ITG_FLAG_REUSE_SLICES_1: this plan kept no slices of this T1"
                           : "ITG_FLAG_REUSE_SLICES_2: this plan kept no slices of this T2");
@@ -1494,8 +1494,8 @@ itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void*
   std::string err;
   std::vector<int> cands;
   if (prec != ITG_PREC_FP64) {
-    cands = {0, 2};  // split tiles 64 x 64 and 128 x 64
-    if (!cplx) cands.push_back(3);  // 64 x 64 with A in registers
+    cands = {0};
+    if (!cplx) cands = {0, 2, 3};  // 64 x 64, 128 x 64, 64 x 64 with A in registers
   } else {
     cands = {kDefaultCfg};  // the FP64 GEMM has one tile shape
   }

@@ -388,7 +388,7 @@ constexpr double kSliceRadix = 254.0;  // digits in [-127, 127]
 constexpr double kSliceLead = 127.0;   // |first digit| <= 127
 // Longest contracted extent of one pair of the split GEMM: the level sums
 // (at most kSliceCount products of two digits per k) stay below 2^31 in
-// INT32 for 2*K (the complex form stacks two K halves): 6 * 127^2 * 16384 <
+// INT32 for 2*K (a component of a complex product sums two): 6 * 127^2 * 16384 <
 // 2^31. Longer pairs are cut into K chunks summed in FP64.
 constexpr int kSplitKChunk = 8192;
 
@@ -430,25 +430,28 @@ struct SliceOperands {
 };
 // Two launches over the same grid (the blocks of both operands, A's first):
 // partial row maxima (as exponents, into pmax), then the slices (planes) and
-// the row exponents (exps). Complex operands: nsets = 3 slice sets (re, im,
-// -im); plane buffers hold nsets x the per-set bytes.
+// the row exponents (exps). Complex operands have two slice sets (re, im) under
+// one exponent per row; plane buffers hold split_sets() x the per-set bytes.
 // Workgroup w slices tile wgmap[w] = (block, tile index within the block:
 // row tile * kparts + K part).
-hipError_t launch_slice(hipStream_t s, int prec, int cplx, int nsets, const SliceBlock* blocks,
+inline int split_sets(int cplx) { return cplx ? 2 : 1; }
+hipError_t launch_slice(hipStream_t s, int prec, int cplx, const SliceBlock* blocks,
                         const int2* wgmap, int64_t grid, const SliceOperands& ops);
-// Tile shape of the split GEMM: 64 x 64 (wmb = 1, 256 threads, tile table of
-// gemm cfg 0) or 128 x 64 (wmb = 2, 512 threads, tile table of gemm cfg 2).
-// Complex: one launch per output component comp (0 = re, 1 = im); `sets`
-// packs the slice sets (0 re, 1 im, 2 -im) of A and B for the two K halves:
-// bits 0-1 A half 0, 2-3 B half 0, 4-5 A half 1, 6-7 B half 1. Both complex
-// operands are sliced with 3 sets.
-// aim: take each pair's factor from alpha_im instead of alpha (the second
-// pass of a product with complex per-pair factors).
-hipError_t launch_split_gemm(hipStream_t s, int prec, int cplx, int wmb, int comp, int sets,
-                             const SplitPair* pairs, const GemmGroup* groups,
-                             const GemmTile* tiles, int64_t grid, const void* planesA, const void* planesB,
-                             const void* expA, const void* expB, void* C, double ga,
-                             double beta, int aim = 0);
+// Split GEMM of real data. wmb 1: 64 x 64 tiles (tile table of cfg 0); 2: 128 x
+// 64 (cfg 2); 3: 64 x 64 with the A operand in registers (cfg 0).
+hipError_t launch_split_gemm(hipStream_t s, int prec, int wmb, const SplitPair* pairs,
+                             const GemmGroup* groups, const GemmTile* tiles, int64_t grid,
+                             const void* planesA, const void* planesB, const void* expA,
+                             const void* expB, void* C, double ga, double beta);
+// Split GEMM of complex data, 64 x 64 tiles (tile table of cfg 0). conja,
+// conjb: the operand is conjugated. aim: take each pair's factor from
+// alpha_im instead of alpha (the second pass of a product with complex
+// per-pair factors).
+hipError_t launch_split_gemm_cplx(hipStream_t s, int prec, bool conja, bool conjb,
+                                  const SplitPair* pairs, const GemmGroup* groups,
+                                  const GemmTile* tiles, int64_t grid, const void* planesA,
+                                  const void* planesB, const void* expA, const void* expB,
+                                  void* C, double ga, double beta, int aim);
 // x[i] = beta * x[i] for i < n (complex when cplx).
 hipError_t launch_scale(hipStream_t s, int cplx, void* x, int64_t n, double b_re, double b_im);
 // Float32 / ComplexF32 at the boundary: x64[i] = x32[i] (n elements; cplx:

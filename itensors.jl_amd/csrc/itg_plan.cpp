@@ -1248,8 +1248,7 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
     ep->split_kmax = std::max<int64_t>(ep->split_kmax, dA[bp].K);
     const int64_t kpad = dA[bp].K == 0 ? 0 : dA[bp].Kpad;
     first[p] = (int32_t)sp.size();
-    int64_t k0 = 0;
-    do {
+    for (int64_t k0 = 0; k0 < kpad;) {  // none for an empty K
       const int64_t len = std::min<int64_t>(kpad - k0, kSplitKChunk);
       x.a_planes = dA[bp].plane_off;
       x.b_planes = dB[bq].plane_off;
@@ -1258,9 +1257,10 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
       x.kpad = (int32_t)len;
       sp.push_back(x);
       k0 += len;
-    } while (k0 < kpad);
+    }
   }
   first[pairs.size()] = (int32_t)sp.size();
+  if (sp.empty()) sp.push_back(SplitPair{});
   std::vector<GemmGroup> sg(ep->h_groups);
   for (GemmGroup& G : sg) {
     G.p0 = first[G.p0];
@@ -1480,7 +1480,7 @@ size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_c
   if (prec != 0 && ksplit_takes_split_prec(ep)) prec = 0;
   if (prec == 0 && ep.ks_grid > 0) b += align256((size_t)ep.ks_elems * es);
   if (prec != 0 && ep.split_ok) {
-    const size_t ns = cplx ? 3 : 1;
+    const size_t ns = (size_t)split_sets(cplx);
     b += align256((size_t)ep.sA_plane_bytes * ns) + align256((size_t)ep.sB_plane_bytes * ns);
     b += align256((size_t)ep.sA_rows * 4) + align256((size_t)ep.sB_rows * 4);
     b += align256((size_t)ep.sA_pmax * 4) + align256((size_t)ep.sB_pmax * 4);
@@ -1499,20 +1499,6 @@ size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_c
 }
 
 namespace {
-
-// Slice sets of the two K halves of a complex split product (see
-// launch_split_gemm): Re C = Re A Re B - Im A Im B, Im C = Re A Im B + Im A Re B,
-// with Im A -> -Im A under conj(A) and Im B -> -Im B under conj(B).
-int split_sets(int comp, bool conja, bool conjb) {
-  const int ima = conja ? 2 : 1, imb = conjb ? 2 : 1, nimb = conjb ? 1 : 2;
-  int a0, b0, a1, b1;
-  if (comp == 0) {
-    a0 = 0, b0 = 0, a1 = ima, b1 = nimb;
-  } else {
-    a0 = 0, b0 = imb, a1 = ima, b1 = 0;
-  }
-  return a0 | (b0 << 2) | (a1 << 4) | (b1 << 6);
-}
 
 // Brackets the launches made in its lifetime with timer events (no-op when
 // the timer is null).
@@ -1539,7 +1525,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     *err = "this split-precision form is not available";
     return hipErrorNotSupported;
   }
-  const int nsets = cplx ? 3 : 1;
+  const int nsets = split_sets(cplx);
   const void* A = ep.swap ? T2 : T1;
   const void* B = ep.swap ? T1 : T2;
   const bool conja = (flags & (ep.swap ? 2u : 1u)) != 0;
@@ -1597,11 +1583,11 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     const SliceBlock* desc = (const SliceBlock*)ep.s_desc.p;
     TimeScope ts(kt, "slice_max_kernel+slice_kernel", s);
     if (!reuse[0] && !reuse[1])
-      e = launch_slice(s, prec, cplx, nsets, desc, (const int2*)ep.s_wgmap.p, ep.s_grid, ops);
+      e = launch_slice(s, prec, cplx, desc, (const int2*)ep.s_wgmap.p, ep.s_grid, ops);
     else if (!reuse[0])
-      e = launch_slice(s, prec, cplx, nsets, desc, (const int2*)ep.s_wgmap.p, ep.sA_grid, ops);
+      e = launch_slice(s, prec, cplx, desc, (const int2*)ep.s_wgmap.p, ep.sA_grid, ops);
     else
-      e = launch_slice(s, prec, cplx, nsets, desc + ep.sA_blocks, (const int2*)ep.s_wgmapB.p,
+      e = launch_slice(s, prec, cplx, desc + ep.sA_blocks, (const int2*)ep.s_wgmapB.p,
                        ep.sB_grid, ops);
     if (e != hipSuccess) {
       *err = std::string("slice launch: ") + hipGetErrorString(e);
@@ -1613,9 +1599,9 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
       ep.kept_src[side] = side == 0 ? A : B;
       ep.kept_sets[side] = nsets;
     }
-  // cfg 2: 128 x 64 split tiles (three-stage); cfg 3 (real data): 64 x 64
-  // with A in registers; otherwise 64 x 64
-  const int wmb = cfg == 2 ? 2 : (cfg == 3 && !cplx ? 3 : 1);
+  // real data, cfg 2: 128 x 64 split tiles; cfg 3: 64 x 64 with A in
+  // registers; otherwise, and for complex data, 64 x 64
+  const int wmb = cplx ? 1 : (cfg == 2 ? 2 : (cfg == 3 ? 3 : 1));
   const int tcfg = wmb == 2 ? 2 : 0;  // the FP64 tile table of the same shape
   if ((e = ensure_gemm_launch(ep, tcfg, s, may_build)) != hipSuccess) {
     *err = e == hipErrorNotReady ? std::string(kTablesMissing)
@@ -1623,6 +1609,18 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     return e;
   }
   GemmLaunch& gl = *ep.launches[tcfg];
+  // out = ga * sum_p f_p P_p + beta * out, f_p the real (part 0) or imaginary
+  // factors of the pairs
+  auto products = [&](void* out, double ga, double beta, int part) {
+    TimeScope ts(kt, "split_gemm_kernel", s);
+    const SplitPair* pairs = (const SplitPair*)ep.s_pairs.p;
+    const GemmGroup* groups = (const GemmGroup*)ep.s_groups.p;
+    const GemmTile* tiles = (const GemmTile*)gl.tiles.p;
+    return cplx ? launch_split_gemm_cplx(s, prec, conja, conjb, pairs, groups, tiles, gl.grid,
+                                         planesA, planesB, expA, expB, out, ga, beta, part)
+                : launch_split_gemm(s, prec, wmb, pairs, groups, tiles, gl.grid, planesA, planesB,
+                                    expA, expB, out, ga, beta);
+  };
   if (split_cplx_scale(ep, cplx, a_im != 0.0)) {
     // R = alpha * sum_p (a_p + i b_p) P_p + beta * R: the split kernel scales
     // each pair by a real factor, so form S1 = sum_p a_p P_p and S2 =
@@ -1632,13 +1630,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     void* S1 = w;
     void* S2 = ep.cplx_pair_alpha ? (void*)(w + cbytes) : nullptr;
     for (int part = 0; part < (S2 ? 2 : 1) && e == hipSuccess; ++part)
-      for (int comp = 0; comp < 2 && e == hipSuccess; ++comp) {
-        TimeScope ts(kt, "split_gemm_kernel", s);
-        e = launch_split_gemm(s, prec, cplx, wmb, comp, split_sets(comp, conja, conjb),
-                              (const SplitPair*)ep.s_pairs.p, (const GemmGroup*)ep.s_groups.p,
-                              (const GemmTile*)gl.tiles.p, gl.grid, planesA, planesB, expA, expB,
-                              part ? S2 : S1, 1.0, 0.0, part);
-      }
+      e = products(part ? S2 : S1, 1.0, 0.0, part);
     if (e != hipSuccess) {
       *err = std::string("split gemm launch: ") + hipGetErrorString(e);
       return e;
@@ -1678,13 +1670,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     }
     beta_k = 1.0;
   }
-  for (int comp = 0; comp < (cplx ? 2 : 1) && e == hipSuccess; ++comp) {
-    TimeScope ts(kt, "split_gemm_kernel", s);
-    e = launch_split_gemm(s, prec, cplx, wmb, comp, split_sets(comp, conja, conjb),
-                          (const SplitPair*)ep.s_pairs.p, (const GemmGroup*)ep.s_groups.p,
-                          (const GemmTile*)gl.tiles.p, gl.grid, planesA, planesB, expA, expB, C, a_re,
-                          beta_k);
-  }
+  e = products(C, a_re, beta_k, 0);
   if (e != hipSuccess) {
     *err = std::string("split gemm launch: ") + hipGetErrorString(e);
     return e;

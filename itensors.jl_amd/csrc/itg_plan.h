@@ -183,7 +183,7 @@ struct ExecPlan {
   DevBuf s_wgmap, s_wgmapB;
   // digit planes and row exponents kept for a fixed operand (side 0 = A,
   // 1 = B) by ITG_FLAG_KEEP_SLICES_*: the source pointer they were made from
-  // and the number of slice sets (1 real, 3 complex); 0 = none kept
+  // and the number of slice sets (1 real, 2 complex); 0 = none kept
   DevBuf kept[2];
   const void* kept_src[2] = {nullptr, nullptr};
   int kept_sets[2] = {0, 0};

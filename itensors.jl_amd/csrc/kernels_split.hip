@@ -25,8 +25,10 @@
 //    The error is that of the two representations plus the dropped levels
 //    L >= S (same order), about 1e-13 relative Frobenius for N(0,1) data;
 //    no rounding occurs in the products or the INT32 sums.
-// Tiles: 256 threads = 4 wave64s (2x2), (64*WMB) x 64 per workgroup,
-// (32*WMB) x 32 per wave; K steps of 32 (two chunks) double-buffered in LDS.
+//    Complex data have two slice sets per operand (re, im) under one exponent
+//    per row; a kernel of its own forms both components of C in one pass.
+// Tiles: 64 x 64 (or 128 x 64) per workgroup, 32 x 32 per wave64; K steps of 32
+// (two chunks) in a ring of LDS stages.
 // Stages are fetched with global_load_lds_dwordx4 (HBM/L2 -> LDS without
 // registers): one wave instruction moves the 64 rows of one (plane, chunk),
 // issued a full K step ahead of the MFMAs that consume it. In LDS a stage is
@@ -34,6 +36,8 @@
 // l/32) is read with consecutive lanes on consecutive 16-byte slots (no bank
 // conflicts). The MFMA is issued as D = B^T A^T so that each lane's
 // accumulators run down a column of C (contiguous column-major stores).
+#include <utility>
+
 #include "itg_internal.h"
 
 namespace itg {
@@ -267,12 +271,12 @@ __global__ void __launch_bounds__(kThreads)
 
 // Pass 2: row exponent E = max of the row's partials (0 for an all-zero row),
 // then the S slices of every element of the tile.
-// nsets: slice sets written per element -- 1 (real) or 3 (re, im, -im:
-// complex); set s of block b starts at planes + nsets*plane_off + s*S*R*Kpad.
+// Slice sets per element: 1 (real) or 2 (re, im: complex); set s of block b
+// starts at planes + sets*plane_off + s*S*R*Kpad.
 template <int S, int CPLX>
 __global__ void __launch_bounds__(kThreads)
     slice_kernel(const SliceBlock* __restrict__ blocks, const int2* __restrict__ wgmap,
-                 SliceOperands ops, int nsets) {
+                 SliceOperands ops) {
   __shared__ int32_t sexp[kSliceRows];
   __shared__ int64_t srow[kSliceRows];
   const SliceTile t = slice_tile(blocks, wgmap, blockIdx.x);
@@ -309,7 +313,7 @@ __global__ void __launch_bounds__(kThreads)
   constexpr int kItems = kSliceRows * kChunks / kThreads;
   static_assert(kSliceRows * kChunks % kThreads == 0, "items per thread");
   constexpr int NB = CPLX ? 1 : kItems;
-  constexpr int NC = CPLX ? 3 : 1;  // re, im, -im
+  constexpr int NC = CPLX ? 2 : 1;  // re, im
   for (int i0 = 0; i0 < kItems; i0 += NB) {
     double xr[NB][16], xi[NB][CPLX ? 16 : 1];
     int eq[NB], grq[NB], chq[NB];
@@ -355,15 +359,13 @@ __global__ void __launch_bounds__(kThreads)
     for (int q = 0; q < NB; ++q) {
       if (!lq[q]) continue;
       const int e = eq[q];
-      // one slice set at a time (re, then im and -im for complex data: the
-      // digits of -im are those of im negated), so only one set's packed
-      // digits are live: with all three at once the complex kernel needed a
-      // full register file and ran one wave per SIMD
+      // one slice set at a time (re, then im for complex data), so only one
+      // set's packed digits are live: with all at once the complex kernel
+      // needed a full register file and ran one wave per SIMD
       int8_t* dst =
-          planes + (int64_t)nsets * d.plane_off + ((int64_t)chq[q] * d.R + grq[q]) * 16;
+          planes + NC * d.plane_off + ((int64_t)chq[q] * d.R + grq[q]) * 16;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        if (c >= nsets) break;
         uint32_t packed[S][4];
 #pragma unroll
         for (int i = 0; i < S; ++i)
@@ -377,8 +379,7 @@ __global__ void __launch_bounds__(kThreads)
           for (int i = 0; i < S; ++i) {
             const double v = rint(y);
             y = (y - v) * kSliceRadix;
-            const int32_t dg = c == 2 ? -(int32_t)v : (int32_t)v;
-            packed[i][j >> 2] |= ((uint32_t)(dg & 0xff)) << (8 * (j & 3));
+            packed[i][j >> 2] |= ((uint32_t)((int32_t)v & 0xff)) << (8 * (j & 3));
           }
         }
 #pragma unroll
@@ -392,6 +393,7 @@ __global__ void __launch_bounds__(kThreads)
 
 constexpr int BN = 64, BKB = 32;  // BKB: K bytes per LDS stage (two 16-byte chunks)
 
+typedef const __attribute__((address_space(4))) SplitPair* const_pair_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
@@ -401,13 +403,6 @@ __device__ inline void load_lds16(const int8_t* g, v4i* lds_base) {
   __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)lds_base, 16, 0, 0);
 }
 
-// Complex data (CPLX = 1): one launch per output component `comp`; the
-// component is a K-stacked real product over two halves, e.g.
-//   Re C = [Re A | Im A] . [Re B ; -Im B],  Im C = [Re A | Im A] . [Im B ; Re B],
-// with the slice sets of each half packed in `sets` (bits 0-1 / 2-3: A / B
-// set of half 0, bits 4-5 / 6-7: half 1), accumulated into the same INT32
-// levels (both halves share the row and column scales), and written to the
-// interleaved complex output.
 // s_waitcnt vmcnt(N) (expcnt and lgkmcnt left at their maxima).
 template <int N>
 __device__ inline void wait_vmcnt() {
@@ -456,13 +451,13 @@ __device__ inline v4i lds_read16_untracked(uint32_t addr) {
 // still takes three quarters of its time, without its fills a little over
 // half; a stage waits for its slowest load, which an L2 miss makes long, so
 // the ring is as deep as the LDS allows.
-template <int S, int CPLX, int WM>
+template <int S, int WM>
 __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
     split_gemm_kernel(const SplitPair* __restrict__ pairs, const GemmGroup* __restrict__ groups,
                       const GemmTile* __restrict__ tiles, const int8_t* __restrict__ planesA,
                       const int8_t* __restrict__ planesB, const int32_t* __restrict__ expA,
                       const int32_t* __restrict__ expB, double* __restrict__ Cg, double ga,
-                      double beta, int comp, int sets, int nsetsA, int nsetsB, int aim) {
+                      double beta) {
   constexpr int BM = 32 * WM;
   constexpr int NW = 2 * WM;                    // waves
   constexpr int NSTAGE = WM == 2 ? 3 : 4;
@@ -546,22 +541,12 @@ __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
     for (int r = 0; r < 16; ++r)
       eb[r] = expB[pr.b_exp + min(n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh, grp.N - 1)];
 
-    for (int h = 0; h < (CPLX ? 2 : 1); ++h) {
-    // slice sets (0 = re, 1 = im, 2 = -im) of this half, chosen by the host
-    // for the output component and the conj flags
-    if (CPLX) {
-      const int seta = h == 0 ? (sets & 3) : ((sets >> 4) & 3);
-      const int setb = h == 0 ? ((sets >> 2) & 3) : ((sets >> 6) & 3);
-      pa = planesA + (int64_t)nsetsA * pr.a_planes + pr.a_koff + (int64_t)seta * S * pr.a_pstride;
-      pb = planesB + (int64_t)nsetsB * pr.b_planes + pr.b_koff + (int64_t)setb * S * pr.b_pstride;
-    } else {
-      pa = planesA + pr.a_planes + pr.a_koff;
-      pb = planesB + pr.b_planes + pr.b_koff;
-    }
+    pa = planesA + pr.a_planes + pr.a_koff;
+    pb = planesB + pr.b_planes + pr.b_koff;
     // Stage ring: step s computes from stage s % NSTAGE and fetches step
     // s + NSTAGE - 1 into the stage step s - 1 used (every wave finished
     // reading it before the barrier that closed step s - 1). Every wave is
-    // past the previous half's / pair's last barrier, so all stages are free.
+    // past the previous pair's last barrier, so all stages are free.
     const int nsteps = kpad / BKB;
     issue(0, 0);
     int pre = 1;  // stages issued ahead of the first step
@@ -607,7 +592,6 @@ __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
       stage_barrier();
       if (++st == NSTAGE) st = 0;
     }
-    }  // halves
 
     // FP64 recombination of the levels, scaled per row/column
 #pragma unroll
@@ -617,7 +601,7 @@ __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
       for (int L = NL - 2; L >= 0; --L) h = fma(h, kInvRadix, (double)lev[L][r]);
       double v = ldexp(h * kInvLead2, ea + eb[r]);
       if (ea == kNonFinite || eb[r] == kNonFinite) v = __builtin_nan("");
-      acc[r] = fma(ga * (aim ? pr.alpha_im : pr.alpha), v, acc[r]);
+      acc[r] = fma(ga * pr.alpha, v, acc[r]);
     }
   }
 
@@ -627,10 +611,277 @@ __global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
   for (int r = 0; r < 16; ++r) {
     const int gn = n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh;
     if (gn >= grp.N) continue;
-    const int64_t o0 = grp.off_c + gm + (int64_t)gn * grp.ldc;
-    const int64_t o = CPLX ? 2 * o0 + comp : o0;
+    const int64_t o = grp.off_c + gm + (int64_t)gn * grp.ldc;
     double out = acc[r];
     if (beta != 0.0) out = fma(beta, Cg[o], out);
+    Cg[o] = out;
+  }
+}
+
+// f(0), f(1), ... with each argument a compile-time constant.
+template <class F, int... N>
+__device__ __attribute__((always_inline)) inline void static_for(F f,
+                                                                 std::integer_sequence<int, N...>) {
+  (f(std::integral_constant<int, N>{}), ...);
+}
+// The products of S digits by S in the order (0, 0), (0, 1), ..., (0, S - 1),
+// (1, 0), ..., (1, S - 2), ...: number of the first one of digit i of the
+// first factor, and that digit of product n.
+template <int S>
+constexpr int digit_first(int i) {
+  return i * S - i * (i - 1) / 2;
+}
+template <int S>
+constexpr int digit_row(int n) {
+  int i = 0;
+  while (n >= digit_first<S>(i + 1)) ++i;
+  return i;
+}
+
+// Whether dword q of S digits may be negated behind MFMA q + first of two
+// quarters in a row: digit q / 4 after its last product with the old sign
+// (first quarter; `old` false: it has none) and before its first with the new
+// one, in the quarter that starts at MFMA `now`.
+template <int S>
+constexpr bool negation_fits(int first, bool old, int now) {
+  for (int q = 0; q < 4 * S; ++q) {
+    const int i = q / 4, at = q + first;
+    if (old && at < digit_first<S>(i + 1) - 1) return false;
+    if (at >= now + digit_first<S>(i)) return false;
+  }
+  return true;
+}
+
+// The four digits of a dword negated (a digit is at most 127 in magnitude):
+// with l = the low seven bits, each byte is 128 - l with its sign bit flipped
+// where the digit was not negative.
+__device__ inline int negate_digits(int x) {
+  const uint32_t h = 0x80808080u, u = (uint32_t)x;
+  return (int)((~(u | h) + 0x01010101u) ^ (~u & h));
+}
+
+// Complex split GEMM, both components of C in one pass: 64 x 64 tiles, four
+// waves of 32 x 32, one workgroup (one wave per SIMD) per CU. With A = ar + i
+// ai and B = br + i bi a K step forms ar br and -ai bi into the levels of Re
+// C, ar bi and ai br into those of Im C: 84 MFMAs per 24 fragment reads and
+// 48 KB of fills, half of either per MFMA of a pass per component.
+// DIFF: exactly one operand is conjugated (+ai bi, -ai br); negim: Im C is
+// negated (B conjugated).
+// Stages form one sequence over the pairs of the group: step s computes from
+// stage s % 3 and fills step s + 2 into the stage step s - 1 read, also across
+// the end of a pair, so the fills of the next pair run under this one's
+// recombination. The barrier that opens the next stage comes before the last
+// quarter of a step's MFMAs, and the next step's first fragments are read
+// under that quarter.
+// Against a pass per component (a 32 x 32 block of one component per wave, two
+// waves per SIMD), MI355X: 7680 x 1536 x 6144 5.68 -> 4.47 ms, 1000^3 0.101 ->
+// 0.071, 300^3 33 -> 22 us, 2000 x 64 x 2000 51 -> 48 us. It is bound by power:
+// the matrix pipe is busy 73 % of the cycles at 1.8 GHz; the same product of
+// zeros takes 3.36 ms, at 2.4 GHz. Without the negations (4 %) or with the
+// compiler's instruction order (6 % slower) the balance is the same.
+template <int S, bool DIFF>
+__global__ void __launch_bounds__(kThreads, 1)
+    split_gemm_cplx_kernel(const SplitPair* __restrict__ pairs,
+                           const GemmGroup* __restrict__ groups,
+                           const GemmTile* __restrict__ tiles, const int8_t* __restrict__ planesA,
+                           const int8_t* __restrict__ planesB, const int32_t* __restrict__ expA,
+                           const int32_t* __restrict__ expB, double2* __restrict__ Cg, double ga,
+                           double beta, int negim, int aim) {
+  constexpr int BM = 64;
+  constexpr int NSTAGE = 3;
+  constexpr int NL = S;
+  constexpr int OP_ST = 2 * S * 2 * BM;  // 16-byte LDS slots of one operand's stage: [re, im
+                                         // digit planes][chunk][row]
+  constexpr int NLD = 2 * S;             // fills a wave issues per stage (both operands)
+  constexpr int NP = S * (S + 1) / 2;    // digit products of a quarter step
+  static_assert(S + NLD <= NP, "a quarter holds S reads and the fills");
+  // The 4 S dwords of ai are negated one behind each MFMA, in place: from
+  // MFMA kNeg of the third quarter, digit i after its last product there and
+  // before its first in the fourth; with DIFF (third quarter negated, fourth
+  // not) also from MFMA kNegDiff of the second.
+  constexpr int kNeg = S + 1, kNegDiff = S + 2;
+  static_assert(negation_fits<S>(kNeg, true, NP) && negation_fits<S>(kNegDiff, false, NP),
+                "negation order");
+  __shared__ v4i lds[NSTAGE * 2 * OP_ST];
+  // read through the scalar cache (the plan's tables do not change)
+  const const_pair_t ptab = (const_pair_t)(uintptr_t)pairs;
+
+  const GemmTile& tt = tiles[blockIdx.x];
+  if (tt.g < 0) return;
+  const GemmGroup grp = groups[tt.g];
+  const int m0 = tt.m0, n0 = tt.n0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
+  const int l32 = lane & 31, lh = lane >> 5;
+  // rows this lane fetches; rows past the block are clamped onto its last
+  // row (they only feed outputs that are never stored)
+  uint32_t aoff = (uint32_t)min(m0 + lane, grp.M - 1) * 16u;
+  uint32_t boff = (uint32_t)min(n0 + lane, grp.N - 1) * 16u;
+
+  double acc_re[16], acc_im[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc_re[r] = acc_im[r] = 0.0;
+
+  // The fills: pair fp, K byte fk; a wave takes chunk wave & 1 of the digit
+  // planes of parity wave >> 1. Past the last step every lane fetches the
+  // first row of the last pair again, into a stage nobody reads, so that
+  // every step issues the same loads and waits for the same count.
+  int fp = grp.p0, fk = 0, fkpad = 0;
+  const int8_t *fa = nullptr, *fb = nullptr;
+  int64_t fas = 0, fbs = 0;
+  auto open_pair = [&]() {
+    const bool live = fp < grp.p1;
+    const __attribute__((address_space(4))) SplitPair& pr = ptab[live ? fp : grp.p1 - 1];
+    fas = pr.a_pstride;
+    fbs = pr.b_pstride;
+    fa = planesA + 2 * pr.a_planes + pr.a_koff + (wave >> 1) * fas +
+         (int64_t)(wave & 1) * grp.M * 16;
+    fb = planesB + 2 * pr.b_planes + pr.b_koff + (wave >> 1) * fbs +
+         (int64_t)(wave & 1) * grp.N * 16;
+    fk = 0;
+    fkpad = pr.kpad;
+    aoff = live ? aoff : 0u;
+    boff = live ? boff : 0u;
+  };
+  v4i* fst = nullptr;  // slot of (plane wave >> 1, chunk wave & 1) of the stage being filled
+  auto fill_load = [&](int t) {  // load t of 2 S
+    if (t < S)
+      load_lds16(fa + 2 * t * fas + aoff, fst + t * 4 * BM);
+    else
+      load_lds16(fb + 2 * (t - S) * fbs + boff, fst + OP_ST + (t - S) * 4 * BM);
+  };
+  auto fill_next = [&]() {
+    fa += (int64_t)grp.M * BKB;
+    fb += (int64_t)grp.N * BKB;
+    fk += BKB;
+    if (fk >= fkpad) {
+      ++fp;
+      open_pair();
+    }
+  };
+  auto fill = [&](int st) {
+    fst = lds + st * 2 * OP_ST + wave * BM;
+#pragma unroll
+    for (int t = 0; t < NLD; ++t) fill_load(t);
+    fill_next();
+  };
+  // fragment of digit plane i of an operand's stage
+  auto frag = [&](const v4i* op, int i, int w0) { return op[(i * 2 + lh) * BM + w0 + l32]; };
+
+  v4i ar[S], br[S];
+  int st = 0;
+  if (grp.p0 < grp.p1) {
+    open_pair();
+    fill(0);
+    fill(1);
+    wait_vmcnt<NLD>();
+    stage_barrier();
+#pragma unroll
+    for (int i = 0; i < S; ++i) ar[i] = frag(lds, i, wm0);
+#pragma unroll
+    for (int i = 0; i < S; ++i) br[i] = frag(lds + OP_ST, i, wn0);
+  }
+
+  for (int p = grp.p0; p < grp.p1; ++p) {
+    const __attribute__((address_space(4))) SplitPair& pr = ptab[p];
+    const int kpad = pr.kpad;
+    v16i re[NL], im[NL];
+#pragma unroll
+    for (int L = 0; L < NL; ++L) re[L] = im[L] = v16i{0};
+    const int32_t *xa = expA + pr.a_exp, *xb = expB + pr.b_exp;
+    const int ea = xa[(uint32_t)min(m0 + wm0 + l32, grp.M - 1)];
+    int eb[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      eb[r] = xb[(uint32_t)min(n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh, grp.N - 1)];
+
+    for (int k0 = 0; k0 < kpad; k0 += BKB) {
+      const v4i* sA = lds + st * 2 * OP_ST;
+      const v4i* sB = sA + OP_ST;
+      fst = lds + (st == 0 ? 2 : st - 1) * 2 * OP_ST + wave * BM;
+      if (++st == NSTAGE) st = 0;
+      const v4i* nA = lds + st * 2 * OP_ST;
+      const v4i* nB = nA + OP_ST;
+      // One quarter of the step: the digit products a b into lev, with
+      // after(n) issued behind MFMA n. A wave issues in order and an MFMA
+      // keeps the matrix pipe busy for several issues, so reads, fills and
+      // negations placed between MFMAs cost nothing; before a quarter they
+      // would leave the pipe idle (the order is pinned).
+      auto products = [&](const v4i (&a)[S], const v4i (&b)[S], v16i (&lev)[NL],
+                          auto after) __attribute__((always_inline)) {
+        static_for([&](auto n) __attribute__((always_inline)) {
+          constexpr int i = digit_row<S>(n), j = n - digit_first<S>(i);
+          lev[i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j], a[i], lev[i + j], 0, 0, 0);
+          after(n);
+          __builtin_amdgcn_sched_barrier(0);
+        }, std::make_integer_sequence<int, S * (S + 1) / 2>{});
+      };
+      v4i ai[S], bi[S];
+      // dword q of the 4 S dwords of ai
+      auto negate = [&](auto q) __attribute__((always_inline)) {
+        if constexpr (q >= 0 && q < 4 * S) ai[q / 4][q % 4] = negate_digits(ai[q / 4][q % 4]);
+      };
+      products(ar, br, re, [&](auto n) __attribute__((always_inline)) {
+        if constexpr (n < S) bi[n] = frag(sB, S + n, wn0);
+      });
+      products(ar, bi, im, [&](auto n) __attribute__((always_inline)) {
+        if constexpr (n < S)
+          ai[n] = frag(sA, S + n, wm0);
+        else if constexpr (n < S + NLD)
+          fill_load(n - S);
+        if constexpr (DIFF) negate(std::integral_constant<int, n - kNegDiff>{});
+      });
+      products(ai, br, im, [&](auto n) __attribute__((always_inline)) {
+        if constexpr (DIFF) negate(std::integral_constant<int, n + NP - kNegDiff>{});
+        negate(std::integral_constant<int, n - kNeg>{});
+      });
+      fill_next();
+      wait_vmcnt<NLD>();
+      stage_barrier();
+      // the next step's first fragments (past the last step: a stage nobody
+      // reads, values unused)
+      products(ai, bi, re, [&](auto n) __attribute__((always_inline)) {
+        if constexpr (n < S)
+          ar[n] = frag(nA, n, wm0);
+        else if constexpr (n < 2 * S)
+          br[n - S] = frag(nB, n - S, wn0);
+        negate(std::integral_constant<int, n + NP - kNeg>{});
+      });
+    }
+
+    // FP64 recombination of the levels, scaled per row/column
+    const double al = ga * (aim ? pr.alpha_im : pr.alpha);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      auto join = [&](const v16i (&lev)[NL]) {
+        double h = (double)lev[NL - 1][r];
+#pragma unroll
+        for (int L = NL - 2; L >= 0; --L) h = fma(h, kInvRadix, (double)lev[L][r]);
+        const double v = ldexp(h * kInvLead2, ea + eb[r]);
+        return (ea == kNonFinite || eb[r] == kNonFinite) ? __builtin_nan("") : v;
+      };
+      const double vr = join(re), vi = join(im);
+      acc_re[r] = fma(al, vr, acc_re[r]);
+      acc_im[r] = fma(al, negim ? -vi : vi, acc_im[r]);
+      __builtin_amdgcn_sched_barrier(0);  // one output at a time: few registers
+    }
+  }
+  wait_vmcnt<0>();  // no fill outlives the workgroup
+
+  const int gm = m0 + wm0 + l32;
+  if (gm >= grp.M) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int gn = n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh;
+    if (gn >= grp.N) continue;
+    const int64_t o = grp.off_c + gm + (int64_t)gn * grp.ldc;
+    double2 out = make_double2(acc_re[r], acc_im[r]);
+    if (beta != 0.0) {
+      const double2 c = Cg[o];
+      out.x = fma(beta, c.x, out.x);
+      out.y = fma(beta, c.y, out.y);
+    }
     Cg[o] = out;
   }
 }
@@ -805,7 +1056,7 @@ __global__ void __launch_bounds__(128, 1)
 
 int split_slices(int prec) { return prec == 2 ? kSliceCount : 0; }
 
-hipError_t launch_slice(hipStream_t s, int prec, int cplx, int nsets, const SliceBlock* blocks,
+hipError_t launch_slice(hipStream_t s, int prec, int cplx, const SliceBlock* blocks,
                         const int2* wgmap, int64_t grid, const SliceOperands& ops) {
   if (grid == 0) return hipSuccess;
   if (prec != 2) return hipErrorNotSupported;
@@ -814,12 +1065,12 @@ hipError_t launch_slice(hipStream_t s, int prec, int cplx, int nsets, const Slic
     ITG_LAUNCH((slice_max_kernel<1>), g, blk, 0, s, blocks, wgmap, ops);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    ITG_LAUNCH((slice_kernel<kSliceCount, 1>), g, blk, 0, s, blocks, wgmap, ops, nsets);
+    ITG_LAUNCH((slice_kernel<kSliceCount, 1>), g, blk, 0, s, blocks, wgmap, ops);
   } else {
     ITG_LAUNCH((slice_max_kernel<0>), g, blk, 0, s, blocks, wgmap, ops);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    ITG_LAUNCH((slice_kernel<kSliceCount, 0>), g, blk, 0, s, blocks, wgmap, ops, 1);
+    ITG_LAUNCH((slice_kernel<kSliceCount, 0>), g, blk, 0, s, blocks, wgmap, ops);
   }
   return hipGetLastError();
 }
@@ -828,45 +1079,48 @@ int64_t slice_block_wgs(int32_t rows, int32_t kparts) {
   return (int64_t)((rows + kSliceRows - 1) / kSliceRows) * kparts;
 }
 
-namespace {
-template <int CPLX, int WM>
-hipError_t launch_sg(hipStream_t s, int comp, int sets, const SplitPair* pairs,
-                     const GemmGroup* groups, const GemmTile* tiles, int64_t grid,
-                     const void* planesA, const void* planesB, const void* expA,
-                     const void* expB, void* C, double ga, double beta, int aim) {
-  const int ns = CPLX ? 3 : 1;
-  ITG_LAUNCH((split_gemm_kernel<kSliceCount, CPLX, WM>), dim3((unsigned)grid),
-                     dim3(128 * WM), 0, s, pairs, groups, tiles, (const int8_t*)planesA,
-                     (const int8_t*)planesB, (const int32_t*)expA, (const int32_t*)expB,
-                     (double*)C, ga, beta, CPLX ? comp : 0, CPLX ? sets : 0, ns, ns, aim);
-  return hipGetLastError();
-}
-}  // namespace
-
-hipError_t launch_split_gemm(hipStream_t s, int prec, int cplx, int wmb, int comp, int sets,
-                             const SplitPair* pairs, const GemmGroup* groups, const GemmTile* tiles,
-                             int64_t grid, const void* planesA, const void* planesB,
-                             const void* expA, const void* expB, void* C, double ga,
-                             double beta, int aim) {
+hipError_t launch_split_gemm(hipStream_t s, int prec, int wmb, const SplitPair* pairs,
+                             const GemmGroup* groups, const GemmTile* tiles, int64_t grid,
+                             const void* planesA, const void* planesB, const void* expA,
+                             const void* expB, void* C, double ga, double beta) {
   if (grid == 0) return hipSuccess;
   if (prec != 2) return hipErrorNotSupported;
-  if (wmb == 3) {  // A in registers (real data; 64 x 64 tile table)
-    if (cplx || aim) return hipErrorInvalidValue;
-    ITG_LAUNCH((split_gemm_areg_kernel<kSliceCount>), dim3((unsigned)grid), dim3(128), 0,
-                       s, pairs, groups, tiles, (const int8_t*)planesA, (const int8_t*)planesB,
-                       (const int32_t*)expA, (const int32_t*)expB, (double*)C, ga, beta);
-    return hipGetLastError();
-  }
-  if (wmb != 1 && wmb != 2) return hipErrorInvalidValue;
-  if (cplx)
-    return wmb == 2 ? launch_sg<1, 4>(s, comp, sets, pairs, groups, tiles, grid, planesA, planesB,
-                                      expA, expB, C, ga, beta, aim)
-                    : launch_sg<1, 2>(s, comp, sets, pairs, groups, tiles, grid, planesA, planesB,
-                                      expA, expB, C, ga, beta, aim);
-  return wmb == 2 ? launch_sg<0, 4>(s, comp, sets, pairs, groups, tiles, grid, planesA, planesB,
-                                    expA, expB, C, ga, beta, aim)
-                  : launch_sg<0, 2>(s, comp, sets, pairs, groups, tiles, grid, planesA, planesB,
-                                    expA, expB, C, ga, beta, aim);
+  const dim3 g((unsigned)grid);
+  const int8_t *pa = (const int8_t*)planesA, *pb = (const int8_t*)planesB;
+  const int32_t *ea = (const int32_t*)expA, *eb = (const int32_t*)expB;
+  double* c = (double*)C;
+  if (wmb == 3)
+    ITG_LAUNCH((split_gemm_areg_kernel<kSliceCount>), g, dim3(128), 0, s, pairs, groups, tiles, pa,
+               pb, ea, eb, c, ga, beta);
+  else if (wmb == 2)
+    ITG_LAUNCH((split_gemm_kernel<kSliceCount, 4>), g, dim3(512), 0, s, pairs, groups, tiles, pa,
+               pb, ea, eb, c, ga, beta);
+  else if (wmb == 1)
+    ITG_LAUNCH((split_gemm_kernel<kSliceCount, 2>), g, dim3(256), 0, s, pairs, groups, tiles, pa,
+               pb, ea, eb, c, ga, beta);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t launch_split_gemm_cplx(hipStream_t s, int prec, bool conja, bool conjb,
+                                  const SplitPair* pairs, const GemmGroup* groups,
+                                  const GemmTile* tiles, int64_t grid, const void* planesA,
+                                  const void* planesB, const void* expA, const void* expB,
+                                  void* C, double ga, double beta, int aim) {
+  if (grid == 0) return hipSuccess;
+  if (prec != 2) return hipErrorNotSupported;
+#define ITG_LAUNCH_CPLX(DIFF)                                                                 \
+  ITG_LAUNCH((split_gemm_cplx_kernel<kSliceCount, DIFF>), dim3((unsigned)grid), dim3(kThreads), \
+             0, s, pairs, groups, tiles, (const int8_t*)planesA, (const int8_t*)planesB,      \
+             (const int32_t*)expA, (const int32_t*)expB, (double2*)C, ga, beta, (int)conjb,   \
+             aim)
+  if (conja != conjb)
+    ITG_LAUNCH_CPLX(true);
+  else
+    ITG_LAUNCH_CPLX(false);
+#undef ITG_LAUNCH_CPLX
+  return hipGetLastError();
 }
 
 }  // namespace itg
