@@ -110,11 +110,9 @@ itg_status itg_synchronize(itg_handle* h);
 const char* itg_version(void);
 
 /* Tile shape of the split-precision GEMM for later contractions on this
- * handle: 0 = per plan (the autotuned shape, else chosen by size),
- * 1 = 64 x 64, 2 = 128 x 64, 3 = 64 x 64 with the A operand held in
- * registers (real data; complex plans use 1). All shapes give the same
- * result bit for bit. No counterpart in NDTensors, whose BLAS call has no
- * tile shape; for tests and tuning. ITG_ERR_INVALID outside 0..3. */
+ * handle, 0..3: there is one shape, 64 x 64, so every value selects it. No
+ * counterpart in NDTensors, whose BLAS call has no tile shape.
+ * ITG_ERR_INVALID outside 0..3. */
 itg_status itg_set_split_tile(itg_handle* h, int tile);
 
 /* Kernel family of the contractions planned on this handle from now on (a
@@ -471,9 +469,9 @@ itg_status itg_batch_plan_destroy(itg_batch_plan* p);
 
 /* ------------------------------------------------------------- autotuner */
 
-/* Time the GEMM tile shapes on this plan's pairs and keep the fastest for
- * this plan and (dtype, prec); plans not tuned themselves use the choice
- * cached for their (shape bucket, dtype, prec). Synchronises the stream. */
+/* Prepare the plan for (dtype, prec): runs it once, R = T1*T2, so that its
+ * launch tables and the workspace exist, and waits. The GEMM kernels have one
+ * tile shape each, so there is nothing to choose. Synchronises the stream. */
 itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype,
                            void* R, const void* T1, const void* T2, itg_prec prec);
 

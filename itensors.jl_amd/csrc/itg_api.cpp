@@ -58,9 +58,6 @@ struct itg_handle {
   // dense plan cache (LRU)
   std::list<std::pair<std::string, std::unique_ptr<ExecPlan>>> dense_lru;
   std::unordered_map<std::string, decltype(dense_lru)::iterator> dense_map;
-  // autotuned tile cfg per (bucket, cplx, prec)
-  std::map<std::string, int> tuned;
-  int split_tile = 0;  // itg_set_split_tile (0 = per plan)
   int backend = kBackendAuto;  // itg_set_gemm_backend: plans created from now on
   int bs_order = ITG_BS_ORDER_SEQUENTIAL;  // itg_set_blocksparse_order: likewise
   // itg_graph_begin / _end: the stream being captured, and the caller's
@@ -269,15 +266,6 @@ struct DeviceGuard {
   }
 };
 
-std::string tune_key(const ExecPlan& ep, int cplx, int prec) {
-  // bucket by the log2 of the largest block dim and the transpose form
-  int b = 0;
-  while ((int64_t(1) << b) < ep.max_dim && b < 40) ++b;
-  char buf[96];
-  std::snprintf(buf, sizeof buf, "b%d_c%d_p%d_t%d%d", b, cplx, prec, ep.ta, ep.tb);
-  return buf;
-}
-
 // The handle's timer while timing is on and the stream is not being captured.
 KernelTimer* active_timer(itg_handle* h) {
   if (!h->timing || !h->timer) return nullptr;
@@ -285,14 +273,6 @@ KernelTimer* active_timer(itg_handle* h) {
   if (hipStreamIsCapturing(h->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
     return nullptr;
   return h->timer.get();
-}
-
-int pick_cfg(itg_handle* h, const ExecPlan& ep, int cplx, int prec) {
-  if (prec != 0 && h->split_tile > 0) return h->split_tile == 1 ? 0 : h->split_tile;
-  if (ep.tuned[cplx][prec] >= 0) return ep.tuned[cplx][prec];
-  auto it = h->tuned.find(tune_key(ep, cplx, prec));
-  if (it != h->tuned.end()) return it->second;
-  return kDefaultCfg;
 }
 
 itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void* T1,
@@ -303,8 +283,7 @@ itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void*
   hipError_t e = ensure_ws(h, exec_workspace_bytes(ep, cplx, prec, a_im != 0.0));
   if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
   std::string err;
-  const int cfg = pick_cfg(h, ep, cplx, prec);
-  e = exec_run(ep, cplx, prec, cfg, h->stream, h->ws, T1, T2, R, flags, a_re, a_im, b_re, b_im,
+  e = exec_run(ep, cplx, prec, h->stream, h->ws, T1, T2, R, flags, a_re, a_im, b_re, b_im,
                &err, active_timer(h));
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
@@ -420,8 +399,7 @@ itg_status bs_execute_on(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void* R
     return fail(h, ITG_ERR_INVALID, msg);
   }
   std::string err;
-  const int cfg = pick_cfg(h, *ep, cplx, (int)prec);
-  hipError_t e = exec_run(*ep, cplx, (int)prec, cfg, h->stream, ws, T1, T2, R, flags, a_re, a_im,
+  hipError_t e = exec_run(*ep, cplx, (int)prec, h->stream, ws, T1, T2, R, flags, a_re, a_im,
                           0.0, 0.0, &err, nullptr, false);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e == hipErrorNotReady) return fail(h, ITG_ERR_INVALID, err);
@@ -577,7 +555,6 @@ itg_status itg_synchronize(itg_handle* h) {
 
 itg_status itg_set_split_tile(itg_handle* h, int tile) {
   if (!h || tile < 0 || tile > 3) return ITG_ERR_INVALID;
-  h->split_tile = tile;
   return ITG_OK;
 }
 
@@ -1483,46 +1460,12 @@ itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void*
   if (prec != ITG_PREC_FP64 && !ep.split_ok) return ITG_OK;
   hipError_t e = ensure_ws(h, exec_workspace_bytes(ep, cplx, (int)prec));
   if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
-  hipEvent_t t0, t1;
-  if ((e = hipEventCreate(&t0)) != hipSuccess) return hip_fail(h, e, "event");
-  if ((e = hipEventCreate(&t1)) != hipSuccess) {
-    (void)hipEventDestroy(t0);
-    return hip_fail(h, e, "event");
-  }
-  int best = -1;
-  float best_ms = 1e30f;
   std::string err;
-  std::vector<int> cands;
-  if (prec != ITG_PREC_FP64) {
-    cands = {0};
-    if (!cplx) cands = {0, 2, 3};  // 64 x 64, 128 x 64, 64 x 64 with A in registers
-  } else {
-    cands = {kDefaultCfg};  // the FP64 GEMM has one tile shape
-  }
-  for (int cfg : cands) {
-    // warm-up, then 3 timed runs
-    e = exec_run(ep, cplx, (int)prec, cfg, h->stream, h->ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err);
-    if (e != hipSuccess) break;
-    (void)hipEventRecord(t0, h->stream);
-    for (int r = 0; r < 3; ++r)
-      (void)exec_run(ep, cplx, (int)prec, cfg, h->stream, h->ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err);
-    (void)hipEventRecord(t1, h->stream);
-    (void)hipEventSynchronize(t1);
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, t0, t1);
-    if (ms < best_ms) {
-      best_ms = ms;
-      best = cfg;
-    }
-  }
-  (void)hipEventDestroy(t0);
-  (void)hipEventDestroy(t1);
+  e = exec_run(ep, cplx, (int)prec, h->stream, h->ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
-  if (best >= 0) {
-    h->tuned[tune_key(ep, cplx, (int)prec)] = best;  // for plans not tuned themselves
-    ep.tuned[cplx][(int)prec] = best;
-  }
+  if ((e = hipStreamSynchronize(h->stream)) != hipSuccess)
+    return hip_fail(h, e, "hipStreamSynchronize");
   return ITG_OK;
 }
 

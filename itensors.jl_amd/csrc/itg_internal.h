@@ -334,11 +334,7 @@ struct GemmTile {
   int32_t m0, n0;  // first row / column
   int32_t pad;
 };
-// Tile shapes by cfg: 0 = 64 x 64 (FP64 and split GEMM), 2 = 128 x 64 (split).
-struct GemmTileCfg {
-  int bm, bn;
-};
-GemmTileCfg gemm_cfg(int cfg);
+constexpr int kGemmTile = 64;  // rows and columns of a tile (FP64 and split GEMM)
 hipError_t launch_gemm_f64(hipStream_t s, int cplx, int ta, int tb, const GemmPair* pairs,
                            const GemmGroup* groups, const GemmTile* tiles, int64_t entries,
                            bool quarters, const void* A, const void* B, void* C, unsigned flags,
@@ -437,14 +433,12 @@ struct SliceOperands {
 inline int split_sets(int cplx) { return cplx ? 2 : 1; }
 hipError_t launch_slice(hipStream_t s, int prec, int cplx, const SliceBlock* blocks,
                         const int2* wgmap, int64_t grid, const SliceOperands& ops);
-// Split GEMM of real data. wmb 1: 64 x 64 tiles (tile table of cfg 0); 2: 128 x
-// 64 (cfg 2); 3: 64 x 64 with the A operand in registers (cfg 0).
-hipError_t launch_split_gemm(hipStream_t s, int prec, int wmb, const SplitPair* pairs,
+// Split GEMM of real data.
+hipError_t launch_split_gemm(hipStream_t s, int prec, const SplitPair* pairs,
                              const GemmGroup* groups, const GemmTile* tiles, int64_t grid,
                              const void* planesA, const void* planesB, const void* expA,
                              const void* expB, void* C, double ga, double beta);
-// Split GEMM of complex data, 64 x 64 tiles (tile table of cfg 0). conja,
-// conjb: the operand is conjugated. aim: take each pair's factor from
+// Split GEMM of complex data. conja, conjb: the operand is conjugated. aim: take each pair's factor from
 // alpha_im instead of alpha (the second pass of a product with complex
 // per-pair factors).
 hipError_t launch_split_gemm_cplx(hipStream_t s, int prec, bool conja, bool conjb,

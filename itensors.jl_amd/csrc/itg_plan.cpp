@@ -779,7 +779,7 @@ std::string build_ksplit(ExecPlan* ep, hipStream_t s) {
   ExecPlan tab;
   tab.h_groups = sg;
   tab.h_pairs = sp;
-  std::vector<GemmTile> tiles_tab = xcd_tile_table(tab, gemm_cfg(0), nullptr);
+  std::vector<GemmTile> tiles_tab = xcd_tile_table(tab, nullptr);
   // skinny: (entry, first row) per workgroup, 256 rows of the long side
   std::vector<int2> rows;
   if (skinny)
@@ -1302,16 +1302,16 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
   return "";
 }
 
-hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, hipStream_t s, bool may_build) {
-  if (ep.launches.count(cfg)) return hipSuccess;
+hipError_t ensure_gemm_launch(ExecPlan& ep, hipStream_t s, bool may_build) {
+  if (ep.launch) return hipSuccess;
   if (!may_build) return hipErrorNotReady;
   std::unique_ptr<GemmLaunch> gl(new GemmLaunch);
-  std::vector<GemmTile> table = xcd_tile_table(ep, gemm_cfg(cfg), gl->quarters);
+  std::vector<GemmTile> table = xcd_tile_table(ep, gl->quarters);
   gl->grid = (int64_t)table.size();
   hipError_t e;
   if ((e = gl->tiles.upload(table.data(), table.size() * sizeof(GemmTile), s)) != hipSuccess)
     return e;
-  ep.launches[cfg] = std::move(gl);
+  ep.launch = std::move(gl);
   return hipSuccess;
 }
 
@@ -1363,13 +1363,13 @@ void quarters_faster(const std::vector<std::vector<double>>& cost, bool faster[2
 // First row and column of tile t of group G, in strips of kStrip tile columns
 // taken row by row; returns its live 16 x 16 blocks.
 constexpr int kStrip = 8;
-int tile_blocks(const GemmGroup& G, GemmTileCfg tc, int32_t t, int* m0, int* n0) {
-  const int tm = (G.M + tc.bm - 1) / tc.bm, tn = (G.N + tc.bn - 1) / tc.bn;
+int tile_blocks(const GemmGroup& G, int32_t t, int* m0, int* n0) {
+  const int tm = (G.M + kGemmTile - 1) / kGemmTile, tn = (G.N + kGemmTile - 1) / kGemmTile;
   const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
   const int width = std::min(kStrip, tn - strip * kStrip);
-  *m0 = r / width * tc.bm;
-  *n0 = (strip * kStrip + r % width) * tc.bn;
-  return ((std::min(G.M - *m0, tc.bm) + 15) / 16) * ((std::min(G.N - *n0, tc.bn) + 15) / 16);
+  *m0 = r / width * kGemmTile;
+  *n0 = (strip * kStrip + r % width) * kGemmTile;
+  return ((std::min(G.M - *m0, kGemmTile) + 15) / 16) * ((std::min(G.N - *n0, kGemmTile) + 15) / 16);
 }
 }  // namespace
 
@@ -1388,7 +1388,7 @@ int tile_blocks(const GemmGroup& G, GemmTileCfg tc, int32_t t, int* m0, int* n0)
 // tiles as the work instead of their live blocks left one XCD with 4 % more
 // than its share in the chi = 4096 U(1) network's last product: both products
 // 618 -> 604 us; split precision, which computes whole tiles, is level.
-std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* quarters) {
+std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, bool* quarters) {
   constexpr int kXcds = 8;
   struct Chunk {
     int32_t g, t0, t1;
@@ -1402,7 +1402,7 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* q
     const GemmGroup& G = ep.h_groups[g];
     gt[g] = (G.M <= 0 || G.N <= 0)
                 ? 0
-                : ((G.M + tc.bm - 1) / tc.bm) * ((G.N + tc.bn - 1) / tc.bn);
+                : ((G.M + kGemmTile - 1) / kGemmTile) * ((G.N + kGemmTile - 1) / kGemmTile);
     total += gt[g];
   }
   const int64_t unit = std::max<int64_t>(1, (total + 8 * kXcds - 1) / (8 * kXcds));
@@ -1414,7 +1414,7 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* q
       double work = 0.0;
       for (int64_t t = t0; t < t1; ++t) {
         int m0, n0;
-        work += tile_blocks(ep.h_groups[g], tc, (int32_t)t, &m0, &n0) * k;
+        work += tile_blocks(ep.h_groups[g], (int32_t)t, &m0, &n0) * k;
       }
       chunks.push_back(Chunk{(int32_t)g, (int32_t)t0, (int32_t)t1, k, work});
     }
@@ -1440,7 +1440,7 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* q
       const GemmGroup& G = ep.h_groups[(size_t)c.g];
       for (int32_t t = c.t0; t < c.t1; ++t) {
         GemmTile T{c.g, 0, 0, 0};
-        const int blocks = tile_blocks(G, tc, t, &T.m0, &T.n0);
+        const int blocks = tile_blocks(G, t, &T.m0, &T.n0);
         bins[x].push_back(T);
         if (quarters) cost[x].push_back(blocks * c.k);
       }
@@ -1513,7 +1513,7 @@ struct TimeScope {
   }
 };
 
-hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, void* ws,
+hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                       const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                       double a_im, double b_re, double b_im, std::string* err,
                       KernelTimer* kt, bool may_build) {
@@ -1599,16 +1599,12 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
       ep.kept_src[side] = side == 0 ? A : B;
       ep.kept_sets[side] = nsets;
     }
-  // real data, cfg 2: 128 x 64 split tiles; cfg 3: 64 x 64 with A in
-  // registers; otherwise, and for complex data, 64 x 64
-  const int wmb = cplx ? 1 : (cfg == 2 ? 2 : (cfg == 3 ? 3 : 1));
-  const int tcfg = wmb == 2 ? 2 : 0;  // the FP64 tile table of the same shape
-  if ((e = ensure_gemm_launch(ep, tcfg, s, may_build)) != hipSuccess) {
+  if ((e = ensure_gemm_launch(ep, s, may_build)) != hipSuccess) {
     *err = e == hipErrorNotReady ? std::string(kTablesMissing)
                                  : std::string("gemm table upload: ") + hipGetErrorString(e);
     return e;
   }
-  GemmLaunch& gl = *ep.launches[tcfg];
+  GemmLaunch& gl = *ep.launch;
   // out = ga * sum_p f_p P_p + beta * out, f_p the real (part 0) or imaginary
   // factors of the pairs
   auto products = [&](void* out, double ga, double beta, int part) {
@@ -1618,7 +1614,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
     const GemmTile* tiles = (const GemmTile*)gl.tiles.p;
     return cplx ? launch_split_gemm_cplx(s, prec, conja, conjb, pairs, groups, tiles, gl.grid,
                                          planesA, planesB, expA, expB, out, ga, beta, part)
-                : launch_split_gemm(s, prec, wmb, pairs, groups, tiles, gl.grid, planesA, planesB,
+                : launch_split_gemm(s, prec, pairs, groups, tiles, gl.grid, planesA, planesB,
                                     expA, expB, out, ga, beta);
   };
   if (split_cplx_scale(ep, cplx, a_im != 0.0)) {
@@ -1687,7 +1683,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, 
 
 }  // namespace
 
-hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, void* ws,
+hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err, KernelTimer* kt,
                     bool may_build) {
@@ -1726,7 +1722,7 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
     return e;
   }
   if (prec != 0 && !ksplit_takes_split_prec(ep))
-    return exec_split(ep, cplx, prec, cfg, s, ws, T1, T2, R, flags, a_re, a_im, b_re, b_im, err,
+    return exec_split(ep, cplx, prec, s, ws, T1, T2, R, flags, a_re, a_im, b_re, b_im, err,
                       kt, may_build);
   const size_t es = cplx ? 16 : 8;
   char* w = (char*)ws;
@@ -1797,12 +1793,12 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
       return e;
     }
   } else {
-  if ((e = ensure_gemm_launch(ep, kDefaultCfg, s, may_build)) != hipSuccess) {
+  if ((e = ensure_gemm_launch(ep, s, may_build)) != hipSuccess) {
     *err = e == hipErrorNotReady ? std::string(kTablesMissing)
                                  : std::string("gemm table upload: ") + hipGetErrorString(e);
     return e;
   }
-  GemmLaunch& gl = *ep.launches[kDefaultCfg];
+  GemmLaunch& gl = *ep.launch;
   {
     TimeScope ts(kt, "gemm_f64_kernel", s);
     e = launch_gemm_f64(s, cplx, ep.ta, ep.tb, (const GemmPair*)ep.g_pairs.p,

@@ -109,7 +109,7 @@ struct PermuteLaunch {
   DevBuf blocks, prefix;
 };
 
-// Workgroup table of a tile shape (FP64: gemm cfg 0; split: cfg 0 or 2).
+// Workgroup table of a plan's GEMM (FP64 and split).
 struct GemmLaunch {
   int64_t grid = 0;   // entries, idle padding included
   bool quarters[2] = {false, false};  // FP64, real / complex: 32 x 32 workgroups
@@ -147,8 +147,7 @@ struct ExecPlan {
   std::vector<GemmPair> h_pairs;
   std::vector<GemmGroup> h_groups;
   std::vector<double> group_cost;  // flops per group (for LPT ordering)
-  std::map<int, std::unique_ptr<GemmLaunch>> launches;  // per tile cfg
-  int tuned[2][3] = {{-1, -1, -1}, {-1, -1, -1}};      // autotuned cfg per (complex, prec)
+  std::unique_ptr<GemmLaunch> launch;
   // split-K form (FP64): few output tiles over long contracted extents; the
   // K range of each output block is cut into slices whose partial sums go
   // to the workspace (ks_elems elements) and are added by the reduce kernel
@@ -222,15 +221,13 @@ void build_permute_tables(PermuteLaunch* pl, int n, const int* perm, const Block
 // alpha_cplx: the call's alpha has a nonzero imaginary part.
 size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_cplx = false);
 // kt (optional) brackets each launch with timer events. may_build = false:
-// the launch tables of the tile shape must already exist (built by an
-// earlier run with the same element type and precision); the call then
+// the launch table must already exist (built by an earlier run); the call then
 // allocates no device memory and fails with hipErrorNotReady otherwise.
-hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, void* ws,
+hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err,
                     KernelTimer* kt = nullptr, bool may_build = true);
-// Tile shape of plans that were not tuned: 64x64, FP64 and split precision
-// alike, whatever the block size.
+// Builds the plan's tile table once (kGemmTile square tiles for every plan).
 // FP64, timed on MI355X against the other shapes (128x128, 128x64, 64x128
 // real; 128x64 complex): the fastest or within 3 % of it for the two-site
 // network's GEMMs at chi = 1024 (one 5120 x 4096 x 1024 block), the chi = 4096
@@ -238,15 +235,14 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, int cfg, hipStream_t s, vo
 // 128x64 0.74), the 256-network batch and a 4096^3 product (2.04-2.11 ms,
 // 128x128 1.99-2.07): the padding and the last wave of large tiles cost more
 // than the panels they save.
-// Split, 64x64 (two workgroups per CU, three LDS stages) against 128x64 (one,
-// four): U(1) chi = 4096 0.43 against 0.51 ms for the two GEMMs, dense complex
-// chi = 1536 11.8 against 12.1 ms, 3001 x 777 x 500 0.039 against 0.046 ms,
-// 4096^3 1.36 against 1.38 ms.
-constexpr int kDefaultCfg = 0;
-hipError_t ensure_gemm_launch(ExecPlan& ep, int cfg, hipStream_t s, bool may_build = true);
-// XCD-balanced tile table for tile shape tc. quarters (optional, two values):
+// Split, against 128x64 (eight waves) and 64x64 with the A operand in
+// registers (two waves): U(1) chi = 4096 0.345 against 0.49 and 0.47 ms for the
+// two GEMMs, 4096^3 1.08 against 1.24 and 1.16, 1000^3 22 against 41 and 37 us,
+// 1100 x 8000 x 1100 0.22 against 0.28 and 0.235.
+hipError_t ensure_gemm_launch(ExecPlan& ep, hipStream_t s, bool may_build = true);
+// XCD-balanced tile table. quarters (optional, two values):
 // whether the FP64 GEMM should run it as quarter tiles (real, complex).
-std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, GemmTileCfg tc, bool* quarters);
+std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, bool* quarters);
 
 // Two consecutive matrix-form fiber contractions run as one pass (see
 // ChainGroup). Built from the two steps' plans; the device tables live here.

@@ -918,8 +918,6 @@ hipError_t launch_ksplit_skinny(hipStream_t s, int cplx, int kc, int ta, int tb,
   return hipGetLastError();
 }
 
-GemmTileCfg gemm_cfg(int cfg) { return GemmTileCfg{cfg == 2 ? 128 : 64, 64}; }
-
 hipError_t launch_gemm_f64(hipStream_t s, int cplx, int ta, int tb, const GemmPair* pairs,
                            const GemmGroup* groups, const GemmTile* tiles, int64_t entries,
                            bool quarters, const void* A, const void* B, void* C, unsigned flags, double ga_re, double ga_im,

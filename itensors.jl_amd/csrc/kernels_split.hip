@@ -27,7 +27,7 @@
 //    no rounding occurs in the products or the INT32 sums.
 //    Complex data have two slice sets per operand (re, im) under one exponent
 //    per row; a kernel of its own forms both components of C in one pass.
-// Tiles: 64 x 64 (or 128 x 64) per workgroup, 32 x 32 per wave64; K steps of 32
+// Tiles: 64 x 64 per workgroup of four waves, 32 x 32 per wave64; K steps of 32
 // (two chunks) in a ring of LDS stages.
 // Stages are fetched with global_load_lds_dwordx4 (HBM/L2 -> LDS without
 // registers): one wave instruction moves the 64 rows of one (plane, chunk),
@@ -391,7 +391,8 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-constexpr int BN = 64, BKB = 32;  // BKB: K bytes per LDS stage (two 16-byte chunks)
+constexpr int kBT = kGemmTile;  // rows and columns of a workgroup's tile
+constexpr int BKB = 32;  // K bytes per LDS stage (two 16-byte chunks)
 
 typedef const __attribute__((address_space(4))) SplitPair* const_pair_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -424,200 +425,6 @@ __device__ inline void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// s_waitcnt lgkmcnt(0) alone.
-__device__ inline void wait_lgkmcnt0() {
-  __builtin_amdgcn_s_waitcnt(0xF | (7 << 4) | (0 << 8) | (3 << 14));
-}
-
-// 16-byte LDS read that the compiler does not track. The compiler's wait
-// insertion makes every LDS read it knows of wait for every outstanding
-// global->LDS fill, including fills of stages nobody reads yet, which
-// flattens a multi-stage ring. The caller waits itself: the stage was
-// completed by an explicit vmcnt wait and barrier, and the destination
-// registers are used only after an explicit wait_lgkmcnt0() that the caller
-// pins with a sched_barrier.
-__device__ inline v4i lds_read16_untracked(uint32_t addr) {
-  v4i v;
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
-  return v;
-}
-
-// WM waves along M (the tile is (32*WM) x 64, 2*WM waves, one 32x32 block
-// each). WM = 2: 64 x 64 tiles, three LDS stages of 24 KB (each fetched two
-// K steps ahead), two workgroups per CU. WM = 4: 128 x 64 tiles, four LDS
-// stages of 36 KB (144 KB, each fetched three K steps ahead), one workgroup
-// (eight waves) per CU. Either way a SIMD runs two waves. The fills bound
-// this kernel more than the matrix cores do: with its MFMAs taken out it
-// still takes three quarters of its time, without its fills a little over
-// half; a stage waits for its slowest load, which an L2 miss makes long, so
-// the ring is as deep as the LDS allows.
-template <int S, int WM>
-__global__ void __launch_bounds__(128 * WM, WM == 2 ? 2 : 1)
-    split_gemm_kernel(const SplitPair* __restrict__ pairs, const GemmGroup* __restrict__ groups,
-                      const GemmTile* __restrict__ tiles, const int8_t* __restrict__ planesA,
-                      const int8_t* __restrict__ planesB, const int32_t* __restrict__ expA,
-                      const int32_t* __restrict__ expB, double* __restrict__ Cg, double ga,
-                      double beta) {
-  constexpr int BM = 32 * WM;
-  constexpr int NW = 2 * WM;                    // waves
-  constexpr int NSTAGE = WM == 2 ? 3 : 4;
-  constexpr int RB = BM / 64;                   // 64-row blocks of the A tile
-  constexpr int NL = S;                         // levels 0..S-1
-  constexpr int A_ST = S * 2 * BM;              // 16-byte LDS slots of one A stage
-  constexpr int B_ST = S * 2 * BN;
-  constexpr int NLD_A = S * 2 * RB;             // wave loads (64 rows x 16 bytes) per A stage
-  constexpr int NLD = NLD_A + S * 2;
-  constexpr int NLD_W = (NLD + NW - 1) / NW;    // most loads a wave issues per stage
-  constexpr int PER = NLD / NW;                 // fewest loads a wave issues per stage
-  // wait until the loads of every stage but the newest `n` have landed (a
-  // wave issuing more than PER per stage waits a little longer than needed)
-  auto wait_newer = [](int n) {
-    if (n >= 2)
-      wait_vmcnt<2 * PER>();
-    else if (n == 1)
-      wait_vmcnt<PER>();
-    else
-      wait_vmcnt<0>();
-  };
-  static_assert(NSTAGE - 2 <= 2, "wait_newer covers at most two newer stages");
-  __shared__ v4i lds[NSTAGE * (A_ST + B_ST)];
-
-  const GemmTile& tt = tiles[blockIdx.x];
-  if (tt.g < 0) return;
-  const GemmGroup grp = groups[tt.g];
-  const int m0 = tt.m0, n0 = tt.n0;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm0 = (wave % WM) * 32, wn0 = (wave / WM) * 32;
-  const int l32 = lane & 31, lh = lane >> 5;
-  // B row fetched by this lane; rows past the block are clamped onto its
-  // last row (they only feed outputs that are never stored)
-  const int brow = min(n0 + lane, grp.N - 1);
-
-  // this lane's outputs: m = m0+wm0+l32 ; n = n0+wn0+(r%4)+8*(r/4)+4*lh
-  double acc[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0;
-
-  for (int p = grp.p0; p < grp.p1; ++p) {
-    const SplitPair pr = pairs[p];
-    const int kpad = pr.kpad;
-    if (kpad <= 0) continue;
-    const int8_t* pa = planesA;
-    const int8_t* pb = planesB;
-    v16i lev[NL];
-#pragma unroll
-    for (int L = 0; L < NL; ++L) lev[L] = v16i{0};
-
-    // the NLD wave loads of the stage at K byte k0, into LDS stage `st`;
-    // wave w issues loads w, w+NW, ...
-    auto issue = [&](int k0, int st) {
-      v4i* sA = lds + st * (A_ST + B_ST);
-      v4i* sB = sA + A_ST;
-      const int c0 = k0 >> 4;
-#pragma unroll
-      for (int t = 0; t < NLD_W; ++t) {
-        const int q = wave + NW * t;
-        if (q >= NLD) break;
-        if (q < NLD_A) {
-          const int rb = q % RB, ch = (q / RB) & 1, pl = q / (2 * RB);
-          const int row = min(m0 + rb * 64 + lane, grp.M - 1);
-          load_lds16(pa + pl * pr.a_pstride + ((int64_t)(c0 + ch) * grp.M + row) * 16,
-                     sA + (pl * 2 + ch) * BM + rb * 64);
-        } else {
-          const int r = q - NLD_A, ch = r & 1, pl = r >> 1;
-          load_lds16(pb + pl * pr.b_pstride + ((int64_t)(c0 + ch) * grp.N + brow) * 16,
-                     sB + (pl * 2 + ch) * BN);
-        }
-      }
-    };
-
-    // this lane's row and column exponents, fetched before the K loop so
-    // that their latency hides under it (indices clamped into the block: a
-    // row or column past the block only feeds outputs that are not stored)
-    const int ea = expA[pr.a_exp + min(m0 + wm0 + l32, grp.M - 1)];
-    int eb[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      eb[r] = expB[pr.b_exp + min(n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh, grp.N - 1)];
-
-    pa = planesA + pr.a_planes + pr.a_koff;
-    pb = planesB + pr.b_planes + pr.b_koff;
-    // Stage ring: step s computes from stage s % NSTAGE and fetches step
-    // s + NSTAGE - 1 into the stage step s - 1 used (every wave finished
-    // reading it before the barrier that closed step s - 1). Every wave is
-    // past the previous pair's last barrier, so all stages are free.
-    const int nsteps = kpad / BKB;
-    issue(0, 0);
-    int pre = 1;  // stages issued ahead of the first step
-    for (; pre < NSTAGE - 1 && pre < nsteps; ++pre) issue(pre * BKB, pre);
-    wait_newer(pre - 1);  // stage 0 landed
-    stage_barrier();
-    int st = 0;
-    for (int s = 0; s < nsteps; ++s) {
-      const v4i* sA = lds + st * (A_ST + B_ST);
-      const v4i* sB = sA + A_ST;
-      // the fill of a later stage first, then the fragments in the order the
-      // MFMAs consume them (A slice 0, the B slices, A slices 1..): the first
-      // MFMA waits for two LDS reads, not fourteen, so a wave's reads overlap
-      // the other waves' MFMAs
-      const int nxt = s + NSTAGE - 1;
-      int nst = st + NSTAGE - 1;
-      if (nst >= NSTAGE) nst -= NSTAGE;
-      if (nxt < nsteps) issue(nxt * BKB, nst);
-      v4i bv[S], av[S];
-      av[0] = sA[lh * BM + wm0 + l32];
-#pragma unroll
-      for (int j = 0; j < S; ++j) bv[j] = sB[(j * 2 + lh) * BN + wn0 + l32];
-#pragma unroll
-      for (int i = 1; i < S; ++i) av[i] = sA[(i * 2 + lh) * BM + wm0 + l32];
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-#pragma unroll
-        for (int j = 0; j < S - i; ++j)  // slice i of A with slice j of B, level i+j
-          lev[i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv[j], av[i], lev[i + j], 0, 0, 0);
-      // All 2S fragment reads are issued before the first MFMA, each into its
-      // own registers, and waited for once. Left to itself the scheduler
-      // reuses one register set for the A slices and waits for every read
-      // with lgkmcnt(0) between MFMA groups, draining the matrix pipe.
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * S, 0);       // DS reads
-      __builtin_amdgcn_sched_group_barrier(0x008, S * (S + 1) / 2, 0);  // MFMAs
-      // The MFMAs only touch registers, so without this fence the scheduler
-      // sinks them below the wait for the next stage, which then serialises
-      // the fetch with the math.
-      __builtin_amdgcn_sched_barrier(0);
-      // stage s + 1 must have landed; the stages issued after it may stay in
-      // flight
-      wait_newer(min(nsteps - 1, s + NSTAGE - 1) - (s + 1));
-      stage_barrier();
-      if (++st == NSTAGE) st = 0;
-    }
-
-    // FP64 recombination of the levels, scaled per row/column
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      double h = (double)lev[NL - 1][r];
-#pragma unroll
-      for (int L = NL - 2; L >= 0; --L) h = fma(h, kInvRadix, (double)lev[L][r]);
-      double v = ldexp(h * kInvLead2, ea + eb[r]);
-      if (ea == kNonFinite || eb[r] == kNonFinite) v = __builtin_nan("");
-      acc[r] = fma(ga * pr.alpha, v, acc[r]);
-    }
-  }
-
-  const int gm = m0 + wm0 + l32;
-  if (gm >= grp.M) return;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int gn = n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh;
-    if (gn >= grp.N) continue;
-    const int64_t o = grp.off_c + gm + (int64_t)gn * grp.ldc;
-    double out = acc[r];
-    if (beta != 0.0) out = fma(beta, Cg[o], out);
-    Cg[o] = out;
-  }
-}
-
 // f(0), f(1), ... with each argument a compile-time constant.
 template <class F, int... N>
 __device__ __attribute__((always_inline)) inline void static_for(F f,
@@ -637,6 +444,83 @@ constexpr int digit_row(int n) {
   while (n >= digit_first<S>(i + 1)) ++i;
   return i;
 }
+
+// The stages of a workgroup's 64 x 64 tile, filled as one sequence over the
+// pairs of its group. A stage holds K bytes k..k+31 of the digit planes of
+// both operands, [operand][plane][chunk][row] x 16 bytes, SETS * S planes per
+// operand; wave w of four fetches chunk w & 1 of the planes of parity w >> 1.
+// Past the last step every lane fetches the first row of the last pair again,
+// into a stage nobody reads, so that every step issues the same loads and
+// waits for the same count. The group has at least one pair.
+template <int S, int SETS>
+struct StageFill {
+  static constexpr int kPlanes = SETS * S;
+  static constexpr int kLoads = kPlanes;              // a wave's, per stage
+  static constexpr int kOperand = kPlanes * 2 * kBT;  // 16-byte slots of one operand
+  static constexpr int kStage = 2 * kOperand;
+  const const_pair_t pairs;
+  const int8_t *planesA, *planesB;
+  const int M, N, p1, wave;
+  int p;              // pair, K byte and padded K of the stage to fill next
+  int k, kpad;
+  const int8_t *a, *b;
+  int64_t as, bs;     // plane strides
+  uint32_t aoff, boff;  // this lane's row: rows past the block are clamped onto its last
+                        // row (they only feed outputs that are never stored)
+  v4i* dst;
+
+  __device__ __attribute__((always_inline)) StageFill(const SplitPair* tab, const GemmGroup& g,
+                                                      const int8_t* pa, const int8_t* pb, int m0,
+                                                      int n0, int lane, int w)
+      : pairs((const_pair_t)(uintptr_t)tab), planesA(pa), planesB(pb), M(g.M), N(g.N), p1(g.p1),
+        wave(w), p(g.p0), k(0), kpad(0), a(nullptr), b(nullptr), as(0), bs(0),
+        aoff((uint32_t)min(m0 + lane, g.M - 1) * 16u),
+        boff((uint32_t)min(n0 + lane, g.N - 1) * 16u), dst(nullptr) {}
+  __device__ __attribute__((always_inline)) void open() {
+    const bool live = p < p1;
+    const __attribute__((address_space(4))) SplitPair& pr = pairs[live ? p : p1 - 1];
+    as = pr.a_pstride;
+    bs = pr.b_pstride;
+    a = planesA + SETS * pr.a_planes + pr.a_koff + (wave >> 1) * as + (int64_t)(wave & 1) * M * 16;
+    b = planesB + SETS * pr.b_planes + pr.b_koff + (wave >> 1) * bs + (int64_t)(wave & 1) * N * 16;
+    k = 0;
+    kpad = pr.kpad;
+    aoff = live ? aoff : 0u;
+    boff = live ? boff : 0u;
+  }
+  __device__ __attribute__((always_inline)) void stage(v4i* st) { dst = st + wave * kBT; }
+  // load t of kLoads into the stage
+  __device__ __attribute__((always_inline)) void load(int t) const {
+    constexpr int h = kPlanes / 2;
+    if (t < h)
+      load_lds16(a + 2 * t * as + aoff, dst + t * 4 * kBT);
+    else
+      load_lds16(b + 2 * (t - h) * bs + boff, dst + kOperand + (t - h) * 4 * kBT);
+  }
+  __device__ __attribute__((always_inline)) void next() {
+    a += (int64_t)M * BKB;
+    b += (int64_t)N * BKB;
+    k += BKB;
+    if (k >= kpad) {
+      ++p;
+      open();
+    }
+  }
+  // both stages ahead of the first step; the first has landed on return
+  __device__ __attribute__((always_inline)) void begin(v4i* lds) {
+    open();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      stage(lds + i * kStage);
+#pragma unroll
+      for (int t = 0; t < kLoads; ++t) load(t);
+      next();
+    }
+    wait_vmcnt<kLoads>();
+    stage_barrier();
+  }
+};
+constexpr int kRing = 3;  // LDS stages
 
 // Whether dword q of S digits may be negated behind MFMA q + first of two
 // quarters in a row: digit q / 4 after its last product with the old sign
@@ -687,12 +571,8 @@ __global__ void __launch_bounds__(kThreads, 1)
                            const int8_t* __restrict__ planesB, const int32_t* __restrict__ expA,
                            const int32_t* __restrict__ expB, double2* __restrict__ Cg, double ga,
                            double beta, int negim, int aim) {
-  constexpr int BM = 64;
-  constexpr int NSTAGE = 3;
-  constexpr int NL = S;
-  constexpr int OP_ST = 2 * S * 2 * BM;  // 16-byte LDS slots of one operand's stage: [re, im
-                                         // digit planes][chunk][row]
-  constexpr int NLD = 2 * S;             // fills a wave issues per stage (both operands)
+  using Fill = StageFill<S, 2>;
+  constexpr int NLD = Fill::kLoads, NL = S;
   constexpr int NP = S * (S + 1) / 2;    // digit products of a quarter step
   static_assert(S + NLD <= NP, "a quarter holds S reads and the fills");
   // The 4 S dwords of ai are negated one behind each MFMA, in place: from
@@ -702,9 +582,7 @@ __global__ void __launch_bounds__(kThreads, 1)
   constexpr int kNeg = S + 1, kNegDiff = S + 2;
   static_assert(negation_fits<S>(kNeg, true, NP) && negation_fits<S>(kNegDiff, false, NP),
                 "negation order");
-  __shared__ v4i lds[NSTAGE * 2 * OP_ST];
-  // read through the scalar cache (the plan's tables do not change)
-  const const_pair_t ptab = (const_pair_t)(uintptr_t)pairs;
+  __shared__ v4i lds[kRing * Fill::kStage];
 
   const GemmTile& tt = tiles[blockIdx.x];
   if (tt.g < 0) return;
@@ -714,77 +592,27 @@ __global__ void __launch_bounds__(kThreads, 1)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
   const int l32 = lane & 31, lh = lane >> 5;
-  // rows this lane fetches; rows past the block are clamped onto its last
-  // row (they only feed outputs that are never stored)
-  uint32_t aoff = (uint32_t)min(m0 + lane, grp.M - 1) * 16u;
-  uint32_t boff = (uint32_t)min(n0 + lane, grp.N - 1) * 16u;
+  Fill fill(pairs, grp, planesA, planesB, m0, n0, lane, wave);
 
   double acc_re[16], acc_im[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc_re[r] = acc_im[r] = 0.0;
 
-  // The fills: pair fp, K byte fk; a wave takes chunk wave & 1 of the digit
-  // planes of parity wave >> 1. Past the last step every lane fetches the
-  // first row of the last pair again, into a stage nobody reads, so that
-  // every step issues the same loads and waits for the same count.
-  int fp = grp.p0, fk = 0, fkpad = 0;
-  const int8_t *fa = nullptr, *fb = nullptr;
-  int64_t fas = 0, fbs = 0;
-  auto open_pair = [&]() {
-    const bool live = fp < grp.p1;
-    const __attribute__((address_space(4))) SplitPair& pr = ptab[live ? fp : grp.p1 - 1];
-    fas = pr.a_pstride;
-    fbs = pr.b_pstride;
-    fa = planesA + 2 * pr.a_planes + pr.a_koff + (wave >> 1) * fas +
-         (int64_t)(wave & 1) * grp.M * 16;
-    fb = planesB + 2 * pr.b_planes + pr.b_koff + (wave >> 1) * fbs +
-         (int64_t)(wave & 1) * grp.N * 16;
-    fk = 0;
-    fkpad = pr.kpad;
-    aoff = live ? aoff : 0u;
-    boff = live ? boff : 0u;
-  };
-  v4i* fst = nullptr;  // slot of (plane wave >> 1, chunk wave & 1) of the stage being filled
-  auto fill_load = [&](int t) {  // load t of 2 S
-    if (t < S)
-      load_lds16(fa + 2 * t * fas + aoff, fst + t * 4 * BM);
-    else
-      load_lds16(fb + 2 * (t - S) * fbs + boff, fst + OP_ST + (t - S) * 4 * BM);
-  };
-  auto fill_next = [&]() {
-    fa += (int64_t)grp.M * BKB;
-    fb += (int64_t)grp.N * BKB;
-    fk += BKB;
-    if (fk >= fkpad) {
-      ++fp;
-      open_pair();
-    }
-  };
-  auto fill = [&](int st) {
-    fst = lds + st * 2 * OP_ST + wave * BM;
-#pragma unroll
-    for (int t = 0; t < NLD; ++t) fill_load(t);
-    fill_next();
-  };
   // fragment of digit plane i of an operand's stage
-  auto frag = [&](const v4i* op, int i, int w0) { return op[(i * 2 + lh) * BM + w0 + l32]; };
+  auto frag = [&](const v4i* op, int i, int w0) { return op[(i * 2 + lh) * kBT + w0 + l32]; };
 
   v4i ar[S], br[S];
   int st = 0;
   if (grp.p0 < grp.p1) {
-    open_pair();
-    fill(0);
-    fill(1);
-    wait_vmcnt<NLD>();
-    stage_barrier();
+    fill.begin(lds);
 #pragma unroll
     for (int i = 0; i < S; ++i) ar[i] = frag(lds, i, wm0);
 #pragma unroll
-    for (int i = 0; i < S; ++i) br[i] = frag(lds + OP_ST, i, wn0);
+    for (int i = 0; i < S; ++i) br[i] = frag(lds + Fill::kOperand, i, wn0);
   }
 
   for (int p = grp.p0; p < grp.p1; ++p) {
-    const __attribute__((address_space(4))) SplitPair& pr = ptab[p];
+    const __attribute__((address_space(4))) SplitPair& pr = fill.pairs[p];
     const int kpad = pr.kpad;
     v16i re[NL], im[NL];
 #pragma unroll
@@ -797,12 +625,12 @@ __global__ void __launch_bounds__(kThreads, 1)
       eb[r] = xb[(uint32_t)min(n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh, grp.N - 1)];
 
     for (int k0 = 0; k0 < kpad; k0 += BKB) {
-      const v4i* sA = lds + st * 2 * OP_ST;
-      const v4i* sB = sA + OP_ST;
-      fst = lds + (st == 0 ? 2 : st - 1) * 2 * OP_ST + wave * BM;
-      if (++st == NSTAGE) st = 0;
-      const v4i* nA = lds + st * 2 * OP_ST;
-      const v4i* nB = nA + OP_ST;
+      const v4i* sA = lds + st * Fill::kStage;
+      const v4i* sB = sA + Fill::kOperand;
+      fill.stage(lds + (st == 0 ? kRing - 1 : st - 1) * Fill::kStage);
+      if (++st == kRing) st = 0;
+      const v4i* nA = lds + st * Fill::kStage;
+      const v4i* nB = nA + Fill::kOperand;
       // One quarter of the step: the digit products a b into lev, with
       // after(n) issued behind MFMA n. A wave issues in order and an MFMA
       // keeps the matrix pipe busy for several issues, so reads, fills and
@@ -829,14 +657,14 @@ __global__ void __launch_bounds__(kThreads, 1)
         if constexpr (n < S)
           ai[n] = frag(sA, S + n, wm0);
         else if constexpr (n < S + NLD)
-          fill_load(n - S);
+          fill.load(n - S);
         if constexpr (DIFF) negate(std::integral_constant<int, n - kNegDiff>{});
       });
       products(ai, br, im, [&](auto n) __attribute__((always_inline)) {
         if constexpr (DIFF) negate(std::integral_constant<int, n + NP - kNegDiff>{});
         negate(std::integral_constant<int, n - kNeg>{});
       });
-      fill_next();
+      fill.next();
       wait_vmcnt<NLD>();
       stage_barrier();
       // the next step's first fragments (past the last step: a stage nobody
@@ -886,29 +714,34 @@ __global__ void __launch_bounds__(kThreads, 1)
   }
 }
 
-// Real split GEMM with the A operand in registers: 64 x 64 tiles, two waves
-// per workgroup, each wave 32 rows x 64 columns (both 32-column B blocks
-// share its A fragments). A fragments come straight from the chunk-major
-// planes into registers (a wave owns its rows, nothing to share), prefetched
-// one K step ahead; B goes through LDS (three stages, filled two steps
-// ahead). Per MFMA this moves half the LDS bytes of the 32x32-per-wave
-// kernels, which the LDS-activity counters show are LDS-bound. 7 levels x 2
-// blocks of INT32 accumulators need one wave per SIMD (two workgroups per
-// CU).
+// Real split GEMM: 64 x 64 tiles, four waves of 32 x 32, two workgroups (two
+// waves per SIMD) per CU. As in the complex kernel the stages form one
+// sequence over the pairs of the group and reads and fills are issued between
+// MFMAs. A step's first seven fragments are read before it begins: the barrier
+// that opens the next stage comes behind the products of digits 0 to 2 of A,
+// after which digits 3 to 5 of B are free; 2 to 0 follow as their last products
+// are issued, and the products of one digit of A run from the last digit of B
+// down, so the fragment read last is needed last.
+// Against stages restarted for every pair, with all reads ahead of the MFMAs
+// (MI355X): the two products of the chi = 4096 U(1) network 410 -> 346 us,
+// 4096^3 1.26 -> 1.08 ms, 1000^3 28.5 -> 22.3 us, 300^3 11 -> 7.8 us, 2000 x 64 x
+// 2000 17 -> 15.3 us. 4096^3 is bound by power like the complex kernel (2.7
+// POP/s in both); the U(1) blocks by the start and the end of their short
+// tiles.
 template <int S>
-__global__ void __launch_bounds__(128, 1)
-    split_gemm_areg_kernel(const SplitPair* __restrict__ pairs,
-                           const GemmGroup* __restrict__ groups, const GemmTile* __restrict__ tiles,
-                           const int8_t* planesA, const int8_t* __restrict__ planesB,
-                           const int32_t* __restrict__ expA, const int32_t* __restrict__ expB,
-                           double* __restrict__ Cg, double ga, double beta) {
-  constexpr int NL = S;
-  constexpr int B_ST = S * 2 * BN;  // 16-byte LDS slots of one B stage
-  constexpr int NLD = S * 2;        // wave loads (64 rows x 16 bytes) per B stage
-  constexpr int NLD_W = NLD / 2;    // per wave (two waves)
-  static_assert(NLD % 2 == 0, "B stage loads split evenly over the two waves");
-  constexpr int NSTAGE = 3;
-  __shared__ v4i lds[NSTAGE * B_ST];
+__global__ void __launch_bounds__(kThreads, 2)
+    split_gemm_real_kernel(const SplitPair* __restrict__ pairs,
+                           const GemmGroup* __restrict__ groups,
+                           const GemmTile* __restrict__ tiles, const int8_t* __restrict__ planesA,
+                           const int8_t* __restrict__ planesB, const int32_t* __restrict__ expA,
+                           const int32_t* __restrict__ expB, double* __restrict__ Cg, double ga,
+                           double beta) {
+  using Fill = StageFill<S, 1>;
+  constexpr int NLD = Fill::kLoads, NL = S;
+  constexpr int NP = S * (S + 1) / 2;  // digit products of a step
+  constexpr int kOpen = digit_first<S>(3) - 1;  // the next stage opens behind this MFMA
+  static_assert(S % 2 == 0 && S + NLD - 1 <= kOpen, "reads and fills fit before the barrier");
+  __shared__ v4i lds[kRing * Fill::kStage];
 
   const GemmTile& tt = tiles[blockIdx.x];
   if (tt.g < 0) return;
@@ -916,140 +749,89 @@ __global__ void __launch_bounds__(128, 1)
   const int m0 = tt.m0, n0 = tt.n0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
   const int l32 = lane & 31, lh = lane >> 5;
-  const int arow = min(m0 + wave * 32 + l32, grp.M - 1);  // A row of this lane's fragment
-  const int brow = min(n0 + lane, grp.N - 1);             // B row this lane fetches
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
+  Fill fill(pairs, grp, planesA, planesB, m0, n0, lane, wave);
 
-  // outputs: m = m0 + 32*wave + l32 ; n = n0 + 32*jb + (r%4) + 8*(r/4) + 4*lh
-  double acc[2][16];
+  double acc[16];
 #pragma unroll
-  for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[jb][r] = 0.0;
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0;
 
-  for (int p = grp.p0; p < grp.p1; ++p) {
-    const SplitPair pr = pairs[p];
-    const int kpad = pr.kpad;
-    if (kpad <= 0) continue;
-    const int8_t* pa = planesA + pr.a_planes + pr.a_koff;
-    const int8_t* pb = planesB + pr.b_planes + pr.b_koff;
-    v16i lev[2][NL];
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-      for (int L = 0; L < NL; ++L) lev[jb][L] = v16i{0};
+  auto frag = [&](const v4i* op, int i, int w0) { return op[(i * 2 + lh) * kBT + w0 + l32]; };
 
-    auto fill_b = [&](int k0, int st) {
-      v4i* sB = lds + st * B_ST;
-      const int c0 = k0 >> 4;
+  v4i a[S], b[S];
+  int st = 0;
+  if (grp.p0 < grp.p1) {
+    fill.begin(lds);
+    a[0] = frag(lds, 0, wm0);
 #pragma unroll
-      for (int t = 0; t < NLD_W; ++t) {
-        const int q = wave + 2 * t, ch = q & 1, pl = q >> 1;
-        load_lds16(pb + pl * pr.b_pstride + ((int64_t)(c0 + ch) * grp.N + brow) * 16,
-                   sB + (pl * 2 + ch) * BN);
-      }
-    };
-    v4i av[S], an[S];
-    auto load_a = [&](int k0) {  // A fragments of the step at K byte k0 -> an
-      const int c = (k0 >> 4) + lh;
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-        an[i] = *reinterpret_cast<const v4i*>(pa + i * pr.a_pstride +
-                                              ((int64_t)c * grp.M + arow) * 16);
-    };
-
-    // prologue: B stage 0, A step 0, B stage 1 (in that order, so that
-    // waiting for all but the last NLD_W loads covers the first two). Past
-    // the last step the prefetches re-fetch the last step (clamped) into a
-    // stage / registers nobody reads, so every step issues the same loads
-    // and waits for the same count.
-    const int nsteps = kpad / BKB;
-    const int klast = (nsteps - 1) * BKB;
-    fill_b(0, 0);
-    load_a(0);
-    fill_b(min(BKB, klast), 1);
-    wait_vmcnt<NLD_W>();
-    stage_barrier();
-#pragma unroll
-    for (int i = 0; i < S; ++i) av[i] = an[i];
-    int st = 0;
-    for (int s = 0; s < nsteps; ++s) {
-      // A of the next step first, then the B fill two steps ahead: the wait
-      // at the end of the step then leaves only that fill in flight
-      load_a(min((s + 1) * BKB, klast));
-      int nst = st + 2;
-      if (nst >= NSTAGE) nst -= NSTAGE;
-      fill_b(min((s + 2) * BKB, klast), nst);
-      // B fragments of this stage; the second block's reads complete under
-      // the first block's MFMAs. Both prefetches stay ahead of the math.
-      const uint32_t sb = lds_base + (uint32_t)(st * B_ST + lh * BN + l32) * 16u;
-      v4i bv[2][S];
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < S; ++j) bv[0][j] = lds_read16_untracked(sb + (j * 2 * BN) * 16);
-      wait_lgkmcnt0();
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < S; ++j) bv[1][j] = lds_read16_untracked(sb + (j * 2 * BN + 32) * 16);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int jb = 0; jb < 2; ++jb) {
-        if (jb == 1) {
-          __builtin_amdgcn_sched_barrier(0);
-          wait_lgkmcnt0();
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int i = 0; i < S; ++i)
-#pragma unroll
-          for (int j = 0; j < S - i; ++j)
-            lev[jb][i + j] =
-                __builtin_amdgcn_mfma_i32_32x32x32_i8(bv[jb][j], av[i], lev[jb][i + j], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<NLD_W>();
-      stage_barrier();
-#pragma unroll
-      for (int i = 0; i < S; ++i) av[i] = an[i];
-      if (++st == NSTAGE) st = 0;
-    }
-    // the last (unused) fill must land before the next pair's prologue
-    // writes the stages again
-    wait_vmcnt<0>();
-    stage_barrier();
-
-    // FP64 recombination of the levels, scaled per row/column
-    const int gm = m0 + wave * 32 + l32;
-    const int ea = (gm < grp.M) ? expA[pr.a_exp + gm] : 0;
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int gn = n0 + jb * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh;
-        const int eb = (gn < grp.N) ? expB[pr.b_exp + gn] : 0;
-        double h = (double)lev[jb][NL - 1][r];
-#pragma unroll
-        for (int L = NL - 2; L >= 0; --L) h = fma(h, kInvRadix, (double)lev[jb][L][r]);
-        double v = ldexp(h * kInvLead2, ea + eb);
-        if (ea == kNonFinite || eb == kNonFinite) v = __builtin_nan("");
-        acc[jb][r] = fma(ga * pr.alpha, v, acc[jb][r]);
-      }
+    for (int j = 0; j < S; ++j) b[j] = frag(lds + Fill::kOperand, j, wn0);
   }
 
-  const int gm = m0 + wave * 32 + l32;
-  if (gm >= grp.M) return;
+  for (int p = grp.p0; p < grp.p1; ++p) {
+    const __attribute__((address_space(4))) SplitPair& pr = fill.pairs[p];
+    const int kpad = pr.kpad;
+    v16i lev[NL];
 #pragma unroll
-  for (int jb = 0; jb < 2; ++jb)
+    for (int L = 0; L < NL; ++L) lev[L] = v16i{0};
+    const int32_t *xa = expA + pr.a_exp, *xb = expB + pr.b_exp;
+    const int ea = xa[(uint32_t)min(m0 + wm0 + l32, grp.M - 1)];
+    int eb[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      eb[r] = xb[(uint32_t)min(n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh, grp.N - 1)];
+
+    for (int k0 = 0; k0 < kpad; k0 += BKB) {
+      const v4i* sA = lds + st * Fill::kStage;
+      fill.stage(lds + (st == 0 ? kRing - 1 : st - 1) * Fill::kStage);
+      if (++st == kRing) st = 0;
+      const v4i* nA = lds + st * Fill::kStage;
+      const v4i* nB = nA + Fill::kOperand;
+      static_for([&](auto n) __attribute__((always_inline)) {
+        // digit j descending: the digits of B freed first are read first
+        constexpr int i = digit_row<S>(n), j = S - 1 - i - (n - digit_first<S>(i));
+        lev[i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j], a[i], lev[i + j], 0, 0, 0);
+        if constexpr (n < S - 1) a[n + 1] = frag(sA, n + 1, wm0);
+        if constexpr (n >= S - 1 && n < S - 1 + NLD) fill.load(n - (S - 1));
+        if constexpr (n == kOpen) {
+          fill.next();
+          wait_vmcnt<NLD>();
+          stage_barrier();
+          a[0] = frag(nA, 0, wm0);
+#pragma unroll
+          for (int q = S - 1; q >= S - 3; --q) b[q] = frag(nB, q, wn0);
+        }
+        if constexpr (i >= 3 && n == digit_first<S>(i + 1) - 1) {
+          constexpr int q = S - 1 - i;  // no later product uses it
+          b[q] = frag(nB, q, wn0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }, std::make_integer_sequence<int, NP>{});
+    }
+
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int gn = n0 + jb * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh;
-      if (gn >= grp.N) continue;
-      const int64_t o = grp.off_c + gm + (int64_t)gn * grp.ldc;
-      double out = acc[jb][r];
-      if (beta != 0.0) out = fma(beta, Cg[o], out);
-      Cg[o] = out;
+      double h = (double)lev[NL - 1][r];
+#pragma unroll
+      for (int L = NL - 2; L >= 0; --L) h = fma(h, kInvRadix, (double)lev[L][r]);
+      double v = ldexp(h * kInvLead2, ea + eb[r]);
+      if (ea == kNonFinite || eb[r] == kNonFinite) v = __builtin_nan("");
+      acc[r] = fma(ga * pr.alpha, v, acc[r]);
     }
+  }
+  wait_vmcnt<0>();  // no fill outlives the workgroup
+
+  const int gm = m0 + wm0 + l32;
+  if (gm >= grp.M) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int gn = n0 + wn0 + (r & 3) + 8 * (r >> 2) + 4 * lh;
+    if (gn >= grp.N) continue;
+    const int64_t o = grp.off_c + gm + (int64_t)gn * grp.ldc;
+    double out = acc[r];
+    if (beta != 0.0) out = fma(beta, Cg[o], out);
+    Cg[o] = out;
+  }
 }
 
 }  // namespace
@@ -1079,27 +861,15 @@ int64_t slice_block_wgs(int32_t rows, int32_t kparts) {
   return (int64_t)((rows + kSliceRows - 1) / kSliceRows) * kparts;
 }
 
-hipError_t launch_split_gemm(hipStream_t s, int prec, int wmb, const SplitPair* pairs,
+hipError_t launch_split_gemm(hipStream_t s, int prec, const SplitPair* pairs,
                              const GemmGroup* groups, const GemmTile* tiles, int64_t grid,
                              const void* planesA, const void* planesB, const void* expA,
                              const void* expB, void* C, double ga, double beta) {
   if (grid == 0) return hipSuccess;
   if (prec != 2) return hipErrorNotSupported;
-  const dim3 g((unsigned)grid);
-  const int8_t *pa = (const int8_t*)planesA, *pb = (const int8_t*)planesB;
-  const int32_t *ea = (const int32_t*)expA, *eb = (const int32_t*)expB;
-  double* c = (double*)C;
-  if (wmb == 3)
-    ITG_LAUNCH((split_gemm_areg_kernel<kSliceCount>), g, dim3(128), 0, s, pairs, groups, tiles, pa,
-               pb, ea, eb, c, ga, beta);
-  else if (wmb == 2)
-    ITG_LAUNCH((split_gemm_kernel<kSliceCount, 4>), g, dim3(512), 0, s, pairs, groups, tiles, pa,
-               pb, ea, eb, c, ga, beta);
-  else if (wmb == 1)
-    ITG_LAUNCH((split_gemm_kernel<kSliceCount, 2>), g, dim3(256), 0, s, pairs, groups, tiles, pa,
-               pb, ea, eb, c, ga, beta);
-  else
-    return hipErrorInvalidValue;
+  ITG_LAUNCH((split_gemm_real_kernel<kSliceCount>), dim3((unsigned)grid), dim3(kThreads), 0, s,
+             pairs, groups, tiles, (const int8_t*)planesA, (const int8_t*)planesB,
+             (const int32_t*)expA, (const int32_t*)expB, (double*)C, ga, beta);
   return hipGetLastError();
 }
 

@@ -172,10 +172,8 @@ def _handle(dev):
 
 
 def set_split_tile(tile: int, device=None) -> None:
-    """Tile shape of the split-precision GEMM on `device`: 0 = per plan
-    (autotuned, else by size), 1 = 64 x 64, 2 = 128 x 64, 3 = 64 x 64 with
-    the A operand in registers (real data; complex uses 1). The shapes agree
-    bit for bit; this exists for tests and tuning."""
+    """Tile shape of the split-precision GEMM on `device`, 0..3: there is one
+    shape, 64 x 64, so every value selects it."""
     dev = torch.device(device) if device is not None else torch.device(
         "cuda", torch.cuda.current_device())
     h = _handle(dev)
