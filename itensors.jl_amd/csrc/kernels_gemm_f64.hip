@@ -25,17 +25,18 @@
 //
 // K loop: the slices (16 real or 8 complex values of k) of all pairs form one
 // sequence. Slice s is multiplied from one LDS buffer while slice s + 1 goes
-// from registers to the other and slice s + 2 is loaded, one barrier per
-// slice; the fragments of each half slice are read while the other half's
-// MFMAs run. What bounds it: the FP64 matrix pipe (76 TF/s measured with
-// MFMAs alone; one instruction takes 64 cycles) and, with it, every vector
-// instruction, which FP64 MFMAs do not overlap. The loop before this one
-// spent about 150 of them per slice and wave on addresses, masks and alpha
-// and waited for each slice's loads within the slice; this one spends about
-// 8, in 16-byte loads and LDS accesses. Measured, 64x64 tiles, MI355X:
-// 4096^3 real 2.63 -> 2.21 ms, 2048^3 complex 0.95 ms (72 TF/s); the grouped
-// products of the chi = 4096 U(1) network 0.385 -> 0.313 ms each; dense
-// chi = 1024 network (5120 x 4096 x 1024) 0.84 -> 0.71 ms.
+// from registers to the other, slice s + 2 is in registers and slice s + 3 is
+// loaded, one barrier per slice; the fragments of each half slice are read
+// while the other half's MFMAs run. What bounds it: the FP64 matrix pipe (76
+// TF/s measured with MFMAs alone; one instruction takes 64 cycles) and, with
+// it, every vector instruction, which FP64 MFMAs do not overlap (about 8 per
+// slice and wave, in 16-byte loads and LDS accesses). A slice's MFMAs take 0.5
+// us on a CU with one workgroup, less than a load that misses L2: with one
+// slice in registers (four waves per SIMD) instead of two (three waves),
+// 4096^3 took 2.08 instead of 1.95 ms, 3001 x 1777 x 2049 432 instead of 418 us,
+// 4800 x 495 x 2100 218 instead of 206, the chi = 1024 dense network's two
+// products (5120 x 4096 x 1024) 1.365 instead of 1.307 ms; complex products,
+// the chi = 4096 U(1) network's (0.60 ms for both) and small ones are level.
 //
 // Complex data (interleaved re/im) uses the 4-real-product form on the same
 // tiles, with conj(A)/conj(B) folded into the sign of the imaginary parts.
@@ -92,10 +93,10 @@ struct Operand {
   // LDS distance of a thread's consecutive chunks
   static constexpr int kStep = KC ? kThreads / kChunksK * 16 : kThreads / RC * kRowBytes;
 
-  double2 v[NCH];     // the slice in flight
+  double2 v[2][NCH];  // the slices in flight
   const char* base;   // uniform: the next fast slice's first element
   uint32_t off[NCH];  // byte offsets of this thread's chunks from base
-  uint32_t mask;      // masked slices: bits 2 r, 2 r + 1 for the halves of chunk r
+  uint32_t mask[2];   // masked slices: bits 2 r, 2 r + 1 for the halves of chunk r
   int wr, rd;         // LDS offsets: first chunk written, first fragment read
 
   // chunk r of this thread: first row / first k inside the tile
@@ -139,12 +140,13 @@ struct Operand {
   }
   // Buffer loads: a scalar base and a 32-bit lane offset, with no address
   // arithmetic on the vector ALU.
+  template <int B>
   __device__ __forceinline__ void load_fast(int64_t ld) {
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, 0xffffffffu, 0x00027000);
 #pragma unroll
     for (int r = 0; r < NCH; ++r)
-      v[r] = __builtin_bit_cast(
+      v[B][r] = __builtin_bit_cast(
           double2, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[r], 0, 0));
     base += (KC ? 1 : ld) * (BK * ES);
   }
@@ -152,17 +154,18 @@ struct Operand {
   // chunks past the end re-read values of the slice (KC: the last two before
   // the end, which may start one value before the slice), and mask says
   // which elements count.
+  template <int B>
   __device__ __forceinline__ void load_tail(int64_t ld, int krem, int tid) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(base) - ES, 0, 0xffffffffu, 0x00027000);
-    mask = 0u;
+    mask[B] = 0u;
 #pragma unroll
     for (int r = 0; r < NCH; ++r) {
       const int k = kofs(tid, r);
       const int back = max(k - (krem - (KC ? CE : 1)), 0);
-      if (k < krem) mask |= 1u << (2 * r);
-      if (k + (KC ? CE - 1 : 0) < krem) mask |= 2u << (2 * r);
-      v[r] = __builtin_bit_cast(
+      if (k < krem) mask[B] |= 1u << (2 * r);
+      if (k + (KC ? CE - 1 : 0) < krem) mask[B] |= 2u << (2 * r);
+      v[B][r] = __builtin_bit_cast(
           double2, __builtin_amdgcn_raw_buffer_load_b128(
                        rs, (int)(off[r] + ES - (uint32_t)back * (KC ? 1u : (uint32_t)ld) * ES), 0,
                        0));
@@ -171,59 +174,64 @@ struct Operand {
   // any slice of a pair without fast loads (a block of one row, one
   // contracted value, or one that does not fit): element by element from
   // clamped addresses
+  template <int B>
   __device__ __forceinline__ void load_slow(const double* __restrict__ X, int64_t block,
                                             int64_t ld, int r0, int rows, int k0, int K,
                                             int tid) {
-    mask = 0u;
+    mask[B] = 0u;
 #pragma unroll
     for (int r = 0; r < NCH; ++r) {
 #pragma unroll
       for (int e = 0; e < CE; ++e) {
         const int g = r0 + row(tid, r) + (KC ? 0 : e), k = k0 + kofs(tid, r) + (KC ? e : 0);
-        if (g < rows && k < K) mask |= (CPLX ? 3u : 1u << e) << (2 * r);
+        if (g < rows && k < K) mask[B] |= (CPLX ? 3u : 1u << e) << (2 * r);
         const int64_t gc = min(g, rows - 1), kc = min(k, K - 1);
         const int64_t o = block + (KC ? gc * ld + kc : kc * ld + gc);
         if (CPLX)
-          v[r] = reinterpret_cast<const double2*>(X)[o];
+          v[B][r] = reinterpret_cast<const double2*>(X)[o];
         else if (e == 0)
-          v[r].x = X[o];
+          v[B][r].x = X[o];
         else
-          v[r].y = X[o];
+          v[B][r].y = X[o];
       }
     }
   }
+  template <int B>
   __device__ __forceinline__ void store_fast(char* S) const {
 #pragma unroll
     for (int r = 0; r < NCH; ++r) {
       Chunk c;
-      c.x = v[r].x;
-      c.y = v[r].y;
+      c.x = v[B][r].x;
+      c.y = v[B][r].y;
       *reinterpret_cast<Chunk*>(S + wr + r * kStep) = c;
     }
   }
   // slow: load_slow's, at the chunks' unmoved places; else load_tail's, where
   // the last value of an odd end is the second of the chunk that was re-read
+  template <int B>
   __device__ __forceinline__ void store_masked(char* S, int tid, bool slow) const {
 #pragma unroll
     for (int r = 0; r < NCH; ++r) {
-      const bool in0 = mask >> (2 * r) & 1u, in1 = mask >> (2 * r + 1) & 1u;
+      const bool in0 = mask[B] >> (2 * r) & 1u, in1 = mask[B] >> (2 * r + 1) & 1u;
       Chunk c;
-      c.x = !CPLX && KC && !slow && !in1 ? v[r].y : v[r].x;
+      c.x = !CPLX && KC && !slow && !in1 ? v[B][r].y : v[B][r].x;
       c.x = in0 ? c.x : 0.0;
-      c.y = in1 ? v[r].y : 0.0;
+      c.y = in1 ? v[B][r].y : 0.0;
       char* d = !CPLX && !KC && slow ? S + at(row(tid, r), kofs(tid, r)) : S + wr + r * kStep;
       *reinterpret_cast<Chunk*>(d) = c;
     }
   }
+  template <int B>
   __device__ __forceinline__ void conj() {
 #pragma unroll
-    for (int r = 0; r < NCH; ++r) v[r].y = -v[r].y;
+    for (int r = 0; r < NCH; ++r) v[B][r].y = -v[B][r].y;
   }
+  template <int B>
   __device__ __forceinline__ void scale(double re, double im) {
 #pragma unroll
     for (int r = 0; r < NCH; ++r)
-      v[r] = CPLX ? make_double2(re * v[r].x - im * v[r].y, re * v[r].y + im * v[r].x)
-                  : make_double2(re * v[r].x, re * v[r].y);
+      v[B][r] = CPLX ? make_double2(re * v[B][r].x - im * v[B][r].y, re * v[B][r].y + im * v[B][r].x)
+                  : make_double2(re * v[B][r].x, re * v[B][r].y);
   }
   // The fragments of one wave for half a slice (Q = 0, 1), two values per
   // row: f[h][i], row w0 + 16 i + l16. Real: the MFMA steps h = 0, 1 take
@@ -262,7 +270,7 @@ typedef const __attribute__((address_space(4))) GemmGroup* GroupTable;
 typedef const __attribute__((address_space(4))) GemmTile* TileTable;
 
 template <int CPLX, int TA, int TB>
-__global__ void __launch_bounds__(kThreads, CPLX ? 3 : 4)  // waves per SIMD
+__global__ void __launch_bounds__(kThreads, 3)  // waves per SIMD
     gemm_f64_kernel(const GemmPair* __restrict__ pairs, const GemmGroup* __restrict__ groups,
                     const GemmTile* __restrict__ tiles, int quarters,
                     const double* __restrict__ Ag, const double* __restrict__ Bg,
@@ -299,49 +307,63 @@ __global__ void __launch_bounds__(kThreads, CPLX ? 3 : 4)  // waves per SIMD
   // a chunk of two rows needs two rows
   const bool wide = CPLX || ((TA || M >= 2) && (!TB || N >= 2));
 
-  // The slices of all pairs form one sequence: one slice is multiplied from
-  // LDS while the next one is in registers, on its way there.
+  // The slices of all pairs form one sequence: slice s is multiplied from LDS
+  // buffer s % 2 while slices s + 1 and s + 2 are in registers, on their way
+  // there, in the sets of the same parity.
   OpA a;
   OpB b;
   const PairTable ptab = (PairTable)(uintptr_t)pairs;
+  // of the slice loaded last
   int p = grp->pf, k0 = 0, K = grp->K;
   int64_t off_a = grp->off_a, off_b = grp->off_b;
   int lda = grp->lda, ldb = grp->ldb;
-  bool masked = false, fast = false;   // of the slice in registers; of its pair
-  bool special = false;                // conj or alpha to apply to its pair
-  double al_re = 1.0, al_im = 0.0;
-  auto load = [&]() __attribute__((always_inline)) {
-    masked = !fast || k0 + BK > K;
-    if (!masked) {
-      a.load_fast(lda);
-      b.load_fast(ldb);
-    } else if (fast) {
-      a.load_tail(lda, K - k0, tid);
-      b.load_tail(ldb, K - k0, tid);
+  // of the slice in each set
+  bool masked[2], fast[2];  // fast: of its pair
+  bool special[2];          // conj or alpha to apply
+  double al_re[2], al_im[2];
+  auto same_pair = [&](auto set) __attribute__((always_inline)) {  // as the other set's
+    constexpr int B = decltype(set)::value;
+    fast[B] = fast[B ^ 1];
+    special[B] = special[B ^ 1];
+    al_re[B] = al_re[B ^ 1];
+    al_im[B] = al_im[B ^ 1];
+  };
+  auto load = [&](auto set) __attribute__((always_inline)) {
+    constexpr int B = decltype(set)::value;
+    masked[B] = !fast[B] || k0 + BK > K;
+    if (!masked[B]) {
+      a.template load_fast<B>(lda);
+      b.template load_fast<B>(ldb);
+    } else if (fast[B]) {
+      a.template load_tail<B>(lda, K - k0, tid);
+      b.template load_tail<B>(ldb, K - k0, tid);
     } else {
-      a.load_slow(Ag, off_a, lda, m0, M, k0, K, tid);
-      b.load_slow(Bg, off_b, ldb, n0, N, k0, K, tid);
+      a.template load_slow<B>(Ag, off_a, lda, m0, M, k0, K, tid);
+      b.template load_slow<B>(Bg, off_b, ldb, n0, N, k0, K, tid);
     }
   };
   // the first slice of pair p
-  auto load_first = [&]() __attribute__((always_inline)) {
+  auto load_first = [&](auto set) __attribute__((always_inline)) {
+    constexpr int B = decltype(set)::value;
     k0 = 0;
-    fast = wide && K >= 2 && OpA::fits(lda, m0, M) && OpB::fits(ldb, n0, N);
-    if (fast) {
+    fast[B] = wide && K >= 2 && OpA::fits(lda, m0, M) && OpB::fits(ldb, n0, N);
+    if (fast[B]) {
       a.start(Ag, off_a, lda, m0, M, tid);
       b.start(Bg, off_b, ldb, n0, N, tid);
     }
-    load();
+    load(set);
     const double are = ptab[p].alpha_re, aim = ptab[p].alpha_im;
-    al_re = ga_re * are - ga_im * aim;
-    al_im = ga_re * aim + ga_im * are;
-    special = al_re != 1.0 || (CPLX && (al_im != 0.0 || (flags & 3u)));
+    al_re[B] = ga_re * are - ga_im * aim;
+    al_im[B] = ga_re * aim + ga_im * are;
+    special[B] = al_re[B] != 1.0 || (CPLX && (al_im[B] != 0.0 || (flags & 3u)));
   };
-  // issue the loads of the next slice; false when there is none
-  auto load_next = [&]() __attribute__((always_inline)) -> bool {
+  // issue the loads of the slice after the last one into a set; false when
+  // there is none
+  auto load_next = [&](auto set) __attribute__((always_inline)) -> bool {
     k0 += BK;
     if (k0 < K) {
-      load();
+      same_pair(set);
+      load(set);
       return true;
     }
     do {
@@ -352,25 +374,29 @@ __global__ void __launch_bounds__(kThreads, CPLX ? 3 : 4)  // waves per SIMD
     off_b = ptab[p].off_b;
     lda = ptab[p].lda;
     ldb = ptab[p].ldb;
-    load_first();
+    load_first(set);
     return true;
   };
-  auto adjust = [&]() __attribute__((always_inline)) {
-    if (special) {
+  auto adjust = [&](auto set) __attribute__((always_inline)) {
+    constexpr int B = decltype(set)::value;
+    if (special[B]) {
       asm volatile("; conj, alpha");  // stays a branch: it is almost never taken
-      if (CPLX && (flags & 1u)) a.conj();
-      if (CPLX && (flags & 2u)) b.conj();
-      if (al_re != 1.0 || (CPLX && al_im != 0.0)) a.scale(al_re, al_im);
+      if (CPLX && (flags & 1u)) a.template conj<B>();
+      if (CPLX && (flags & 2u)) b.template conj<B>();
+      if (al_re[B] != 1.0 || (CPLX && al_im[B] != 0.0))
+        a.template scale<B>(al_re[B], al_im[B]);
     }
   };
-  auto store_any = [&](char* S) __attribute__((always_inline)) {
-    adjust();
-    if (!masked) {
-      a.store_fast(S);
-      b.store_fast(S + OpA::kBytes);
+  auto store_any = [&](auto set) __attribute__((always_inline)) {
+    constexpr int B = decltype(set)::value;
+    char* S = smem[B];
+    adjust(set);
+    if (!masked[B]) {
+      a.template store_fast<B>(S);
+      b.template store_fast<B>(S + OpA::kBytes);
     } else {
-      a.store_masked(S, tid, !fast);
-      b.store_masked(S + OpA::kBytes, tid, !fast);
+      a.template store_masked<B>(S, tid, !fast[B]);
+      b.template store_masked<B>(S + OpA::kBytes, tid, !fast[B]);
     }
   };
 
@@ -421,60 +447,74 @@ __global__ void __launch_bounds__(kThreads, CPLX ? 3 : 4)  // waves per SIMD
             }
       }
     };
-    // one slice from S; the registers (a full slice) go to T and the next
-    // full slice of the pair is loaded. The halves of a slice are read one
-    // half ahead of their MFMAs; T was last read before the previous barrier.
-    auto steady = [&](const char* S, char* T) __attribute__((always_inline)) {
-      adjust();
-      a.store_fast(T);
-      b.store_fast(T + OpA::kBytes);
-      frags(1, S);
+    // Slice s from its buffer: slice s + 1 (full) goes from its registers to
+    // the other buffer and slice s + 3, a full one of the pair loaded last, is
+    // loaded into them. The halves of a slice are read one half ahead of their
+    // MFMAs; the other buffer was last read before the previous barrier.
+    auto steady = [&](auto buf) __attribute__((always_inline)) {
+      constexpr int B = decltype(buf)::value;
+      adjust(std::integral_constant<int, B ^ 1>{});
+      a.template store_fast<B ^ 1>(smem[B ^ 1]);
+      b.template store_fast<B ^ 1>(smem[B ^ 1] + OpA::kBytes);
+      frags(1, smem[B]);
       __builtin_amdgcn_sched_barrier(0);
-      a.load_fast(lda);
-      b.load_fast(ldb);
+      a.template load_fast<B ^ 1>(lda);
+      b.template load_fast<B ^ 1>(ldb);
       mfmas(0);
       __builtin_amdgcn_sched_barrier(0);
       lds_barrier();
-      frags(0, T);
+      frags(0, smem[B ^ 1]);
       __builtin_amdgcn_sched_barrier(0);
       mfmas(1);
       __builtin_amdgcn_sched_barrier(0);
     };
-    if (K > 0) {
-      load_first();
-      store_any(smem[0]);
-      bool more = load_next();
+    // the same for any slices s + 1 (there is one) and s + 3: have_after says
+    // whether there is a slice s + 2, have_next then whether there is s + 3
+    auto any = [&](auto buf, bool& have_next, bool& have_after) __attribute__((always_inline)) {
+      constexpr int B = decltype(buf)::value;
+      const std::integral_constant<int, B ^ 1> next{};
+      store_any(next);
+      frags(1, smem[B]);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(0);
+      have_next = have_after && load_next(next);
       lds_barrier();
-      int buf = 0;
+      frags(0, smem[B ^ 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(1);
+    };
+    if (K > 0) {
+      const std::integral_constant<int, 0> even{};
+      const std::integral_constant<int, 1> odd{};
+      load_first(even);
+      bool have1 = load_next(odd), have0 = false;  // the sets hold slices to come
+      store_any(even);
+      if (have1) have0 = load_next(even);
+      lds_barrier();
       frags(0, smem[0]);
-      while (more) {
-        // Slices whose successor is a full slice of the same pair, then one
-        // whose successor may be a partial slice or the next pair's first.
-        int n = masked ? 0 : (K - k0) / BK - 1;
-        k0 += max(n, 0) * BK;
-        if (n > 0 && buf) {
-          steady(smem[1], smem[0]);
-          buf = 0;
-          --n;
+      int buf = 0;
+      for (;;) {
+        // buffer 0 is next. Slices whose third successors are full slices of
+        // the pair loaded last, two by two, while neither set is masked.
+        if (have0 && !masked[0] && !masked[1]) {
+          int n = (K - k0) / BK - 1;
+          if (n >= 2) {
+            n &= ~1;
+            k0 += n * BK;
+            do {
+              steady(even);
+              same_pair(odd);  // set 1 may have held the pair before
+              steady(odd);
+              n -= 2;
+            } while (n);
+          }
         }
-        for (; n >= 2; n -= 2) {
-          steady(smem[0], smem[1]);
-          steady(smem[1], smem[0]);
-        }
-        if (n > 0) {
-          steady(smem[0], smem[1]);
-          buf = 1;
-        }
-        store_any(smem[buf ^ 1]);
-        frags(1, smem[buf]);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(0);
-        more = load_next();
-        lds_barrier();
-        buf ^= 1;
-        frags(0, smem[buf]);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(1);
+        if (!have1) break;
+        any(even, have1, have0);
+        buf = 1;
+        if (!have0) break;
+        any(odd, have0, have1);
+        buf = 0;
       }
       frags(1, smem[buf]);
       __builtin_amdgcn_sched_barrier(0);
