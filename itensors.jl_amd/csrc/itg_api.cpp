@@ -275,16 +275,41 @@ KernelTimer* active_timer(itg_handle* h) {
   return h->timer.get();
 }
 
+// The handle's workspace for a run that needs `need` bytes. *parts: whether it
+// also holds the partial buffer of the plan's part form. That form is only
+// faster: where the workspace cannot grow for it (out of memory, or a stream
+// under capture) the plan runs without.
+hipError_t ready_ws(itg_handle* h, ExecPlan& ep, int cplx, int prec, size_t need, bool* parts) {
+  *parts = false;
+  if (ep.strategy == ExecPlan::GEMM && prec == ITG_PREC_FP64 && ep.ks_grid == 0)
+    (void)ensure_gemm_launch(ep, h->stream);  // a failure is exec_run's to report
+  const size_t extra = exec_part_bytes(ep, cplx, prec);
+  if (extra) {
+    const size_t want = ((need + 255) & ~(size_t)255) + extra;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (h->ws_bytes >= want)
+      *parts = true;
+    else if (hipStreamIsCapturing(h->stream, &cs) == hipSuccess &&
+             cs == hipStreamCaptureStatusNone && ensure_ws(h, want) == hipSuccess)
+      *parts = true;
+    if (*parts) return hipSuccess;
+    (void)hipGetLastError();
+  }
+  return ensure_ws(h, need);
+}
+
 itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void* T1,
                     const void* T2, void* R, unsigned flags, const double* alpha,
                     const double* beta) {
   const double a_re = alpha ? alpha[0] : 1.0, a_im = (alpha && cplx) ? alpha[1] : 0.0;
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
-  hipError_t e = ensure_ws(h, exec_workspace_bytes(ep, cplx, prec, a_im != 0.0));
-  if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
   std::string err;
+  bool parts = false;
+  hipError_t e = ready_ws(h, ep, cplx, prec, exec_workspace_bytes(ep, cplx, prec, a_im != 0.0),
+                          &parts);
+  if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
   e = exec_run(ep, cplx, prec, h->stream, h->ws, T1, T2, R, flags, a_re, a_im, b_re, b_im,
-               &err, active_timer(h));
+               &err, active_timer(h), true, parts);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
   return ITG_OK;
@@ -399,8 +424,10 @@ itg_status bs_execute_on(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void* R
     return fail(h, ITG_ERR_INVALID, msg);
   }
   std::string err;
+  const size_t extra = exec_part_bytes(*ep, cplx, (int)prec);
+  const bool parts = extra && ((need + 255) & ~(size_t)255) + extra <= ws_bytes;
   hipError_t e = exec_run(*ep, cplx, (int)prec, h->stream, ws, T1, T2, R, flags, a_re, a_im,
-                          0.0, 0.0, &err, nullptr, false);
+                          0.0, 0.0, &err, nullptr, false, parts);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e == hipErrorNotReady) return fail(h, ITG_ERR_INVALID, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
@@ -1458,10 +1485,12 @@ itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void*
   DeviceGuard g(h->device);
   ExecPlan& ep = *p->ep;
   if (prec != ITG_PREC_FP64 && !ep.split_ok) return ITG_OK;
-  hipError_t e = ensure_ws(h, exec_workspace_bytes(ep, cplx, (int)prec));
+  bool parts = false;
+  hipError_t e = ready_ws(h, ep, cplx, (int)prec, exec_workspace_bytes(ep, cplx, (int)prec), &parts);
   if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
   std::string err;
-  e = exec_run(ep, cplx, (int)prec, h->stream, h->ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err);
+  e = exec_run(ep, cplx, (int)prec, h->stream, h->ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err,
+               nullptr, true, parts);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
   if ((e = hipStreamSynchronize(h->stream)) != hipSuccess)

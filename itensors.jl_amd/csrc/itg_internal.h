@@ -89,7 +89,7 @@ struct GemmGroup {
   int32_t pf;
   int64_t off_a, off_b;
   int32_t K, lda, ldb;
-  int32_t pad;
+  int32_t part;  // FP64 GEMM: nonzero if C is the partial buffer (off_c within it; no beta)
 };
 inline void set_first_pair(GemmGroup* g, const GemmPair* pairs) {
   g->pf = g->p0;
@@ -335,10 +335,21 @@ struct GemmTile {
   int32_t pad;
 };
 constexpr int kGemmTile = 64;  // rows and columns of a tile (FP64 and split GEMM)
+// P: buffer of the groups with `part` set (null when there are none).
 hipError_t launch_gemm_f64(hipStream_t s, int cplx, int ta, int tb, const GemmPair* pairs,
                            const GemmGroup* groups, const GemmTile* tiles, int64_t entries,
-                           bool quarters, const void* A, const void* B, void* C, unsigned flags,
-                           double ga_re, double ga_im, double beta_re, double beta_im);
+                           bool quarters, const void* A, const void* B, void* C, void* P,
+                           unsigned flags, double ga_re, double ga_im, double beta_re,
+                           double beta_im);
+// A 64 x 64 (or edge) tile of C computed in S parts along K: C = sum of the
+// partial blocks at P[poff + s*M*N], s = 0..S-1 in order (M x N,
+// column-major), + beta * C (beta == 0 does not read C).
+struct GemmJoin {
+  int64_t poff, off_c;
+  int32_t M, N, ldc, S;
+};
+hipError_t launch_gemm_join(hipStream_t s, int cplx, const GemmJoin* joins, int64_t n,
+                            const void* P, void* C, double beta_re, double beta_im);
 
 // Split-K form of the grouped FP64 GEMM: the GEMM kernel writes S partial
 // sums of each output block (one per slice of its contracted extent) into a

@@ -779,7 +779,7 @@ std::string build_ksplit(ExecPlan* ep, hipStream_t s) {
   ExecPlan tab;
   tab.h_groups = sg;
   tab.h_pairs = sp;
-  std::vector<GemmTile> tiles_tab = xcd_tile_table(tab, nullptr);
+  std::vector<GemmTile> tiles_tab = xcd_tile_table(tab);
   // skinny: (entry, first row) per workgroup, 256 rows of the long side
   std::vector<int2> rows;
   if (skinny)
@@ -1306,71 +1306,206 @@ hipError_t ensure_gemm_launch(ExecPlan& ep, hipStream_t s, bool may_build) {
   if (ep.launch) return hipSuccess;
   if (!may_build) return hipErrorNotReady;
   std::unique_ptr<GemmLaunch> gl(new GemmLaunch);
-  std::vector<GemmTile> table = xcd_tile_table(ep, gl->quarters);
+  PartTables pt;
+  const std::vector<GemmTile> table = xcd_tile_table(ep, gl->form, &pt);
   gl->grid = (int64_t)table.size();
-  hipError_t e;
-  if ((e = gl->tiles.upload(table.data(), table.size() * sizeof(GemmTile), s)) != hipSuccess)
-    return e;
+  gl->part_grid = (int64_t)pt.tiles.size();
+  gl->njoin = (int64_t)pt.joins.size();
+  gl->part_elems = pt.elems;
+  // one buffer, one copy
+  std::vector<char> host;
+  host.reserve(table.size() * sizeof(GemmTile) + pt.tiles.size() * sizeof(GemmTile) +
+               pt.groups.size() * sizeof(GemmGroup) + pt.pairs.size() * sizeof(GemmPair) +
+               pt.joins.size() * sizeof(GemmJoin) + 64);
+  auto put = [&](const void* p, size_t n) {
+    const size_t at = (host.size() + 15) & ~(size_t)15;
+    host.resize(at);
+    host.insert(host.end(), (const char*)p, (const char*)p + n);
+    return at;
+  };
+  const size_t o_tiles = put(table.data(), table.size() * sizeof(GemmTile));
+  const size_t o_ptiles = put(pt.tiles.data(), pt.tiles.size() * sizeof(GemmTile));
+  const size_t o_groups = put(pt.groups.data(), pt.groups.size() * sizeof(GemmGroup));
+  const size_t o_pairs = put(pt.pairs.data(), pt.pairs.size() * sizeof(GemmPair));
+  const size_t o_joins = put(pt.joins.data(), pt.joins.size() * sizeof(GemmJoin));
+  hipError_t e = gl->tab.upload(host.data(), host.size(), s);
+  if (e != hipSuccess) return e;
+  const char* base = (const char*)gl->tab.p;
+  gl->tiles = (const GemmTile*)(base + o_tiles);
+  gl->part_tiles = (const GemmTile*)(base + o_ptiles);
+  gl->part_groups = (const GemmGroup*)(base + o_groups);
+  gl->part_pairs = (const GemmPair*)(base + o_pairs);
+  gl->joins = (const GemmJoin*)(base + o_joins);
   ep.launch = std::move(gl);
   return hipSuccess;
 }
 
 namespace {
-// Whether the FP64 GEMM runs a table of 64 x 64 tiles faster as four 32 x 32
-// quarters each. cost[x]: of the tiles of XCD x, in their order (16 x 16 blocks
-// times contracted values). A quarter costs 1.42 (real) or 1.08 (complex: four
-// products per value loaded) of a fourth of its tile on a full CU, but a
-// product with fewer tiles than the chip has CUs, or a few long ones, leaves
-// CUs idle: the tiles are laid on the XCD's 32 CUs in order, each on the least
-// loaded, and a CU that holds few of them runs slower by `lone` (one, two,
-// three tiles; latency is not hidden). A lone quarter, bound by latency alone,
-// takes about as long as the MFMAs of its whole tile. Measured on MI355X, whole
-// -> quarters (K = 2048 unless said): real 512 x 1024 79 -> 58 us, 1024 x 1024
-// 91 -> 113, 2048 x 2048 272 -> 386; 128 x 1280 x 128 (K = 128) 9.4 -> 6.5 us;
-// complex 1024 x 1024 273 -> 289, the chi = 1500 U(1) network's last product
-// 134 -> 112 us.
-void quarters_faster(const std::vector<std::vector<double>>& cost, bool faster[2]) {
-  constexpr int kCus = 32, kMaxTiles = 256;  // per XCD; beyond 8 tiles a CU whole tiles win
-  const double lone[2][3] = {{1.32, 1.23, 1.08}, {1.15, 1.02, 1.0}};
-  const double quarter[2] = {1.42, 1.08};
-  double t_whole[2] = {0.0, 0.0}, t_quarters[2] = {0.0, 0.0};
-  faster[0] = faster[1] = false;
-  for (const std::vector<double>& c : cost)
-    if (c.size() > kMaxTiles) return;
-  for (const std::vector<double>& c : cost) {
-    std::pair<double, int> cu[kCus];  // load, tiles: a heap, least load first
-    std::fill(cu, cu + kCus, std::make_pair(0.0, 0));
-    double all = 0.0, longest = 0.0;
-    for (double t : c) {
-      std::pop_heap(cu, cu + kCus, std::greater<>());
-      cu[kCus - 1].first += t;
-      ++cu[kCus - 1].second;
-      std::push_heap(cu, cu + kCus, std::greater<>());
-      all += t;
-      longest = std::max(longest, t);
+constexpr int kCus = 32;  // per XCD
+// The CUs of an XCD as a heap, least load first.
+struct CuHeap {
+  struct Cu {
+    double load;
+    int tiles;
+  } cu[kCus];
+  CuHeap() { std::fill(cu, cu + kCus, Cu{0.0, 0}); }
+  double least() const { return cu[0].load; }
+  void add(double t) {  // to the least loaded
+    const Cu x{cu[0].load + t, cu[0].tiles + 1};
+    int i = 0;
+    for (int c = 1; c < kCus; c = 2 * i + 1) {
+      if (c + 1 < kCus && cu[c + 1].load < cu[c].load) ++c;
+      if (cu[c].load >= x.load) break;
+      cu[i] = cu[c];
+      i = c;
     }
-    for (int x = 0; x < 2; ++x) {
-      for (const auto& u : cu)
-        if (u.second)
-          t_whole[x] =
-              std::max(t_whole[x], u.first * (u.second <= 3 ? lone[x][u.second - 1] : 1.0));
-      t_quarters[x] = std::max({t_quarters[x], quarter[x] * all / kCus, 0.97 * longest});
+    cu[i] = x;
+  }
+};
+
+// How the FP64 GEMM runs a table of 64 x 64 tiles fastest. cost[x]: of the tiles
+// of XCD x, in their order (16 x 16 blocks times contracted values). The tiles
+// are laid on the XCD's 32 CUs in order, each on the least loaded, and a CU
+// that holds few of them runs slower by `lone` (one, two, three tiles; latency
+// is not hidden).
+// Quarters: a quarter costs 1.55 (real) or 1.35 (complex: four products per
+// value loaded) of a fourth of its tile on a full CU, but a product with fewer
+// tiles than the chip has CUs, or a few long ones, leaves CUs idle. A lone
+// quarter, bound by latency alone, takes about as long as the MFMAs of its
+// whole tile. Measured on MI355X, whole -> quarters: real 512 x 1024 x 2048 80 ->
+// 51 us, 128 x 1280 x 128 9.0 -> 5.5, 1000^3 43 -> 51, 2000^3 271 -> 368; complex 512 x
+// 1024 x 513 71 -> 47, 1300 x 701 x 400 58 -> 66.
+// Parts: a tile that would end after its XCD's share of the work is cut along K
+// into parts of an eighth of that share (a quarter where the share is less than
+// two of the longest tiles), of at least kPartK contracted values each;
+// cut[x][i] is the number of parts. A part costs 1.5 us beyond its MFMAs, the
+// join 4 us and the partial blocks' traffic.
+// They are taken where they come out 5 % (complex, which gains less than the
+// model says: 18 %) faster than whole tiles. Measured, whole -> parts with the
+// join: real 3001 x 1777 x 2049 374 -> 352 us, 4800 x 495 x 2100 195 -> 184, 1100 x
+// 3000 x 1700 217 -> 192, 2500^3 531 -> 500, 640 x 640 x 4000 147 -> 79 (quarters 94);
+// 2000^3 272 -> 288, 1000^3 43 -> 55 and 1700 x 1700 x 900 90 -> 119 stay whole. Complex
+// 1500 x 1500 x 700 247 -> 230, the last product of the chi = 1500 U(1) network 7 %
+// faster than in quarters; 2100 x 1101 x 500 180 -> 185 and 1300 x 701 x 400 58 -> 71
+// stay whole.
+constexpr int kMaxParts = 16, kPartK = 128;
+void choose_form(const std::vector<std::vector<double>>& cost,
+                 const std::vector<std::vector<double>>& depth, TileForm form[2],
+                 std::vector<std::vector<int>>* cut) {
+  const double lone[2][3] = {{1.32, 1.23, 1.08}, {1.15, 1.02, 1.0}};
+  const double quarter[2] = {1.55, 1.35};
+  const double us[2] = {525.0, 131.0};  // cost of a microsecond: 4 (complex 16) cycles per unit
+  double t_whole[2] = {0.0, 0.0}, t_quarters[2] = {0.0, 0.0}, t_parts[2] = {0.0, 0.0};
+  form[0] = form[1] = TileForm::kWhole;
+  cut->assign(cost.size(), {});
+  std::vector<double> share(cost.size(), 0.0), longest(cost.size(), 0.0);
+  for (size_t x = 0; x < cost.size(); ++x)
+    for (double t : cost[x]) share[x] += t / kCus, longest[x] = std::max(longest[x], t);
+  bool any = false;
+  double part_bytes = 0.0;  // of real data
+  for (size_t x = 0; x < cost.size(); ++x) {
+    const std::vector<double>& c = cost[x];
+    const double part = share[x] * (share[x] < 2.0 * longest[x] ? 0.25 : 0.125);
+    CuHeap whole, mixed;
+    bool cuts = false;
+    (*cut)[x].assign(c.size(), 1);
+    for (size_t i = 0; i < c.size(); ++i) {
+      if ((cuts ? mixed : whole).least() + c[i] > 1.02 * share[x]) {
+        const int n = (int)std::min(
+            {(double)kMaxParts, std::ceil(c[i] / part), std::floor(depth[x][i] / kPartK)});
+        if (n > 1) {
+          (*cut)[x][i] = n;
+          part_bytes += n * 8.0 * 256.0 * c[i] / depth[x][i];
+          if (!cuts) mixed = whole;
+          cuts = any = true;
+          whole.add(c[i]);
+          continue;
+        }
+      }
+      whole.add(c[i]);
+      if (cuts) mixed.add(c[i]);
+    }
+    for (int z = 0; z < 2; ++z) {
+      CuHeap parts = cuts ? mixed : whole;
+      for (size_t i = 0; cuts && i < c.size(); ++i)
+        if ((*cut)[x][i] > 1)
+          for (int q = 0; q < (*cut)[x][i]; ++q) parts.add(c[i] / (*cut)[x][i] + 1.5 * us[z]);
+      auto slowest = [&](const CuHeap& h) {
+        double t = 0.0;
+        for (const auto& u : h.cu)
+          if (u.tiles) t = std::max(t, u.load * (u.tiles <= 3 ? lone[z][u.tiles - 1] : 1.0));
+        return t;
+      };
+      t_whole[z] = std::max(t_whole[z], slowest(whole));
+      t_parts[z] = std::max(t_parts[z], slowest(parts));
+      t_quarters[z] = std::max({t_quarters[z], quarter[z] * share[x], 0.97 * longest[x]});
     }
   }
-  for (int x = 0; x < 2; ++x) faster[x] = t_quarters[x] < 0.9 * t_whole[x];
+  for (int z = 0; z < 2; ++z) {
+    double best = t_whole[z];
+    if (t_quarters[z] < 0.9 * t_whole[z]) {
+      form[z] = TileForm::kQuarters;
+      best = t_quarters[z];
+    }
+    const double join = (4.0 + (z ? 2 : 1) * part_bytes * 2.5 / 6e6) * us[z];
+    if (any && t_parts[z] + join < std::min(best, (z ? 0.82 : 0.95) * t_whole[z]))
+      form[z] = TileForm::kParts;
+  }
 }
 
-// First row and column of tile t of group G, in strips of kStrip tile columns
-// taken row by row; returns its live 16 x 16 blocks.
-constexpr int kStrip = 8;
-int tile_blocks(const GemmGroup& G, int32_t t, int* m0, int* n0) {
-  const int tm = (G.M + kGemmTile - 1) / kGemmTile, tn = (G.N + kGemmTile - 1) / kGemmTile;
-  const int strip = t / (tm * kStrip), r = t - strip * tm * kStrip;
-  const int width = std::min(kStrip, tn - strip * kStrip);
-  *m0 = r / width * kGemmTile;
-  *n0 = (strip * kStrip + r % width) * kGemmTile;
-  return ((std::min(G.M - *m0, kGemmTile) + 15) / 16) * ((std::min(G.N - *n0, kGemmTile) + 15) / 16);
+// The groups, pairs and joins of the parts of one tile (n of them, cut along
+// the concatenated contracted values of its group at multiples of a slice
+// within a pair, so that no cut makes a partial slice); appends the parts'
+// entries to *entries.
+void cut_tile(const ExecPlan& ep, const GemmTile& T, int n, PartTables* pt,
+              std::vector<GemmTile>* entries) {
+  constexpr int kSlice = 16;
+  const GemmGroup& G = ep.h_groups[(size_t)T.g];
+  const int M = std::min(G.M - T.m0, kGemmTile), N = std::min(G.N - T.n0, kGemmTile);
+  int64_t klen = 0;
+  for (int p = G.p0; p < G.p1; ++p) klen += std::max(ep.h_pairs[(size_t)p].K, 0);
+  int p = G.p0, kin = 0;     // the next part's first value: kin of pair p
+  int64_t done = 0;          // values before it
+  GemmJoin J{pt->elems, G.off_c + T.m0 + (int64_t)T.n0 * G.ldc, M, N, G.ldc, 0};
+  for (int q = 1; q <= n; ++q) {
+    const int64_t to = klen * q / n;
+    GemmGroup h = G;
+    h.M = M;
+    h.N = N;
+    h.ldc = M;
+    h.off_c = J.poff + (int64_t)J.S * M * N;
+    h.part = 1;
+    h.p0 = (int32_t)pt->pairs.size();
+    while (p < G.p1 && (done < to || q == n)) {
+      const GemmPair& pr = ep.h_pairs[(size_t)p];
+      const int left = std::max(pr.K, 0) - kin;
+      int take = left;
+      if (q < n && done + left > to)
+        take = std::min<int64_t>(left, (to - done + kSlice / 2) / kSlice * kSlice);
+      if (take > 0) {
+        GemmPair y = pr;
+        y.K = take;
+        y.off_a += (ep.ta ? kin : (int64_t)kin * pr.lda) + (int64_t)T.m0 * (ep.ta ? pr.lda : 1);
+        y.off_b += (ep.tb ? (int64_t)kin * pr.ldb : kin) + (int64_t)T.n0 * (ep.tb ? 1 : pr.ldb);
+        pt->pairs.push_back(y);
+      }
+      done += take;
+      kin += take;
+      if (take < left) break;
+      ++p;
+      kin = 0;
+    }
+    h.p1 = (int32_t)pt->pairs.size();
+    if (h.p1 == h.p0) continue;
+    set_first_pair(&h, pt->pairs.data());
+    entries->push_back(GemmTile{(int32_t)pt->groups.size(), 0, 0, 0});
+    pt->groups.push_back(h);
+    ++J.S;
+  }
+  pt->elems += (int64_t)J.S * M * N;
+  pt->joins.push_back(J);
 }
+
 }  // namespace
 
 // Workgroup w of a launch is dispatched to XCD w % kXcds. Cut the tiles of
@@ -1388,35 +1523,46 @@ int tile_blocks(const GemmGroup& G, int32_t t, int* m0, int* n0) {
 // tiles as the work instead of their live blocks left one XCD with 4 % more
 // than its share in the chi = 4096 U(1) network's last product: both products
 // 618 -> 604 us; split precision, which computes whole tiles, is level.
-std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, bool* quarters) {
-  constexpr int kXcds = 8;
-  struct Chunk {
-    int32_t g, t0, t1;
-    double k;     // contracted values of one of its tiles
-    double work;  // of all of them
-  };
-  std::vector<Chunk> chunks;
-  int64_t total = 0;
-  std::vector<int32_t> gt(ep.h_groups.size());
+std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, TileForm* form, PartTables* parts) {
+  constexpr int kXcds = 8, kStrip = 8;
+  // the tiles of all groups, each group's in its order; pad: live blocks
+  std::vector<GemmTile> all;
+  std::vector<size_t> first(ep.h_groups.size() + 1, 0);
+  auto sides = [](int n) { return (n + kGemmTile - 1) / kGemmTile; };
+  size_t total = 0;
+  for (const GemmGroup& G : ep.h_groups)
+    if (G.M > 0 && G.N > 0) total += (size_t)sides(G.M) * (size_t)sides(G.N);
+  all.reserve(total);
   for (size_t g = 0; g < ep.h_groups.size(); ++g) {
     const GemmGroup& G = ep.h_groups[g];
-    gt[g] = (G.M <= 0 || G.N <= 0)
-                ? 0
-                : ((G.M + kGemmTile - 1) / kGemmTile) * ((G.N + kGemmTile - 1) / kGemmTile);
-    total += gt[g];
+    first[g] = all.size();
+    if (G.M <= 0 || G.N <= 0) continue;
+    for (int s0 = 0; s0 < G.N; s0 += kStrip * kGemmTile)
+      for (int m0 = 0; m0 < G.M; m0 += kGemmTile) {
+        const int bm = (std::min(G.M - m0, kGemmTile) + 15) / 16;
+        for (int n0 = s0; n0 < std::min(G.N, s0 + kStrip * kGemmTile); n0 += kGemmTile)
+          all.push_back(
+              GemmTile{(int32_t)g, m0, n0, bm * ((std::min(G.N - n0, kGemmTile) + 15) / 16)});
+      }
   }
-  const int64_t unit = std::max<int64_t>(1, (total + 8 * kXcds - 1) / (8 * kXcds));
+  first[ep.h_groups.size()] = all.size();
+  struct Chunk {
+    size_t t0, t1;
+    double k;     // contracted values of one of its tiles
+    double work;  // of all of them
+    double most;  // of the largest one
+  };
+  std::vector<Chunk> chunks;
+  const size_t unit = std::max<size_t>(1, (total + 8 * kXcds - 1) / (8 * kXcds));
   for (size_t g = 0; g < ep.h_groups.size(); ++g) {
     double k = 0;
     for (int p = ep.h_groups[g].p0; p < ep.h_groups[g].p1; ++p) k += std::max(ep.h_pairs[p].K, 1);
-    for (int64_t t0 = 0; t0 < gt[g]; t0 += unit) {
-      const int64_t t1 = std::min<int64_t>(gt[g], t0 + unit);
-      double work = 0.0;
-      for (int64_t t = t0; t < t1; ++t) {
-        int m0, n0;
-        work += tile_blocks(ep.h_groups[g], (int32_t)t, &m0, &n0) * k;
-      }
-      chunks.push_back(Chunk{(int32_t)g, (int32_t)t0, (int32_t)t1, k, work});
+    for (size_t t0 = first[g]; t0 < first[g + 1]; t0 += unit) {
+      const size_t t1 = std::min(first[g + 1], t0 + unit);
+      int64_t blocks = 0;
+      int most = 0;
+      for (size_t t = t0; t < t1; ++t) blocks += all[t].pad, most = std::max(most, all[t].pad);
+      chunks.push_back(Chunk{t0, t1, k, (double)blocks * k, most * k});
     }
   }
   std::stable_sort(chunks.begin(), chunks.end(),
@@ -1431,26 +1577,56 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, bool* quarters) {
     mine[best].push_back(c);
   }
   // an XCD starts its longest tiles first
-  for (auto& m : mine)
-    std::stable_sort(m.begin(), m.end(), [](const Chunk& a, const Chunk& b) { return a.k > b.k; });
-  std::vector<std::vector<GemmTile>> bins(kXcds);
-  std::vector<std::vector<double>> cost(kXcds);  // of each tile: its 16 x 16 blocks times k
-  for (int x = 0; x < kXcds; ++x)
+  std::vector<size_t> count(kXcds, 0);
+  bool few = false;  // tiles, or a few long ones (else the CUs end within an eighth)
+  for (int x = 0; x < kXcds; ++x) {
+    std::stable_sort(mine[x].begin(), mine[x].end(),
+                     [](const Chunk& a, const Chunk& b) { return a.k > b.k; });
     for (const Chunk& c : mine[x]) {
-      const GemmGroup& G = ep.h_groups[(size_t)c.g];
-      for (int32_t t = c.t0; t < c.t1; ++t) {
-        GemmTile T{c.g, 0, 0, 0};
-        const int blocks = tile_blocks(G, t, &T.m0, &T.n0);
-        bins[x].push_back(T);
-        if (quarters) cost[x].push_back(blocks * c.k);
-      }
+      count[x] += c.t1 - c.t0;
+      few = few || 8.0 * c.most > load[x] / kCus;
     }
-  size_t len = 0;
-  for (auto& b : bins) len = std::max(len, b.size());
+  }
+  const size_t len = *std::max_element(count.begin(), count.end());
   std::vector<GemmTile> table(len * kXcds, GemmTile{-1, 0, 0, 0});
+  for (int x = 0; x < kXcds; ++x) {
+    size_t at = (size_t)x;
+    for (const Chunk& c : mine[x])
+      for (size_t t = c.t0; t < c.t1; ++t, at += kXcds) table[at] = all[t];
+  }
+  if (!form) return table;
+  form[0] = form[1] = TileForm::kWhole;
+  if (!few) return table;
+  // of each tile: its 16 x 16 blocks times k, and k
+  std::vector<std::vector<double>> cost(kXcds), depth(kXcds);
   for (int x = 0; x < kXcds; ++x)
-    for (size_t i = 0; i < bins[x].size(); ++i) table[i * kXcds + x] = bins[x][i];
-  if (quarters) quarters_faster(cost, quarters);
+    for (const Chunk& c : mine[x])
+      for (size_t t = c.t0; t < c.t1; ++t) {
+        cost[x].push_back(all[t].pad * c.k);
+        depth[x].push_back(c.k);
+      }
+  std::vector<std::vector<int>> cut;
+  choose_form(cost, depth, form, &cut);
+  if (form[0] != TileForm::kParts && form[1] != TileForm::kParts) return table;
+  parts->groups = ep.h_groups;
+  parts->pairs = ep.h_pairs;
+  std::vector<std::vector<GemmTile>> mixed(kXcds);
+  size_t most = 0;
+  for (int x = 0; x < kXcds; ++x) {
+    std::vector<GemmTile> last;
+    for (size_t i = 0; i < count[x]; ++i) {
+      const GemmTile& T = table[i * kXcds + x];
+      if (cut[x][i] > 1)
+        cut_tile(ep, T, cut[x][i], parts, &last);
+      else
+        mixed[x].push_back(T);
+    }
+    mixed[x].insert(mixed[x].end(), last.begin(), last.end());
+    most = std::max(most, mixed[x].size());
+  }
+  parts->tiles.assign(most * kXcds, GemmTile{-1, 0, 0, 0});
+  for (int x = 0; x < kXcds; ++x)
+    for (size_t i = 0; i < mixed[x].size(); ++i) parts->tiles[i * kXcds + x] = mixed[x][i];
   return table;
 }
 
@@ -1471,6 +1647,18 @@ static bool split_cplx_scale(const ExecPlan& ep, int cplx, bool alpha_cplx) {
 constexpr int64_t kKsSplitPrecK = 1 << 17;
 bool ksplit_takes_split_prec(const ExecPlan& ep) {
   return ep.ks_grid > 0 && ep.ks_maxk >= kKsSplitPrecK;
+}
+
+size_t exec_part_bytes(const ExecPlan& ep, int cplx, int prec) {
+  if (ep.strategy != ExecPlan::GEMM || prec != 0 || ep.ks_grid > 0 || !ep.launch ||
+      ep.launch->form[cplx] != TileForm::kParts)
+    return 0;
+  // A run in the library's fixed scratch buffer gives the same bits as one in a
+  // handle's workspace: no part form where it alone would not fit the former.
+  const size_t base = align256(exec_workspace_bytes(ep, cplx, 0));
+  const size_t extra = align256((size_t)ep.launch->part_elems * (cplx ? 16 : 8));
+  const size_t fixed = ITG_NOALLOC_SCRATCH_BYTES;
+  return base <= fixed && base + extra > fixed ? 0 : extra;
 }
 
 size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_cplx) {
@@ -1611,7 +1799,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
     TimeScope ts(kt, "split_gemm_kernel", s);
     const SplitPair* pairs = (const SplitPair*)ep.s_pairs.p;
     const GemmGroup* groups = (const GemmGroup*)ep.s_groups.p;
-    const GemmTile* tiles = (const GemmTile*)gl.tiles.p;
+    const GemmTile* tiles = gl.tiles;
     return cplx ? launch_split_gemm_cplx(s, prec, conja, conjb, pairs, groups, tiles, gl.grid,
                                          planesA, planesB, expA, expB, out, ga, beta, part)
                 : launch_split_gemm(s, prec, pairs, groups, tiles, gl.grid, planesA, planesB,
@@ -1686,7 +1874,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
 hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err, KernelTimer* kt,
-                    bool may_build) {
+                    bool may_build, bool parts) {
   hipError_t e;
   if (ep.strategy == ExecPlan::DIRECT) {
     {
@@ -1781,7 +1969,7 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
       TimeScope ts(kt, "gemm_f64_kernel", s);
       e = launch_gemm_f64(s, cplx, ep.ta, ep.tb, (const GemmPair*)ep.ks_pairs.p,
                           (const GemmGroup*)ep.ks_groups.p, (const GemmTile*)ep.ks_tiles.p,
-                          ep.ks_grid, false, A, B, w, gflags, a_re, a_im, 0.0, 0.0);
+                          ep.ks_grid, false, A, B, w, nullptr, gflags, a_re, a_im, 0.0, 0.0);
     }
     if (e == hipSuccess) {
       TimeScope ts(kt, "ksplit_reduce_kernel", s);
@@ -1799,12 +1987,24 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
     return e;
   }
   GemmLaunch& gl = *ep.launch;
-  {
+  if (parts && gl.form[cplx] == TileForm::kParts) {
+    // the cut tiles' partial blocks go behind the workspace's other buffers
+    void* P = (char*)ws + align256(exec_workspace_bytes(ep, cplx, 0));
+    {
+      TimeScope ts(kt, "gemm_f64_kernel", s);
+      e = launch_gemm_f64(s, cplx, ep.ta, ep.tb, gl.part_pairs, gl.part_groups, gl.part_tiles,
+                          gl.part_grid, false, A, B, C, P, gflags, a_re, a_im, gbr, gbi);
+    }
+    if (e == hipSuccess) {
+      TimeScope ts(kt, "gemm_join_kernel", s);
+      e = launch_gemm_join(s, cplx, gl.joins, gl.njoin, P, C, gbr, gbi);
+    }
+  } else {
     TimeScope ts(kt, "gemm_f64_kernel", s);
     e = launch_gemm_f64(s, cplx, ep.ta, ep.tb, (const GemmPair*)ep.g_pairs.p,
-                        (const GemmGroup*)ep.g_groups.p, (const GemmTile*)gl.tiles.p, gl.grid,
-                        gl.quarters[cplx], A, B, C, gflags, a_re,
-                        a_im, gbr, gbi);
+                        (const GemmGroup*)ep.g_groups.p, gl.tiles, gl.grid,
+                        gl.form[cplx] == TileForm::kQuarters, A, B, C, nullptr, gflags, a_re, a_im,
+                        gbr, gbi);
   }
   if (e != hipSuccess) {
     char what[160];

@@ -109,11 +109,25 @@ struct PermuteLaunch {
   DevBuf blocks, prefix;
 };
 
-// Workgroup table of a plan's GEMM (FP64 and split).
+// How the FP64 GEMM runs a plan's tiles: whole, each as four 32 x 32 quarters,
+// or with some of them cut into parts along K (see GemmJoin).
+enum class TileForm { kWhole, kQuarters, kParts };
+
+// Workgroup tables of a plan's GEMM. tiles / grid: the whole tiles (split
+// precision, and FP64 in the other two forms). The part form has tables of
+// its own: the tiles it leaves whole and the parts, the plan's groups and
+// pairs followed by those of the parts, and the join of every cut tile.
 struct GemmLaunch {
   int64_t grid = 0;   // entries, idle padding included
-  bool quarters[2] = {false, false};  // FP64, real / complex: 32 x 32 workgroups
-  DevBuf tiles;       // GemmTile per entry
+  TileForm form[2] = {TileForm::kWhole, TileForm::kWhole};  // FP64, real / complex
+  DevBuf tab;         // all tables
+  const GemmTile* tiles = nullptr;
+  int64_t part_grid = 0, njoin = 0;
+  int64_t part_elems = 0;  // of the partial buffer
+  const GemmTile* part_tiles = nullptr;
+  const GemmGroup* part_groups = nullptr;
+  const GemmPair* part_pairs = nullptr;
+  const GemmJoin* joins = nullptr;
 };
 
 struct ExecPlan {
@@ -217,7 +231,8 @@ void build_permute_tables(PermuteLaunch* pl, int n, const int* perm, const Block
                           const std::vector<int64_t>* dst_offs, const std::vector<uint8_t>* fresh,
                           std::vector<PermBlock>* blocks, std::vector<int64_t>* prefix);
 
-// Launch the plan. ws: workspace of at least exec_workspace_bytes().
+// Launch the plan. ws: workspace of at least exec_workspace_bytes(); parts: and of
+// exec_part_bytes() behind it, so the FP64 GEMM may run in its part form.
 // alpha_cplx: the call's alpha has a nonzero imaginary part.
 size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_cplx = false);
 // kt (optional) brackets each launch with timer events. may_build = false:
@@ -226,7 +241,7 @@ size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_c
 hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err,
-                    KernelTimer* kt = nullptr, bool may_build = true);
+                    KernelTimer* kt = nullptr, bool may_build = true, bool parts = false);
 // Builds the plan's tile table once (kGemmTile square tiles for every plan).
 // FP64, timed on MI355X against the other shapes (128x128, 128x64, 64x128
 // real; 128x64 complex): the fastest or within 3 % of it for the two-site
@@ -240,9 +255,21 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
 // two GEMMs, 4096^3 1.08 against 1.24 and 1.16, 1000^3 22 against 41 and 37 us,
 // 1100 x 8000 x 1100 0.22 against 0.28 and 0.235.
 hipError_t ensure_gemm_launch(ExecPlan& ep, hipStream_t s, bool may_build = true);
-// XCD-balanced tile table. quarters (optional, two values):
-// whether the FP64 GEMM should run it as quarter tiles (real, complex).
-std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, bool* quarters);
+// Bytes of the partial buffer that exec_run needs beyond exec_workspace_bytes()
+// to run the plan in its part form: 0 if it has none or it is not built yet.
+size_t exec_part_bytes(const ExecPlan& ep, int cplx, int prec);
+// The tables of the part form on the host (empty when no tile is cut).
+struct PartTables {
+  std::vector<GemmTile> tiles;
+  std::vector<GemmGroup> groups;
+  std::vector<GemmPair> pairs;
+  std::vector<GemmJoin> joins;
+  int64_t elems = 0;
+};
+// XCD-balanced tile table. form (optional, two values: real, complex): how
+// the FP64 GEMM should run it, with the tables of the part form in *parts.
+std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, TileForm* form = nullptr,
+                                     PartTables* parts = nullptr);
 
 // Two consecutive matrix-form fiber contractions run as one pass (see
 // ChainGroup). Built from the two steps' plans; the device tables live here.

@@ -274,7 +274,8 @@ __global__ void __launch_bounds__(kThreads, 3)  // waves per SIMD
     gemm_f64_kernel(const GemmPair* __restrict__ pairs, const GemmGroup* __restrict__ groups,
                     const GemmTile* __restrict__ tiles, int quarters,
                     const double* __restrict__ Ag, const double* __restrict__ Bg,
-                    double* __restrict__ Cg, unsigned flags, double ga_re, double ga_im,
+                    double* __restrict__ Call, double* __restrict__ Pall, unsigned flags,
+                    double ga_re, double ga_im,
                     double beta_re, double beta_im) {
   constexpr int NPLANE = CPLX ? 2 : 1;
   using OpA = Operand<CPLX, TA ? 1 : 0>;
@@ -294,6 +295,8 @@ __global__ void __launch_bounds__(kThreads, 3)  // waves per SIMD
   if (tile->g < 0) return;  // padding slot of the XCD-balanced table
   const GroupTable grp = (GroupTable)(uintptr_t)(groups + tile->g);
   const int ldc = grp->ldc;
+  double* const Cg = grp->part ? Pall : Call;
+  const bool use_beta = !grp->part && (beta_re != 0.0 || beta_im != 0.0);
   const int m0 = tile->m0 + (quarter & 1) * side, n0 = tile->n0 + (quarter >> 1) * side;
   if (m0 >= grp->M || n0 >= grp->N) return;
   // rows and columns of this workgroup: [m0, M) x [n0, N)
@@ -524,7 +527,6 @@ __global__ void __launch_bounds__(kThreads, 3)  // waves per SIMD
     // v_mfma_f64_16x16x4_f64 leaves D[i][j] in lane j + 16*(i%4), register
     // i/4 (rows interleaved across the four lane groups), so with D = (A B)^T
     // this lane holds C[m = l16][n = lk + 4*r] of each 16x16 block.
-    const bool use_beta = (beta_re != 0.0 || beta_im != 0.0);
 #pragma unroll
     for (int i = 0; i < NM; ++i) {
       const int gm = m0 + w_m + i * 16 + l16;
@@ -590,6 +592,45 @@ __global__ void __launch_bounds__(kThreads, 3)  // waves per SIMD
     run(c1, c2, w_m, w_n);
   else
     run(c1, c1, w_m, w_n);
+}
+
+// C of the tiles computed in parts along K: four workgroups per tile, each
+// thread up to four elements of it, every part's value added in order. Beta is
+// applied as the GEMM's epilogue does.
+template <int CPLX>
+__global__ void __launch_bounds__(kThreads)
+    gemm_join_kernel(const GemmJoin* __restrict__ joins, const double* __restrict__ P,
+                     double* __restrict__ C, double beta_re, double beta_im) {
+  const GemmJoin J = joins[blockIdx.x >> 2];
+  const bool use_beta = (beta_re != 0.0 || beta_im != 0.0);
+  const int mn = J.M * J.N;
+  for (int e = (int)(blockIdx.x & 3) * kThreads + (int)threadIdx.x; e < mn; e += 4 * kThreads) {
+    const int n = e / J.M, m = e - n * J.M;
+    const int64_t o = J.off_c + m + (int64_t)n * J.ldc;
+    if (CPLX) {
+      const double2* p = reinterpret_cast<const double2*>(P) + J.poff + e;
+      double2 v = p[0];
+#pragma unroll 4
+      for (int q = 1; q < J.S; ++q) {
+        const double2 w = p[(int64_t)q * mn];
+        v.x += w.x;
+        v.y += w.y;
+      }
+      if (use_beta) {
+        const double2 c = reinterpret_cast<double2*>(C)[o];
+        v.x += beta_re * c.x - beta_im * c.y;
+        v.y += beta_re * c.y + beta_im * c.x;
+      }
+      reinterpret_cast<double2*>(C)[o] = v;
+    } else {
+      const double* p = P + J.poff + e;
+      double v = p[0];
+#pragma unroll 4
+      for (int q = 1; q < J.S; ++q) v += p[(int64_t)q * mn];
+      if (use_beta) v = fma(beta_re, C[o], v);
+      C[o] = v;
+    }
+  }
 }
 
 // The block of output element e, found by binary search over the blocks'
@@ -958,18 +999,33 @@ hipError_t launch_ksplit_skinny(hipStream_t s, int cplx, int kc, int ta, int tb,
   return hipGetLastError();
 }
 
+hipError_t launch_gemm_join(hipStream_t s, int cplx, const GemmJoin* joins, int64_t n,
+                            const void* P, void* C, double beta_re, double beta_im) {
+  if (n == 0) return hipSuccess;
+  if (n > INT32_MAX / 4) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(4 * n));
+  if (cplx)
+    ITG_LAUNCH((gemm_join_kernel<1>), grid, dim3(kThreads), 0, s, joins, (const double*)P,
+               (double*)C, beta_re, beta_im);
+  else
+    ITG_LAUNCH((gemm_join_kernel<0>), grid, dim3(kThreads), 0, s, joins, (const double*)P,
+               (double*)C, beta_re, beta_im);
+  return hipGetLastError();
+}
+
 hipError_t launch_gemm_f64(hipStream_t s, int cplx, int ta, int tb, const GemmPair* pairs,
                            const GemmGroup* groups, const GemmTile* tiles, int64_t entries,
-                           bool quarters, const void* A, const void* B, void* C, unsigned flags, double ga_re, double ga_im,
-                           double beta_re, double beta_im) {
+                           bool quarters, const void* A, const void* B, void* C, void* P,
+                           unsigned flags, double ga_re, double ga_im, double beta_re,
+                           double beta_im) {
   const int64_t grid = quarters ? 4 * entries : entries;
   if (grid == 0) return hipSuccess;
   if (entries % 8 || grid > INT32_MAX) return hipErrorInvalidValue;
 #define ITG_GEMM_CASE(c, a, b)                                                                   \
   if ((cplx != 0) == c && (ta != 0) == a && (tb != 0) == b) {                                    \
     ITG_LAUNCH((gemm_f64_kernel<c, a, b>), dim3((unsigned)grid), dim3(kThreads), 0, s, pairs,    \
-               groups, tiles, (int)quarters, (const double*)A, (const double*)B, (double*)C, flags, ga_re, \
-               ga_im, beta_re, beta_im);                                                         \
+               groups, tiles, (int)quarters, (const double*)A, (const double*)B, (double*)C,     \
+               (double*)P, flags, ga_re, ga_im, beta_re, beta_im);                               \
     return hipGetLastError();                                                                    \
   }
   ITG_GEMM_CASE(0, 0, 0)
