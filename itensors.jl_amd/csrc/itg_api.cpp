@@ -300,7 +300,7 @@ hipError_t ready_ws(itg_handle* h, ExecPlan& ep, int cplx, int prec, size_t need
 
 itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void* T1,
                     const void* T2, void* R, unsigned flags, const double* alpha,
-                    const double* beta) {
+                    const double* beta, unsigned f32 = 0) {
   const double a_re = alpha ? alpha[0] : 1.0, a_im = (alpha && cplx) ? alpha[1] : 0.0;
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
   std::string err;
@@ -309,9 +309,30 @@ itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void*
                           &parts);
   if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
   e = exec_run(ep, cplx, prec, h->stream, h->ws, T1, T2, R, flags, a_re, a_im, b_re, b_im,
-               &err, active_timer(h), true, parts);
+               &err, active_timer(h), true, parts, f32);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
+  return ITG_OK;
+}
+
+// Float32 / ComplexF32 data (dt): FP64 (MFMA) whatever the precision mode, as
+// Float32 values are exact in FP64 and the split form has nothing to emulate.
+// Operands that the plan permutes are read as they are; the others are
+// widened first.
+itg_status run_plan32(itg_handle* h, ExecPlan& ep, itg_dtype dt, int64_t n1, const void* T1,
+                      int64_t n2, const void* T2, int64_t nR, void* R, unsigned flags,
+                      const double* alpha, const double* beta) {
+  const int cplx = dt == ITG_C64;
+  const unsigned f32 = exec_reads_f32(ep);
+  Wide w;
+  itg_status st = widen_operands(h, dt, f32 & 1u ? 0 : n1, T1, f32 & 2u ? 0 : n2, T2, nR, &w);
+  if (st != ITG_OK) return st;
+  st = run_plan(h, ep, cplx, ITG_PREC_FP64, f32 & 1u ? T1 : w.t1, f32 & 2u ? T2 : w.t2, w.r, flags,
+                alpha, nullptr, f32);
+  if (st != ITG_OK) return st;
+  hipError_t e = launch_narrow(h->stream, cplx, nR, w.r, R, beta ? beta[0] : 0.0,
+                               (beta && cplx) ? beta[1] : 0.0);
+  if (e != hipSuccess) return hip_fail(h, e, "narrow launch");
   return ITG_OK;
 }
 
@@ -784,23 +805,6 @@ itg_status itg_contract_dense_ex(itg_handle* h, itg_dtype dtype, int NR, const i
     return fail(h, ITG_ERR_UNSUPPORTED, "tensor with more than 2^31-1 elements");
   if (nR == 0) return ITG_OK;
   if (!R || (n1 > 0 && !T1) || (n2 > 0 && !T2)) return fail(h, ITG_ERR_INVALID, "null data pointer");
-  if (dtype32(dtype)) {
-    // FP64 (MFMA) on widened copies, whatever the precision mode: Float32
-    // values are exact in FP64, so the split form has nothing to emulate
-    DeviceGuard g(h->device);
-    Wide w;
-    itg_status st = widen_operands(h, dtype, n1, T1, n2, T2, nR, &w);
-    if (st != ITG_OK) return st;
-    st = itg_contract_dense_ex(h, wide_of(dtype), NR, dimsR, labelsR, w.r, N1, dims1, labels1,
-                               w.t1, N2, dims2, labels2, w.t2, alpha, nullptr, ITG_PREC_FP64,
-                               flags);
-    if (st != ITG_OK) return st;
-    const int c = dtype == ITG_C64;
-    hipError_t e = launch_narrow(h->stream, c, nR, w.r, R, beta ? beta[0] : 0.0,
-                                 (beta && c) ? beta[1] : 0.0);
-    if (e != hipSuccess) return hip_fail(h, e, "narrow launch");
-    return ITG_OK;
-  }
   const int cplx = dtype == ITG_C128;
   DeviceGuard g(h->device);
 
@@ -858,6 +862,8 @@ itg_status itg_contract_dense_ex(itg_handle* h, itg_dtype dtype, int NR, const i
       h->dense_lru.pop_back();
     }
   }
+  if (dtype32(dtype))
+    return run_plan32(h, *ep, dtype, n1, T1, n2, T2, nR, R, flags, alpha, beta);
   return run_plan(h, *ep, cplx, (int)prec, T1, T2, R, flags, alpha, beta);
 }
 
@@ -1229,24 +1235,14 @@ itg_status itg_bs_execute(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void* 
   if (p->pairs.empty()) return ITG_OK;
   if (!R || !T1 || !T2) return fail(h, ITG_ERR_INVALID, "null data pointer");
   if (p->device != h->device) return fail(h, ITG_ERR_INVALID, "plan built on another device");
-  if (dtype32(dtype)) {
-    DeviceGuard g(h->device);
-    Wide w;
-    itg_status st = widen_operands(h, dtype, extent_of(p->b1, false), T1,
-                                   extent_of(p->b2, false), T2, p->bR.nnz, &w);
-    if (st != ITG_OK) return st;
-    st = itg_bs_execute(h, p, wide_of(dtype), w.r, w.t1, w.t2, alpha, pair_alpha,
-                        ITG_PREC_FP64, flags & kFlagConj);
-    if (st != ITG_OK) return st;
-    hipError_t e = launch_narrow(h->stream, dtype == ITG_C64, p->bR.nnz, w.r, R, 0.0, 0.0);
-    if (e != hipSuccess) return hip_fail(h, e, "narrow launch");
-    return ITG_OK;
-  }
-  const int cplx = dtype == ITG_C128;
+  const int cplx = dtype == ITG_C128 || dtype == ITG_C64;
   DeviceGuard g(h->device);
   ExecPlan* ep = nullptr;
   itg_status st = plan_for_factors(h, p, pair_alpha, cplx, true, &ep);
   if (st != ITG_OK) return st;
+  if (dtype32(dtype))
+    return run_plan32(h, *ep, dtype, extent_of(p->b1, false), T1, extent_of(p->b2, false), T2,
+                      p->bR.nnz, R, flags & kFlagConj, alpha, nullptr);
   if ((st = check_reuse(h, *ep, cplx, (int)prec, T1, T2, flags)) != ITG_OK) return st;
   return run_plan(h, *ep, cplx, (int)prec, T1, T2, R, flags, alpha, nullptr);
 }

@@ -153,7 +153,15 @@ inline hipError_t launch_kernel(void (*kernel)(KArgs...), dim3 grid, dim3 block,
 // `esize` is 1 for Float64 and 2 for ComplexF64.
 
 // Element types of the data-movement kernels.
-enum EltCode { kEltF64 = 0, kEltC128 = 1, kEltF32 = 2, kEltC64 = 3 };
+enum EltCode {
+  kEltF64 = 0,
+  kEltC128 = 1,
+  kEltF32 = 2,
+  kEltC64 = 3,
+  // permutations only: Float32 / ComplexF32 source, FP64 destination
+  kEltF32ToF64 = 4,
+  kEltC64ToC128 = 5,
+};
 // Grouped permutation. tile_prefix has nblk+1 entries (workgroups before
 // block b). elt: EltCode (0 / 1 = the cplx flag of the FP64 paths). nzflags
 // (optional, nblk ints, cleared by the launcher): set to 1 for every block

@@ -1871,10 +1871,16 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
 
 }  // namespace
 
+unsigned exec_reads_f32(const ExecPlan& ep) {
+  if (ep.strategy != ExecPlan::GEMM) return 0u;
+  const unsigned a = ep.permA ? 1u : 0u, b = ep.permB ? 1u : 0u;
+  return ep.swap ? a << 1 | b : a | b << 1;
+}
+
 hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err, KernelTimer* kt,
-                    bool may_build, bool parts) {
+                    bool may_build, bool parts, unsigned f32) {
   hipError_t e;
   if (ep.strategy == ExecPlan::DIRECT) {
     {
@@ -1917,10 +1923,14 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
   const void* A = ep.swap ? T2 : T1;
   const void* B = ep.swap ? T1 : T2;
   unsigned gflags = ep.swap ? (((flags & 1u) << 1) | ((flags & 2u) >> 1)) : (flags & kFlagConj);
+  // element code of a permutation of operand `op` (a bit of f32)
+  auto elt = [&](unsigned op) {
+    return f32 & op ? (cplx ? (int)kEltC64ToC128 : (int)kEltF32ToF64) : cplx;
+  };
   if (ep.permA) {
     {
       TimeScope ts(kt, "permute_kernel", s);
-      e = launch_permute(s, cplx, ep.pA.nm, (const PermBlock*)ep.pA.blocks.p,
+      e = launch_permute(s, elt(ep.swap ? 2u : 1u), ep.pA.nm, (const PermBlock*)ep.pA.blocks.p,
                          (const int64_t*)ep.pA.prefix.p, ep.pA.nblk, ep.pA.tiles, A,
                          w, 1.0, 0.0, 0.0, 0.0);
     }
@@ -1934,7 +1944,7 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
   if (ep.permB) {
     {
       TimeScope ts(kt, "permute_kernel", s);
-      e = launch_permute(s, cplx, ep.pB.nm, (const PermBlock*)ep.pB.blocks.p,
+      e = launch_permute(s, elt(ep.swap ? 1u : 2u), ep.pB.nm, (const PermBlock*)ep.pB.blocks.p,
                          (const int64_t*)ep.pB.prefix.p, ep.pB.nblk, ep.pB.tiles, B,
                          w, 1.0, 0.0, 0.0, 0.0);
     }

@@ -241,7 +241,11 @@ size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_c
 hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err,
-                    KernelTimer* kt = nullptr, bool may_build = true, bool parts = false);
+                    KernelTimer* kt = nullptr, bool may_build = true, bool parts = false,
+                    unsigned f32 = 0);
+// Operands (bit 0: T1, bit 1: T2) that exec_run may be given as Float32 /
+// ComplexF32 data (its f32) in FP64 precision: those that it permutes first.
+unsigned exec_reads_f32(const ExecPlan& ep);
 // Builds the plan's tile table once (kGemmTile square tiles for every plan).
 // FP64, timed on MI355X against the other shapes (128x128, 128x64, 64x128
 // real; 128x64 complex): the fastest or within 3 % of it for the two-site
