@@ -266,6 +266,14 @@ struct DeviceGuard {
   }
 };
 
+// A plan of few contracted values may run on the GEMM, with a small workspace,
+// or on kernels that need none: the workspace is made with the plan, so that a
+// first run under capture finds it. (A failure is the run's to report.)
+void reserve_plan_ws(itg_handle* h, const ExecPlan& ep) {
+  if (ep.fp64_only && ensure_ws(h, exec_workspace_bytes(ep, 1, 0)) != hipSuccess)
+    (void)hipGetLastError();
+}
+
 // The handle's timer while timing is on and the stream is not being captured.
 KernelTimer* active_timer(itg_handle* h) {
   if (!h->timing || !h->timer) return nullptr;
@@ -281,7 +289,8 @@ KernelTimer* active_timer(itg_handle* h) {
 // under capture) the plan runs without.
 hipError_t ready_ws(itg_handle* h, ExecPlan& ep, int cplx, int prec, size_t need, bool* parts) {
   *parts = false;
-  if (ep.strategy == ExecPlan::GEMM && prec == ITG_PREC_FP64 && ep.ks_grid == 0)
+  if (ep.strategy == ExecPlan::GEMM && (prec == ITG_PREC_FP64 || ep.fp64_only) &&
+      ep.ks_grid == 0)
     (void)ensure_gemm_launch(ep, h->stream);  // a failure is exec_run's to report
   const size_t extra = exec_part_bytes(ep, cplx, prec);
   if (extra) {
@@ -399,6 +408,7 @@ itg_status plan_for_factors(itg_handle* h, itg_bs_plan* p, const double* pair_al
         build_exec_plan(p->st, p->b1, p->b2, p->bR, p->pairs, pa.data(), h->stream, np.get(),
                         p->backend);
     if (!err.empty()) return fail(h, ITG_ERR_HIP, err);
+    reserve_plan_ws(h, *np);
     it = p->ep_alpha.emplace(pa, std::move(np)).first;
   }
   *out = it->second.get();
@@ -1044,6 +1054,7 @@ itg_status itg_bs_plan_create(itg_handle* h, int N1, int64_t nblk1, const int64_
     std::string err = build_exec_plan(p->st, p->b1, p->b2, p->bR, p->pairs, nullptr, h->stream,
                                       p->ep.get(), p->backend);
     if (!err.empty()) return fail(h, ITG_ERR_HIP, err);
+    reserve_plan_ws(h, *p->ep);
   }
   *out = p.release();
   return ITG_OK;
@@ -1576,6 +1587,7 @@ itg_status itg_batch_plan_create(itg_handle* h, itg_dtype dtype, int64_t nbatch,
   p->ep.reset(new ExecPlan);
   m = build_exec_plan(st, L1, L2, LR, pairs, nullptr, h->stream, p->ep.get(), h->backend);
   if (!m.empty()) return fail(h, ITG_ERR_HIP, m);
+  reserve_plan_ws(h, *p->ep);
   *out = p.release();
   return ITG_OK;
 }

@@ -430,14 +430,15 @@ std::string build_fiber_mv(const Structure& st, const BlockList& TA, const Block
   return "";
 }
 
-// FIBER tables. Returns false (nothing built) when the shape does not suit:
+// FIBER tables, of the matrix form or of the loop form. Returns false (nothing
+// built) when the shape does not suit:
 // the smaller operand is not at most a quarter of the larger, the larger has
 // no free mode, too few fibers, or too many B-free elements per output block.
 // On an upload failure returns true with *err set.
 bool build_fiber_tables(const Structure& st, const BlockList& b1, const BlockList& b2,
                         const BlockList& bR, const std::vector<PairSpec>& pairs,
                         const std::vector<std::pair<size_t, size_t>>& granges,
-                        const double* pair_alpha, hipStream_t s, ExecPlan* ep,
+                        const double* pair_alpha, bool matrix, hipStream_t s, ExecPlan* ep,
                         std::string* err) {
   const int NR = st.NR, nk = st.nk;
   // operand sizes over the blocks the pairs touch
@@ -498,8 +499,7 @@ bool build_fiber_tables(const Structure& st, const BlockList& b1, const BlockLis
     comp_granges[(size_t)c].push_back(gi);
   }
 
-  // The matrix form when every group has few enough slots and outputs.
-  {
+  if (matrix) {  // when every group has few enough slots and outputs
     bool fits = true;
     for (size_t c = 0; c < comp_granges.size() && fits; ++c) {
       std::map<int64_t, int64_t> kOfA;  // distinct A blocks -> K
@@ -527,6 +527,7 @@ bool build_fiber_tables(const Structure& st, const BlockList& b1, const BlockLis
         return true;
       }
     }
+    return false;
   }
 
   std::vector<FiberGroup> fg(comp_granges.size());
@@ -823,6 +824,7 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
   // per-pair shape figures
   double mnk = 0.0, mn = 0.0, flops = 0.0;
   int64_t maxdim = 0;
+  std::vector<double> pk(pairs.size()), pm(pairs.size()), pn(pairs.size());
   for (size_t p = 0; p < pairs.size(); ++p) {
     const int32_t* d1 = b1.d(pairs[p].blk1);
     const int32_t* d2 = b2.d(pairs[p].blk2);
@@ -834,6 +836,9 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
       else
         N *= d2[st.r_pos[r]];
     }
+    pk[p] = K;
+    pm[p] = M;
+    pn[p] = N;
     mnk += M * N * K;
     mn += M * N;
     flops += 2.0 * M * N * K;
@@ -864,10 +869,11 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
     }
   };
 
-  if (!use_gemm) {
+  // The loop form of the fiber kernel, or the strided kernel.
+  auto build_strided = [&]() -> std::string {
     std::string ferr;
     if (backend != kBackendGeneric &&
-        build_fiber_tables(st, b1, b2, bR, pairs, granges, pair_alpha, s, ep, &ferr)) {
+        build_fiber_tables(st, b1, b2, bR, pairs, granges, pair_alpha, false, s, ep, &ferr)) {
       ep->strategy = ExecPlan::FIBER;
       return ferr;
     }
@@ -954,6 +960,15 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
         (e = ep->d_wgg.upload(wgg.data(), wgg.size() * sizeof(int32_t), s)) != hipSuccess)
       return std::string("device table upload failed: ") + hipGetErrorString(e);
     return "";
+  };
+  if (!use_gemm) {
+    std::string ferr;
+    if (backend != kBackendGeneric &&
+        build_fiber_tables(st, b1, b2, bR, pairs, granges, pair_alpha, true, s, ep, &ferr)) {
+      ep->strategy = ExecPlan::FIBER;
+      return ferr;
+    }
+    if (backend != kBackendAuto || nk == 0 || kavg < 2.0) return build_strided();
   }
 
   // ------------------------------------------------------------- GEMM
@@ -1033,6 +1048,53 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
   };
   Choice c1 = evaluate(true), c2 = evaluate(false);
   Choice& ch = (c2.cost < c1.cost) ? c2 : c1;
+  if (!use_gemm) {
+    // Few contracted values and no matrix form: the GEMM or the strided kernels,
+    // by estimates of their times in us (fitted to MI355X runs). The GEMM
+    // spends 0.6 on a pair's slice, one tile per workgroup, and 4.5 on each
+    // permutation; the strided kernel 0.25 on a contracted value (dependent
+    // loads) and 1 on a million products; the loop form of the fiber kernel,
+    // which goes before it where it applies (build_fiber_tables), about 0.1 on
+    // each output and contracted value of a fiber. Measured, before -> GEMM: 2000
+    // x 16 x 2000 65 -> 12 us, 300 x 12 x 400 7.7 -> 4.1, 50 x 20 x 60 10 -> 4.4, 1000 x 4
+    // x 1000 7.2 -> 5.7, both products of the U(1) network at chi = 126 26 -> 15 and
+    // at 230 65 -> 18, fiber kernel 200 x 10 x 3000 657 -> 5, a chi = 200 U(1)
+    // gradient's kernels 893 -> 248; 17 x 6 x 13 x 40 with a permuted operand 5.2
+    // -> 9.2 stays. The products stay in FP64 in every precision mode and their
+    // permuted copies fit the fixed scratch buffer, as the strided kernels
+    // need neither.
+    double klen = 0.0, npair = 0.0, tiles = 0.0, parts = 0.0, fiber = 0.0, fibers = 0.0;
+    const bool big2 = b2.nnz > b1.nnz;
+    for (const auto& gr : granges) {
+      double k = 0.0, f = 0.0;
+      for (size_t p = gr.first; p < gr.second; ++p) {
+        k += pk[p];
+        f += pk[p] * (big2 ? pm[p] : pn[p]);
+      }
+      const double m = pm[gr.first], n = pn[gr.first];
+      klen = std::max(klen, k);
+      npair = std::max(npair, (double)(gr.second - gr.first));
+      fiber = std::max(fiber, f);
+      fibers += big2 ? n : m;
+      tiles += std::ceil(m / kGemmTile) * std::ceil(n / kGemmTile);
+      parts += std::ceil(m * n / kDirectElemsPerWG);
+    }
+    auto elems = [](const BlockList& T) {
+      double n = 0.0;
+      for (int64_t b = 0; b < T.nblk(); ++b) n += (double)block_size(T, b);
+      return n;
+    };
+    const double copied =
+        (ch.permA ? elems(P) : 0.0) + (ch.permB ? elems(Q) : 0.0) + (permC ? elems(bR) : 0.0);
+    const int nperm = (int)ch.permA + (int)ch.permB + (int)permC;
+    const double t_gemm = 4.0 + 0.6 * npair * std::max(1.0, tiles / 768.0) + 4.5 * nperm +
+                          copied * 16.0 / 3e6 + mn * 8.0 / 4e6 + mnk / 1.5e7;
+    double t_strided = 4.0 + 0.25 * klen * std::max(1.0, parts / 2048.0) + mnk / 1e6;
+    if (fibers >= 256.0 && 4 * std::min(b1.nnz, b2.nnz) <= std::max(b1.nnz, b2.nnz))
+      t_strided = 5.0 + 0.1 * fiber;
+    if (t_gemm > 0.8 * t_strided || copied * 16.0 > (double)(28 << 20)) return build_strided();
+    ep->fp64_only = true;
+  }
   ep->swap = swap;
   ep->permC = permC;
   ep->permA = ch.permA;
@@ -1141,6 +1203,12 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
     return std::string("device table upload failed: ") + hipGetErrorString(e);
   std::string kerr = build_ksplit(ep, s);
   if (!kerr.empty()) return kerr;
+  if (ep->fp64_only) {
+    // as the strided kernels, ready to run without building anything
+    if (ep->ks_grid == 0 && (e = ensure_gemm_launch(*ep, s)) != hipSuccess)
+      return std::string("device table upload failed: ") + hipGetErrorString(e);
+    return "";
+  }
   std::string serr = build_split_tables(ep, P, Q, Mp, Nq, ch.Xp, ch.Xq, pairs, swap, s);
   if (!serr.empty()) return serr;
   return "";
@@ -1650,6 +1718,7 @@ bool ksplit_takes_split_prec(const ExecPlan& ep) {
 }
 
 size_t exec_part_bytes(const ExecPlan& ep, int cplx, int prec) {
+  if (ep.fp64_only) prec = 0;
   if (ep.strategy != ExecPlan::GEMM || prec != 0 || ep.ks_grid > 0 || !ep.launch ||
       ep.launch->form[cplx] != TileForm::kParts)
     return 0;
@@ -1663,6 +1732,7 @@ size_t exec_part_bytes(const ExecPlan& ep, int cplx, int prec) {
 
 size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_cplx) {
   if (ep.strategy != ExecPlan::GEMM) return 0;
+  if (ep.fp64_only) prec = 0;
   const size_t es = cplx ? 16 : 8;
   size_t b = 0;
   if (prec != 0 && ksplit_takes_split_prec(ep)) prec = 0;
@@ -1683,7 +1753,7 @@ size_t exec_workspace_bytes(const ExecPlan& ep, int cplx, int prec, bool alpha_c
     if (ep.permB) b += align256((size_t)ep.nnzB * es);
   }
   if (ep.permC) b += align256((size_t)ep.nnzC * es);
-  return b + 1024;
+  return b ? b + 1024 : 0;
 }
 
 namespace {
@@ -1881,6 +1951,7 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
                     const void* T1, const void* T2, void* R, unsigned flags, double a_re,
                     double a_im, double b_re, double b_im, std::string* err, KernelTimer* kt,
                     bool may_build, bool parts, unsigned f32) {
+  if (ep.fp64_only) prec = 0;
   hipError_t e;
   if (ep.strategy == ExecPlan::DIRECT) {
     {

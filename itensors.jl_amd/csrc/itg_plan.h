@@ -161,6 +161,7 @@ struct ExecPlan {
   std::vector<GemmPair> h_pairs;
   std::vector<GemmGroup> h_groups;
   std::vector<double> group_cost;  // flops per group (for LPT ordering)
+  bool fp64_only = false;  // GEMM of few contracted values: FP64 in every precision mode
   std::unique_ptr<GemmLaunch> launch;
   // split-K form (FP64): few output tiles over long contracted extents; the
   // K range of each output block is cut into slices whose partial sums go
@@ -206,7 +207,8 @@ struct ExecPlan {
 // must be contiguous, in plan order). alpha per pair is taken from
 // pair_alpha (2 doubles per pair) or 1.
 // backend: kBackendAuto lets the shape decide (GEMM for a flop-weighted
-// mean contracted extent >= 24, else FIBER or DIRECT); kBackendGemm takes
+// mean contracted extent >= 24, else the matrix form of FIBER, else by an
+// estimate GEMM in FP64, FIBER or DIRECT); kBackendGemm takes
 // the GEMM (TTGT on MFMA) whenever a mode is contracted; kBackendGeneric
 // takes the generic strided kernel (DIRECT: no permutation, no MFMA) for
 // every contraction.

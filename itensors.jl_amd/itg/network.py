@@ -280,9 +280,9 @@ class BatchedSequence:
     place instead of permuting it (the Z of the two-site network before its
     product with R). The result's index order is the fold's either way."""
 
-    # contracted extent below which the planner's automatic choice is not the
-    # grouped GEMM (the library's kBackendAuto rule, flop-weighted mean
-    # contracted extent >= 24)
+    # contracted extent (flop-weighted mean) from which the planner's automatic
+    # choice is the grouped GEMM; below it is the fiber kernel's matrix form
+    # where that applies, else whichever kernel the planner estimates fastest
     _GEMM_MIN_K = 24
 
     def __init__(self, networks, *, prec=None, reorder=True):
