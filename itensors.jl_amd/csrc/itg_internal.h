@@ -410,6 +410,13 @@ constexpr int kSplitKChunk = 8192;
 // One block of an operand to slice: rows x K read through mode strides.
 constexpr int kSliceRows = 64;    // rows per slicing workgroup
 constexpr int kSliceKPart = 128;  // K elements per slicing workgroup
+// One-pass slicing (real data, K <= 2048): a workgroup keeps all of K of its
+// rows in registers, 16 values for each of two chunks of the planes per thread.
+// kOnceRowsMin bounds K: a workgroup of fewer rows would write less than 64
+// bytes in a run.
+constexpr int kOnceThreads = 256;
+constexpr int kOnceChunks = 2 * kOnceThreads;  // chunks of a workgroup: its rows x Kpad / 16
+constexpr int kOnceRowsMin = 4;
 struct SliceBlock {
   int64_t off;        // element offset of the block in the FP64 operand
   int64_t plane_off;  // byte offset of slice plane 0 (R x Kpad bytes per plane,
@@ -420,7 +427,7 @@ struct SliceBlock {
   int32_t kparts;     // ceil(Kpad / kSliceKPart): workgroups along K
   int32_t nrm, nkm;   // number of row / K modes
   int32_t side;       // operand: 0 = A, 1 = B (one launch slices both)
-  int32_t pad;
+  int32_t once;       // rows of a one-pass workgroup (0: K is too long for it)
   int32_t rdim[kSliceModes], rstr[kSliceModes];
   int32_t kdim[kSliceModes], kstr[kSliceModes];
 };
@@ -436,6 +443,8 @@ struct SplitPair {
 int split_slices(int prec);  // slices per value for a precision mode (0: none)
 // Workgroups of one block: ceil(rows / kSliceRows) x kparts.
 int64_t slice_block_wgs(int32_t rows, int32_t kparts);
+// Rows of a one-pass workgroup for a block of `rows` rows (SliceBlock::once).
+int32_t slice_once_rows(int32_t rows, int32_t kpad);
 // The buffers of the two operands of a split GEMM; SliceBlock::side picks.
 struct SliceOperands {
   const double* src[2];  // FP64 operand (complex: interleaved)
@@ -443,15 +452,20 @@ struct SliceOperands {
   int32_t* exps[2];      // row exponents
   int32_t* pmax[2];      // partial row exponents
 };
-// Two launches over the same grid (the blocks of both operands, A's first):
-// partial row maxima (as exponents, into pmax), then the slices (planes) and
-// the row exponents (exps). Complex operands have two slice sets (re, im) under
-// one exponent per row; plane buffers hold split_sets() x the per-set bytes.
-// Workgroup w slices tile wgmap[w] = (block, tile index within the block:
-// row tile * kparts + K part).
+// The workgroups of a slicing launch; w takes tile map[w] = (block, tile index
+// within the block). once: one pass over blocks whose SliceBlock::once is set
+// (tile = row tile). two: two passes over the same grid, partial row maxima (as
+// exponents, into pmax), then the slices (tile = row tile * kparts + K part).
+struct SliceGrid {
+  const int2 *once, *two;
+  int64_t n_once, n_two;
+};
+// The slices (planes) and the row exponents (exps) of an operand, or of both.
+// Complex operands (two passes) have two slice sets (re, im) under one exponent
+// per row; plane buffers hold split_sets() x the per-set bytes.
 inline int split_sets(int cplx) { return cplx ? 2 : 1; }
 hipError_t launch_slice(hipStream_t s, int prec, int cplx, const SliceBlock* blocks,
-                        const int2* wgmap, int64_t grid, const SliceOperands& ops);
+                        const SliceGrid& grid, const SliceOperands& ops);
 // Split GEMM of real data.
 hipError_t launch_split_gemm(hipStream_t s, int prec, const SplitPair* pairs,
                              const GemmGroup* groups, const GemmTile* tiles, int64_t grid,

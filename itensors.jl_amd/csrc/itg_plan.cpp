@@ -1253,10 +1253,9 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
                                const std::vector<PairSpec>& pairs, bool swap, hipStream_t s) {
   ep->split_ok = false;
   auto side = [&](const BlockList& T, const std::vector<int>& rows, const std::vector<int>& ks,
-                  std::vector<SliceBlock>* out, std::vector<int64_t>* prefix, int64_t* plane_bytes,
-                  int64_t* nrows, int64_t* npmax) -> std::string {
+                  std::vector<SliceBlock>* out, int64_t* plane_bytes, int64_t* nrows,
+                  int64_t* npmax) -> std::string {
     out->resize(T.nblk());
-    prefix->assign(T.nblk() + 1, 0);
     int64_t pb = 0, er = 0, pm = 0;
     for (int64_t b = 0; b < T.nblk(); ++b) {
       SliceBlock& d = (*out)[b];
@@ -1272,13 +1271,13 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
       d.K = (int32_t)K;
       d.Kpad = (int32_t)((K + 31) / 32 * 32);
       d.kparts = (d.Kpad + kSliceKPart - 1) / kSliceKPart;
+      d.once = slice_once_rows(d.R, d.Kpad);
       d.plane_off = pb;
       d.exp_off = er;
       d.pmax_off = pm;
       pb += (int64_t)kSliceCount * R * d.Kpad;
       er += R;
       pm += (int64_t)d.kparts * R;
-      (*prefix)[b + 1] = (*prefix)[b] + slice_block_wgs(d.R, d.kparts);
     }
     *plane_bytes = pb;
     *nrows = er;
@@ -1286,11 +1285,9 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
     return "";
   };
   std::vector<SliceBlock> dA, dB;
-  std::vector<int64_t> pA, pB;
-  std::string err =
-      side(P, Mp, Xp, &dA, &pA, &ep->sA_plane_bytes, &ep->sA_rows, &ep->sA_pmax);
+  std::string err = side(P, Mp, Xp, &dA, &ep->sA_plane_bytes, &ep->sA_rows, &ep->sA_pmax);
   if (err.empty())
-    err = side(Q, Nq, Xq, &dB, &pB, &ep->sB_plane_bytes, &ep->sB_rows, &ep->sB_pmax);
+    err = side(Q, Nq, Xq, &dB, &ep->sB_plane_bytes, &ep->sB_rows, &ep->sB_pmax);
   if (!err.empty()) {
     ep->split_why = err;
     return "";  // the FP64 path still works
@@ -1336,36 +1333,33 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
   }
   // one slicing grid over both operands: A's blocks, then B's (side 1)
   std::vector<SliceBlock> dAB(dA);
-  std::vector<int64_t> pAB(pA);
-  for (size_t b = 0; b < dB.size(); ++b) {
-    SliceBlock d = dB[b];
+  for (SliceBlock d : dB) {
     d.side = 1;
     dAB.push_back(d);
-    pAB.push_back(pA.back() + pB[b + 1]);
   }
   // workgroup -> (block, tile within the block): one table read per
   // workgroup instead of a search over the blocks' workgroup prefix
-  auto wgmap = [](const std::vector<int64_t>& prefix) {
-    std::vector<int2> m((size_t)std::max<int64_t>(prefix.back(), 1), int2{0, 0});
-    for (size_t b = 0; b + 1 < prefix.size(); ++b)
-      for (int64_t w = prefix[b]; w < prefix[b + 1]; ++w)
-        m[(size_t)w] = int2{(int)b, (int)(w - prefix[b])};
-    return m;
-  };
-  const std::vector<int2> mAB = wgmap(pAB), mB = wgmap(pB);
+  std::vector<int2> map;
+  int64_t most = 0;
+  for (int list = 0; list < 3; ++list) {
+    for (size_t b = 0; b < dAB.size(); ++b) {
+      const SliceBlock& d = dAB[b];
+      int64_t n = 0;
+      if (list == 0 && d.once) n = (d.R + d.once - 1) / d.once;
+      if (list == 2 || (list == 1 && !d.once)) n = slice_block_wgs(d.R, d.kparts);
+      ep->s_tiles[list][d.side] += n;
+      if ((most = std::max(most, ep->s_tiles[list][0] + ep->s_tiles[list][1])) > INT32_MAX)
+        return "slicing grid too large";
+      for (int64_t w = 0; w < n; ++w) map.push_back(int2{(int)b, (int)w});
+    }
+  }
+  if (map.empty()) map.push_back(int2{0, 0});
   hipError_t e;
-  ep->sA_blocks = (int64_t)dA.size();
-  ep->sA_grid = pA.back();
-  ep->sB_grid = pB.back();
-  if (pAB.back() > INT32_MAX) return "slicing grid too large";
   if ((e = ep->s_desc.upload(dAB.data(), dAB.size() * sizeof(SliceBlock), s)) != hipSuccess ||
-      (e = ep->s_wgmap.upload(mAB.data(), mAB.size() * sizeof(int2), s)) != hipSuccess ||
-      (e = ep->s_wgmapB.upload(mB.data(), mB.size() * sizeof(int2), s)) != hipSuccess ||
+      (e = ep->s_wgmap.upload(map.data(), map.size() * sizeof(int2), s)) != hipSuccess ||
       (e = ep->s_pairs.upload(sp.data(), sp.size() * sizeof(SplitPair), s)) != hipSuccess ||
       (e = ep->s_groups.upload(sg.data(), sg.size() * sizeof(GemmGroup), s)) != hipSuccess)
     return std::string("device table upload failed: ") + hipGetErrorString(e);
-  ep->s_blocks = (int64_t)dAB.size();
-  ep->s_grid = pAB.back();
   ep->split_ok = true;
   return "";
 }
@@ -1838,15 +1832,18 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
     ops.exps[1] = (int32_t*)expB;
     ops.pmax[0] = (int32_t*)pmaxA;
     ops.pmax[1] = (int32_t*)pmaxB;
-    const SliceBlock* desc = (const SliceBlock*)ep.s_desc.p;
+    // list l of s_wgmap without the tiles of a reused operand
+    int64_t first[4] = {0}, n[3];
+    for (int l = 0; l < 3; ++l) {
+      first[l + 1] = first[l] + ep.s_tiles[l][0] + ep.s_tiles[l][1];
+      if (reuse[0]) first[l] += ep.s_tiles[l][0];
+      n[l] = (reuse[0] ? 0 : ep.s_tiles[l][0]) + (reuse[1] ? 0 : ep.s_tiles[l][1]);
+    }
+    const int2* map = (const int2*)ep.s_wgmap.p;
+    const int two = cplx ? 2 : 1;
+    const SliceGrid grid{map + first[0], map + first[two], cplx ? 0 : n[0], n[two]};
     TimeScope ts(kt, "slice_max_kernel+slice_kernel", s);
-    if (!reuse[0] && !reuse[1])
-      e = launch_slice(s, prec, cplx, desc, (const int2*)ep.s_wgmap.p, ep.s_grid, ops);
-    else if (!reuse[0])
-      e = launch_slice(s, prec, cplx, desc, (const int2*)ep.s_wgmap.p, ep.sA_grid, ops);
-    else
-      e = launch_slice(s, prec, cplx, desc + ep.sA_blocks, (const int2*)ep.s_wgmapB.p,
-                       ep.sB_grid, ops);
+    e = launch_slice(s, prec, cplx, (const SliceBlock*)ep.s_desc.p, grid, ops);
     if (e != hipSuccess) {
       *err = std::string("slice launch: ") + hipGetErrorString(e);
       return e;

@@ -184,17 +184,15 @@ struct ExecPlan {
   bool cplx_pair_alpha = false;  // some per-pair alpha has an imaginary part
   int64_t split_kmax = 0;        // largest contracted extent of a pair
   std::string split_why;         // reason when !split_ok
-  int64_t s_blocks = 0, s_grid = 0;  // slicing grid over both operands
   int64_t sA_plane_bytes = 0, sB_plane_bytes = 0, sA_rows = 0, sB_rows = 0;
   int64_t sA_pmax = 0, sB_pmax = 0;  // partial row exponents (ints)
   DevBuf s_desc, s_pairs, s_groups;  // s_groups: h_groups over the K-chunked pairs
-  // slicing grids: workgroup w of the launch over both operands slices tile
-  // s_wgmap[w] = (block index into s_desc, tile index within the block); A's
-  // blocks are s_desc[0, sA_blocks) and its tiles the first sA_grid entries;
-  // a launch over B alone uses s_desc + sA_blocks with s_wgmapB (sB_grid
-  // workgroups, block indices counted from B's first block)
-  int64_t sA_blocks = 0, sA_grid = 0, sB_grid = 0;
-  DevBuf s_wgmap, s_wgmapB;
+  // slicing grids: s_wgmap holds the tiles (block index into s_desc, tile index
+  // within the block) of three lists, each A's tiles, then B's: one pass, two
+  // passes over the blocks with a K too long for one, two passes over all blocks
+  // (complex data). s_tiles[list][side]: entries
+  int64_t s_tiles[3][2] = {};
+  DevBuf s_wgmap;
   // digit planes and row exponents kept for a fixed operand (side 0 = A,
   // 1 = B) by ITG_FLAG_KEEP_SLICES_*: the source pointer they were made from
   // and the number of slice sets (1 real, 2 complex); 0 = none kept

@@ -1,7 +1,8 @@
 // Split-precision grouped GEMM for gfx950: FP64 operands emulated with
 // integer slices on the INT8 matrix cores (Ozaki-style error-free splitting).
 //
-// 1. slice_kernel, once per operand: for every row r of every block (rows =
+// 1. slice_once_kernel (real data, K up to 2048) or slice_max_kernel and
+//    slice_kernel, once per operand: for every row r of every block (rows =
 //    the GEMM's M modes for A, N modes for B; the K modes are the columns),
 //    E_r = the smallest integer with max_k |x_rk| < 2^E_r, and
 //        x_rk = 2^E_r / 127 * sum_{i=0..S-1} v_i,rk * 254^(-i) + residue,
@@ -48,6 +49,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 256;
+constexpr int kXcds = 8;
 constexpr double kInvRadix = 1.0 / kSliceRadix;               // rounded: 2^-53 relative
 constexpr double kInvLead2 = 1.0 / (kSliceLead * kSliceLead);  // rounded: 2^-53 relative
 constexpr int kNonFinite = 0x7fff;   // row exponent of a row holding Inf / NaN
@@ -269,6 +271,33 @@ __global__ void __launch_bounds__(kThreads)
         max(max(ered[0][tid], ered[1][tid]), max(ered[2][tid], ered[3][tid]));
 }
 
+// The S digits of 16 values x of a row with exponent e (kNonFinite: all zero),
+// 16 bytes to each of the planes at dst, pstride apart.
+template <int S>
+__device__ __forceinline__ void slice_digits(const double (&x)[16], int e, int8_t* dst,
+                                             int64_t pstride) {
+  uint32_t packed[S][4];
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) packed[i][w] = 0u;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    // x / 2^E is exact (|.| < 1), the scale by 127 rounds once
+    double y = ldexp(e == kNonFinite ? 0.0 : x[j], -e) * kSliceLead;
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      const double v = rint(y);
+      y = (y - v) * kSliceRadix;
+      packed[i][j >> 2] |= ((uint32_t)((int32_t)v & 0xff)) << (8 * (j & 3));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    *reinterpret_cast<v4i*>(dst + i * pstride) =
+        v4i{(int)packed[i][0], (int)packed[i][1], (int)packed[i][2], (int)packed[i][3]};
+}
+
 // Pass 2: row exponent E = max of the row's partials (0 for an all-zero row),
 // then the S slices of every element of the tile.
 // Slice sets per element: 1 (real) or 2 (re, im: complex); set s of block b
@@ -315,7 +344,7 @@ __global__ void __launch_bounds__(kThreads)
   constexpr int NB = CPLX ? 1 : kItems;
   constexpr int NC = CPLX ? 2 : 1;  // re, im
   for (int i0 = 0; i0 < kItems; i0 += NB) {
-    double xr[NB][16], xi[NB][CPLX ? 16 : 1];
+    double xr[NB][16], xi[NB][16];  // xi: complex data
     int eq[NB], grq[NB], chq[NB];
     bool lq[NB];
 #pragma unroll
@@ -341,14 +370,13 @@ __global__ void __launch_bounds__(kThreads)
         off[j] = ro + (ch * 16 + j < d.K ? kw.off : 0);
         kw.step(d);
       }
-      const bool ok = e != kNonFinite;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const bool in = ok && ch * 16 + j < d.K;
+        const bool in = ch * 16 + j < d.K;
         if (CPLX) {
           const double2 v = reinterpret_cast<const double2*>(x)[off[j]];
           xr[q][j] = in ? v.x : 0.0;
-          xi[q][CPLX ? j : 0] = in ? v.y : 0.0;
+          xi[q][j] = in ? v.y : 0.0;
         } else {
           const double v = x[off[j]];
           xr[q][j] = in ? v : 0.0;
@@ -366,28 +394,105 @@ __global__ void __launch_bounds__(kThreads)
           planes + NC * d.plane_off + ((int64_t)chq[q] * d.R + grq[q]) * 16;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        uint32_t packed[S][4];
-#pragma unroll
-        for (int i = 0; i < S; ++i)
-#pragma unroll
-          for (int w = 0; w < 4; ++w) packed[i][w] = 0u;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          // x / 2^E is exact (|.| < 1), the scale by 127 rounds once
-          double y = ldexp(c == 0 ? xr[q][j] : xi[q][CPLX ? j : 0], -e) * kSliceLead;
-#pragma unroll
-          for (int i = 0; i < S; ++i) {
-            const double v = rint(y);
-            y = (y - v) * kSliceRadix;
-            packed[i][j >> 2] |= ((uint32_t)((int32_t)v & 0xff)) << (8 * (j & 3));
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < S; ++i)
-          *reinterpret_cast<v4i*>(dst + (c * S + i) * pstride) =
-              v4i{(int)packed[i][0], (int)packed[i][1], (int)packed[i][2], (int)packed[i][3]};
+        slice_digits<S>(c == 0 ? xr[q] : xi[q], e, dst + c * S * pstride, pstride);
       }
     }
+  }
+}
+
+// Two values at any multiple of 8 bytes.
+struct __attribute__((aligned(8))) Chunk {
+  double x, y;
+};
+
+// One pass, for blocks whose K fits a workgroup (d.once rows x Kpad / 16 chunks
+// <= kOnceChunks): a thread loads the values of its two chunks, the rows'
+// exponents are the maxima of their chunks' (LDS), and the slices are formed
+// from the values in registers. Bound by memory: 8 bytes read and 6 written per
+// value. Four workgroups a CU (114 registers) overlap one's loads with another's
+// digits: 256 threads and up to K = 2048 took 132 us for the operands of the U(1)
+// chi = 4096 apply's two products (two passes: 186), 512 threads 143, 1024
+// threads 174. 16384 x 512: 24 us rows first, 26 us K first (two passes: 40, 59);
+// 16384 x 2048: 146 and 112 (161 and 190); 30 x 2000: 7.7 (19). With few rows a
+// tile uses only part of each line, so neighbours run on one XCD, whose L2 holds
+// the line (16384 x 2048 rows first without that: 236 us), and chunks that are
+// contiguous in the operand are read 16 bytes at a time (143 us of the apply's
+// 155 with 512 threads). Complex data (two passes) would need twice the registers.
+template <int S>
+__global__ void __launch_bounds__(kOnceThreads, 4)
+    slice_once_kernel(const SliceBlock* __restrict__ blocks, const int2* __restrict__ map,
+                      SliceOperands ops) {
+  __shared__ int32_t sexp[kOnceThreads];
+  __shared__ int64_t srow[kOnceThreads];
+  constexpr int NI = kOnceChunks / kOnceThreads;
+  static_assert(kOnceChunks / 2 <= kOnceThreads, "Kpad >= 32: at most a row per thread");
+  // consecutive tiles to one XCD (workgroup w runs on XCD w % 8)
+  const int n = gridDim.x, xcd = blockIdx.x % kXcds, per = n / kXcds, rem = n % kXcds;
+  const int2 m = map[xcd * per + min(xcd, rem) + (int)blockIdx.x / kXcds];
+  const SliceBlock& d = blocks[m.x];
+  const int tid = threadIdx.x;
+  const int r0 = m.y * d.once, rows = min(d.once, d.R - r0), chunks = d.Kpad / 16;
+  const double* x = ops.src[d.side] + d.off;
+  int8_t* planes = ops.planes[d.side] + d.plane_off;
+  if (tid < rows) {
+    srow[tid] = mode_offset((uint32_t)(r0 + tid), d.nrm, d.rdim, d.rstr);
+    sexp[tid] = kZeroRow;
+  }
+  __syncthreads();
+  // Consecutive threads take consecutive rows of a chunk. Every load is
+  // unconditional, from a chunk clamped into the tile (one past it stores
+  // nothing) and a k clamped into the row (padding).
+  double v[NI][16];
+  int row[NI], ch[NI];
+  bool live[NI];
+#pragma unroll
+  for (int q = 0; q < NI; ++q) {
+    const int it0 = tid + q * kOnceThreads, it = min(it0, rows * chunks - 1);
+    live[q] = it0 == it;
+    ch[q] = it / rows;
+    row[q] = it - ch[q] * rows;
+    const int64_t ro = srow[row[q]];
+    const int k0 = ch[q] * 16;
+    if (d.nkm == 1 && d.kstr[0] == 1 && k0 + 16 <= d.K) {
+#pragma unroll
+      for (int j = 0; j < 16; j += 2) {
+        const Chunk c = *reinterpret_cast<const Chunk*>(x + ro + k0 + j);
+        v[q][j] = c.x;
+        v[q][j + 1] = c.y;
+      }
+    } else if (d.nkm == 1) {
+      const int64_t ks = d.kstr[0];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[q][j] = x[ro + (int64_t)min(k0 + j, d.K - 1) * ks];
+    } else {
+      KWalk kw;
+      kw.init((uint32_t)k0, d);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        v[q][j] = x[ro + (k0 + j < d.K ? kw.off : 0)];
+        kw.step(d);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NI; ++q) {
+    double mag = 0.0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      if (ch[q] * 16 + j >= d.K) v[q][j] = 0.0;
+      mag = fmax(mag, isfinite(v[q][j]) ? fabs(v[q][j]) : INFINITY);
+    }
+    if (live[q]) atomicMax(&sexp[row[q]], mag_exponent(mag));
+  }
+  __syncthreads();
+  const int64_t pstride = (int64_t)d.R * d.Kpad;
+#pragma unroll
+  for (int q = 0; q < NI; ++q) {
+    if (!live[q]) continue;
+    int e = sexp[row[q]];
+    if (e == kZeroRow) e = 0;
+    if (ch[q] == 0) ops.exps[d.side][d.exp_off + r0 + row[q]] = e;
+    slice_digits<S>(v[q], e, planes + ((int64_t)ch[q] * d.R + r0 + row[q]) * 16, pstride);
   }
 }
 
@@ -839,22 +944,35 @@ __global__ void __launch_bounds__(kThreads, 2)
 int split_slices(int prec) { return prec == 2 ? kSliceCount : 0; }
 
 hipError_t launch_slice(hipStream_t s, int prec, int cplx, const SliceBlock* blocks,
-                        const int2* wgmap, int64_t grid, const SliceOperands& ops) {
-  if (grid == 0) return hipSuccess;
+                        const SliceGrid& grid, const SliceOperands& ops) {
   if (prec != 2) return hipErrorNotSupported;
-  const dim3 g((unsigned)grid), blk(kThreads);
+  hipError_t e;
+  if (grid.n_once > 0) {
+    ITG_LAUNCH((slice_once_kernel<kSliceCount>), dim3((unsigned)grid.n_once), dim3(kOnceThreads),
+               0, s, blocks, grid.once, ops);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (grid.n_two == 0) return hipSuccess;
+  const dim3 g((unsigned)grid.n_two), blk(kThreads);
   if (cplx) {
-    ITG_LAUNCH((slice_max_kernel<1>), g, blk, 0, s, blocks, wgmap, ops);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    ITG_LAUNCH((slice_kernel<kSliceCount, 1>), g, blk, 0, s, blocks, wgmap, ops);
+    ITG_LAUNCH((slice_max_kernel<1>), g, blk, 0, s, blocks, grid.two, ops);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    ITG_LAUNCH((slice_kernel<kSliceCount, 1>), g, blk, 0, s, blocks, grid.two, ops);
   } else {
-    ITG_LAUNCH((slice_max_kernel<0>), g, blk, 0, s, blocks, wgmap, ops);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    ITG_LAUNCH((slice_kernel<kSliceCount, 0>), g, blk, 0, s, blocks, wgmap, ops);
+    ITG_LAUNCH((slice_max_kernel<0>), g, blk, 0, s, blocks, grid.two, ops);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    ITG_LAUNCH((slice_kernel<kSliceCount, 0>), g, blk, 0, s, blocks, grid.two, ops);
   }
   return hipGetLastError();
+}
+
+int32_t slice_once_rows(int32_t rows, int32_t kpad) {
+  if (rows <= 0 || kpad <= 0) return 0;
+  const int32_t cap = kOnceChunks / (kpad / 16) / kOnceRowsMin * kOnceRowsMin;
+  if (cap == 0) return 0;
+  // as few row tiles as hold the rows, of even size
+  const int32_t tiles = (rows + cap - 1) / cap, even = (rows + tiles - 1) / tiles;
+  return (even + kOnceRowsMin - 1) / kOnceRowsMin * kOnceRowsMin;
 }
 
 int64_t slice_block_wgs(int32_t rows, int32_t kparts) {
