@@ -103,7 +103,11 @@ typedef struct itg_bs_plan itg_bs_plan;
 itg_status itg_init(int device, itg_handle** out);
 itg_status itg_destroy(itg_handle* h);
 const char* itg_last_error(const itg_handle* h);
-/* Enqueue subsequent work on `stream` (a hipStream_t; NULL = null stream). */
+/* Enqueue subsequent work on `stream` (a hipStream_t; NULL = null stream). Work
+ * queued before stays on its stream. The caller orders its own data; the
+ * handle's workspaces the library orders itself: a call that uses them waits on
+ * its stream for the last such call on another (the first time this happens on
+ * a handle, for the device). */
 itg_status itg_set_stream(itg_handle* h, void* stream);
 itg_status itg_synchronize(itg_handle* h);
 /* Library version, "major.minor.patch". */
@@ -186,7 +190,14 @@ itg_status itg_timer_read(itg_handle* h, int64_t i, const char** name, int64_t* 
 typedef struct itg_graph itg_graph;
 itg_status itg_graph_begin(itg_handle* h);
 itg_status itg_graph_end(itg_handle* h, itg_graph** out);
-/* Launch the graph on the handle's stream (stream-ordered, returns at once). */
+/* Launch the graph on the handle's stream (stream-ordered, returns at once).
+ * Through the handle that recorded it, its use of the handle's workspaces is
+ * ordered with the handle's other calls, as itg_set_stream says. Replays that
+ * the library does not launch (the caller captured the stream by other means),
+ * or launches through another handle, are not: they must not overlap, on other
+ * streams, each other or the recording handle's eager calls, where both use a
+ * workspace. Recorded FP64 contractions without permuted, widened or split-K
+ * operands, and those of fewer than 24 values, never share one with eager calls. */
 itg_status itg_graph_launch(itg_handle* h, itg_graph* g);
 itg_status itg_graph_destroy(itg_graph* g);
 

@@ -51,7 +51,17 @@ struct itg_handle {
   size_t ws_bytes = 0;
   void* ws32 = nullptr;        // FP64 copies of Float32 / ComplexF32 operands
   size_t ws32_bytes = 0;
+  // workspace of the recorded runs of products that needed none until they were
+  // computed in parts or from permuted copies (see ready_ws): a replay of such a
+  // product does not touch what eager calls use
+  void* ws_cap = nullptr;
+  size_t ws_cap_bytes = 0;
   std::vector<void*> retired;  // earlier workspaces, freed by itg_destroy
+  // the workspaces' users in order across streams (WsUse)
+  hipStream_t ws_stream = nullptr;  // the last user's
+  bool ws_used = false, ws_multi = false;
+  hipEvent_t ws_done = nullptr;  // ws_multi: recorded behind the last user
+  bool cap_ws = false;           // a workspace's user has been recorded since itg_graph_begin
   bool timing = false;         // itg_timer_enable
   std::unique_ptr<KernelTimer> timer;
   std::vector<std::string> timer_names;  // snapshot behind itg_timer_read's `name`
@@ -70,6 +80,8 @@ struct itg_handle {
 struct itg_graph {
   int device = 0;
   hipGraphExec_t exec = nullptr;
+  const itg_handle* recorder = nullptr;
+  bool ws = false;  // uses a workspace of the recorder
 };
 
 struct itg_bs_plan {
@@ -147,6 +159,61 @@ hipError_t grow(itg_handle* h, void** buf, size_t* cur, size_t bytes) {
 }
 
 hipError_t ensure_ws(itg_handle* h, size_t bytes) { return grow(h, &h->ws, &h->ws_bytes, bytes); }
+
+bool captured(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
+// Calls that a capture forbids although they leave it alone (allocations, waits
+// for other streams), allowed to this thread for the scope.
+class RelaxedCapture {
+ public:
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
+// The scope of one use of the handle's workspaces. A handle may be given another
+// stream between two calls: work on the new one then waits for the last user
+// of the workspaces on the old. One event per use once that has happened; before
+// (nearly every handle keeps one stream) nothing is recorded, and the first
+// change waits for the device: the old stream may no longer exist. A recorded
+// run is ordered by the launch of its graph.
+class WsUse {
+ public:
+  hipError_t begin(itg_handle* h) {
+    if (captured(h->stream)) {
+      h->cap_ws = true;
+      return hipSuccess;
+    }
+    hipError_t e = hipSuccess;
+    if (h->ws_used && h->ws_stream != h->stream) {
+      if (h->ws_multi) {
+        e = hipStreamWaitEvent(h->stream, h->ws_done, 0);
+      } else {
+        RelaxedCapture r;
+        if (!h->ws_done) e = hipEventCreateWithFlags(&h->ws_done, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipDeviceSynchronize();
+        h->ws_multi = e == hipSuccess;
+      }
+    }
+    if (e == hipSuccess) h_ = h;
+    return e;
+  }
+  ~WsUse() {
+    if (!h_) return;
+    h_->ws_used = true;
+    h_->ws_stream = h_->stream;
+    if (h_->ws_multi && hipEventRecord(h_->ws_done, h_->stream) != hipSuccess)
+      (void)hipStreamSynchronize(h_->stream);
+  }
+
+ private:
+  itg_handle* h_ = nullptr;
+};
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -266,14 +333,6 @@ struct DeviceGuard {
   }
 };
 
-// A plan of few contracted values may run on the GEMM, with a small workspace,
-// or on kernels that need none: the workspace is made with the plan, so that a
-// first run under capture finds it. (A failure is the run's to report.)
-void reserve_plan_ws(itg_handle* h, const ExecPlan& ep) {
-  if (ep.fp64_only && ensure_ws(h, exec_workspace_bytes(ep, 1, 0)) != hipSuccess)
-    (void)hipGetLastError();
-}
-
 // The handle's timer while timing is on and the stream is not being captured.
 KernelTimer* active_timer(itg_handle* h) {
   if (!h->timing || !h->timer) return nullptr;
@@ -283,28 +342,33 @@ KernelTimer* active_timer(itg_handle* h) {
   return h->timer.get();
 }
 
-// The handle's workspace for a run that needs `need` bytes. *parts: whether it
+// The workspace for a run that needs `need` bytes, in *ws. *parts: whether it
 // also holds the partial buffer of the plan's part form. That form is only
-// faster: where the workspace cannot grow for it (out of memory, or a stream
-// under capture) the plan runs without.
-hipError_t ready_ws(itg_handle* h, ExecPlan& ep, int cplx, int prec, size_t need, bool* parts) {
+// faster: where the workspace cannot grow for it (out of memory) the plan runs
+// without. A recorded run of a part form or of a GEMM of few contracted values
+// has a workspace that only recorded runs use, made while recording if need be.
+hipError_t ready_ws(itg_handle* h, ExecPlan& ep, int cplx, int prec, size_t need, bool* parts,
+                    void** ws) {
   *parts = false;
   if (ep.strategy == ExecPlan::GEMM && (prec == ITG_PREC_FP64 || ep.fp64_only) &&
       ep.ks_grid == 0)
     (void)ensure_gemm_launch(ep, h->stream);  // a failure is exec_run's to report
   const size_t extra = exec_part_bytes(ep, cplx, prec);
-  if (extra) {
-    const size_t want = ((need + 255) & ~(size_t)255) + extra;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (h->ws_bytes >= want)
-      *parts = true;
-    else if (hipStreamIsCapturing(h->stream, &cs) == hipSuccess &&
-             cs == hipStreamCaptureStatusNone && ensure_ws(h, want) == hipSuccess)
-      *parts = true;
-    if (*parts) return hipSuccess;
+  hipError_t e = hipSuccess;
+  if ((extra || (ep.fp64_only && need)) && captured(h->stream)) {
+    RelaxedCapture r;
+    e = grow(h, &h->ws_cap, &h->ws_cap_bytes, extra ? al256(need) + extra : need);
+    *parts = extra && e == hipSuccess;
+    if (e == hipSuccess) *ws = h->ws_cap;
+    if (e == hipSuccess || !extra) return e;
     (void)hipGetLastError();
+  } else if (extra) {
+    *parts = ensure_ws(h, al256(need) + extra) == hipSuccess;
+    if (!*parts) (void)hipGetLastError();
   }
-  return ensure_ws(h, need);
+  if (!*parts) e = ensure_ws(h, need);
+  *ws = h->ws;
+  return e;
 }
 
 itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void* T1,
@@ -313,11 +377,15 @@ itg_status run_plan(itg_handle* h, ExecPlan& ep, int cplx, int prec, const void*
   const double a_re = alpha ? alpha[0] : 1.0, a_im = (alpha && cplx) ? alpha[1] : 0.0;
   const double b_re = beta ? beta[0] : 0.0, b_im = (beta && cplx) ? beta[1] : 0.0;
   std::string err;
+  const size_t need = exec_workspace_bytes(ep, cplx, prec, a_im != 0.0);
   bool parts = false;
-  hipError_t e = ready_ws(h, ep, cplx, prec, exec_workspace_bytes(ep, cplx, prec, a_im != 0.0),
-                          &parts);
+  void* ws = nullptr;
+  hipError_t e = ready_ws(h, ep, cplx, prec, need, &parts, &ws);
   if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
-  e = exec_run(ep, cplx, prec, h->stream, h->ws, T1, T2, R, flags, a_re, a_im, b_re, b_im,
+  WsUse use;
+  if ((need || parts) && (e = use.begin(h)) != hipSuccess)
+    return hip_fail(h, e, "workspace order");
+  e = exec_run(ep, cplx, prec, h->stream, ws, T1, T2, R, flags, a_re, a_im, b_re, b_im,
                &err, active_timer(h), true, parts, f32);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
@@ -333,14 +401,17 @@ itg_status run_plan32(itg_handle* h, ExecPlan& ep, itg_dtype dt, int64_t n1, con
                       const double* alpha, const double* beta) {
   const int cplx = dt == ITG_C64;
   const unsigned f32 = exec_reads_f32(ep);
+  WsUse use;
+  hipError_t e = use.begin(h);
+  if (e != hipSuccess) return hip_fail(h, e, "workspace order");
   Wide w;
   itg_status st = widen_operands(h, dt, f32 & 1u ? 0 : n1, T1, f32 & 2u ? 0 : n2, T2, nR, &w);
   if (st != ITG_OK) return st;
   st = run_plan(h, ep, cplx, ITG_PREC_FP64, f32 & 1u ? T1 : w.t1, f32 & 2u ? T2 : w.t2, w.r, flags,
                 alpha, nullptr, f32);
   if (st != ITG_OK) return st;
-  hipError_t e = launch_narrow(h->stream, cplx, nR, w.r, R, beta ? beta[0] : 0.0,
-                               (beta && cplx) ? beta[1] : 0.0);
+  e = launch_narrow(h->stream, cplx, nR, w.r, R, beta ? beta[0] : 0.0,
+                    (beta && cplx) ? beta[1] : 0.0);
   if (e != hipSuccess) return hip_fail(h, e, "narrow launch");
   return ITG_OK;
 }
@@ -408,7 +479,6 @@ itg_status plan_for_factors(itg_handle* h, itg_bs_plan* p, const double* pair_al
         build_exec_plan(p->st, p->b1, p->b2, p->bR, p->pairs, pa.data(), h->stream, np.get(),
                         p->backend);
     if (!err.empty()) return fail(h, ITG_ERR_HIP, err);
-    reserve_plan_ws(h, *np);
     it = p->ep_alpha.emplace(pa, std::move(np)).first;
   }
   *out = it->second.get();
@@ -504,8 +574,10 @@ itg_status itg_destroy(itg_handle* h) {
       h->stream = h->pre_capture;
     }
     for (Stage& st : h->stages) free_stage(&st);
-    if (h->ws || !h->retired.empty()) (void)hipStreamSynchronize(h->stream);
+    if (h->ws || h->ws_cap || !h->retired.empty()) (void)hipStreamSynchronize(h->stream);
     if (h->ws) (void)hipFree(h->ws);
+    if (h->ws_cap) (void)hipFree(h->ws_cap);
+    if (h->ws_done) (void)hipEventDestroy(h->ws_done);
     if (h->ws32) (void)hipFree(h->ws32);
     for (void* p : h->retired) (void)hipFree(p);
     h->dense_map.clear();
@@ -545,6 +617,7 @@ itg_status itg_graph_begin(itg_handle* h) {
     return hip_fail(h, e, "hipStreamBeginCapture");
   }
   h->capturing = true;
+  h->cap_ws = false;
   return ITG_OK;
 }
 
@@ -564,6 +637,8 @@ itg_status itg_graph_end(itg_handle* h, itg_graph** out) {
   }
   std::unique_ptr<itg_graph> ig(new itg_graph);
   ig->device = h->device;
+  ig->recorder = h;
+  ig->ws = h->cap_ws;
   e = hipGraphInstantiate(&ig->exec, gr, nullptr, nullptr, 0);
   (void)hipGraphDestroy(gr);
   if (e != hipSuccess) return hip_fail(h, e, "hipGraphInstantiate");
@@ -576,7 +651,10 @@ itg_status itg_graph_launch(itg_handle* h, itg_graph* gph) {
   if (gph->device != h->device) return fail(h, ITG_ERR_INVALID, "graph built on another device");
   if (h->capturing) return fail(h, ITG_ERR_INVALID, "cannot launch a graph while capturing");
   DeviceGuard g(h->device);
-  hipError_t e = hipGraphLaunch(gph->exec, h->stream);
+  WsUse use;
+  hipError_t e = gph->ws && gph->recorder == h ? use.begin(h) : hipSuccess;
+  if (e != hipSuccess) return hip_fail(h, e, "workspace order");
+  e = hipGraphLaunch(gph->exec, h->stream);
   if (e != hipSuccess) return hip_fail(h, e, "hipGraphLaunch");
   return ITG_OK;
 }
@@ -1054,7 +1132,6 @@ itg_status itg_bs_plan_create(itg_handle* h, int N1, int64_t nblk1, const int64_
     std::string err = build_exec_plan(p->st, p->b1, p->b2, p->bR, p->pairs, nullptr, h->stream,
                                       p->ep.get(), p->backend);
     if (!err.empty()) return fail(h, ITG_ERR_HIP, err);
-    reserve_plan_ws(h, *p->ep);
   }
   *out = p.release();
   return ITG_OK;
@@ -1492,11 +1569,16 @@ itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void*
   DeviceGuard g(h->device);
   ExecPlan& ep = *p->ep;
   if (prec != ITG_PREC_FP64 && !ep.split_ok) return ITG_OK;
+  const size_t need = exec_workspace_bytes(ep, cplx, (int)prec);
   bool parts = false;
-  hipError_t e = ready_ws(h, ep, cplx, (int)prec, exec_workspace_bytes(ep, cplx, (int)prec), &parts);
+  void* ws = nullptr;
+  hipError_t e = ready_ws(h, ep, cplx, (int)prec, need, &parts, &ws);
   if (e != hipSuccess) return hip_fail(h, e, "workspace allocation");
+  WsUse use;
+  if ((need || parts) && (e = use.begin(h)) != hipSuccess)
+    return hip_fail(h, e, "workspace order");
   std::string err;
-  e = exec_run(ep, cplx, (int)prec, h->stream, h->ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err,
+  e = exec_run(ep, cplx, (int)prec, h->stream, ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err,
                nullptr, true, parts);
   if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
   if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
@@ -1587,7 +1669,6 @@ itg_status itg_batch_plan_create(itg_handle* h, itg_dtype dtype, int64_t nbatch,
   p->ep.reset(new ExecPlan);
   m = build_exec_plan(st, L1, L2, LR, pairs, nullptr, h->stream, p->ep.get(), h->backend);
   if (!m.empty()) return fail(h, ITG_ERR_HIP, m);
-  reserve_plan_ws(h, *p->ep);
   *out = p.release();
   return ITG_OK;
 }
