@@ -1610,21 +1610,25 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, TileForm* form, PartTab
   first[ep.h_groups.size()] = all.size();
   struct Chunk {
     size_t t0, t1;
-    double k;     // contracted values of one of its tiles
+    double k;     // contracted values of one of its tiles, an empty pair counted as one
+    double live;  // the same, an empty pair counted as none: what can be cut
     double work;  // of all of them
     double most;  // of the largest one
   };
   std::vector<Chunk> chunks;
   const size_t unit = std::max<size_t>(1, (total + 8 * kXcds - 1) / (8 * kXcds));
   for (size_t g = 0; g < ep.h_groups.size(); ++g) {
-    double k = 0;
-    for (int p = ep.h_groups[g].p0; p < ep.h_groups[g].p1; ++p) k += std::max(ep.h_pairs[p].K, 1);
+    double k = 0, live = 0;
+    for (int p = ep.h_groups[g].p0; p < ep.h_groups[g].p1; ++p) {
+      k += std::max(ep.h_pairs[p].K, 1);
+      live += std::max(ep.h_pairs[p].K, 0);
+    }
     for (size_t t0 = first[g]; t0 < first[g + 1]; t0 += unit) {
       const size_t t1 = std::min(first[g + 1], t0 + unit);
       int64_t blocks = 0;
       int most = 0;
       for (size_t t = t0; t < t1; ++t) blocks += all[t].pad, most = std::max(most, all[t].pad);
-      chunks.push_back(Chunk{t0, t1, k, (double)blocks * k, most * k});
+      chunks.push_back(Chunk{t0, t1, k, live, (double)blocks * k, most * k});
     }
   }
   std::stable_sort(chunks.begin(), chunks.end(),
@@ -1659,13 +1663,13 @@ std::vector<GemmTile> xcd_tile_table(const ExecPlan& ep, TileForm* form, PartTab
   if (!form) return table;
   form[0] = form[1] = TileForm::kWhole;
   if (!few) return table;
-  // of each tile: its 16 x 16 blocks times k, and k
+  // of each tile: its 16 x 16 blocks times k, and the values that can be cut
   std::vector<std::vector<double>> cost(kXcds), depth(kXcds);
   for (int x = 0; x < kXcds; ++x)
     for (const Chunk& c : mine[x])
       for (size_t t = c.t0; t < c.t1; ++t) {
         cost[x].push_back(all[t].pad * c.k);
-        depth[x].push_back(c.k);
+        depth[x].push_back(c.live);
       }
   std::vector<std::vector<int>> cut;
   choose_form(cost, depth, form, &cut);
