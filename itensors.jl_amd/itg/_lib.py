@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 
 import numpy as np
@@ -160,13 +161,21 @@ def ptr64(a):
     return a.ctypes.data_as(I64P), a
 
 
-_I64_ARRAYS = [ctypes.c_int64 * max(n, 1) for n in range(16)]
+# by length: a C array made of the bytes of its values
+_I64_ARRAY = [(ctypes.c_int64 * max(n, 1)).from_buffer_copy for n in range(16)]
+_I64_BYTES = [lambda: bytes(8)] + [struct.Struct(f"={n}q").pack for n in range(1, 16)]
 
 
 def ints(seq):
     """A C array of a short sequence (labels, dims), passed where an Int*
-    argument is expected: a tenth of the cost of going through numpy."""
-    return _I64_ARRAYS[len(seq)](*seq) if len(seq) < 16 else (ctypes.c_int64 * len(seq))(*seq)
+    argument is expected: 0.6 us, a tenth of the cost of going through numpy,
+    which still takes (or refuses) what is not a short sequence of Int64 values."""
+    try:
+        n = len(seq)
+        return _I64_ARRAY[n](_I64_BYTES[n](*seq))
+    except (IndexError, TypeError, struct.error):
+        a = i64(seq)
+        return (ctypes.c_int64 * max(a.size, 1)).from_buffer_copy(a if a.size else bytes(8))
 
 
 def ptr32(a):
