@@ -823,7 +823,6 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
   const int NR = st.NR, nk = st.nk;
   // per-pair shape figures
   double mnk = 0.0, mn = 0.0, flops = 0.0;
-  int64_t maxdim = 0;
   std::vector<double> pk(pairs.size()), pm(pairs.size()), pn(pairs.size());
   for (size_t p = 0; p < pairs.size(); ++p) {
     const int32_t* d1 = b1.d(pairs[p].blk1);
@@ -842,10 +841,8 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
     mnk += M * N * K;
     mn += M * N;
     flops += 2.0 * M * N * K;
-    maxdim = std::max<int64_t>(maxdim, (int64_t)std::max(M, N));
   }
   ep->flops = flops;
-  ep->max_dim = maxdim;
   const double kavg = mn > 0 ? mnk / mn : 0.0;
   const bool use_gemm = backend == kBackendGeneric ? false
                        : backend == kBackendGemm  ? nk > 0
@@ -1155,7 +1152,6 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
   // GEMM pairs and groups
   ep->h_pairs.resize(pairs.size());
   ep->h_groups.resize(granges.size());
-  ep->group_cost.resize(granges.size());
   for (size_t p = 0; p < pairs.size(); ++p) {
     const int64_t bp = swap ? pairs[p].blk2 : pairs[p].blk1;
     const int64_t bq = swap ? pairs[p].blk1 : pairs[p].blk2;
@@ -1190,11 +1186,7 @@ std::string build_exec_plan(const Structure& st, const BlockList& b1, const Bloc
     g.ldc = (int32_t)std::max<int64_t>(M, 1);
     g.p0 = (int32_t)granges[gi].first;
     g.p1 = (int32_t)granges[gi].second;
-    double cost = 0;
     set_first_pair(&g, ep->h_pairs.data());
-    for (size_t q = granges[gi].first; q < granges[gi].second; ++q)
-      cost += 2.0 * (double)M * (double)N * (double)ep->h_pairs[q].K;
-    ep->group_cost[gi] = cost;
   }
   if ((e = ep->g_pairs.upload(ep->h_pairs.data(), ep->h_pairs.size() * sizeof(GemmPair), s)) !=
           hipSuccess ||

@@ -160,7 +160,6 @@ struct ExecPlan {
   DevBuf g_pairs, g_groups;
   std::vector<GemmPair> h_pairs;
   std::vector<GemmGroup> h_groups;
-  std::vector<double> group_cost;  // flops per group (for LPT ordering)
   bool fp64_only = false;  // GEMM of few contracted values: FP64 in every precision mode
   std::unique_ptr<GemmLaunch> launch;
   // split-K form (FP64): few output tiles over long contracted extents; the
@@ -177,7 +176,6 @@ struct ExecPlan {
   int64_t ks_ngroups = 0;   // (block, slice) entries of the split tables
   DevBuf ks_pairs, ks_groups, ks_tiles, ks_red;
   double flops = 0.0;                                   // real flops (2*M*N*K summed)
-  int64_t max_dim = 0;
   // split precision (real data): slice tables of the A-side operand P and
   // the B-side operand Q, read in place (no permutation), and the pair table
   bool split_ok = false;
