@@ -1330,21 +1330,29 @@ std::string build_split_tables(ExecPlan* ep, const BlockList& P, const BlockList
     dAB.push_back(d);
   }
   // workgroup -> (block, tile within the block): one table read per
-  // workgroup instead of a search over the blocks' workgroup prefix
-  std::vector<int2> map;
-  int64_t most = 0;
-  for (int list = 0; list < 3; ++list) {
-    for (size_t b = 0; b < dAB.size(); ++b) {
-      const SliceBlock& d = dAB[b];
-      int64_t n = 0;
-      if (list == 0 && d.once) n = (d.R + d.once - 1) / d.once;
-      if (list == 2 || (list == 1 && !d.once)) n = slice_block_wgs(d.R, d.kparts);
-      ep->s_tiles[list][d.side] += n;
-      if ((most = std::max(most, ep->s_tiles[list][0] + ep->s_tiles[list][1])) > INT32_MAX)
-        return "slicing grid too large";
-      for (int64_t w = 0; w < n; ++w) map.push_back(int2{(int)b, (int)w});
-    }
+  // workgroup instead of a search over the blocks' workgroup prefix. A block
+  // with a one-pass form has tiles of both forms.
+  for (const SliceBlock& d : dAB) {
+    const int64_t two = slice_block_wgs(d.R, d.kparts);
+    if (d.once) ep->s_once[d.side] += (d.R + d.once - 1) / d.once;
+    (d.once ? ep->s_two_once : ep->s_two_long)[d.side] += two;
   }
+  const int64_t n_once = ep->s_once[0] + ep->s_once[1];
+  const int64_t n_two = ep->s_two_once[0] + ep->s_two_once[1] + ep->s_two_long[0] +
+                        ep->s_two_long[1];
+  if (std::max(n_once, n_two) > INT32_MAX) return "slicing grid too large";
+  std::vector<int2> map((size_t)(n_once + n_two));
+  size_t at = 0;
+  auto tiles = [&](size_t b, int64_t n) {
+    for (int64_t w = 0; w < n; ++w) map[at++] = int2{(int)b, (int)w};
+  };
+  for (size_t b = 0; b < dAB.size(); ++b)
+    if (dAB[b].once) tiles(b, (dAB[b].R + dAB[b].once - 1) / dAB[b].once);
+  // A's one-pass blocks, A's others, B's others, B's one-pass blocks
+  for (int part = 0; part < 4; ++part)
+    for (size_t b = 0; b < dAB.size(); ++b)
+      if (dAB[b].side == part / 2 && (dAB[b].once != 0) == (part == 0 || part == 3))
+        tiles(b, slice_block_wgs(dAB[b].R, dAB[b].kparts));
   if (map.empty()) map.push_back(int2{0, 0});
   hipError_t e;
   if ((e = ep->s_desc.upload(dAB.data(), dAB.size() * sizeof(SliceBlock), s)) != hipSuccess ||
@@ -1828,16 +1836,25 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
     ops.exps[1] = (int32_t*)expB;
     ops.pmax[0] = (int32_t*)pmaxA;
     ops.pmax[1] = (int32_t*)pmaxB;
-    // list l of s_wgmap without the tiles of a reused operand
-    int64_t first[4] = {0}, n[3];
-    for (int l = 0; l < 3; ++l) {
-      first[l + 1] = first[l] + ep.s_tiles[l][0] + ep.s_tiles[l][1];
-      if (reuse[0]) first[l] += ep.s_tiles[l][0];
-      n[l] = (reuse[0] ? 0 : ep.s_tiles[l][0]) + (reuse[1] ? 0 : ep.s_tiles[l][1]);
-    }
+    // the tiles of the operands that are not reused
+    const int64_t* once = ep.s_once;
+    const int64_t* two = ep.s_two_long;
+    const int64_t both[2] = {ep.s_two_once[0] + two[0], ep.s_two_once[1] + two[1]};
+    auto count = [&](const int64_t (&n)[2]) {
+      return (reuse[0] ? 0 : n[0]) + (reuse[1] ? 0 : n[1]);
+    };
     const int2* map = (const int2*)ep.s_wgmap.p;
-    const int two = cplx ? 2 : 1;
-    const SliceGrid grid{map + first[0], map + first[two], cplx ? 0 : n[0], n[two]};
+    const int2* map2 = map + once[0] + once[1];
+    SliceGrid grid;
+    grid.once = map + (reuse[0] ? once[0] : 0);
+    grid.n_once = cplx ? 0 : count(ep.s_once);
+    if (cplx) {
+      grid.two = map2 + (reuse[0] ? both[0] : 0);
+      grid.n_two = count(both);
+    } else {
+      grid.two = map2 + ep.s_two_once[0] + (reuse[0] ? two[0] : 0);
+      grid.n_two = count(ep.s_two_long);
+    }
     TimeScope ts(kt, "slice_max_kernel+slice_kernel", s);
     e = launch_slice(s, prec, cplx, (const SliceBlock*)ep.s_desc.p, grid, ops);
     if (e != hipSuccess) {

@@ -185,11 +185,12 @@ struct ExecPlan {
   int64_t sA_plane_bytes = 0, sB_plane_bytes = 0, sA_rows = 0, sB_rows = 0;
   int64_t sA_pmax = 0, sB_pmax = 0;  // partial row exponents (ints)
   DevBuf s_desc, s_pairs, s_groups;  // s_groups: h_groups over the K-chunked pairs
-  // slicing grids: s_wgmap holds the tiles (block index into s_desc, tile index
-  // within the block) of three lists, each A's tiles, then B's: one pass, two
-  // passes over the blocks with a K too long for one, two passes over all blocks
-  // (complex data). s_tiles[list][side]: entries
-  int64_t s_tiles[3][2] = {};
+  // slicing grids: s_wgmap holds tiles (block index into s_desc, tile index within
+  // the block): those of the one-pass form, A's blocks before B's, then those of the
+  // two-pass form over A's one-pass blocks, A's others, B's others and B's one-pass
+  // blocks, so that the tiles of the others alone (real data) and of all blocks
+  // (complex data), of one operand or of both, are runs of it. Entries by operand:
+  int64_t s_once[2] = {}, s_two_once[2] = {}, s_two_long[2] = {};
   DevBuf s_wgmap;
   // digit planes and row exponents kept for a fixed operand (side 0 = A,
   // 1 = B) by ITG_FLAG_KEEP_SLICES_*: the source pointer they were made from
