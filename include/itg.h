@@ -480,9 +480,12 @@ itg_status itg_batch_plan_destroy(itg_batch_plan* p);
 
 /* ------------------------------------------------------------- autotuner */
 
-/* Prepare the plan for (dtype, prec): runs it once, R = T1*T2, so that its
- * launch tables and the workspace exist, and waits. The GEMM kernels have one
- * tile shape each, so there is nothing to choose. Synchronises the stream. */
+/* Time the tile shapes of the FP64 GEMM (64 x 64 and their 32 x 32 quarters) on
+ * this plan's pairs and keep the faster one for this plan and element type, in
+ * place of the planner's estimate. The shapes agree bit for bit. The split GEMM
+ * has one shape, and a plan whose tiles are computed in parts along K keeps that
+ * form: for these, as for all, R = T1*T2 is computed and the launch tables and
+ * the workspace exist afterwards. Synchronises the stream. */
 itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype,
                            void* R, const void* T1, const void* T2, itg_prec prec);
 

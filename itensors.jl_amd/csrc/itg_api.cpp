@@ -1578,10 +1578,39 @@ itg_status itg_bs_autotune(itg_handle* h, itg_bs_plan* p, itg_dtype dtype, void*
   if ((need || parts) && (e = use.begin(h)) != hipSuccess)
     return hip_fail(h, e, "workspace order");
   std::string err;
-  e = exec_run(ep, cplx, (int)prec, h->stream, ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err,
-               nullptr, true, parts);
-  if (e == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
-  if (e != hipSuccess) return fail(h, ITG_ERR_HIP, err);
+  auto run = [&]() {
+    return exec_run(ep, cplx, (int)prec, h->stream, ws, T1, T2, R, 0u, 1.0, 0.0, 0.0, 0.0, &err,
+                    active_timer(h), true, parts);
+  };
+  auto failed = [&](hipError_t x) {
+    if (x == hipErrorNotSupported) return fail(h, ITG_ERR_UNSUPPORTED, err);
+    return err.empty() ? hip_fail(h, x, "autotune") : fail(h, ITG_ERR_HIP, err);
+  };
+  if ((e = run()) != hipSuccess) return failed(e);
+  // Each output value is summed in the same order in 64 x 64 tiles and in their
+  // 32 x 32 quarters: these two shapes are timed. A plan that is computed in parts
+  // stays so (its sums have another order), and the split GEMM has one shape.
+  if ((prec == ITG_PREC_FP64 || ep.fp64_only) && ep.launch &&
+      ep.launch->form[cplx] != TileForm::kParts) {
+    const TileForm was = ep.launch->form[cplx];
+    constexpr int kRuns = 3;
+    hipEvent_t t[2] = {nullptr, nullptr};
+    float ms[2] = {0.0f, 0.0f};
+    const TileForm forms[2] = {TileForm::kWhole, TileForm::kQuarters};
+    for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreate(&t[i]);
+    for (int f = 0; f < 2 && e == hipSuccess; ++f) {
+      ep.launch->form[cplx] = forms[f];
+      if ((e = run()) != hipSuccess || (e = hipEventRecord(t[0], h->stream)) != hipSuccess) break;
+      for (int r = 0; r < kRuns && e == hipSuccess; ++r) e = run();
+      if (e == hipSuccess) e = hipEventRecord(t[1], h->stream);
+      if (e == hipSuccess) e = hipEventSynchronize(t[1]);
+      if (e == hipSuccess) e = hipEventElapsedTime(&ms[f], t[0], t[1]);
+    }
+    ep.launch->form[cplx] = e != hipSuccess ? was : forms[ms[1] < ms[0] ? 1 : 0];
+    for (hipEvent_t x : t)
+      if (x) (void)hipEventDestroy(x);
+    if (e != hipSuccess) return failed(e);
+  }
   if ((e = hipStreamSynchronize(h->stream)) != hipSuccess)
     return hip_fail(h, e, "hipStreamSynchronize");
   return ITG_OK;
