@@ -230,7 +230,11 @@ itg_status itg_convert(itg_handle* h, itg_dtype from, const void* src, itg_dtype
  * Replaces NDTensors.permutedims!(::Exposed{<:Array}, ...) with @strided
  * (NDTensors/src/array/permutedims.jl:5-24) and the alpha/beta variants used
  * by the scalar contraction paths
- * (NDTensors/src/abstractarray/tensoralgebra/contract.jl:88-113). */
+ * (NDTensors/src/abstractarray/tensoralgebra/contract.jl:88-113).
+ * Stream-ordered: returns with the permutation queued on the handle's stream;
+ * src and dst stay valid until it has run, and the host or another stream waits
+ * (itg_synchronize) before it reads dst or changes src. dims and perm may change
+ * on return. Not under stream capture (it uploads its tables): ITG_ERR_HIP. */
 itg_status itg_permute(itg_handle* h, itg_dtype dtype, int ndim,
                        const int64_t* dims, const int32_t* perm,
                        const void* src, void* dst,
@@ -403,7 +407,8 @@ itg_status itg_bs_chain_destroy(itg_bs_chain* c);
  * passes in offsR) = permutedims(src block b, perm). dims of each block are
  * N x nblk (block b at dims[b*N..]). Replaces permutedims!(R::BlockSparseTensor,
  * T::BlockSparseTensor, perm) (NDTensors/src/blocksparse/blocksparsetensor.jl:834-881)
- * for the common case of matching block lists. */
+ * for the common case of matching block lists. Stream-ordered and not for use
+ * under stream capture, as itg_permute. */
 itg_status itg_bs_permute(itg_handle* h, itg_dtype dtype, int N, int64_t nblk,
                           const int64_t* blockdims, const int64_t* offs_src,
                           const int64_t* offs_dst, const int32_t* perm,
