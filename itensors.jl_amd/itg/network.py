@@ -83,10 +83,16 @@ class ContractionSequence:
             elif reorder and C is not None and step[0] == "dense" and \
                     ND.gemm_backend() == "Auto" and \
                     _contracted_extent(a_it, step[5][0]) < BatchedSequence._GEMM_MIN_K:
-                # dense steps have no plan to ask: a step with a short
-                # contracted extent runs on the strided or fiber kernels
-                # (any output order costs the same), so its output takes the
-                # order a GEMM-shaped next step reads in place
+                # dense steps have no plan to ask. A step with a short
+                # contracted extent usually runs on the fiber or strided
+                # kernels, where any output order costs the same, so its
+                # output takes the order a GEMM-shaped next step reads in
+                # place: the w = 5, d = 2 networks save a permutation. Where
+                # the matrix form does not apply (w d > 16) the planner may
+                # take the GEMM for it; the order then moves that permutation
+                # to this step, or leaves it on the fiber kernel (w d = 20 at
+                # chi = 24: 55 us against 52 in fold order; 200: 266 against
+                # 118; 400: 571 against 643).
                 order = self._order_for_next(cur.inds, C.inds)
                 if order != tuple(cur.inds):
                     step, cur = self._build_step(a_it, B, out_inds=order)
@@ -274,8 +280,8 @@ class BatchedSequence:
     share one allocation.
 
     reorder: an intermediate made by a step with a short contracted extent
-    (the strided or fiber kernels, which write any mode order at the same
-    cost) holds the indices the next step contracts last, in the order the
+    (usually the fiber or strided kernels, which write any mode order at the
+    same cost) holds the indices the next step contracts last, in the order the
     next operand holds them, so that a GEMM-shaped next step reads it in
     place instead of permuting it (the Z of the two-site network before its
     product with R). The result's index order is the fold's either way."""
