@@ -55,9 +55,11 @@ __device__ inline double axpby(double a_re, double, double x, double b_re, doubl
 }
 __device__ inline double2 axpby(double a_re, double a_im, double2 x, double b_re, double b_im,
                                 double2 y, bool use_beta) {
-  double2 r;
-  r.x = a_re * x.x - a_im * x.y;
-  r.y = a_re * x.y + a_im * x.x;
+  double2 r = x;  // alpha = 1 copies: 1 * (inf + 0i), multiplied out, is (inf, nan)
+  if (a_re != 1.0 || a_im != 0.0) {
+    r.x = a_re * x.x - a_im * x.y;
+    r.y = a_re * x.y + a_im * x.x;
+  }
   if (use_beta) {
     r.x += b_re * y.x - b_im * y.y;
     r.y += b_re * y.y + b_im * y.x;
