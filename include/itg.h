@@ -166,7 +166,8 @@ itg_status itg_set_blocksparse_order(itg_handle* h, int order);
  * clears the totals and starts; (h, 0) stops. itg_timer_read synchronizes
  * the stream and reports entry i (0 <= i < itg_timer_count) as a kernel
  * name, its launch count and its summed duration in milliseconds; `name`
- * stays valid until the next timer call on the handle. */
+ * stays valid until the next timer call on the handle. Slicing is one entry per
+ * contraction, "slice_max_kernel+slice_kernel", in one pass or in two. */
 itg_status itg_timer_enable(itg_handle* h, int enable);
 int64_t itg_timer_count(itg_handle* h);
 itg_status itg_timer_read(itg_handle* h, int64_t i, const char** name, int64_t* calls,

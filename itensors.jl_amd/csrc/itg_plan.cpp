@@ -1877,6 +1877,7 @@ hipError_t exec_split(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
       grid.two = map2 + ep.s_two_once[0] + (reuse[0] ? two[0] : 0);
       grid.n_two = count(ep.s_two_long);
     }
+    // the section's name, whichever of the slicing kernels run
     TimeScope ts(kt, "slice_max_kernel+slice_kernel", s);
     e = launch_slice(s, prec, cplx, (const SliceBlock*)ep.s_desc.p, grid, ops);
     if (e != hipSuccess) {

@@ -246,17 +246,11 @@ hipError_t exec_run(ExecPlan& ep, int cplx, int prec, hipStream_t s, void* ws,
 // ComplexF32 data (its f32) in FP64 precision: those that it permutes first.
 unsigned exec_reads_f32(const ExecPlan& ep);
 // Builds the plan's tile table once (kGemmTile square tiles for every plan).
-// FP64, timed on MI355X against the other shapes (128x128, 128x64, 64x128
-// real; 128x64 complex): the fastest or within 3 % of it for the two-site
-// network's GEMMs at chi = 1024 (one 5120 x 4096 x 1024 block), the chi = 4096
-// U(1) blocks (about 410 on a side: 0.63 ms for the two GEMMs, 128x128 0.86,
-// 128x64 0.74), the 256-network batch and a 4096^3 product (2.04-2.11 ms,
-// 128x128 1.99-2.07): the padding and the last wave of large tiles cost more
-// than the panels they save.
-// Split, against 128x64 (eight waves) and 64x64 with the A operand in
-// registers (two waves): U(1) chi = 4096 0.345 against 0.49 and 0.47 ms for the
-// two GEMMs, 4096^3 1.08 against 1.24 and 1.16, 1000^3 22 against 41 and 37 us,
-// 1100 x 8000 x 1100 0.22 against 0.28 and 0.235.
+// Larger tiles (FP64: 128x128, 128x64, 64x128; split: 128x64, and 64x64 with A in
+// registers) were timed on MI355X while these kernels had them: in FP64 17 to 37 %
+// slower on the chi = 4096 U(1) blocks (about 410 on a side), level within 4 % on
+// 4096^3; in split precision 36 to 42 % slower on the U(1) blocks, 7 to 15 % on
+// 4096^3. Their padding and last wave cost more than the panels they save.
 hipError_t ensure_gemm_launch(ExecPlan& ep, hipStream_t s, bool may_build = true);
 // Bytes of the partial buffer that exec_run needs beyond exec_workspace_bytes()
 // to run the plan in its part form: 0 if it has none or it is not built yet.
