@@ -165,10 +165,16 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() > 0 else ctypes.c_void_p(0)
 
 
-def _handle(dev):
+def _handle_on(dev):
+    """The handle of a device, set to the current stream, and that stream."""
     h = _lib.handle_for(dev.index if dev.index is not None else torch.cuda.current_device())
-    h.set_stream(torch.cuda.current_stream(dev).cuda_stream)
-    return h
+    s = torch.cuda.current_stream(dev)
+    h.set_stream(s.cuda_stream)
+    return h, s
+
+
+def _handle(dev):
+    return _handle_on(dev)[0]
 
 
 def set_split_tile(tile: int, device=None) -> None:
@@ -919,13 +925,16 @@ def permutedims_(R, T, perm, alpha=1.0, beta=0.0):
     block-sparse tensors the union-of-blocks form of permutedims!."""
     if isinstance(T, BlockSparseTensor):
         return _bs_permutedims_(R, T, perm, alpha, beta)
-    h = _handle(T.data.device)
+    h, stream = _handle_on(T.data.device)
     d, _k = _lib.ptr64(_lib.i64(T.dims))
     pp, _kp = _lib.ptr32([int(x) for x in perm])
     a, _ka = _lib.scalar2(alpha)
     b, _kb = _lib.scalar2(beta)
     h.check(_lib.lib().itg_permute(h.h, _dtype_code(T.eltype), T.ndims, d, pp, _ptr(T.data),
                                    _ptr(R.data), a, b))
+    # queued: memory of another stream is not handed out again before it has run
+    T.data.record_stream(stream)
+    R.data.record_stream(stream)
     return R
 
 
@@ -938,7 +947,7 @@ def permutedims(T, perm):
         dims = tuple(T.dims[p - 1] for p in perm)
         R = DenseTensor(torch.empty_like(T.data), dims)
         return permutedims_(R, T, perm)
-    h = _handle(T.data.device)
+    h, stream = _handle_on(T.data.device)
     N = T.ndims
     if len(perm) != N:
         raise ValueError("permutation length does not match the tensor")
@@ -962,6 +971,7 @@ def permutedims(T, perm):
         _lib.ptr64(np.ascontiguousarray(a)) for a in (bd.reshape(-1), offs, dst))
     h.check(_lib.lib().itg_bs_permute(h.h, _dtype_code(T.eltype), N, nb, pbd, poffs, pdst, p32,
                                       _ptr(T.data), _ptr(out)))
+    T.data.record_stream(stream)  # as in permutedims_
     if N > 1:
         moved = map(operator.itemgetter(*(p - 1 for p in perm)), blocks)
     else:
